@@ -14,6 +14,8 @@ import os
 import shutil
 import subprocess
 import sys
+import tempfile
+from concurrent.futures import ThreadPoolExecutor
 from pathlib import Path
 
 PKG = Path(__file__).resolve().parent
@@ -53,11 +55,18 @@ def _run(cmd: list[str]) -> None:
 
 def build_library() -> Path:
     LIB_DIR.mkdir(exist_ok=True)
-    sources = [str(CSRC / "swmi_kernels.hip"), str(CSRC / "swmi_engine.hip"), str(CSRC / "swmi_noalloc.hip"),
-               str(CSRC / "swmi_server.cpp")]
-    tmp = LIB.with_suffix(".so.tmp")
-    _run([HIPCC, *HIP_FLAGS, "-shared", "-I", str(ROOT / "include"), "-o", str(tmp), *sources])
-    os.replace(tmp, LIB)
+    parts = [(src, []) for src in ("swmi_kernels.hip", "swmi_engine.hip", "swmi_noalloc.hip", "swmi_server.cpp")]
+    parts += [("swmi_bond.hip", [f"-DSWMI_BOND_TW64={tw64}", f"-DSWMI_BOND_DBG={dbg}"])
+              for tw64 in ("true", "false") for dbg in ("true", "false")]
+    with tempfile.TemporaryDirectory() as tmp, ThreadPoolExecutor(min(8, os.cpu_count() or 1)) as pool:
+        objects = [str(Path(tmp) / f"{i}.o") for i in range(len(parts))]
+        compiles = [pool.submit(_run, [HIPCC, *HIP_FLAGS, *defs, "-I", str(ROOT / "include"), "-c", str(CSRC / src), "-o", obj])
+                    for (src, defs), obj in zip(parts, objects)]
+        for c in compiles:
+            c.result()
+        out = LIB.with_suffix(".so.tmp")
+        _run([HIPCC, f"--offload-arch={ARCH}", "-shared", "-o", str(out), *objects])
+    os.replace(out, LIB)
     return LIB
 
 

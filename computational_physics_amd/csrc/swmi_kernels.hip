@@ -20,1135 +20,10 @@
 // per-group data except on the sweeps that rotate (one in 7.5).
 // Reference behaviour: ising/src/swendsen_wang_amd_gpu.cpp:78-467 (four kernels per sweep) and the CPU
 // labeller ising/src/swendsen_wang_cpu.cpp:13-205; the kernels here are written for wave64 CDNA4.
-#include <hip/hip_runtime.h>
-
-#include <algorithm>
-#include <type_traits>
-
-#include "swmi_internal.h"
+#include "swmi_device.h"
 
 namespace swmi
 {
-    __device__ __forceinline__ uint32_t Uniform(const uint32_t v) { return __builtin_amdgcn_readfirstlane(v); }
-
-    // The buffers are reached through pointers stored in the lattice descriptor, which the compiler sees
-    // as generic (FLAT) addresses; FLAT accesses wait on both the memory and the LDS counters. Every
-    // buffer access goes through a global-address-space view instead.
-    template <typename T>
-    using gptr = __attribute__((address_space(1))) T*;
-
-    template <typename T>
-    __device__ __forceinline__ gptr<T> Glob(T* p)
-    {
-        return (gptr<T>)(p);
-    }
-
-    // plain vector types (HIP's uint2/uint4 classes cannot be assigned through address-space-1 pointers)
-    using u32x2 = uint32_t __attribute__((ext_vector_type(2)));
-    using u32x4 = uint32_t __attribute__((ext_vector_type(4)));
-
-    // Buffer views (raw: stride 0, byte offsets). The hardware checks a lane's offset against the view's
-    // size and drops a store past it, which lets a lane opt out of a store without an exec mask.
-    using Rsrc = __amdgpu_buffer_rsrc_t;
-    constexpr uint32_t kNoStore = 0x80000000u;   // a lane offset past every view
-    template <typename T>
-    __device__ __forceinline__ Rsrc MakeRsrc(T* base, const uint32_t bytes)
-    {
-        return __builtin_amdgcn_make_buffer_rsrc(static_cast<void*>(base), 0, static_cast<int>(bytes), 0x00020000);
-    }
-
-    // bit `lane` of a wave-uniform mask, as a per-lane predicate (v_cndmask on the SGPR pair)
-    __device__ __forceinline__ bool LaneBit(const uint64_t mask) { return __builtin_amdgcn_inverse_ballot_w64(mask); }
-
-    // 64-bit shifts by 0..64 (a shift by 64 yields 0; the hardware would use the count modulo 64)
-    __device__ __forceinline__ uint64_t Shr(const uint64_t v, const uint32_t s) { return s >= 64u ? 0ull : v >> s; }
-    __device__ __forceinline__ uint64_t Shl(const uint64_t v, const uint32_t s) { return s >= 64u ? 0ull : v << s; }
-
-    __device__ __forceinline__ uint32_t ReadLane(const uint32_t v, const uint32_t lane)
-    {
-        return static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(v), static_cast<int>(lane)));
-    }
-
-    // Numerical Recipes pair k of random/src/lcg32.cpp:18-24.
-    __device__ __forceinline__ void ParamsOf(const uint32_t k, uint32_t& a, uint32_t& c)
-    {
-        const bool b0 = (k & 1u) != 0u, b1 = (k & 2u) != 0u, b2 = (k & 4u) != 0u;
-        const uint32_t a01 = b0 ? 2891336453u : 1372383749u;
-        const uint32_t a23 = b0 ? 32310901u : 2024337845u;
-        const uint32_t c01 = b0 ? 1640531513u : 1289706101u;
-        const uint32_t c23 = b0 ? 626627237u : 797082193u;
-        a = b2 ? 29943829u : (b1 ? a23 : a01);
-        c = b2 ? 1013904223u : (b1 ? c23 : c01);
-    }
-
-    // Offset added to the rotation at update `it` (random/src/lcg32.cpp:56-64): state[it & 63] + (it even).
-    __device__ __forceinline__ uint32_t ShuffleShift(const uint32_t st, const uint32_t it)
-    {
-        return ReadLane(st, it & 63u) + ((it & 1u) ? 0u : 1u);
-    }
-
-    // ---- random flip rule: MurmurHash3 (Austin Appleby, public domain). The cluster with canonical root r
-    // flips iff the top bit of Fmix32(r ^ key) is set; key = MurmurHash3_x86_32 of the 4-byte lcg32
-    // iteration count before the sweep, seeded with the lattice seed. ----
-    __device__ __forceinline__ uint32_t Fmix32(uint32_t h)
-    {
-        h ^= h >> 16;
-        h *= 0x85EBCA6Bu;
-        h ^= h >> 13;
-        h *= 0xC2B2AE35u;
-        h ^= h >> 16;
-        return h;
-    }
-
-    __device__ __forceinline__ uint32_t FlipKey(const uint32_t seed, const uint32_t iteration)
-    {
-        uint32_t k = iteration * 0xCC9E2D51u;
-        k = (k << 15) | (k >> 17);
-        k *= 0x1B873593u;
-        uint32_t h = seed ^ k;
-        h = (h << 13) | (h >> 19);
-        h = h * 5u + 0xE6546B64u;
-        return Fmix32(h ^ 4u);
-    }
-
-    // ---- union-find in LDS. Nodes are named by their byte offset into the workgroup's parent array P
-    // (so no instruction scales an index into an address); parents satisfy P[x] <= x, so roots are cluster
-    // minima. ----
-    __device__ __forceinline__ uint32_t* At(uint32_t* P, const uint32_t off)
-    {
-        return reinterpret_cast<uint32_t*>(reinterpret_cast<char*>(P) + off);
-    }
-
-    __device__ __forceinline__ uint32_t LdsLoad(const uint32_t* p)
-    {
-        return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-    }
-
-    // An empty asm statement that reads v: v's load completes before this point, so it cannot be sunk past a
-    // later branch (an early exit) and is waited for together with the loads issued beside it.
-    __device__ __forceinline__ void Issued(const uint32_t v)
-    {
-        asm volatile("" ::"v"(v));
-    }
-
-    __device__ __forceinline__ void Issued(const uint64_t v)
-    {
-        asm volatile("" ::"v"(v));
-    }
-
-    // An empty asm statement that needs the uniform value v in scalar registers here: a descriptor field read
-    // this way is fetched at this point, with the others read beside it, not at its first use.
-    template <typename T>
-    __device__ __forceinline__ void HeldScalar(const T v)
-    {
-        asm volatile("" ::"s"(v));
-    }
-
-    __device__ __forceinline__ void LdsMin(uint32_t* p, const uint32_t v)
-    {
-        (void)__hip_atomic_fetch_min(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-    }
-
-    // ---- union-find in HBM over the roots of edge-reaching clusters, one node per slot (every block numbers
-    // its edge roots densely, so a block's nodes share a few cache lines). Entry of slot c: (key << 32) | parent
-    // slot, where a root's key is its site index and a non-root holds its parent's key. Links are made with
-    // agent-scope 64-bit atomicMin (the 8 XCD L2s are not coherent with each other for plain stores), which
-    // orders by key first: a parent's key never exceeds its child's, so a tree's root is the minimum site of
-    // its component. Chase loads are relaxed atomic loads (never hoisted by the compiler); a stale value is an
-    // earlier parent, still an ancestor, and every link is decided by an atomicMin that returns the true value,
-    // so staleness only costs retries and longer paths. ----
-    __device__ __forceinline__ uint64_t SlotEntry(const uint32_t key, const uint32_t slot)
-    {
-        return (static_cast<uint64_t>(key) << 32) | slot;
-    }
-
-    __device__ __forceinline__ uint64_t CachedLoad64(gptr<uint64_t> p)
-    {
-        return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-    }
-
-    // Loads of the merge's chases. FRESH reads the entry as it is now, past the CU's cache (agent scope);
-    // otherwise the load may hit a line the CU cached earlier in the kernel. Fresh loads cost memory traffic
-    // and save retries: they pay where the merge is latency-bound, i.e. where all its blocks are resident at
-    // once (LaunchMerge chooses).
-    template <bool FRESH>
-    __device__ __forceinline__ uint64_t ChaseLoad64(gptr<uint64_t> p)
-    {
-        return __hip_atomic_load(p, __ATOMIC_RELAXED, FRESH ? __HIP_MEMORY_SCOPE_AGENT : __HIP_MEMORY_SCOPE_WORKGROUP);
-    }
-
-    __device__ __forceinline__ uint64_t SlotLinkMin(gptr<uint64_t> p, const uint64_t v)
-    {
-        return __hip_atomic_fetch_min(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-
-    // Union of the clusters of slots a and b (keys ka, kb), the loop of the reference Merge
-    // (swendsen_wang_amd_gpu.cpp:368-401) on slot entries. The ends start as the listed roots k_bond_label
-    // wrote (entry = (own key << 32) | self), so the first link is tried at once, without chasing: when a
-    // concurrent union got there first, atomicMin returns the parent found and the loop continues from it.
-    // Both ends are chased together (their loads in flight at once); a start node more than one hop from its
-    // root is pointed at the root (the atomic returns nothing, so the wave does not wait for it). A slot out
-    // of range or a parent with a larger key can only come from a broken invariant, which is reported through
-    // the lattice's error flag instead of being followed.
-    template <bool FRESH>
-    __device__ void SlotUnion(gptr<uint64_t> E, uint32_t a, uint32_t ka, uint32_t b, uint32_t kb, const uint32_t nslots,
-                              gptr<uint32_t> err)
-    {
-        if (a < nslots && b < nslots && ka != kb)
-        {
-            if (ka > kb)
-            {
-                const uint32_t t = a, tk = ka;
-                a = b;
-                ka = kb;
-                b = t;
-                kb = tk;
-            }
-            const uint64_t old = SlotLinkMin(&E[b], SlotEntry(ka, a));
-            if (old == SlotEntry(kb, b) || static_cast<uint32_t>(old) == a)
-                return;
-            b = static_cast<uint32_t>(old);
-            kb = static_cast<uint32_t>(old >> 32);
-        }
-        for (;;)
-        {
-            if (a >= nslots || b >= nslots)
-                break;
-            const uint32_t a0 = a, b0 = b;
-            uint64_t ea = ChaseLoad64<FRESH>(&E[a]), eb = ChaseLoad64<FRESH>(&E[b]);
-            uint32_t ha = 0, hb = 0;
-            bool bad = false;
-            while (static_cast<uint32_t>(ea) != a || static_cast<uint32_t>(eb) != b)
-            {
-                const uint32_t pa = static_cast<uint32_t>(ea), qa = static_cast<uint32_t>(ea >> 32);
-                const uint32_t pb = static_cast<uint32_t>(eb), qb = static_cast<uint32_t>(eb >> 32);
-                if (pa >= nslots || qa > ka || pb >= nslots || qb > kb)
-                {
-                    bad = true;
-                    break;
-                }
-                if (pa != a)
-                {
-                    a = pa;
-                    ka = qa;
-                    ea = ChaseLoad64<FRESH>(&E[a]);
-                    ++ha;
-                }
-                if (pb != b)
-                {
-                    b = pb;
-                    kb = qb;
-                    eb = ChaseLoad64<FRESH>(&E[b]);
-                    ++hb;
-                }
-            }
-            if (bad)
-                break;
-            if (ha > 1)
-                (void)SlotLinkMin(&E[a0], SlotEntry(ka, a));
-            if (hb > 1)
-                (void)SlotLinkMin(&E[b0], SlotEntry(kb, b));
-            if (a == b)
-                return;
-            if (ka > kb)
-            {
-                const uint32_t t = a, tk = ka;
-                a = b;
-                ka = kb;
-                b = t;
-                kb = tk;
-            }
-            const uint64_t old = SlotLinkMin(&E[b], SlotEntry(ka, a));
-            if (old == SlotEntry(kb, b))
-                return;
-            b = static_cast<uint32_t>(old);
-            kb = static_cast<uint32_t>(old >> 32);
-        }
-        (void)__hip_atomic_fetch_or(err, kErrLabelRange, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-
-    // Key of the canonical root (the minimum site) of the cluster of slot c, whose entry e the caller loaded;
-    // c_max bounds the slots. A chase that leaves the slots or meets a parent with a larger key clears ok.
-    __device__ __forceinline__ uint32_t SlotRootKey(gptr<uint64_t> E, uint32_t c, uint64_t e, const uint32_t c_max, bool& ok)
-    {
-        uint32_t k = static_cast<uint32_t>(e >> 32);
-        while (static_cast<uint32_t>(e) != c)
-        {
-            const uint32_t p = static_cast<uint32_t>(e), kp = static_cast<uint32_t>(e >> 32);
-            if (p >= c_max || kp > k)
-            {
-                ok = false;
-                break;
-            }
-            c = p;
-            k = kp;
-            e = CachedLoad64(&E[c]);
-        }
-        return static_cast<uint32_t>(e >> 32);
-    }
-
-    // ---- work decomposition ----
-    // Workgroups are dispatched round-robin over the 8 XCDs; give each XCD a contiguous range of blocks
-    // so that blocks that share cache lines (spin rows, halos) meet in the same L2.
-    __device__ __forceinline__ uint32_t RemapBlock(const uint32_t units)
-    {
-        const uint32_t per = (units + kNumXcd - 1) / kNumXcd;
-        return (blockIdx.x % kNumXcd) * per + blockIdx.x / kNumXcd;
-    }
-
-    // Lattice of block b in the work list; a work list of one lattice is passed as a null pointer, which
-    // saves the dependent load of the block's entry before the descriptor.
-    __device__ __forceinline__ uint32_t LatticeOf(const uint32_t* __restrict__ block_lat, const uint32_t b)
-    {
-        return block_lat ? block_lat[b] : 0u;
-    }
-
-    struct Block
-    {
-        uint32_t lb;       // block index within its lattice
-        uint32_t sx, sy;   // block column, block row
-        uint32_t wyb;      // first wave row of the block
-        uint32_t nwr;      // wave rows in the block
-        uint32_t stride;   // sites between consecutive wave rows (64 * tiles_x)
-        uint32_t base;     // first site of the block
-    };
-
-    __device__ __forceinline__ Block DecodeBlock(const LatDesc& d, const uint32_t b)
-    {
-        Block bl;
-        bl.lb = b - d.block_base;
-        bl.sx = bl.lb % d.tiles_x;
-        bl.sy = bl.lb / d.tiles_x;
-        bl.wyb = bl.sy * kWavesPerBlock * d.twr;
-        bl.nwr = min(kWavesPerBlock * d.twr, d.nwr_y - bl.wyb);
-        bl.stride = 64u * d.tiles_x;
-        bl.base = bl.wyb * bl.stride + bl.sx * 64u;
-        return bl;
-    }
-
-    __device__ __forceinline__ uint32_t BlockBase(const LatDesc& d, const uint32_t sx, const uint32_t sy)
-    {
-        return sy * kWavesPerBlock * d.twr * 64u * d.tiles_x + sx * 64u;
-    }
-
-    __device__ __forceinline__ uint32_t SiteOf(const uint32_t base, const uint32_t stride, const uint32_t q)
-    {
-        return base + (q >> 6) * stride + (q & 63u);
-    }
-
-    // ---- the flip rule (reference FlipClusters_Kernel, swendsen_wang_amd_gpu.cpp:445-467) ----
-    // Row-major site index of a padded site index p (d.n0 is the row pitch, d.n0v the lattice width).
-    __device__ __forceinline__ uint32_t RealSite(const LatDesc& d, const uint32_t p)
-    {
-        return d.n0v == d.n0 ? p : (p / d.n0) * d.n0v + p % d.n0;
-    }
-
-    // The flip rule for the cluster whose canonical root is the padded site `root`. The pitch and the width
-    // are even, so a padded index and its row-major index have the same parity.
-    __device__ __forceinline__ uint32_t FlipBit(const LatDesc& d, const uint32_t root, const bool random_rule, const uint32_t key)
-    {
-        return random_rule ? (Fmix32(RealSite(d, root) ^ key) >> 31) : (root & 1u);
-    }
-
-    // A block's flip bitmap has one bit per label index: bit q (q < qcap) for the cluster rooted at block-local
-    // index q that stays inside the block, the rule applied to the root's own site; bit qcap + s for the
-    // edge-reaching cluster whose root holds slot s, the rule applied to its canonical root (set by the
-    // resolve). Word w of the rule part: bit j for q = 32w + j (block bases and row strides are even, so under
-    // the parity rule q's parity is its site's parity).
-    __device__ __forceinline__ uint32_t RuleWord(const LatDesc& d, const Block& bl, const uint32_t w, const bool random_rule,
-                                                 const uint32_t key)
-    {
-        if (!random_rule)
-            return 0xAAAAAAAAu;
-        uint32_t v = 0;
-        for (uint32_t j = 0; j < 32u; ++j)
-            v |= FlipBit(d, SiteOf(bl.base, bl.stride, 32u * w + j), true, key) << j;
-        return v;
-    }
-
-    // =============================================================================================
-    // k_bond_label
-    // =============================================================================================
-    // Down bonds are deduplicated before any union: lanes l-1 and l lie in the same "overlap interval"
-    // when they share their row run above and their row run below (mask C); only the first down bond
-    // of every interval can join two different clusters. With M = C << 1 (continuation) and
-    // S1 = (D << 1) & M, the positions that follow an earlier bond of the same interval are
-    // S1 | (M & ((M + S1) ^ M)) (carries of S1 run through the ones of M).
-    __device__ __forceinline__ uint64_t FirstBondPerInterval(const uint64_t D, const uint64_t C, const uint64_t rowstart)
-    {
-        const uint64_t M = (C << 1) & ~rowstart;
-        const uint64_t S1 = (D << 1) & M;
-        const uint64_t later = S1 | (M & ((M + S1) ^ M));
-        return D & ~later;
-    }
-
-    // Union of the pairs (a, b) held by the lanes, all lanes in lockstep. Each step moves the ends that
-    // are not roots up (two parents, halving the path); when both are roots the larger is linked under the
-    // smaller with atomicMin, and a lost race continues with the value found (the loop of the reference
-    // Merge, swendsen_wang_amd_gpu.cpp:368-401). Lanes with nothing to do hold a == b; only lanes that
-    // link issue the atomic (idle lanes would all hit the same word). a and b are byte offsets into P.
-    __device__ __forceinline__ void LdsUnionLockstep(uint32_t* P, uint32_t a, uint32_t b)
-    {
-        while (__ballot(a != b))
-        {
-            // lanes that are done (a == b) only read P[a]; they follow no pointer and write nothing, so
-            // their a may name a node another wave has not written yet
-            const bool act = a != b;
-            const uint32_t pa = LdsLoad(At(P, a));
-            const uint32_t pb = LdsLoad(At(P, b));
-            const bool roots = (pa == a) && (pb == b);
-            const bool up = act && !roots;
-            const uint32_t lo = min(a, b), hi = max(a, b);
-            uint32_t old = hi;
-            if (act && roots)
-                old = __hip_atomic_fetch_min(At(P, hi), lo, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-            const bool linked = roots && old == hi;
-            // ends that are not roots move two steps up and point their node at the grandparent (path
-            // halving, monotone like every write to P)
-            const uint32_t ga = up ? LdsLoad(At(P, pa)) : 0u;
-            const uint32_t gb = up ? LdsLoad(At(P, pb)) : 0u;
-            if (up && ga != pa)
-                LdsMin(At(P, a), ga);
-            if (up && gb != pb)
-                LdsMin(At(P, b), gb);
-            if (act)
-            {
-                a = roots ? (linked ? hi : lo) : ga;
-                b = roots ? (linked ? hi : old) : gb;
-            }
-        }
-    }
-
-    // Per wavefront (tile) the rows are processed top to bottom with the loads of the next kCh rows in
-    // flight together. Bonds are computed on wave-uniform 64-bit masks: S (spin up), U1/U2 (draw below
-    // threshold), B (bond to the right neighbour inside the tile), D (bond to the site below).
-    // 64-wide tiles keep the previous row's roots resolved in registers (Rp). A row run's label is the
-    // minimum of its first site and the roots its down bonds reach (one LDS atomicMin per bonded lane into
-    // the run's slot); a bond to any other root links that root under the minimum with one atomicMin, and
-    // only a link that loses a race goes through the lockstep union.
-    // Narrow tiles record one union per overlap interval of consecutive rows in a per-wave LDS queue,
-    // worked off 64 at a time whenever it fills.
-    // Nodes of the LDS union-find are byte offsets into P. After the final find, the root of every
-    // cluster that reaches the block edge carries kPFlag in its own entry, so a site's label (root index,
-    // plus kEdgeFlag) is P[root] >> 2.
-    // DBG: the inspection modes (injected bonds instead of generated ones, bond recording) are compiled in;
-    // the sweep kernel proper has neither branch.
-    // PAD: the lattice is stored with a row pitch d.n0 above its width d.n0v; in the last tile column only
-    // the lanes up to d.elast hold sites (mask d.vlast), the rest are padding: they bond to nothing, their
-    // draws are unused, and the row's last site bonds across the lattice edge instead of lane tw - 1.
-    template <uint32_t TWR_MAX, bool TW64, bool DBG, bool PAD>
-    __device__ __forceinline__ void BondLabel(const LatDesc* __restrict__ descs, const uint32_t* __restrict__ block_lat,
-                                              const uint32_t total_blocks)
-    {
-        // All loads of a chunk of rows are issued before its first store: on this hardware the memory
-        // counter that a load waits on also counts the stores issued before it.
-        constexpr uint32_t kCh = TWR_MAX < 16 ? TWR_MAX : 16;
-        constexpr uint32_t kRows = TWR_MAX < 16 ? TWR_MAX : 16;   // rows resolved together at the end
-        constexpr uint32_t kSites = kWavesPerBlock * TWR_MAX * 64;
-        constexpr uint32_t kQw = 128u;                             // per-wave LDS words of Q
-        constexpr uint32_t kPFlag = 1u << 17;
-        static_assert(kSites * 4u <= (1u << 16), "byte offsets must fit the 16-bit halves of a queue entry");
-        static_assert((kPFlag >> 2) == kEdgeFlag, "a flagged root entry shifts into a flagged label");
-        __shared__ uint32_t P[kSites];
-        // per wave: 64-wide tiles keep the run minima of the current row in words 0-63 and give each lane a
-        // word of its own in 64-127 (the target of LDS operations a lane has no use for, so that they need
-        // no exec mask); narrow tiles keep their union queue here
-        __shared__ uint32_t Q[kWavesPerBlock * kQw];
-        __shared__ uint32_t FB[2u * kSites / 32u];   // flip bits of a pending flip, by label index (root or qcap + slot)
-        __shared__ uint64_t s_first_B[kWavesPerBlock];
-        __shared__ uint64_t AC[8];              // Numerical Recipes pairs (c << 32 | a) by selector
-        __shared__ uint32_t s_nslot;            // slots given to the block's edge-reaching clusters
-
-        const uint32_t b = RemapBlock(total_blocks);
-        if (b >= total_blocks)
-            return;
-        if (threadIdx.x < 8u)
-        {
-            uint32_t a, c;
-            ParamsOf(threadIdx.x, a, c);
-            AC[threadIdx.x] = (static_cast<uint64_t>(c) << 32) | a;
-        }
-        if (threadIdx.x == 0)
-            s_nslot = 0u;
-        const LatDesc& d = descs[LatticeOf(block_lat, b)];
-        const Block bl = DecodeBlock(d, b);
-        const uint32_t lane = threadIdx.x & 63u;
-        const uint32_t lane4 = lane * 4u;
-        const uint32_t w = Uniform(threadIdx.x >> 6);
-
-        const uint32_t n0 = d.n0, n1 = d.n1, twr = d.twr;
-        const uint32_t tw = TW64 ? 64u : d.tw, rpw = TW64 ? 1u : d.rpw;
-        const uint32_t lx = lane & (tw - 1u);
-        const uint32_t lrow = TW64 ? 0u : lane / tw;
-        const uint32_t x = bl.sx * tw + lx;
-        const bool lastcol = PAD && bl.sx + 1u == d.tiles_x;
-        const uint64_t vmask = lastcol ? d.vlast : ~0ull;   // lanes that hold sites
-        const uint32_t elane = lastcol ? d.elast : tw - 1u;  // lx of a lattice row's last site in this tile
-        const bool rbound = lx == elane;
-        const bool injected = DBG && d.bond_in != nullptr;
-        const uint32_t thr = d.threshold;
-        const gptr<uint32_t> stp = Glob(d.state);
-        const gptr<uint8_t> dump = DBG ? Glob(d.bond_dump) : nullptr;
-        const gptr<uint8_t> spins = Glob(d.spins);
-        const gptr<uint32_t> rotp = Glob(d.rot);
-        const gptr<const uint8_t> bond_in = Glob(d.bond_in);
-
-        const uint32_t r_begin = w * twr;
-        const uint32_t nrow = bl.nwr > r_begin ? min(twr, bl.nwr - r_begin) : 0u;
-        // buffer views of this block's part of the per-site arrays (row offsets in scalar registers, the lane
-        // offset in a vector register, no per-row vector addresses)
-        const uint32_t span = (bl.nwr - 1u) * bl.stride + 64u;   // sites from the block's first to its last
-        const Rsrc rs_spins = MakeRsrc(d.spins + bl.base, span);
-        const Rsrc rs_rng = MakeRsrc(d.rng + bl.base, span * 4u);
-        const Rsrc rs_local = MakeRsrc(d.local + bl.base, span * 2u);
-        const gptr<const uint32_t> fbits_g = Glob(static_cast<const uint32_t*>(d.fbits)) + bl.lb * d.fsw;
-        const uint32_t nwaves = (bl.nwr + twr - 1u) / twr;
-        const bool last_wave = w + 1u == nwaves;
-        const uint32_t sx_r = bl.sx + 1u == d.tiles_x ? 0u : bl.sx + 1u;   // block column to the right
-        const uint32_t sy_b = bl.sy + 1u == d.blocks_y ? 0u : bl.sy + 1u;   // block row below
-        // the two sides of the halo array (by sweep parity)
-        const gptr<const uint8_t> halo_s0 = Glob(static_cast<const uint8_t*>(d.halo));
-        const gptr<const uint8_t> halo_s1 = halo_s0 + d.n_blocks * d.halo_stride;
-
-        // Everything the block reads that needs only the descriptor is loaded together, before any of it is
-        // used, so that the round trips overlap: the lattice's counters (read before this kernel stores any
-        // state), the block's flip bits (they matter only under a pending flip: the edge-reaching clusters'
-        // bits from k_resolve; before them in FB the rule words of the clusters inside the block, constant
-        // under the parity rule) and every candidate for the spin below the tile (which one is used depends on
-        // the counters). The descriptor fields these loads need are fetched first, in one batch, and the loads
-        // carry no condition (in-range addresses, values unused where they do not apply), so that the compiler
-        // neither fetches a field at its first use nor waits for every load at the end of a branch.
-        HeldScalar(d.state);
-        HeldScalar(d.fbits);
-        HeldScalar(d.halo);
-        HeldScalar(d.ecol_stride);
-        HeldScalar(d.halo_stride);
-        HeldScalar(d.qcap);
-        HeldScalar(d.fsw);
-        HeldScalar(d.n_blocks);
-        const uint32_t it0 = injected ? 0u : stp[kStIteration];
-        const uint32_t it_end = injected ? 0u : stp[kStItEnd];
-        const uint32_t applied = injected ? 0u : stp[kStApplied];
-        const uint32_t y_last = (bl.wyb + r_begin + (nrow > 0 ? nrow : 1u) - 1u) * rpw + lrow;
-        const uint32_t y_below = nrow > 0 ? ((y_last + 1u == n1) ? 0u : y_last + 1u) : 0u;
-        const uint32_t below = (r_begin + nrow) * bl.stride + lx;   // the site below the tile, inside the block
-        const uint32_t below_halo = (sy_b * d.tiles_x + bl.sx) * d.halo_stride + d.ecol_stride + lx;
-        const uint32_t hd_spin = spins[y_below * n0 + x];
-        // (the label-only pass over injected bonds has no flip bits and no halos: those loads belong to the sweep,
-        // where `injected` is false at compile time)
-        uint32_t fbw = 0, hd_lab = 0, hd_sv = 0, hd_h0 = 0, hd_h1 = 0;
-        if (!injected)
-        {
-            // fsw <= 256: a block has at most 2 * 64 + 2 * kWavesPerBlock * 64 boundary sites, 4 * edge_cap / 32
-            // words of slots (the engine checks the bound), so one word per thread
-            fbw = fbits_g[min(static_cast<uint32_t>(threadIdx.x), d.fsw - 1u)];
-            hd_lab = __builtin_amdgcn_raw_buffer_load_b16(rs_local, below * 2u, 0, 0);
-            hd_sv = __builtin_amdgcn_raw_buffer_load_b8(rs_spins, below, 0, 0);
-            hd_h0 = halo_s0[below_halo];
-            hd_h1 = halo_s1[below_halo];
-            Issued(fbw);   // not sunk into the branch that stores it
-        }
-
-        // sweep schedule: a lattice past its last sweep is left alone by the whole sweep
-        const bool act = injected || it0 < it_end;
-        if (bl.lb == 0 && threadIdx.x == 0)
-        {
-            stp[kStActive] = act ? 1u : 0u;
-            if (act && d.flip_rule != 0u)
-                stp[kStFlipKey] = FlipKey(d.seed, it0);   // an inactive lattice keeps the key of its pending flip
-            if (act && !injected)
-                stp[kStHaloSide] = (it0 >> 1) & 1u;
-        }
-        if (!act)
-            return;
-        // The previous sweep's flip is still pending (applied != iteration): it is applied here, each site
-        // as it is loaded, from its label and the block's flip bits; the flipped spins are stored as the
-        // rows are processed. That flip belongs to the sweep that started at iteration it0 - 2.
-        const bool pending = !injected && applied != it0;
-        const uint32_t it1 = it0 + 1u;
-        const uint32_t it2 = it1 + 1u;
-        const bool rot1 = !injected && (it1 % 15u == 0u);
-        const bool rot2 = !injected && (it2 % 15u == 0u);
-
-        // halos: this sweep writes the block's first column and first wave row into its side of the halo
-        // array; the other side holds the neighbours' flipped halos of the pending flip
-        const uint32_t hside = (it0 >> 1) & 1u;
-        const gptr<const uint8_t> halo_g = hside ? halo_s0 : halo_s1;
-        const Rsrc rs_halo = MakeRsrc(d.halo + (hside * d.n_blocks + bl.lb) * d.halo_stride, d.halo_stride);
-        const uint32_t hcol_off = (lx == 0u && !injected) ? lrow : kNoStore;   // first column: one lane per lattice row
-        uint32_t* const Qw = Q + w * kQw;
-        uint32_t* const Pl = At(P, lane4);   // this lane's entry of wave row 0
-        uint32_t* const dummy = Qw + 64u + lane;
-        // a full queue (>= 64 entries) is worked off right away; the tail moves to the front
-        const auto drain64 = [&](uint32_t& qlen) {
-            const uint32_t e = Qw[lane];
-            LdsUnionLockstep(P, e >> 16, e & 0xFFFFu);
-            const uint32_t rem = qlen - 64u;
-            const uint32_t t = Qw[64u + lane];
-            if (lane < rem)
-                Qw[lane] = t;
-            qlen = rem;
-        };
-
-        // lane masks: first column of a lattice row, lanes with a right neighbour inside the wave row,
-        // lanes whose down neighbour sits in the same wave row
-        uint64_t rowstart = 1;
-        if (!TW64)
-            for (uint32_t j = tw; j < 64u; j += tw)
-                rowstart |= 1ull << j;
-        const uint64_t redge = rowstart << elane;   // the last site of every lattice row of the wave row
-        const uint64_t in_right = PAD ? (vmask & ~redge) : ~redge;
-        const uint64_t low = TW64 ? 0ull : ((1ull << (64u - tw)) - 1ull);
-        const uint64_t lanes_below = (1ull << lane) - 1ull;
-
-        // pending flip: the block's flip bits (loaded into FB above), one per label index (k_resolve wrote the
-        // bit of every cluster: by root index, or by qcap + slot for an edge-reaching one), so a site's flip is
-        // the bit at its label's index
-        const auto flip_of = [&](const uint32_t lab) { return (LdsLoad(&FB[(lab & 0x7FFFu) >> 5]) >> (lab & 31u)) & 1u; };
-
-        // spins below the tile (down halo), needed last but fetched first. Under a pending flip, below the
-        // block the neighbour's halo holds the flipped spin; inside the block the spin and label of the site
-        // below are carried across the barrier in the lane's spare LDS word (writing them there needs the
-        // loaded values, so these loads complete before the wave that owns the site may store its flipped
-        // spin) and flipped after it, with the block's flip bits.
-        uint32_t halo_down = 0;
-        const bool carry = nrow > 0 && pending && !last_wave;
-        // The block's flip bits and rule words, the carried site below and the barrier that publishes them: run
-        // by every wave after the loads of its first chunk of rows are issued, so that this work and the
-        // barrier overlap their round trip.
-        const auto meet = [&]() {
-            if (!injected)
-            {
-                if (threadIdx.x < d.fsw)
-                    FB[d.qcap / 32u + threadIdx.x] = fbw;
-                if (d.flip_rule == 0u)
-                    for (uint32_t i = threadIdx.x; i < bl.nwr * 2u; i += 256u)   // bl.nwr * 64 root indices, 32 per word
-                        FB[i] = RuleWord(d, bl, i, false, 0u);
-                else if (pending)   // the random rule's words, with the key of the pending flip's sweep
-                    for (uint32_t i = threadIdx.x; i < bl.nwr * 2u; i += 256u)
-                        FB[i] = RuleWord(d, bl, i, true, FlipKey(d.seed, it0 - 2u));
-            }
-            if (nrow > 0)
-            {
-                if (!pending)
-                    halo_down = hd_spin;
-                else if (carry)
-                    __hip_atomic_store(dummy, (hd_lab << 8) | (hd_sv & 0xFFu), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-                else
-                    halo_down = hside ? hd_h0 : hd_h1;
-            }
-            __syncthreads();   // AC, FB, the carried site below
-            if (carry)
-            {
-                const uint32_t v = LdsLoad(dummy);
-                const uint32_t lab = v >> 8;
-                halo_down = (v & 0xFFu) ^ flip_of(lab);
-            }
-        };
-
-        uint64_t last_B = 0, last_D = 0, down_bits = 0, right_bits = 0;
-        uint32_t qlen = 0;
-        uint32_t Rp = 0;   // 64-wide tiles: root of this lane's site in the previous row
-        uint64_t prev_S = 0, prev_U2 = 0, prev_B = 0, prev_Ball = 0;
-        uint32_t prev_site = 0;
-        uint32_t colv = 0;   // 64-wide tiles: lane r collects the first-column spin of row r
-        {
-            // the chunk loop exists twice: sweeps without a group rotation (13 in 15) carry no rotation code
-            // (and twice more for the sweeps that apply a pending flip on load, the rule after any sweep)
-            const auto chunks = [&](auto rotating, auto flipping) {
-            constexpr bool kRot = decltype(rotating)::value;
-            constexpr bool kPend = decltype(flipping)::value;
-            // rows loaded together: a flip on load also keeps the labels in flight, so half as many
-            constexpr uint32_t kC = kPend && kCh > 1u ? kCh / 2u : kCh;
-            // what one chunk of rows loads per lane: the spin byte, the lcg32 state and, under a pending flip,
-            // the label of its site in each row; one right-halo spin and one rotation offset per row (lane i:
-            // row r0 + i of the chunk)
-            struct Chunk
-            {
-                uint32_t sp[kC], aux[kC], lab[kC], h, g_rot;
-            };
-            // The loads carry no condition (rows past the tile re-read its last row, values unused), so that
-            // they issue back to back and their latencies overlap.
-            const auto load = [&](const uint32_t r0, Chunk& c) {
-                const uint32_t lrow_ch = r_begin + min(r0 + (lane % kC), nrow - 1u);
-                // right halo of a 64-wide tile: under a pending flip the right neighbour's flipped first column
-                c.h = 0;
-                if (TW64)
-                    c.h = pending ? halo_g[(bl.sy * d.tiles_x + sx_r) * d.halo_stride + lrow_ch]
-                                  : spins[(bl.wyb + lrow_ch) * n0 + sx_r * 64u];
-                // rotation offsets of the chunk's groups, needed on rotating sweeps only
-                c.g_rot = kRot ? rotp[(bl.base + lrow_ch * bl.stride) >> 6] : 0u;
-#pragma unroll
-                for (uint32_t i = 0; i < kC; ++i)
-                {
-                    // row base in scalar registers, the lane offset in a vector register
-                    const uint32_t wr = r_begin + min(r0 + i, nrow - 1u);
-                    const uint32_t rowoff = Uniform(wr * bl.stride);
-                    c.sp[i] = __builtin_amdgcn_raw_buffer_load_b8(rs_spins, lane, rowoff, 0);
-                    c.aux[i] = injected ? (bond_in + bl.base + rowoff)[lane] : __builtin_amdgcn_raw_buffer_load_b32(rs_rng, lane4, rowoff * 4u, 0);
-                    c.lab[i] = kPend ? __builtin_amdgcn_raw_buffer_load_b16(rs_local, lane * 2u, rowoff * 2u, 0) : 0u;
-                }
-            };
-            const auto process = [&](const uint32_t r0, Chunk& c) {
-                uint32_t(&sp)[kC] = c.sp;
-                const uint32_t(&aux)[kC] = c.aux;
-                const uint32_t(&lab)[kC] = c.lab;
-                const uint32_t h = c.h, g_rot = c.g_rot;
-                if (kPend)
-                {
-#pragma unroll
-                    for (uint32_t i = 0; i < kC; ++i)
-                        sp[i] ^= flip_of(lab[i]);
-                }
-                const uint64_t HR = TW64 ? __ballot((h & 1u) != 0u) : 0ull;
-
-#pragma unroll
-                for (uint32_t i = 0; i < kC; ++i)
-                {
-                    const uint32_t r = r0 + i;
-                    if (r < nrow)
-                    {
-                        const uint32_t wr = r_begin + r;
-                        const uint32_t site = bl.base + wr * bl.stride + lane;
-                        const uint64_t S = __ballot((sp[i] & 1u) != 0u);
-                        if (TW64)
-                            colv = LaneBit(1ull << r) ? static_cast<uint32_t>(S) : colv;   // bit 0 of S: lane 0's spin
-                        else
-                            __builtin_amdgcn_raw_buffer_store_b8(static_cast<uint8_t>(sp[i] & 1u), rs_halo, hcol_off, wr * rpw, 0);
-                        if (wr == 0 && !injected)
-                            __builtin_amdgcn_raw_buffer_store_b8(static_cast<uint8_t>(sp[i] & 1u), rs_halo, d.ecol_stride + lane, 0, 0);
-                        uint64_t Ball, U2;
-                        if (!injected)
-                        {
-                            // two LCG32_State<64>::Update of the group of this wave row
-                            // (random/src/lcg32.cpp:51-84); a rotation by `shift` moves lane
-                            // (i + shift) & 63's selector to lane i
-                            uint32_t ks = sp[i] & kSelMask, st = aux[i], shift = 0;
-                            if (kRot && rot1)
-                            {
-                                shift = ShuffleShift(st, it1) & 63u;
-                                ks = static_cast<uint32_t>(__shfl(static_cast<int>(ks), static_cast<int>((lane + shift) & 63u)));
-                            }
-                            uint64_t ac = AC[ks >> kSelShift];
-                            st = static_cast<uint32_t>(ac) * st + static_cast<uint32_t>(ac >> 32);
-                            const uint32_t u1 = st;
-                            if (kRot && rot2)
-                            {
-                                const uint32_t s2 = ShuffleShift(st, it2) & 63u;
-                                shift += s2;
-                                ks = static_cast<uint32_t>(__shfl(static_cast<int>(ks), static_cast<int>((lane + s2) & 63u)));
-                                ac = AC[ks >> kSelShift];
-                            }
-                            st = static_cast<uint32_t>(ac) * st + static_cast<uint32_t>(ac >> 32);
-                            __builtin_amdgcn_raw_buffer_store_b32(st, rs_rng, lane4, Uniform(wr * bl.stride) * 4u, 0);
-                            if (kRot)
-                            {
-                                spins[site] = static_cast<uint8_t>((sp[i] & 1u) | ks);
-                                if (lane == 0)
-                                    rotp[site >> 6] = (ReadLane(g_rot, i) + shift) & 63u;
-                            }
-                            else if (kPend)
-                                __builtin_amdgcn_raw_buffer_store_b8(static_cast<uint8_t>(sp[i]), rs_spins, lane, Uniform(wr * bl.stride), 0);
-                            const uint64_t U1 = __ballot(u1 < thr);
-                            U2 = __ballot(st < thr);
-                            // right neighbour's spin: next lane, or for a row's last site the halo (64-wide
-                            // tiles) or the first column of the same lattice row (narrow tiles: one tile
-                            // column)
-                            uint64_t RS;
-                            if (!PAD)
-                                RS = TW64 ? ((S >> 1) | (((HR >> i) & 1ull) << 63))
-                                          : (((S >> 1) & in_right) | ((S << (tw - 1u)) & ~in_right));
-                            else
-                                RS = TW64 ? (((S >> 1) & ~redge) | (((HR >> i) & 1ull) << elane))
-                                          : (((S >> 1) & ~redge) | ((S << elane) & redge));
-                            Ball = ~(S ^ RS) & U1;
-                        }
-                        else
-                        {
-                            Ball = __ballot((aux[i] & 1u) != 0u);
-                            U2 = __ballot((aux[i] & 2u) != 0u);
-                        }
-                        if (PAD)
-                        {
-                            Ball &= vmask;
-                            U2 &= vmask;
-                        }
-                        const uint64_t B = Ball & in_right;
-                        const uint64_t edge = Ball & redge;
-                        if (TW64)
-                            right_bits |= (PAD ? ((edge >> elane) & 1ull) : (edge >> 63)) << r;
-                        else
-                            for (uint32_t j = 0; j < rpw; ++j)
-                                right_bits |= ((edge >> (j * tw + elane)) & 1ull) << (r * rpw + j);
-                        if (r == 0)
-                            s_first_B[w] = B;
-
-                        const uint32_t row_b = wr * 256u;   // byte offset of the wave row in P
-                        if (TW64)
-                        {
-                            // slot of this lane's row run: the number of run starts after lane 0 up to this
-                            // lane; the first lane of the run initialises it with its own node
-                            uint32_t* const Mk = Qw + __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(~B >> 32),
-                                                                               __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(~B), 0u));
-                            const uint32_t self = row_b + lane4;
-                            __hip_atomic_store(LaneBit(~(B << 1)) ? Mk : dummy, self, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-                            // the row's entries start as roots (overwritten below), so chases end on them
-                            __hip_atomic_store(At(P, self), self, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-                            const uint64_t D = r == 0 ? 0ull : (injected ? prev_U2 : (~(prev_S ^ S) & prev_U2));
-                            if (r > 0)
-                                LdsMin(LaneBit(D) ? Mk : dummy, Rp);
-                            uint32_t root = LdsLoad(Mk);
-                            // bonds to a root other than the run's minimum link that root under it
-                            const uint64_t mg = D & __ballot(Rp != root);
-                            if (mg != 0ull)
-                            {
-                                const uint32_t old = __hip_atomic_fetch_min(LaneBit(mg) ? At(P, Rp) : dummy, root, __ATOMIC_RELAXED,
-                                                                            __HIP_MEMORY_SCOPE_WORKGROUP);
-                                // Rp was no longer a root (another lane linked it first): join the two trees
-                                const uint64_t more = mg & __ballot(old != Rp && old != root);
-                                if (more != 0ull)
-                                {
-                                    const bool mo = LaneBit(more);
-                                    LdsUnionLockstep(P, mo ? root : 0u, mo ? old : 0u);
-                                }
-                                // the run's minimum may itself have been linked under another root
-                                for (;;)
-                                {
-                                    const uint32_t pr = LdsLoad(At(P, root));
-                                    if (!__ballot(pr != root))
-                                        break;
-                                    root = pr;
-                                }
-                            }
-                            if (dump && r > 0)
-                                dump[prev_site] = static_cast<uint8_t>((LaneBit(prev_Ball) ? 1u : 0u) | (LaneBit(D) ? 2u : 0u));
-                            *At(Pl, row_b) = root;
-                            Rp = root;
-                        }
-                        else
-                        {
-                            // every site starts under the first site of its row run
-                            const uint64_t below = ~B & lanes_below;
-                            const uint32_t run_start = below ? 64u - static_cast<uint32_t>(__clzll(below)) : 0u;
-                            *At(Pl, row_b) = row_b + run_start * 4u;
-                            if (r > 0)
-                            {
-                                // bonds of the previous wave row to the row below: queue one union per overlap
-                                // interval
-                                const uint64_t SD = (Shr(prev_S, tw) & low) | Shl(S, 64u - tw);
-                                const uint64_t D = injected ? prev_U2 : (~(prev_S ^ SD) & prev_U2);
-                                const uint64_t tgtB = Shr(prev_B, tw) | Shl(B, 64u - tw);
-                                const uint64_t K = FirstBondPerInterval(D, prev_B & tgtB, rowstart);
-                                if (LaneBit(K))
-                                {
-                                    const uint32_t top = row_b - 256u + lane4;
-                                    const uint32_t bot = (lane < 64u - tw) ? top + tw * 4u : row_b + lane4 - (64u - tw) * 4u;
-                                    const uint32_t pos = qlen + __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(K >> 32),
-                                                                                         __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(K), 0u));
-                                    Qw[pos] = (top << 16) | bot;
-                                }
-                                qlen += static_cast<uint32_t>(__popcll(K));
-                                if (qlen >= 64u)
-                                    drain64(qlen);
-                                if (dump)
-                                    dump[prev_site] = static_cast<uint8_t>((LaneBit(prev_Ball) ? 1u : 0u) | (LaneBit(D) ? 2u : 0u));
-                            }
-                        }
-                        prev_S = S;
-                        prev_U2 = U2;
-                        prev_B = B;
-                        prev_Ball = Ball;
-                        prev_site = site;
-                    }
-                }
-            };
-            // a tile of at most kC rows is one chunk, starting at row 0; the first chunk's loads go out before
-            // the barrier (a wave without rows loads nothing and only meets the others there)
-            Chunk c0;
-            if (nrow > 0)
-                load(0u, c0);
-            meet();
-            if (nrow == 0)
-                return;
-            process(0u, c0);
-            for (uint32_t r0 = kC; r0 < (TWR_MAX <= kC ? 0u : nrow); r0 += kC)
-            {
-                Chunk c;
-                load(r0, c);
-                process(r0, c);
-            }
-            };
-            if (rot1 || rot2)
-            {
-                if (pending)
-                    chunks(std::true_type{}, std::true_type{});
-                else
-                    chunks(std::true_type{}, std::false_type{});
-            }
-            else if (pending)
-                chunks(std::false_type{}, std::true_type{});
-            else
-                chunks(std::false_type{}, std::false_type{});
-        }
-        if (nrow > 0)
-        {
-            if (TW64 && !injected)   // first column of the tile's rows (rpw == 1): one store per wave
-                __builtin_amdgcn_raw_buffer_store_b8(static_cast<uint8_t>(colv & 1u), rs_halo, lane < nrow ? r_begin + lane : kNoStore, 0, 0);
-
-            // bonds out of the last wave row: into the same wave row (tw < 64), into the next tile of the
-            // block, or across the block edge
-            {
-                const uint32_t wr = r_begin + nrow - 1u;
-                // halo spins arrive in the lanes that need them (lanes >= 64 - tw)
-                const uint64_t H = __ballot((halo_down & 1u) != 0u);
-                const uint64_t SD = TW64 ? H : ((Shr(prev_S, tw) & low) | (H & ~low));
-                const uint64_t D = injected ? prev_U2 : (~(prev_S ^ SD) & prev_U2);
-                if (!TW64)
-                {
-                    const uint64_t Din = D & low;
-                    const uint64_t K = FirstBondPerInterval(Din, prev_B & Shr(prev_B, tw), rowstart);
-                    if (LaneBit(K))
-                    {
-                        const uint32_t pos = qlen + __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(K >> 32),
-                                                                             __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(K), 0u));
-                        const uint32_t top = wr * 256u + lane4;
-                        Qw[pos] = (top << 16) | (top + tw * 4u);
-                    }
-                    qlen += static_cast<uint32_t>(__popcll(K));
-                    if (qlen >= 64u)
-                        drain64(qlen);
-                }
-                if (dump)
-                    dump[prev_site] = static_cast<uint8_t>((LaneBit(prev_Ball) ? 1u : 0u) | (LaneBit(D) ? 2u : 0u));
-                last_B = prev_B;
-                if (last_wave)
-                    down_bits = D & ~low;
-                else
-                    last_D = D & ~low;
-            }
-
-            // the rest of the queued unions of this tile (fewer than 64)
-            if (!TW64 && qlen > 0)
-            {
-                const uint32_t e = (lane < qlen) ? Qw[lane] : 0u;
-                LdsUnionLockstep(P, e >> 16, e & 0xFFFFu);
-            }
-        }
-        __syncthreads();
-
-        // unions across the tile edges inside the block
-        if (nrow > 0 && !last_wave)
-        {
-            const uint32_t wr = r_begin + nrow - 1u;
-            const uint64_t Bbot = s_first_B[w + 1u];
-            const uint64_t tgtB = TW64 ? Bbot : Shl(Bbot, 64u - tw);
-            const bool go = LaneBit(FirstBondPerInterval(last_D, last_B & tgtB, rowstart));
-            const uint32_t top = wr * 256u + lane4;
-            LdsUnionLockstep(P, go ? top : 0u, go ? top + 256u - (64u - tw) * 4u : 0u);
-        }
-        __syncthreads();
-
-        // every site's block-local root (kRows chases in flight per lane). A tile of at most kRows rows
-        // keeps its roots in registers; taller tiles write them back into P.
-        const bool one_chunk = TWR_MAX <= kRows || nrow <= kRows;
-        uint32_t xs[kRows];
-        // (a wave of a partial block may own no rows: its part of P was never written and is not chased)
-        for (uint32_t r0 = 0; r0 < (TWR_MAX <= kRows ? (nrow > 0 ? 1u : 0u) : nrow); r0 += kRows)
-        {
-#pragma unroll
-            for (uint32_t i = 0; i < kRows; ++i)
-                xs[i] = (r_begin + ((r0 + i < nrow) ? r0 + i : r0)) * 256u + lane4;
-            // two steps per round; a round ends the chase once a step moved no lane of any row. The
-            // differences are summed in vector registers (16 values below 2^17 cannot wrap to zero). Parents
-            // only decrease, so a chase ends within kSites steps; more rounds mean a broken forest, which is
-            // reported instead of followed.
-            for (uint32_t round = 0;; ++round)
-            {
-                if (round * 2u > kSites)
-                {
-                    if (lane == 0)
-                        (void)__hip_atomic_fetch_or(stp + kStErr, kErrLabelRange, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                    break;
-                }
-                uint32_t ys[kRows];
-                uint32_t moved = 0;
-#pragma unroll
-                for (uint32_t i = 0; i < kRows; ++i)
-                {
-                    ys[i] = LdsLoad(At(P, xs[i]));
-                    moved += ys[i] ^ xs[i];
-                }
-                if (!__ballot(moved != 0u))
-                    break;
-                moved = 0;
-#pragma unroll
-                for (uint32_t i = 0; i < kRows; ++i)
-                {
-                    xs[i] = LdsLoad(At(P, ys[i]));
-                    moved += xs[i] ^ ys[i];
-                }
-                if (!__ballot(moved != 0u))
-                    break;
-            }
-            if (!one_chunk)
-            {
-#pragma unroll
-                for (uint32_t i = 0; i < kRows; ++i)
-                    if (r0 + i < nrow)
-                        *At(Pl, (r_begin + r0 + i) * 256u) = xs[i];
-            }
-        }
-        // (taller tiles: a flagged entry is a root's own, first flagged by the edge marks, later holding its
-        // slot label; either way the site is its own root)
-        const auto root_of = [&](const uint32_t r) {
-            if (one_chunk)
-                return xs[r];
-            const uint32_t v = LdsLoad(At(Pl, (r_begin + r) * 256u));
-            return v >= kPFlag ? (r_begin + r) * 256u + lane4 : v;
-        };
-        __syncthreads();   // no chase may meet a flagged entry
-
-        // Sites on the block edge flag their root (lanes off the edge flag their own word of Q). The edge
-        // lanes of a row are `side`, plus every lane of the block's first and last lattice rows. The marks of
-        // up to kRows rows are issued together and return the root's entry as it was: the lane that found it
-        // unflagged (the cluster's first mark) gives the cluster the next slot of the block (one LDS counter,
-        // one addition per wave and chunk of rows), writes the slot's union-find entry (a root keyed by the
-        // root's site) and makes the root's entry in P kPFlag | (qcap + slot) << 2, so that after the barrier
-        // every site of the cluster reads the label 0x8000 | (qcap + slot). A block has at most as many edge
-        // roots as boundary sites, within its slot capacity; more would be a broken invariant, reported
-        // through the error flag.
-        const uint64_t side = TW64 ? (PAD ? (1ull | (1ull << elane)) : 0x8000000000000001ull) : __ballot(lx == 0 || rbound);
-        const uint64_t top_first = r_begin == 0 ? (TW64 ? vmask : (__ballot(lrow == 0) & vmask)) : 0ull;
-        const uint64_t bottom_last = last_wave ? (TW64 ? vmask : (__ballot(lrow == rpw - 1u) & vmask)) : 0ull;
-        const uint32_t qcap = d.qcap, bslots = kWavesPerBlock * d.edge_cap;
-        const Rsrc rs_cpar = MakeRsrc(d.cpar + bslots * bl.lb, bslots * 8u);
-        // full tiles (the rule) take the row count and the first/last row masks at compile time
-        const bool full = TWR_MAX <= kRows && nrow == kRows;
-        const auto mark_rows = [&](auto full_t, const uint32_t r0) {
-            constexpr bool kFull = decltype(full_t)::value;
-            uint32_t old[kRows], root[kRows];
-#pragma unroll
-            for (uint32_t i = 0; i < kRows; ++i)
-            {
-                old[i] = kPFlag;
-                root[i] = 0u;
-                const uint32_t r = r0 + i;
-                if (kFull || r < nrow)
-                {
-                    const bool last = kFull ? i + 1u == kRows : r + 1u == nrow;
-                    const uint64_t m = side | (r == 0u ? top_first : 0ull) | (last ? bottom_last : 0ull);
-                    root[i] = root_of(r);
-                    const uint32_t o = __hip_atomic_fetch_or(LaneBit(m) ? At(P, root[i]) : dummy, kPFlag, __ATOMIC_RELAXED,
-                                                             __HIP_MEMORY_SCOPE_WORKGROUP);
-                    old[i] = LaneBit(m) ? o : kPFlag;
-                }
-            }
-            uint64_t F[kRows];
-            uint32_t total = 0;
-#pragma unroll
-            for (uint32_t i = 0; i < kRows; ++i)
-            {
-                F[i] = __ballot(old[i] < kPFlag);
-                total += static_cast<uint32_t>(__popcll(F[i]));
-            }
-            if (total == 0u)
-                return;
-            uint32_t base = 0;
-            if (lane == 0u)
-                base = __hip_atomic_fetch_add(&s_nslot, total, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-            base = __builtin_amdgcn_readfirstlane(base);
-#pragma unroll
-            for (uint32_t i = 0; i < kRows; ++i)
-            {
-                const bool first = LaneBit(F[i]);
-                const uint32_t pos = base + __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(F[i] >> 32),
-                                                                      __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(F[i]), 0u));
-                __hip_atomic_store(first ? At(P, root[i]) : dummy, kPFlag | ((qcap + min(pos, bslots - 1u)) << 2),
-                                   __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-                const u32x2 entry = {bslots * bl.lb + pos, SiteOf(bl.base, bl.stride, root[i] >> 2)};   // (site << 32) | slot
-                __builtin_amdgcn_raw_buffer_store_b64(entry, rs_cpar, first ? pos * 8u : kNoStore, 0, 0);
-                base += static_cast<uint32_t>(__popcll(F[i]));
-            }
-        };
-        if (full)
-            mark_rows(std::true_type{}, 0u);
-        else if (one_chunk)
-            mark_rows(std::false_type{}, 0u);
-        else
-            for (uint32_t r0 = 0; r0 < nrow; r0 += kRows)
-                mark_rows(std::false_type{}, r0);
-        __syncthreads();   // every slot label in place
-
-        // labels out: the block-local labels, and (label << 16) | root index of the block's first and last
-        // column and first and last wave row for the merge and the halo flips. The outputs go through buffer
-        // views of this block's part of each array; a lane with nothing to store gets an offset past the
-        // view, and the hardware drops that store (no exec mask).
-        const Rsrc rs_ecol = MakeRsrc(d.ecol + 2u * bl.lb * d.ecol_stride, 8u * d.ecol_stride);
-        const uint32_t ecol_off = LaneBit(side) ? ((rbound ? d.ecol_stride : 0u) + r_begin * rpw + lrow) * 4u : kNoStore;
-        const Rsrc rs_erow = MakeRsrc(d.erow + 2u * 64u * bl.lb, 2u * 64u * 4u);
-        const auto emit = [&](const uint32_t r, const uint32_t root) {
-            const uint32_t wr = r_begin + r;
-            const uint32_t rowoff = wr * bl.stride;   // sites from the block's first site
-            const uint32_t lab = LdsLoad(At(P, root)) >> 2;
-            const uint32_t e = (lab << 16) | (root >> 2);
-            __builtin_amdgcn_raw_buffer_store_b16(static_cast<uint16_t>(lab), rs_local, lane * 2u, rowoff * 2u, 0);
-            __builtin_amdgcn_raw_buffer_store_b32(e, rs_ecol, ecol_off, r * rpw * 4u, 0);
-            if (wr == 0u)
-                __builtin_amdgcn_raw_buffer_store_b32(e, rs_erow, lane4, 0, 0);
-            if (wr + 1u == bl.nwr)
-                __builtin_amdgcn_raw_buffer_store_b32(e, rs_erow, lane4, 256u, 0);
-        };
-        const auto rows_do = [&](auto full_t, auto&& f) {
-            constexpr bool kFull = decltype(full_t)::value;
-#pragma unroll
-            for (uint32_t i = 0; i < kRows; ++i)
-                if (kFull || i < nrow)
-                    f(i, xs[i]);
-        };
-        const auto for_rows = [&](auto&& f) {
-            if (full)
-                rows_do(std::true_type{}, f);
-            else if (one_chunk)
-                rows_do(std::false_type{}, f);
-            else
-                for (uint32_t r = 0; r < nrow; ++r)
-                    f(r, root_of(r));
-        };
-        for_rows(emit);
-        const gptr<uint64_t> bb = Glob(d.bbits) + kBbitWords * bl.lb;
-        if (lane == 0)
-        {
-            if (last_wave)
-                bb[0] = down_bits;
-            bb[1u + w] = right_bits;
-        }
-        if (threadIdx.x == 0)
-        {
-            const uint32_t n = LdsLoad(&s_nslot);
-            Glob(d.edge_count)[kWavesPerBlock * bl.lb] = min(n, bslots);
-            if (n > bslots)
-                (void)__hip_atomic_fetch_or(stp + kStErr, kErrLabelRange, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
-    }
-
-    // 64-wide tiles of up to 16 rows: eight workgroups per CU (the register budget of 8 waves per SIMD is
-    // asked for explicitly; the compiler keeps the excess scalar registers in vector lanes). Narrow tiles
-    // keep the default budget (the cap would spill vector registers to scratch), and taller tiles are
-    // limited by their LDS anyway.
-    template <uint32_t TWR_MAX, bool DBG>
-    __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8, 8))) void k_bond_label(
-        const LatDesc* __restrict__ descs, const uint32_t* __restrict__ block_lat, const uint32_t total_blocks)
-    {
-        BondLabel<TWR_MAX, true, DBG, false>(descs, block_lat, total_blocks);
-    }
-
-    template <uint32_t TWR_MAX, bool TW64, bool DBG, bool PAD>
-    __global__ __launch_bounds__(256) void k_bond_label_any(const LatDesc* __restrict__ descs, const uint32_t* __restrict__ block_lat,
-                                                            const uint32_t total_blocks)
-    {
-        BondLabel<TWR_MAX, TW64, DBG, PAD>(descs, block_lat, total_blocks);
-    }
-
     // =============================================================================================
     // k_merge: unions across block edges (reference MergeLabels_Kernel, swendsen_wang_amd_gpu.cpp:280-329)
     // =============================================================================================
@@ -2013,30 +888,10 @@ namespace swmi
     // =============================================================================================
     // launch wrappers
     // =============================================================================================
-    static inline uint32_t XcdGrid(const uint32_t units) { return ((units + kNumXcd - 1) / kNumXcd) * kNumXcd; }
-
+    // defined in swmi_bond.hip, one part per combination
     template <bool TW64, bool DBG>
-    static void LaunchBondLabelT(const LatDesc* d_desc, const uint32_t* d_block_lat, const uint32_t total_blocks,
-                                 const uint32_t max_twr, const bool pad, hipStream_t stream)
-    {
-        const uint32_t g = XcdGrid(total_blocks);
-        const auto launch = [&](auto kernel) { kernel<<<g, 256, 0, stream>>>(d_desc, d_block_lat, total_blocks); };
-        if (pad)   // padded lattices: two tile-height bounds
-        {
-            if (max_twr <= 16)
-                launch(k_bond_label_any<16, TW64, DBG, true>);
-            else
-                launch(k_bond_label_any<64, TW64, DBG, true>);
-        }
-        else if (max_twr <= 8)
-            TW64 ? launch(k_bond_label<8, DBG>) : launch(k_bond_label_any<8, false, DBG, false>);
-        else if (max_twr <= 16)
-            TW64 ? launch(k_bond_label<16, DBG>) : launch(k_bond_label_any<16, false, DBG, false>);
-        else if (max_twr <= 32)
-            launch(k_bond_label_any<32, TW64, DBG, false>);
-        else
-            launch(k_bond_label_any<64, TW64, DBG, false>);
-    }
+    void LaunchBondLabelT(const LatDesc* d_desc, const uint32_t* d_block_lat, uint32_t total_blocks, uint32_t max_twr, bool pad,
+                          hipStream_t stream);
 
     void LaunchBondLabel(const LatDesc* d_desc, const uint32_t* d_block_lat, const uint32_t total_blocks, const uint32_t max_twr,
                          const bool all_tw64, const bool pad, const bool debug, hipStream_t stream)
