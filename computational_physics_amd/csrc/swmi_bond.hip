@@ -96,18 +96,14 @@ namespace swmi
         __shared__ uint32_t Q[kWavesPerBlock * kQw];
         __shared__ uint32_t FB[2u * kSites / 32u];   // flip bits of a pending flip, by label index (root or qcap + slot)
         __shared__ uint64_t s_first_B[kWavesPerBlock];
-        __shared__ uint64_t AC[8];              // Numerical Recipes pairs (c << 32 | a) by selector
+        // Numerical Recipes pairs (c << 32 | a) by selector: words 0-7 one update, words 8-15 the jump from the stored
+        // states to this sweep's
+        __shared__ uint64_t AC[16];
         __shared__ uint32_t s_nslot;            // slots given to the block's edge-reaching clusters
 
         const uint32_t b = RemapBlock(total_blocks);
         if (b >= total_blocks)
             return;
-        if (threadIdx.x < 8u)
-        {
-            uint32_t a, c;
-            ParamsOf(threadIdx.x, a, c);
-            AC[threadIdx.x] = (static_cast<uint64_t>(c) << 32) | a;
-        }
         if (threadIdx.x == 0)
             s_nslot = 0u;
         const LatDesc& d = descs[LatticeOf(block_lat, b)];
@@ -159,6 +155,7 @@ namespace swmi
         // carry no condition (in-range addresses, values unused where they do not apply), so that the compiler
         // neither fetches a field at its first use nor waits for every load at the end of a branch.
         HeldScalar(d.state);
+        HeldScalar(d.rng_it);
         HeldScalar(d.fbits);
         HeldScalar(d.halo);
         HeldScalar(d.ecol_stride);
@@ -169,6 +166,7 @@ namespace swmi
         const uint32_t it0 = injected ? 0u : stp[kStIteration];
         const uint32_t it_end = injected ? 0u : stp[kStItEnd];
         const uint32_t applied = injected ? 0u : stp[kStApplied];
+        const uint32_t rng_it = injected ? 0u : *Glob(static_cast<const uint32_t*>(d.rng_it));
         const uint32_t y_last = (bl.wyb + r_begin + (nrow > 0 ? nrow : 1u) - 1u) * rpw + lrow;
         const uint32_t y_below = nrow > 0 ? ((y_last + 1u == n1) ? 0u : y_last + 1u) : 0u;
         const uint32_t below = (r_begin + nrow) * bl.stride + lx;   // the site below the tile, inside the block
@@ -209,6 +207,11 @@ namespace swmi
         const uint32_t it2 = it1 + 1u;
         const bool rot1 = !injected && (it1 % 15u == 0u);
         const bool rot2 = !injected && (it2 % 15u == 0u);
+        // The stored states are those of iteration rng_it: a lane's (a, c) stays the same until the next rotation,
+        // so the state after the sweep's first update is one affine step away, u1 = A st + C with (A, C) the pair
+        // applied it1 - rng_it times, and the sweep needs to store no state. A rotating sweep stores the state at
+        // which the pairs change (it0, or it1 when the second update rotates): at most 15 updates are jumped.
+        const uint32_t n_jump = min((rot1 ? it0 : it1) - rng_it, 15u);
 
         // halos: this sweep writes the block's first column and first wave row into its side of the halo
         // array; the other side holds the neighbours' flipped halos of the pending flip
@@ -259,6 +262,18 @@ namespace swmi
         const auto meet = [&]() {
             if (!injected)
             {
+                if (threadIdx.x < 8u)
+                {
+                    uint32_t a, c, ja = 1u, jc = 0u;
+                    ParamsOf(threadIdx.x, a, c);
+                    for (uint32_t i = 0; i < n_jump; ++i)
+                    {
+                        ja *= a;
+                        jc = a * jc + c;
+                    }
+                    AC[threadIdx.x] = (static_cast<uint64_t>(c) << 32) | a;
+                    AC[8u + threadIdx.x] = (static_cast<uint64_t>(jc) << 32) | ja;
+                }
                 if (threadIdx.x < d.fsw)
                     FB[d.qcap / 32u + threadIdx.x] = fbw;
                 if (d.flip_rule == 0u)
@@ -363,24 +378,21 @@ namespace swmi
                             // two LCG32_State<64>::Update of the group of this wave row
                             // (random/src/lcg32.cpp:51-84); a rotation by `shift` moves lane
                             // (i + shift) & 63's selector to lane i
-                            uint32_t ks = sp[i] & kSelMask, st = aux[i], shift = 0;
-                            if (kRot && rot1)
-                            {
-                                shift = ShuffleShift(st, it1) & 63u;
-                                ks = static_cast<uint32_t>(__shfl(static_cast<int>(ks), static_cast<int>((lane + shift) & 63u)));
-                            }
+                            uint32_t ks = sp[i] & kSelMask, shift = 0;
+                            const uint64_t jump = AC[8u + (ks >> kSelShift)];
                             uint64_t ac = AC[ks >> kSelShift];
-                            st = static_cast<uint32_t>(ac) * st + static_cast<uint32_t>(ac >> 32);
-                            const uint32_t u1 = st;
-                            if (kRot && rot2)
+                            uint32_t u1 = static_cast<uint32_t>(jump) * aux[i] + static_cast<uint32_t>(jump >> 32);
+                            if (kRot)
                             {
-                                const uint32_t s2 = ShuffleShift(st, it2) & 63u;
-                                shift += s2;
-                                ks = static_cast<uint32_t>(__shfl(static_cast<int>(ks), static_cast<int>((lane + s2) & 63u)));
+                                // the state jumped to is the one the rotation works on and the one stored
+                                __builtin_amdgcn_raw_buffer_store_b32(u1, rs_rng, lane4, Uniform(wr * bl.stride) * 4u, 0);
+                                shift = ShuffleShift(u1, rot1 ? it1 : it2) & 63u;
+                                ks = static_cast<uint32_t>(__shfl(static_cast<int>(ks), static_cast<int>((lane + shift) & 63u)));
                                 ac = AC[ks >> kSelShift];
+                                if (rot1)
+                                    u1 = static_cast<uint32_t>(ac) * u1 + static_cast<uint32_t>(ac >> 32);
                             }
-                            st = static_cast<uint32_t>(ac) * st + static_cast<uint32_t>(ac >> 32);
-                            __builtin_amdgcn_raw_buffer_store_b32(st, rs_rng, lane4, Uniform(wr * bl.stride) * 4u, 0);
+                            const uint32_t st = static_cast<uint32_t>(ac) * u1 + static_cast<uint32_t>(ac >> 32);
                             if (kRot)
                             {
                                 spins[site] = static_cast<uint8_t>((sp[i] & 1u) | ks);

@@ -202,7 +202,7 @@ namespace swmi
         const Geometry g = GeometryOf(c.n0, c.n1, c.tile_rows);
         const uint64_t n = static_cast<uint64_t>(g.pitch) * c.n1, groups = n / 64;
         return n * (1 + 4 + 2) + groups * (3 * 8 + 4) + static_cast<uint64_t>(kBbitWords) * 8 * g.n_blocks +
-               4ull * (kLatStateWords + 4ull * c.max_samples) + 4ull * 2 * kWavesPerBlock * g.n_blocks +
+               4ull * (kLatStateWords + 4ull * c.max_samples) + 4 + 4ull * 2 * kWavesPerBlock * g.n_blocks +
                static_cast<uint64_t>(kWavesPerBlock) * g.n_blocks * (8ull * g.edge_cap + 4) + 8ull * g.ecol_stride * g.n_blocks +
                4ull * 2 * 64 * g.n_blocks + 4ull * g.fsw * g.n_blocks + 2ull * g.halo_stride * g.n_blocks;
     }
@@ -215,7 +215,7 @@ namespace swmi
 
     uint64_t Lattice::Bytes() const
     {
-        return spins.bytes() + rng.bytes() + masks.bytes() + rot.bytes() + local.bytes() + parent.bytes() + cpar.bytes() +
+        return spins.bytes() + rng.bytes() + rng_it.bytes() + masks.bytes() + rot.bytes() + local.bytes() + parent.bytes() + cpar.bytes() +
                bbits.bytes() + state.bytes() + partials.bytes() + edge_count.bytes() + ecol.bytes() + erow.bytes() + fbits.bytes() +
                halo.bytes() + bond_dump.bytes() + bond_in.bytes();
     }
@@ -229,6 +229,7 @@ namespace swmi
         n_groups = static_cast<uint32_t>(np / 64);
         spins.allocate(np);
         rng.allocate(np);
+        rng_it.allocate(1);
         masks.allocate(3ull * n_groups);
         rot.allocate(n_groups);
         local.allocate(np);
@@ -255,7 +256,7 @@ namespace swmi
         threshold = BondThreshold(p_add);
         bond_dump.reset();
         Check(hipMemsetAsync(edge_count.ptr, 0, edge_count.bytes(), stream), "edge list init");
-        LaunchInitState(state.ptr, state_words, c.max_samples, 0xFFFFFFFFu, 0u, 0u, stream);
+        LaunchInitState(state.ptr, rng_it.ptr, state_words, c.max_samples, 0xFFFFFFFFu, 0u, 0u, stream);
         if (np != n)   // padding columns hold spin 0
             Check(hipMemsetAsync(spins.ptr, 0, np, stream), "spin init");
         LaunchHotStart(spins.ptr, n, c.spin_seed, cfg.n0, g.pitch, stream);
@@ -330,6 +331,7 @@ LatDesc swmi_engine::Desc(const Lattice& l, uint32_t block_base) const
     LatDesc d = GeometryDesc(l.g, l.cfg.n0, l.cfg.n1);
     d.spins = l.spins.ptr;
     d.rng = l.rng.ptr;
+    d.rng_it = l.rng_it.ptr;
     d.masks = l.masks.ptr;
     d.rot = l.rot.ptr;
     d.local = l.local.ptr;
@@ -560,6 +562,12 @@ void swmi_engine::OneLattice(const Lattice& l, const uint8_t* bond_in)
         d_one_desc.allocate(1);
     Check(hipMemcpyAsync(d_one_desc.ptr, &d, sizeof(d), hipMemcpyHostToDevice, stream), "descriptor upload");
     Check(hipStreamSynchronize(stream), "descriptor upload");
+}
+
+void swmi_engine::AdvanceRng(const Lattice& l)
+{
+    LaunchAdvanceRng(l.spins.ptr, l.rng.ptr, l.np, l.state.ptr, l.rng_it.ptr, stream);
+    LaunchCheck("rng launch");
 }
 
 void swmi_engine::MaterializeOne(const Lattice& l)
@@ -1008,7 +1016,10 @@ int swmi_rng_export(swmi_engine* engine, uint32_t lattice, uint32_t* states, uin
     return Guard([&] {
         Lattice& l = Eng(engine)->At(lattice);
         if (states)
+        {
+            engine->AdvanceRng(l);
             Check(hipMemcpyAsync(states, l.rng.ptr, l.np * 4, hipMemcpyDeviceToHost, engine->stream), "rng export");
+        }
         if (masks)
             Check(hipMemcpyAsync(masks, l.masks.ptr, 3ull * l.n_groups * 8, hipMemcpyDeviceToHost, engine->stream), "rng export");
         if (rot)
@@ -1055,7 +1066,8 @@ int swmi_checkpoint(swmi_engine* engine, uint32_t lattice, void* buffer, uint64_
         Lattice& l = Eng(engine)->At(lattice);
         if (!buffer || bytes < CheckpointBytes(l))
             throw SwmiError(SWMI_ERR_INVALID, "checkpoint buffer too small (" + std::to_string(CheckpointBytes(l)) + " bytes needed)");
-        engine->MaterializeOne(l);   // the checkpoint holds the chain's spins, with no flip pending
+        engine->MaterializeOne(l);   // the checkpoint holds the chain's spins, with no flip pending,
+        engine->AdvanceRng(l);       // and the generator's states of its iteration
         CheckpointHeader h{};
         std::memcpy(h.magic, "SWMICKP1", 8);
         h.n0 = l.cfg.n0;
@@ -1114,7 +1126,8 @@ int swmi_restore(swmi_engine* engine, uint32_t lattice, const void* buffer, uint
         put(l.masks.ptr, 24ull * l.n_groups);
         put(l.rot.ptr, 4ull * l.n_groups);
         put(l.state.ptr, 4ull * l.state_words);
-        LaunchSetApplied(l.state.ptr, engine->stream);   // a checkpoint's spins hold the chain's state
+        LaunchSetApplied(l.state.ptr, engine->stream);   // a checkpoint's spins and states hold the chain's
+        LaunchSetRngCurrent(l.state.ptr, l.rng_it.ptr, engine->stream);
         Check(hipStreamSynchronize(engine->stream), "restore");
         l.cfg.seed = c.seed;
         l.cfg.flip_rule = c.flip_rule;

@@ -139,6 +139,7 @@ namespace swmi
         uint32_t state_words = 0;
         DeviceBuffer<uint8_t> spins;
         DeviceBuffer<uint32_t> rng;
+        DeviceBuffer<uint32_t> rng_it;
         DeviceBuffer<uint64_t> masks;
         DeviceBuffer<uint32_t> rot;
         DeviceBuffer<uint16_t> local;
@@ -234,6 +235,8 @@ struct swmi_engine
     // captured graphs when enabled.
     void Run(uint32_t n, uint32_t sep, int32_t sample_mode);
     void OneLattice(const swmi::Lattice& l, const uint8_t* bond_in);
+    // brings lattice l's stored lcg32 states to its current iteration
+    void AdvanceRng(const swmi::Lattice& l);
     // OneLattice, then applies lattice l's pending flip
     void MaterializeOne(const swmi::Lattice& l);
     uint64_t TotalSites() const;

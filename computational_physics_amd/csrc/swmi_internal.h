@@ -9,7 +9,9 @@
 //
 // HBM layout of one lattice (n = n0*n1 padded sites, n % 64 == 0, groups of 64 sites):
 //   spins    uint8[n]        bit 0: spin {0,1}; bits 3-5: the site's current lcg32 parameter selector
-//   rng      uint32[n]       per-site lcg32 state (lane i of group g = site 64g+i)
+//   rng      uint32[n]       per-site lcg32 state (lane i of group g = site 64g+i) of iteration *rng_it: between two
+//                            rotations a state is an affine function of the stored one, so a sweep computes it
+//                            and only the sweeps that rotate (two in 15) store states
 //   masks    uint64[3*n/64]  initial (a,c) selector of each lane as three bit planes (read-only)
 //   rot      uint32[n/64]    rotation offset of each group's (a,c) arrays (updated on rotating sweeps)
 //   local    uint16[n]       block label of each site: the block-local index q of its cluster's root, or for a
@@ -69,6 +71,7 @@ namespace swmi
     {
         uint8_t* spins;
         uint32_t* rng;
+        uint32_t* rng_it;        // iteration the states in rng belong to
         const uint64_t* masks;
         uint32_t* rot;
         uint16_t* local;
@@ -162,13 +165,17 @@ namespace swmi
                            hipStream_t stream);
     // a lattice's spin array was replaced: no flip is pending
     void LaunchSetApplied(uint32_t* state, hipStream_t stream);
+    // the rng array was replaced by the states of the lattice's current iteration
+    void LaunchSetRngCurrent(const uint32_t* state, uint32_t* rng_it, hipStream_t stream);
+    // brings the rng array of np sites to the lattice's current iteration
+    void LaunchAdvanceRng(const uint8_t* spins, uint32_t* rng, uint64_t np, const uint32_t* state, uint32_t* rng_it, hipStream_t stream);
     // allocation-free labelling: descriptor d into d_desc, fresh d.state
     void LaunchNoAllocSetup(const LatDesc& d, LatDesc* d_desc, hipStream_t stream);
     void LaunchObservables(const LatDesc* d_desc, const uint32_t* d_block_lat, uint32_t total_blocks, uint32_t sample_mode,
                            hipStream_t stream);
     void LaunchFinalizeSamples(const LatDesc* d_desc, uint32_t n_lattices, uint32_t sample_mode, hipStream_t stream);
-    void LaunchInitState(uint32_t* state, uint32_t words, uint32_t series_cap, uint32_t it_end, uint32_t it_meas, uint32_t sep2,
-                         hipStream_t stream);
+    void LaunchInitState(uint32_t* state, uint32_t* rng_it, uint32_t words, uint32_t series_cap, uint32_t it_end, uint32_t it_meas,
+                         uint32_t sep2, hipStream_t stream);
     void LaunchSetSchedule(uint32_t* state, uint32_t sweeps, uint32_t warmup, uint32_t n_sep, hipStream_t stream);
     void LaunchInitRng(uint8_t* spins, uint32_t* rng, uint64_t* masks, uint32_t* rot, uint32_t n_groups, uint32_t seed,
                        hipStream_t stream);

@@ -437,6 +437,11 @@ namespace swmi
             const uint32_t it = stp[kStIteration];
             stp[kStApplied] = it;
             stp[kStIteration] = it + 2u;
+            // a rotating sweep stored the states at which its lanes' pairs changed
+            if ((it + 1u) % 15u == 0u)
+                *Glob(d.rng_it) = it;
+            else if ((it + 2u) % 15u == 0u)
+                *Glob(d.rng_it) = it + 1u;
         }
     }
 
@@ -706,9 +711,12 @@ namespace swmi
     }
 
     // Fresh per-lattice state: counters and moments zero, no sweep limit unless it_end says otherwise.
-    __global__ __launch_bounds__(256) void k_init_state(uint32_t* __restrict__ state, const uint32_t words, const uint32_t series_cap,
-                                                        const uint32_t it_end, const uint32_t it_meas, const uint32_t sep2)
+    __global__ __launch_bounds__(256) void k_init_state(uint32_t* __restrict__ state, uint32_t* __restrict__ rng_it, const uint32_t words,
+                                                        const uint32_t series_cap, const uint32_t it_end, const uint32_t it_meas,
+                                                        const uint32_t sep2)
     {
+        if (threadIdx.x == 0)
+            *rng_it = 0u;
         for (uint32_t i = threadIdx.x; i < words; i += blockDim.x)
         {
             uint32_t v = 0;
@@ -724,6 +732,44 @@ namespace swmi
                 v = sep2;
             state[i] = v;
         }
+    }
+
+    __global__ void k_set_rng_current(const uint32_t* __restrict__ state, uint32_t* __restrict__ rng_it) { *rng_it = state[kStIteration]; }
+
+    // The states of the lattice's current iteration, for callers that read them (export, checkpoint): four sites per
+    // thread, the pair of each site's selector applied iteration - *rng_it times. k_set_rng_current follows it.
+    __global__ __launch_bounds__(256) void k_advance_rng(const uint32_t* __restrict__ spins4, u32x4* __restrict__ rng4, const uint64_t n4,
+                                                         const uint32_t* __restrict__ state, const uint32_t* __restrict__ rng_it)
+    {
+        __shared__ uint32_t JA[8], JC[8];
+        const uint32_t n = state[kStIteration] - *rng_it;
+        if (n == 0u)
+            return;
+        if (threadIdx.x < 8u)
+        {
+            uint32_t a, c, ja = 1u, jc = 0u;
+            ParamsOf(threadIdx.x, a, c);
+            for (uint32_t i = 0; i < n; ++i)
+            {
+                ja *= a;
+                jc = a * jc + c;
+            }
+            JA[threadIdx.x] = ja;
+            JC[threadIdx.x] = jc;
+        }
+        __syncthreads();
+        const uint64_t i = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+        if (i >= n4)
+            return;
+        const uint32_t sel = spins4[i] >> kSelShift;
+        u32x4 v = rng4[i];
+#pragma unroll
+        for (uint32_t e = 0; e < 4u; ++e)
+        {
+            const uint32_t k = (sel >> (8u * e)) & 7u;
+            v[e] = JA[k] * v[e] + JC[k];
+        }
+        rng4[i] = v;
     }
 
     // Schedule relative to the current iteration: `sweeps` more sweeps (0: no limit), the first `warmup` of
@@ -953,6 +999,19 @@ namespace swmi
 
     void LaunchSetApplied(uint32_t* state, hipStream_t stream) { k_set_applied_one<<<1, 1, 0, stream>>>(state); }
 
+    void LaunchSetRngCurrent(const uint32_t* state, uint32_t* rng_it, hipStream_t stream)
+    {
+        k_set_rng_current<<<1, 1, 0, stream>>>(state, rng_it);
+    }
+
+    void LaunchAdvanceRng(const uint8_t* spins, uint32_t* rng, const uint64_t np, const uint32_t* state, uint32_t* rng_it, hipStream_t stream)
+    {
+        const uint64_t n4 = np / 4;   // np is a multiple of 64
+        k_advance_rng<<<static_cast<uint32_t>((n4 + 255) / 256), 256, 0, stream>>>(reinterpret_cast<const uint32_t*>(spins),
+                                                                                   reinterpret_cast<u32x4*>(rng), n4, state, rng_it);
+        LaunchSetRngCurrent(state, rng_it, stream);
+    }
+
     void LaunchNoAllocSetup(const LatDesc& d, LatDesc* d_desc, hipStream_t stream)
     {
         static_assert(kLatStateWords <= 64, "one wave writes the counters");
@@ -970,10 +1029,10 @@ namespace swmi
         k_finalize_samples<<<n_lattices, 256, 0, stream>>>(d_desc, sample_mode);
     }
 
-    void LaunchInitState(uint32_t* state, const uint32_t words, const uint32_t series_cap, const uint32_t it_end, const uint32_t it_meas,
-                         const uint32_t sep2, hipStream_t stream)
+    void LaunchInitState(uint32_t* state, uint32_t* rng_it, const uint32_t words, const uint32_t series_cap, const uint32_t it_end,
+                         const uint32_t it_meas, const uint32_t sep2, hipStream_t stream)
     {
-        k_init_state<<<1, 256, 0, stream>>>(state, words, series_cap, it_end, it_meas, sep2);
+        k_init_state<<<1, 256, 0, stream>>>(state, rng_it, words, series_cap, it_end, it_meas, sep2);
     }
 
     void LaunchSetSchedule(uint32_t* state, const uint32_t sweeps, const uint32_t warmup, const uint32_t n_sep, hipStream_t stream)
