@@ -9,56 +9,6 @@ namespace swmi
     // =============================================================================================
     // k_bond_label
     // =============================================================================================
-    // Down bonds are deduplicated before any union: lanes l-1 and l lie in the same "overlap interval"
-    // when they share their row run above and their row run below (mask C); only the first down bond
-    // of every interval can join two different clusters. With M = C << 1 (continuation) and
-    // S1 = (D << 1) & M, the positions that follow an earlier bond of the same interval are
-    // S1 | (M & ((M + S1) ^ M)) (carries of S1 run through the ones of M).
-    __device__ __forceinline__ uint64_t FirstBondPerInterval(const uint64_t D, const uint64_t C, const uint64_t rowstart)
-    {
-        const uint64_t M = (C << 1) & ~rowstart;
-        const uint64_t S1 = (D << 1) & M;
-        const uint64_t later = S1 | (M & ((M + S1) ^ M));
-        return D & ~later;
-    }
-
-    // Union of the pairs (a, b) held by the lanes, all lanes in lockstep. Each step moves the ends that
-    // are not roots up (two parents, halving the path); when both are roots the larger is linked under the
-    // smaller with atomicMin, and a lost race continues with the value found (the loop of the reference
-    // Merge, swendsen_wang_amd_gpu.cpp:368-401). Lanes with nothing to do hold a == b; only lanes that
-    // link issue the atomic (idle lanes would all hit the same word). a and b are byte offsets into P.
-    __device__ __forceinline__ void LdsUnionLockstep(uint32_t* P, uint32_t a, uint32_t b)
-    {
-        while (__ballot(a != b))
-        {
-            // lanes that are done (a == b) only read P[a]; they follow no pointer and write nothing, so
-            // their a may name a node another wave has not written yet
-            const bool act = a != b;
-            const uint32_t pa = LdsLoad(At(P, a));
-            const uint32_t pb = LdsLoad(At(P, b));
-            const bool roots = (pa == a) && (pb == b);
-            const bool up = act && !roots;
-            const uint32_t lo = min(a, b), hi = max(a, b);
-            uint32_t old = hi;
-            if (act && roots)
-                old = __hip_atomic_fetch_min(At(P, hi), lo, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-            const bool linked = roots && old == hi;
-            // ends that are not roots move two steps up and point their node at the grandparent (path
-            // halving, monotone like every write to P)
-            const uint32_t ga = up ? LdsLoad(At(P, pa)) : 0u;
-            const uint32_t gb = up ? LdsLoad(At(P, pb)) : 0u;
-            if (up && ga != pa)
-                LdsMin(At(P, a), ga);
-            if (up && gb != pb)
-                LdsMin(At(P, b), gb);
-            if (act)
-            {
-                a = roots ? (linked ? hi : lo) : ga;
-                b = roots ? (linked ? hi : old) : gb;
-            }
-        }
-    }
-
     // Per wavefront (tile) the rows are processed top to bottom with the loads of the next kCh rows in
     // flight together. Bonds are computed on wave-uniform 64-bit masks: S (spin up), U1/U2 (draw below
     // threshold), B (bond to the right neighbour inside the tile), D (bond to the site below).
@@ -155,7 +105,7 @@ namespace swmi
         // carry no condition (in-range addresses, values unused where they do not apply), so that the compiler
         // neither fetches a field at its first use nor waits for every load at the end of a branch.
         HeldScalar(d.state);
-        HeldScalar(d.rng_it);
+        HeldScalar(d.aux);
         HeldScalar(d.fbits);
         HeldScalar(d.halo);
         HeldScalar(d.ecol_stride);
@@ -166,7 +116,7 @@ namespace swmi
         const uint32_t it0 = injected ? 0u : stp[kStIteration];
         const uint32_t it_end = injected ? 0u : stp[kStItEnd];
         const uint32_t applied = injected ? 0u : stp[kStApplied];
-        const uint32_t rng_it = injected ? 0u : *Glob(static_cast<const uint32_t*>(d.rng_it));
+        const uint32_t rng_it = injected ? 0u : Glob(static_cast<const uint32_t*>(d.aux))[kAuxRngIt];
         const uint32_t y_last = (bl.wyb + r_begin + (nrow > 0 ? nrow : 1u) - 1u) * rpw + lrow;
         const uint32_t y_below = nrow > 0 ? ((y_last + 1u == n1) ? 0u : y_last + 1u) : 0u;
         const uint32_t below = (r_begin + nrow) * bl.stride + lx;   // the site below the tile, inside the block
@@ -192,6 +142,8 @@ namespace swmi
         if (bl.lb == 0 && threadIdx.x == 0)
         {
             stp[kStActive] = act ? 1u : 0u;
+            if (act)
+                Glob(d.aux)[kAuxWholeLabels] = 0u;
             if (act && d.flip_rule != 0u)
                 stp[kStFlipKey] = FlipKey(d.seed, it0);   // an inactive lattice keeps the key of its pending flip
             if (act && !injected)
@@ -438,44 +390,10 @@ namespace swmi
                         const uint32_t row_b = wr * 256u;   // byte offset of the wave row in P
                         if (TW64)
                         {
-                            // slot of this lane's row run: the number of run starts after lane 0 up to this
-                            // lane; the first lane of the run initialises it with its own node
-                            uint32_t* const Mk = Qw + __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(~B >> 32),
-                                                                               __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(~B), 0u));
-                            const uint32_t self = row_b + lane4;
-                            __hip_atomic_store(LaneBit(~(B << 1)) ? Mk : dummy, self, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-                            // the row's entries start as roots (overwritten below), so chases end on them
-                            __hip_atomic_store(At(P, self), self, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
                             const uint64_t D = r == 0 ? 0ull : (injected ? prev_U2 : (~(prev_S ^ S) & prev_U2));
-                            if (r > 0)
-                                LdsMin(LaneBit(D) ? Mk : dummy, Rp);
-                            uint32_t root = LdsLoad(Mk);
-                            // bonds to a root other than the run's minimum link that root under it
-                            const uint64_t mg = D & __ballot(Rp != root);
-                            if (mg != 0ull)
-                            {
-                                const uint32_t old = __hip_atomic_fetch_min(LaneBit(mg) ? At(P, Rp) : dummy, root, __ATOMIC_RELAXED,
-                                                                            __HIP_MEMORY_SCOPE_WORKGROUP);
-                                // Rp was no longer a root (another lane linked it first): join the two trees
-                                const uint64_t more = mg & __ballot(old != Rp && old != root);
-                                if (more != 0ull)
-                                {
-                                    const bool mo = LaneBit(more);
-                                    LdsUnionLockstep(P, mo ? root : 0u, mo ? old : 0u);
-                                }
-                                // the run's minimum may itself have been linked under another root
-                                for (;;)
-                                {
-                                    const uint32_t pr = LdsLoad(At(P, root));
-                                    if (!__ballot(pr != root))
-                                        break;
-                                    root = pr;
-                                }
-                            }
                             if (dump && r > 0)
                                 dump[prev_site] = static_cast<uint8_t>((LaneBit(prev_Ball) ? 1u : 0u) | (LaneBit(D) ? 2u : 0u));
-                            *At(Pl, row_b) = root;
-                            Rp = root;
+                            Rp = LabelRow64(P, Qw, dummy, row_b + lane4, B, D, Rp, r > 0);
                         }
                         else
                         {

@@ -131,6 +131,102 @@ namespace swmi
         (void)__hip_atomic_fetch_min(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     }
 
+    // Down bonds are deduplicated before any union: lanes l-1 and l lie in the same "overlap interval"
+    // when they share their row run above and their row run below (mask C); only the first down bond
+    // of every interval can join two different clusters. With M = C << 1 (continuation) and
+    // S1 = (D << 1) & M, the positions that follow an earlier bond of the same interval are
+    // S1 | (M & ((M + S1) ^ M)) (carries of S1 run through the ones of M).
+    __device__ __forceinline__ uint64_t FirstBondPerInterval(const uint64_t D, const uint64_t C, const uint64_t rowstart)
+    {
+        const uint64_t M = (C << 1) & ~rowstart;
+        const uint64_t S1 = (D << 1) & M;
+        const uint64_t later = S1 | (M & ((M + S1) ^ M));
+        return D & ~later;
+    }
+
+    // Union of the pairs (a, b) held by the lanes, all lanes in lockstep. Each step moves the ends that
+    // are not roots up (two parents, halving the path); when both are roots the larger is linked under the
+    // smaller with atomicMin, and a lost race continues with the value found (the loop of the reference
+    // Merge, swendsen_wang_amd_gpu.cpp:368-401). Lanes with nothing to do hold a == b; only lanes that
+    // link issue the atomic (idle lanes would all hit the same word). a and b are byte offsets into P.
+    __device__ __forceinline__ void LdsUnionLockstep(uint32_t* P, uint32_t a, uint32_t b)
+    {
+        while (__ballot(a != b))
+        {
+            // lanes that are done (a == b) only read P[a]; they follow no pointer and write nothing, so
+            // their a may name a node another wave has not written yet
+            const bool act = a != b;
+            const uint32_t pa = LdsLoad(At(P, a));
+            const uint32_t pb = LdsLoad(At(P, b));
+            const bool roots = (pa == a) && (pb == b);
+            const bool up = act && !roots;
+            const uint32_t lo = min(a, b), hi = max(a, b);
+            uint32_t old = hi;
+            if (act && roots)
+                old = __hip_atomic_fetch_min(At(P, hi), lo, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+            const bool linked = roots && old == hi;
+            // ends that are not roots move two steps up and point their node at the grandparent (path
+            // halving, monotone like every write to P)
+            const uint32_t ga = up ? LdsLoad(At(P, pa)) : 0u;
+            const uint32_t gb = up ? LdsLoad(At(P, pb)) : 0u;
+            if (up && ga != pa)
+                LdsMin(At(P, a), ga);
+            if (up && gb != pb)
+                LdsMin(At(P, b), gb);
+            if (act)
+            {
+                a = roots ? (linked ? hi : lo) : ga;
+                b = roots ? (linked ? hi : old) : gb;
+            }
+        }
+    }
+
+    // One row of a 64-wide tile joins the union-find: B are its bonds to the right (inside the tile), D the bonds
+    // from the row above into it, Rp the root of this lane's site in the row above (resolved when that row was
+    // labelled), self this lane's node. A row run's label is the minimum of its first site and the roots its down
+    // bonds reach (one LDS atomicMin per bonded lane into the run's slot of M); a bond to any other root links that
+    // root under the minimum with one atomicMin, and only a link that loses a race goes through the lockstep union.
+    // Returns the root of this lane's site. M: 64 words of the wave; dummy: a word of the lane's own, the target of
+    // LDS operations the lane has no use for. below: some row above may be bonded (D may be non-zero).
+    __device__ __forceinline__ uint32_t LabelRow64(uint32_t* P, uint32_t* M, uint32_t* dummy, const uint32_t self, const uint64_t B,
+                                                   const uint64_t D, const uint32_t Rp, const bool below)
+    {
+        // slot of this lane's row run: the number of run starts after lane 0 up to this lane; the first lane of the
+        // run initialises it with its own node
+        uint32_t* const Mk = M + __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(~B >> 32),
+                                                           __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(~B), 0u));
+        __hip_atomic_store(LaneBit(~(B << 1)) ? Mk : dummy, self, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        // the row's entries start as roots (overwritten below), so chases end on them
+        __hip_atomic_store(At(P, self), self, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        if (below)
+            LdsMin(LaneBit(D) ? Mk : dummy, Rp);
+        uint32_t root = LdsLoad(Mk);
+        // bonds to a root other than the run's minimum link that root under it
+        const uint64_t mg = D & __ballot(Rp != root);
+        if (mg != 0ull)
+        {
+            const uint32_t old = __hip_atomic_fetch_min(LaneBit(mg) ? At(P, Rp) : dummy, root, __ATOMIC_RELAXED,
+                                                        __HIP_MEMORY_SCOPE_WORKGROUP);
+            // Rp was no longer a root (another lane linked it first): join the two trees
+            const uint64_t more = mg & __ballot(old != Rp && old != root);
+            if (more != 0ull)
+            {
+                const bool mo = LaneBit(more);
+                LdsUnionLockstep(P, mo ? root : 0u, mo ? old : 0u);
+            }
+            // the run's minimum may itself have been linked under another root
+            for (;;)
+            {
+                const uint32_t pr = LdsLoad(At(P, root));
+                if (!__ballot(pr != root))
+                    break;
+                root = pr;
+            }
+        }
+        *At(P, self) = root;
+        return root;
+    }
+
     // ---- union-find in HBM over the roots of edge-reaching clusters, one node per slot (every block numbers
     // its edge roots densely, so a block's nodes share a few cache lines). Entry of slot c: (key << 32) | parent
     // slot, where a root's key is its site index and a non-root holds its parent's key. Links are made with

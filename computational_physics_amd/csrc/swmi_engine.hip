@@ -35,6 +35,8 @@ namespace swmi
         // Captured measurement graphs hold groups of (n_sep sweeps + sample) up to about this many sweeps.
         constexpr uint32_t kGraphGroupSweeps = 64;
         constexpr size_t kMaxGraphs = 6;
+        // Sweeps of one k_resident launch (a few milliseconds at most).
+        constexpr uint32_t kResidentLaunchSweeps = 500;
     }
 
     void SetLastError(const std::string& m) { g_error = m; }
@@ -173,6 +175,19 @@ namespace swmi
         return g;
     }
 
+    // One workgroup of kResidentWaves waves takes a lattice whose sites fit its LDS union-find and whose rows, split
+    // into strips over the waves left per tile column, leave at most kResidentRows per strip. Every lattice it takes
+    // is faster there than tiled: 64^2 3 against 24 us per sweep, 128^2 9 against 24 (a 16-row strip is as long a
+    // chain as a 16-row tile, and the sweep has no launches, merge or resolve); a larger one would leave the other
+    // 255 CUs idle for longer.
+    uint32_t ResidentRows(const Geometry& g, const uint32_t n1)
+    {
+        if (static_cast<uint64_t>(g.pitch) * n1 > kResidentSites || g.tiles_x > kResidentWaves)
+            return 0;
+        const uint32_t strips = kResidentWaves / g.tiles_x, rows = (g.nwr_y + strips - 1u) / strips;
+        return rows <= kResidentRows ? rows : 0;
+    }
+
     LatDesc GeometryDesc(const Geometry& g, const uint32_t n0, const uint32_t n1)
     {
         LatDesc d{};
@@ -202,7 +217,7 @@ namespace swmi
         const Geometry g = GeometryOf(c.n0, c.n1, c.tile_rows);
         const uint64_t n = static_cast<uint64_t>(g.pitch) * c.n1, groups = n / 64;
         return n * (1 + 4 + 2) + groups * (3 * 8 + 4) + static_cast<uint64_t>(kBbitWords) * 8 * g.n_blocks +
-               4ull * (kLatStateWords + 4ull * c.max_samples) + 4 + 4ull * 2 * kWavesPerBlock * g.n_blocks +
+               4ull * (kLatStateWords + 4ull * c.max_samples) + 4 * kAuxWords + 4ull * 2 * kWavesPerBlock * g.n_blocks +
                static_cast<uint64_t>(kWavesPerBlock) * g.n_blocks * (8ull * g.edge_cap + 4) + 8ull * g.ecol_stride * g.n_blocks +
                4ull * 2 * 64 * g.n_blocks + 4ull * g.fsw * g.n_blocks + 2ull * g.halo_stride * g.n_blocks;
     }
@@ -215,7 +230,7 @@ namespace swmi
 
     uint64_t Lattice::Bytes() const
     {
-        return spins.bytes() + rng.bytes() + rng_it.bytes() + masks.bytes() + rot.bytes() + local.bytes() + parent.bytes() + cpar.bytes() +
+        return spins.bytes() + rng.bytes() + aux.bytes() + masks.bytes() + rot.bytes() + local.bytes() + parent.bytes() + cpar.bytes() +
                bbits.bytes() + state.bytes() + partials.bytes() + edge_count.bytes() + ecol.bytes() + erow.bytes() + fbits.bytes() +
                halo.bytes() + bond_dump.bytes() + bond_in.bytes();
     }
@@ -229,7 +244,7 @@ namespace swmi
         n_groups = static_cast<uint32_t>(np / 64);
         spins.allocate(np);
         rng.allocate(np);
-        rng_it.allocate(1);
+        aux.allocate(kAuxWords);
         masks.allocate(3ull * n_groups);
         rot.allocate(n_groups);
         local.allocate(np);
@@ -256,7 +271,7 @@ namespace swmi
         threshold = BondThreshold(p_add);
         bond_dump.reset();
         Check(hipMemsetAsync(edge_count.ptr, 0, edge_count.bytes(), stream), "edge list init");
-        LaunchInitState(state.ptr, rng_it.ptr, state_words, c.max_samples, 0xFFFFFFFFu, 0u, 0u, stream);
+        LaunchInitState(state.ptr, aux.ptr, state_words, c.max_samples, 0xFFFFFFFFu, 0u, 0u, stream);
         if (np != n)   // padding columns hold spin 0
             Check(hipMemsetAsync(spins.ptr, 0, np, stream), "spin init");
         LaunchHotStart(spins.ptr, n, c.spin_seed, cfg.n0, g.pitch, stream);
@@ -297,9 +312,9 @@ swmi_engine::~swmi_engine()
 
 void swmi_engine::EnsureSideStreams()
 {
-    if (!fork_event && classes.size() > 1)
+    if (!fork_event && SideStreams() > 0)
         Check(hipEventCreateWithFlags(&fork_event, hipEventDisableTiming), "event create");
-    while (side_streams.size() + 1 < classes.size())
+    while (side_streams.size() < SideStreams())
     {
         hipStream_t s = nullptr;
         Check(hipStreamCreateWithFlags(&s, hipStreamNonBlocking), "hipStreamCreate");
@@ -331,7 +346,7 @@ LatDesc swmi_engine::Desc(const Lattice& l, uint32_t block_base) const
     LatDesc d = GeometryDesc(l.g, l.cfg.n0, l.cfg.n1);
     d.spins = l.spins.ptr;
     d.rng = l.rng.ptr;
-    d.rng_it = l.rng_it.ptr;
+    d.aux = l.aux.ptr;
     d.masks = l.masks.ptr;
     d.rot = l.rot.ptr;
     d.local = l.local.ptr;
@@ -368,7 +383,9 @@ void swmi_engine::Rebuild()
     DropGraphs();
     // slots are compacted: the descriptor array has no holes
     lattices.erase(std::remove(lattices.begin(), lattices.end(), nullptr), lattices.end());
-    // class of a lattice: (64-wide tiles, k_bond_label tile-height bound)
+    // class of a lattice: (64-wide tiles, padding, k_bond_label tile-height bound), or for a lattice that one
+    // workgroup sweeps (tile_rows 0: the caller asks for no tiles of its own) the k_resident build it needs. While
+    // bonds are recorded every lattice is tiled: only k_bond_label records them.
     std::vector<KernelClass> next;
     std::vector<LatDesc> d(lattices.size());
     for (uint32_t i = 0; i < lattices.size(); ++i)
@@ -378,8 +395,12 @@ void swmi_engine::Rebuild()
         const bool pad = l.np != l.n;
         // padded lattices have two tile-height classes (16 and 64)
         const uint32_t t = pad ? (l.g.twr <= 16 ? 16u : 64u) : TwrClass(l.g.twr);
-        auto it = std::find_if(next.begin(), next.end(),
-                               [&](const KernelClass& k) { return k.tw64 == tw64 && k.pad == pad && k.twr_t == t; });
+        const uint32_t rows = recording || l.cfg.tile_rows != 0u ? 0u : ResidentRows(l.g, l.cfg.n1);
+        const bool resident = rows != 0u;
+        const auto same = [&](const KernelClass& k) {
+            return k.tw64 == tw64 && k.pad == pad && k.twr_t == t && k.resident == resident && (!resident || (k.max_rows <= 4u) == (rows <= 4u));
+        };
+        auto it = std::find_if(next.begin(), next.end(), same);
         if (it == next.end())
         {
             next.emplace_back();
@@ -387,16 +408,32 @@ void swmi_engine::Rebuild()
             it->tw64 = tw64;
             it->pad = pad;
             it->twr_t = t;
+            it->resident = resident;
         }
+        it->max_rows = std::max(it->max_rows, rows);
+        it->max_sites = std::max(it->max_sites, static_cast<uint32_t>(l.np));
+        it->slots.push_back(i);
         d[i] = Desc(l, static_cast<uint32_t>(it->block_lat.size()));
         if (it->n_lat++ == 0)
             it->first_slot = i;
         it->block_lat.insert(it->block_lat.end(), l.g.n_blocks, i);
         it->max_twr = std::max(it->max_twr, l.g.twr);
     }
+    n_tiled = static_cast<size_t>(std::stable_partition(next.begin(), next.end(), [](const KernelClass& k) { return !k.resident; }) -
+                                  next.begin());
     // reuse the device work-list buffers of the previous classes where the sizes allow
     for (auto& k : next)
     {
+        const auto slots_of = std::find_if(classes.begin(), classes.end(), [&](KernelClass& o) {
+            return o.d_slots.ptr && o.d_slots.count >= k.slots.size();
+        });
+        if (slots_of != classes.end())
+        {
+            std::swap(k.d_slots.ptr, slots_of->d_slots.ptr);
+            std::swap(k.d_slots.count, slots_of->d_slots.count);
+        }
+        else
+            k.d_slots.allocate(k.slots.size());
         k.total_blocks = static_cast<uint32_t>(k.block_lat.size());
         auto old = std::find_if(classes.begin(), classes.end(), [&](KernelClass& o) {
             return o.d_block_lat.ptr && o.d_block_lat.count >= k.block_lat.size();
@@ -417,9 +454,13 @@ void swmi_engine::Rebuild()
         Check(hipMemcpyAsync(d_desc.ptr, descs.data(), descs.size() * sizeof(LatDesc), hipMemcpyHostToDevice, stream),
               "descriptor upload");
     for (auto& k : classes)
+    {
         Check(hipMemcpyAsync(k.d_block_lat.ptr, k.block_lat.data(), k.block_lat.size() * sizeof(uint32_t), hipMemcpyHostToDevice,
                              stream),
               "work list upload");
+        Check(hipMemcpyAsync(k.d_slots.ptr, k.slots.data(), k.slots.size() * sizeof(uint32_t), hipMemcpyHostToDevice, stream),
+              "lattice list upload");
+    }
     EnsureSideStreams();
 }
 
@@ -427,16 +468,10 @@ void swmi_engine::LaunchCheck(const char* what) { Check(hipGetLastError(), what)
 
 void swmi_engine::EnqueueSweeps(uint32_t n)
 {
-    if (n == 0 || classes.empty())
+    if (n == 0 || n_tiled == 0)
         return;
-    const size_t nc = classes.size();
-    if (nc > 1)
-    {
-        Check(hipEventRecord(fork_event, stream), "fork");
-        for (size_t c = 1; c < nc; ++c)
-            Check(hipStreamWaitEvent(side_streams[c - 1], fork_event, 0), "fork");
-    }
-    for (size_t c = 0; c < nc; ++c)
+    Fork(0, n_tiled - 1);
+    for (size_t c = 0; c < n_tiled; ++c)
     {
         const KernelClass& k = classes[c];
         hipStream_t s = ClassStream(c);
@@ -447,29 +482,77 @@ void swmi_engine::EnqueueSweeps(uint32_t n)
             LaunchResolve(k.Descs(d_desc.ptr), k.WorkList(), k.total_blocks, s);
         }
     }
-    for (size_t c = 1; c < nc; ++c)
-    {
-        Check(hipEventRecord(join_events[c - 1], side_streams[c - 1]), "join");
-        Check(hipStreamWaitEvent(stream, join_events[c - 1], 0), "join");
-    }
+    Join(0, n_tiled - 1);
     LaunchCheck("sweep launch");
 }
 
-void swmi_engine::EnqueueMaterialize()
+void swmi_engine::Fork(const size_t first, const size_t last)
 {
-    for (auto& k : classes)
-        LaunchMaterialize(k.Descs(d_desc.ptr), k.WorkList(), k.total_blocks, stream);
-    LaunchCheck("flip launch");
+    if (first >= last)
+        return;
+    Check(hipEventRecord(fork_event, stream), "fork");
+    for (size_t c = first; c < last; ++c)
+        Check(hipStreamWaitEvent(side_streams[c], fork_event, 0), "fork");
+}
+
+void swmi_engine::Join(const size_t first, const size_t last)
+{
+    for (size_t c = first; c < last; ++c)
+    {
+        Check(hipEventRecord(join_events[c], side_streams[c]), "join");
+        Check(hipStreamWaitEvent(stream, join_events[c], 0), "join");
+    }
+}
+
+void swmi_engine::JoinResident()
+{
+    if (n_tiled > 0 && n_tiled < classes.size())
+        Join(n_tiled - 1, SideStreams());
+}
+
+void swmi_engine::EnqueueResident(const uint32_t sweeps, const uint32_t groups, const int32_t sample_mode)
+{
+    if (n_tiled == classes.size())
+        return;
+    const size_t side = n_tiled == 0 ? 0 : n_tiled - 1;
+    Fork(side, SideStreams());
+    for (size_t c = n_tiled; c < classes.size(); ++c)
+    {
+        const KernelClass& k = classes[c];
+        const auto launch = [&](uint32_t per_group, uint32_t n_groups, int32_t mode) {
+            LaunchResident(d_desc.ptr, k.d_slots.ptr, k.n_lat, k.max_sites, k.max_rows, k.tw64, k.pad, per_group, n_groups, mode,
+                           ClassStream(n_tiled));
+        };
+        if (sample_mode < 0 || sweeps > kResidentLaunchSweeps)
+        {
+            // plain sweeps, or long groups: launches of bounded length, the sample in the group's last one
+            for (uint32_t g = 0; g < groups; ++g)
+                for (uint32_t left = sweeps;;)
+                {
+                    const uint32_t now = std::min(left, kResidentLaunchSweeps);
+                    left -= now;
+                    launch(now, 1u, left == 0u ? sample_mode : -1);
+                    if (left == 0u)
+                        break;
+                }
+            continue;
+        }
+        const uint32_t per = std::max(1u, kResidentLaunchSweeps / std::max(1u, sweeps));
+        for (uint32_t g = 0; g < groups; g += per)
+            launch(sweeps, std::min(per, groups - g), sample_mode);
+    }
+    LaunchCheck("resident sweep launch");
 }
 
 void swmi_engine::EnqueueSample(uint32_t mode)
 {
-    if (descs.empty())
-        return;
-    EnqueueMaterialize();
-    for (auto& k : classes)
+    for (size_t c = 0; c < n_tiled; ++c)
+    {
+        const KernelClass& k = classes[c];
+        LaunchMaterialize(k.Descs(d_desc.ptr), k.WorkList(), k.total_blocks, stream);
         LaunchObservables(k.Descs(d_desc.ptr), k.WorkList(), k.total_blocks, mode, stream);
-    LaunchFinalizeSamples(d_desc.ptr, static_cast<uint32_t>(descs.size()), mode, stream);
+        LaunchFinalizeSamples(d_desc.ptr, k.d_slots.ptr, k.n_lat, mode, stream);
+    }
     LaunchCheck("sample launch");
 }
 
@@ -477,13 +560,26 @@ void swmi_engine::Run(uint32_t n, uint32_t sep, int32_t sample_mode)
 {
     if (classes.empty() || n == 0)
         return;
+    // the resident classes beside the tiled ones
+    if (sample_mode >= 0)
+        EnqueueResident(sep, (n + sep - 1) / sep, sample_mode);   // ising_2d.cpp:132: i += N_Sep while i < n
+    else
+        EnqueueResident(n, 1, -1);
+    RunTiled(n, sep, sample_mode);
+    JoinResident();
+}
+
+void swmi_engine::RunTiled(uint32_t n, uint32_t sep, int32_t sample_mode)
+{
+    if (n_tiled == 0 || n == 0)
+        return;
     const bool sampled = sample_mode >= 0;
     if (sampled && sep > kGraphGroupSweeps)
     {
         // long groups: graphs of plain sweeps, eager samples
         for (uint32_t i = 0; i < n; i += sep)
         {
-            Run(sep, 0, -1);
+            RunTiled(sep, 0, -1);
             EnqueueSample(static_cast<uint32_t>(sample_mode));
         }
         return;
@@ -547,7 +643,7 @@ void swmi_engine::Run(uint32_t n, uint32_t sep, int32_t sample_mode)
         if (sampled)
             enqueue_unit(total_groups - replays * groups);
         else
-            Run(n - replays * unit, 0, -1);   // short graphs or eager sweeps
+            RunTiled(n - replays * unit, 0, -1);   // short graphs or eager sweeps
         return;
     }
     enqueue_unit(sampled ? total_groups : n);
@@ -566,7 +662,7 @@ void swmi_engine::OneLattice(const Lattice& l, const uint8_t* bond_in)
 
 void swmi_engine::AdvanceRng(const Lattice& l)
 {
-    LaunchAdvanceRng(l.spins.ptr, l.rng.ptr, l.np, l.state.ptr, l.rng_it.ptr, stream);
+    LaunchAdvanceRng(l.spins.ptr, l.rng.ptr, l.np, l.state.ptr, l.aux.ptr, stream);
     LaunchCheck("rng launch");
 }
 
@@ -784,7 +880,11 @@ int swmi_sweep(swmi_engine* engine, uint32_t n_sweeps)
 
 int swmi_sample(swmi_engine* engine)
 {
-    return Guard([&] { Eng(engine)->EnqueueSample(kSampleAlways); });
+    return Guard([&] {
+        Eng(engine)->EnqueueResident(0, 1, kSampleAlways);
+        engine->EnqueueSample(kSampleAlways);
+        engine->JoinResident();
+    });
 }
 
 int swmi_run(swmi_engine* engine, uint32_t n_sweeps, uint32_t n_sep)
@@ -1127,7 +1227,7 @@ int swmi_restore(swmi_engine* engine, uint32_t lattice, const void* buffer, uint
         put(l.rot.ptr, 4ull * l.n_groups);
         put(l.state.ptr, 4ull * l.state_words);
         LaunchSetApplied(l.state.ptr, engine->stream);   // a checkpoint's spins and states hold the chain's
-        LaunchSetRngCurrent(l.state.ptr, l.rng_it.ptr, engine->stream);
+        LaunchSetRngCurrent(l.state.ptr, l.aux.ptr, engine->stream);
         Check(hipStreamSynchronize(engine->stream), "restore");
         l.cfg.seed = c.seed;
         l.cfg.flip_rule = c.flip_rule;

@@ -124,6 +124,8 @@ namespace swmi
     // Tile height for tile_rows == 0: the autotuned value for this extent if one was measured in this
     // process, else 16 wave rows.
     uint32_t DefaultTileRows(uint32_t n0, uint32_t n1);
+    // Rows of the strips in which k_resident sweeps a lattice of this geometry: 0 if it does not take it.
+    uint32_t ResidentRows(const Geometry& g, uint32_t n1);
     // k_bond_label specialisation bound for a tile height: 8, 16, 32 or 64.
     uint32_t TwrClass(uint32_t twr);
 
@@ -139,7 +141,7 @@ namespace swmi
         uint32_t state_words = 0;
         DeviceBuffer<uint8_t> spins;
         DeviceBuffer<uint32_t> rng;
-        DeviceBuffer<uint32_t> rng_it;
+        DeviceBuffer<uint32_t> aux;
         DeviceBuffer<uint64_t> masks;
         DeviceBuffer<uint32_t> rot;
         DeviceBuffer<uint16_t> local;
@@ -175,6 +177,10 @@ namespace swmi
         std::vector<uint32_t> block_lat;     // block -> lattice slot
         DeviceBuffer<uint32_t> d_block_lat;
         uint32_t total_blocks = 0;
+        bool resident = false;               // small lattices that k_resident sweeps, one workgroup each
+        uint32_t max_sites = 0, max_rows = 0;   // resident: bounds on the padded sites and the rows of a strip
+        std::vector<uint32_t> slots;         // descriptor slots of the class's lattices
+        DeviceBuffer<uint32_t> d_slots;
         uint32_t n_lat = 0;                  // lattices in the class
         uint32_t first_slot = 0;             // descriptor slot of the class's first lattice
         // The kernels' arguments for this class: a class of one lattice passes that lattice's descriptor and a
@@ -199,12 +205,14 @@ struct swmi_engine
     std::vector<std::unique_ptr<swmi::Lattice>> lattices;
     std::vector<swmi::LatDesc> descs;
     swmi::DeviceBuffer<swmi::LatDesc> d_desc;
-    std::vector<swmi::KernelClass> classes;
+    std::vector<swmi::KernelClass> classes;   // the tiled ones first
+    size_t n_tiled = 0;                       // classes the tiled kernels sweep; the rest are resident
     bool recording = false;   // some lattice records its bonds (selects the inspection build of k_bond_label)
     bool use_graphs = true;
     std::vector<swmi::GraphEntry> graphs;   // valid for the current work lists only
-    // kernel classes are independent: class c > 0 runs on side stream c - 1, forked from and joined
-    // back into the engine stream around every sweep loop (parallel branches in a captured graph)
+    // kernel classes are independent: tiled class c > 0 runs on side stream c - 1, forked from and joined
+    // back into the engine stream around every sweep loop (parallel branches in a captured graph); the resident
+    // classes share one more side stream (the engine stream where no class is tiled)
     std::vector<hipStream_t> side_streams;
     std::vector<hipEvent_t> join_events;
     hipEvent_t fork_event = nullptr;
@@ -224,13 +232,27 @@ struct swmi_engine
     void Rebuild();
     void DropGraphs();
     void LaunchCheck(const char* what);
+    // n sweeps of the tiled classes
     void EnqueueSweeps(uint32_t n);
-    // applies the pending flip of every lattice (engine stream), so that their spin arrays hold the chains
-    void EnqueueMaterialize();
+    // a sample of the lattices of the tiled classes
     void EnqueueSample(uint32_t mode);
+    // `groups` groups of `sweeps` sweeps of the resident classes, a sample after each group when sample_mode >= 0, forked
+    // from the engine stream; JoinResident joins them back
+    void EnqueueResident(uint32_t sweeps, uint32_t groups, int32_t sample_mode);
+    void JoinResident();
+    // Run for the tiled classes
+    void RunTiled(uint32_t n, uint32_t sep, int32_t sample_mode);
+    // work on side streams [first, last) starts after what the engine stream holds now, and the engine stream goes on
+    // after it
+    void Fork(size_t first, size_t last);
+    void Join(size_t first, size_t last);
     // side streams and events for every class beyond the first
     void EnsureSideStreams();
     hipStream_t ClassStream(size_t c) const { return c == 0 ? stream : side_streams[c - 1]; }
+    size_t SideStreams() const
+    {
+        return n_tiled == 0 ? 0 : n_tiled - (classes.size() > n_tiled ? 0 : 1);
+    }
     // n sweeps (with a sample of `sample_mode` after every `sep` sweeps when sample_mode >= 0), through
     // captured graphs when enabled.
     void Run(uint32_t n, uint32_t sep, int32_t sample_mode);

@@ -9,7 +9,7 @@
 //
 // HBM layout of one lattice (n = n0*n1 padded sites, n % 64 == 0, groups of 64 sites):
 //   spins    uint8[n]        bit 0: spin {0,1}; bits 3-5: the site's current lcg32 parameter selector
-//   rng      uint32[n]       per-site lcg32 state (lane i of group g = site 64g+i) of iteration *rng_it: between two
+//   rng      uint32[n]       per-site lcg32 state (lane i of group g = site 64g+i) of iteration aux[kAuxRngIt]: between two
 //                            rotations a state is an affine function of the stored one, so a sweep computes it
 //                            and only the sweeps that rotate (two in 15) store states
 //   masks    uint64[3*n/64]  initial (a,c) selector of each lane as three bit planes (read-only)
@@ -60,6 +60,9 @@ namespace swmi
 {
     constexpr uint32_t kWave = 64;
     constexpr uint32_t kWavesPerBlock = 4;   // tiles per block (workgroup)
+    constexpr uint32_t kResidentSites = 16384;  // largest (padded) lattice that one workgroup sweeps alone (k_resident)
+    constexpr uint32_t kResidentWaves = 16;     // its waves, each with a strip of at most kResidentRows rows
+    constexpr uint32_t kResidentRows = 16;
     constexpr uint32_t kNumXcd = 8;          // MI355X: 8 XCDs, workgroups dispatched round-robin
     constexpr uint16_t kEdgeFlag = 0x8000u;  // cluster reaches the block edge
     constexpr uint32_t kRightWords = kWavesPerBlock;
@@ -71,7 +74,7 @@ namespace swmi
     {
         uint8_t* spins;
         uint32_t* rng;
-        uint32_t* rng_it;        // iteration the states in rng belong to
+        uint32_t* aux;           // counters beside the state that no checkpoint holds: kAuxRngIt, kAuxWholeLabels
         const uint64_t* masks;
         uint32_t* rot;
         uint16_t* local;
@@ -139,6 +142,10 @@ namespace swmi
                        kStMoments = 12;
     static_assert(offsetof(LatState, moments) == 4 * kStMoments, "LatState layout");
 
+    constexpr uint32_t kAuxRngIt = 0;        // iteration the states in rng belong to
+    constexpr uint32_t kAuxWholeLabels = 1;  // 1: local holds every site's canonical site (k_resident), 0: block labels
+    constexpr uint32_t kAuxWords = 2;
+
     enum SampleMode : uint32_t
     {
         kSampleAlways = 0u,  // every lattice, now
@@ -156,6 +163,11 @@ namespace swmi
     void LaunchBondLabel(const LatDesc* d_desc, const uint32_t* d_block_lat, uint32_t total_blocks, uint32_t max_twr,
                          bool all_tw64, bool pad, bool debug, hipStream_t stream);
     void LaunchMerge(const LatDesc* d_desc, const uint32_t* d_block_lat, uint32_t total_blocks, hipStream_t stream);
+    // n_lattices small lattices (descriptors d_slots[i]), one workgroup each: `groups` groups of `sweeps` sweeps with a
+    // sample after each group when sample_mode >= 0. max_sites, max_rows: bounds on their padded sites and on the
+    // rows of a strip (ResidentRows).
+    void LaunchResident(const LatDesc* d_desc, const uint32_t* d_slots, uint32_t n_lattices, uint32_t max_sites, uint32_t max_rows,
+                        bool tw64, bool pad, uint32_t sweeps, uint32_t groups, int32_t sample_mode, hipStream_t stream);
     // end of a sweep: flip bits and halos of every block, then iteration += 2
     void LaunchResolve(const LatDesc* d_desc, const uint32_t* d_block_lat, uint32_t total_blocks, hipStream_t stream);
     // apply a pending flip to the spin array (no-op for lattices without one)
@@ -166,15 +178,17 @@ namespace swmi
     // a lattice's spin array was replaced: no flip is pending
     void LaunchSetApplied(uint32_t* state, hipStream_t stream);
     // the rng array was replaced by the states of the lattice's current iteration
-    void LaunchSetRngCurrent(const uint32_t* state, uint32_t* rng_it, hipStream_t stream);
+    void LaunchSetRngCurrent(const uint32_t* state, uint32_t* aux, hipStream_t stream);
     // brings the rng array of np sites to the lattice's current iteration
-    void LaunchAdvanceRng(const uint8_t* spins, uint32_t* rng, uint64_t np, const uint32_t* state, uint32_t* rng_it, hipStream_t stream);
+    void LaunchAdvanceRng(const uint8_t* spins, uint32_t* rng, uint64_t np, const uint32_t* state, uint32_t* aux, hipStream_t stream);
     // allocation-free labelling: descriptor d into d_desc, fresh d.state
     void LaunchNoAllocSetup(const LatDesc& d, LatDesc* d_desc, hipStream_t stream);
     void LaunchObservables(const LatDesc* d_desc, const uint32_t* d_block_lat, uint32_t total_blocks, uint32_t sample_mode,
                            hipStream_t stream);
-    void LaunchFinalizeSamples(const LatDesc* d_desc, uint32_t n_lattices, uint32_t sample_mode, hipStream_t stream);
-    void LaunchInitState(uint32_t* state, uint32_t* rng_it, uint32_t words, uint32_t series_cap, uint32_t it_end, uint32_t it_meas,
+    // lattices d_slots[0 .. n_lattices)
+    void LaunchFinalizeSamples(const LatDesc* d_desc, const uint32_t* d_slots, uint32_t n_lattices, uint32_t sample_mode,
+                               hipStream_t stream);
+    void LaunchInitState(uint32_t* state, uint32_t* aux, uint32_t words, uint32_t series_cap, uint32_t it_end, uint32_t it_meas,
                          uint32_t sep2, hipStream_t stream);
     void LaunchSetSchedule(uint32_t* state, uint32_t sweeps, uint32_t warmup, uint32_t n_sep, hipStream_t stream);
     void LaunchInitRng(uint8_t* spins, uint32_t* rng, uint64_t* masks, uint32_t* rot, uint32_t n_groups, uint32_t seed,

@@ -439,9 +439,9 @@ namespace swmi
             stp[kStIteration] = it + 2u;
             // a rotating sweep stored the states at which its lanes' pairs changed
             if ((it + 1u) % 15u == 0u)
-                *Glob(d.rng_it) = it;
+                Glob(d.aux)[kAuxRngIt] = it;
             else if ((it + 2u) % 15u == 0u)
-                *Glob(d.rng_it) = it + 1u;
+                Glob(d.aux)[kAuxRngIt] = it + 1u;
         }
     }
 
@@ -562,6 +562,7 @@ namespace swmi
         const uint32_t sub = threadIdx.x >> 4;
         const uint32_t col = (threadIdx.x & 15u) * 4u;
         bool ok = true;
+        const bool whole = Glob(static_cast<const uint32_t*>(d.aux))[kAuxWholeLabels] != 0u;
 
         u32x2 lv[kCh];
         const auto load = [&](const uint32_t r0) {
@@ -579,7 +580,8 @@ namespace swmi
         // phase 1: canonical root of every slot in use
         const gptr<uint64_t> E = Glob(d.cpar);
         const uint32_t c_max = d.n_blocks * slots;
-        ForBlockSlots(d, bl, threadIdx.x, 256u, [&](const uint32_t slot, const uint32_t c) { R[slot] = SlotRootKey(E, c, CachedLoad64(&E[c]), c_max, ok); });
+        if (!whole)
+            ForBlockSlots(d, bl, threadIdx.x, 256u, [&](const uint32_t slot, const uint32_t c) { R[slot] = SlotRootKey(E, c, CachedLoad64(&E[c]), c_max, ok); });
         __syncthreads();
 
         // phase 2: every site's label, four sites per lane
@@ -597,6 +599,11 @@ namespace swmi
 #pragma unroll
                     for (uint32_t e = 0; e < 4; ++e)
                     {
+                        if (whole)   // the label is the canonical site already
+                        {
+                            root[e] = lab[e];
+                            continue;
+                        }
                         const uint32_t i = LabelBit(lab[e], qmax, qcap, slots, ok);
                         root[e] = (lab[e] & kEdgeFlag) ? R[i >= qcap ? i - qcap : 0u] : SiteOf(bl.base, bl.stride, i);
                     }
@@ -663,10 +670,11 @@ namespace swmi
 
     // One workgroup per lattice: reduce the tile partials in a fixed order, append (E, M) to the series
     // and accumulate the FP64 moments (the only FP64 on the device).
-    __global__ __launch_bounds__(256) void k_finalize_samples(const LatDesc* __restrict__ descs, const uint32_t sample_mode)
+    __global__ __launch_bounds__(256) void k_finalize_samples(const LatDesc* __restrict__ descs, const uint32_t* __restrict__ slots,
+                                                              const uint32_t sample_mode)
     {
         __shared__ long long red_e[256], red_m[256];
-        const LatDesc& d = descs[blockIdx.x];
+        const LatDesc& d = descs[slots[blockIdx.x]];
         if (sample_mode == kSampleDue && !SampleDue(d.state))
             return;
         long long e = 0, m = 0;
@@ -711,12 +719,12 @@ namespace swmi
     }
 
     // Fresh per-lattice state: counters and moments zero, no sweep limit unless it_end says otherwise.
-    __global__ __launch_bounds__(256) void k_init_state(uint32_t* __restrict__ state, uint32_t* __restrict__ rng_it, const uint32_t words,
+    __global__ __launch_bounds__(256) void k_init_state(uint32_t* __restrict__ state, uint32_t* __restrict__ aux, const uint32_t words,
                                                         const uint32_t series_cap, const uint32_t it_end, const uint32_t it_meas,
                                                         const uint32_t sep2)
     {
-        if (threadIdx.x == 0)
-            *rng_it = 0u;
+        if (threadIdx.x < kAuxWords)
+            aux[threadIdx.x] = 0u;
         for (uint32_t i = threadIdx.x; i < words; i += blockDim.x)
         {
             uint32_t v = 0;
@@ -734,15 +742,15 @@ namespace swmi
         }
     }
 
-    __global__ void k_set_rng_current(const uint32_t* __restrict__ state, uint32_t* __restrict__ rng_it) { *rng_it = state[kStIteration]; }
+    __global__ void k_set_rng_current(const uint32_t* __restrict__ state, uint32_t* __restrict__ aux) { aux[kAuxRngIt] = state[kStIteration]; }
 
     // The states of the lattice's current iteration, for callers that read them (export, checkpoint): four sites per
-    // thread, the pair of each site's selector applied iteration - *rng_it times. k_set_rng_current follows it.
+    // thread, the pair of each site's selector applied once per update since. k_set_rng_current follows it.
     __global__ __launch_bounds__(256) void k_advance_rng(const uint32_t* __restrict__ spins4, u32x4* __restrict__ rng4, const uint64_t n4,
-                                                         const uint32_t* __restrict__ state, const uint32_t* __restrict__ rng_it)
+                                                         const uint32_t* __restrict__ state, const uint32_t* __restrict__ aux)
     {
         __shared__ uint32_t JA[8], JC[8];
-        const uint32_t n = state[kStIteration] - *rng_it;
+        const uint32_t n = state[kStIteration] - aux[kAuxRngIt];
         if (n == 0u)
             return;
         if (threadIdx.x < 8u)
@@ -999,17 +1007,17 @@ namespace swmi
 
     void LaunchSetApplied(uint32_t* state, hipStream_t stream) { k_set_applied_one<<<1, 1, 0, stream>>>(state); }
 
-    void LaunchSetRngCurrent(const uint32_t* state, uint32_t* rng_it, hipStream_t stream)
+    void LaunchSetRngCurrent(const uint32_t* state, uint32_t* aux, hipStream_t stream)
     {
-        k_set_rng_current<<<1, 1, 0, stream>>>(state, rng_it);
+        k_set_rng_current<<<1, 1, 0, stream>>>(state, aux);
     }
 
-    void LaunchAdvanceRng(const uint8_t* spins, uint32_t* rng, const uint64_t np, const uint32_t* state, uint32_t* rng_it, hipStream_t stream)
+    void LaunchAdvanceRng(const uint8_t* spins, uint32_t* rng, const uint64_t np, const uint32_t* state, uint32_t* aux, hipStream_t stream)
     {
         const uint64_t n4 = np / 4;   // np is a multiple of 64
         k_advance_rng<<<static_cast<uint32_t>((n4 + 255) / 256), 256, 0, stream>>>(reinterpret_cast<const uint32_t*>(spins),
-                                                                                   reinterpret_cast<u32x4*>(rng), n4, state, rng_it);
-        LaunchSetRngCurrent(state, rng_it, stream);
+                                                                                   reinterpret_cast<u32x4*>(rng), n4, state, aux);
+        LaunchSetRngCurrent(state, aux, stream);
     }
 
     void LaunchNoAllocSetup(const LatDesc& d, LatDesc* d_desc, hipStream_t stream)
@@ -1024,15 +1032,16 @@ namespace swmi
         k_observables<<<XcdGrid(total_blocks), 256, 0, stream>>>(d_desc, d_block_lat, total_blocks, sample_mode);
     }
 
-    void LaunchFinalizeSamples(const LatDesc* d_desc, const uint32_t n_lattices, const uint32_t sample_mode, hipStream_t stream)
+    void LaunchFinalizeSamples(const LatDesc* d_desc, const uint32_t* d_slots, const uint32_t n_lattices, const uint32_t sample_mode,
+                               hipStream_t stream)
     {
-        k_finalize_samples<<<n_lattices, 256, 0, stream>>>(d_desc, sample_mode);
+        k_finalize_samples<<<n_lattices, 256, 0, stream>>>(d_desc, d_slots, sample_mode);
     }
 
-    void LaunchInitState(uint32_t* state, uint32_t* rng_it, const uint32_t words, const uint32_t series_cap, const uint32_t it_end,
+    void LaunchInitState(uint32_t* state, uint32_t* aux, const uint32_t words, const uint32_t series_cap, const uint32_t it_end,
                          const uint32_t it_meas, const uint32_t sep2, hipStream_t stream)
     {
-        k_init_state<<<1, 256, 0, stream>>>(state, rng_it, words, series_cap, it_end, it_meas, sep2);
+        k_init_state<<<1, 256, 0, stream>>>(state, aux, words, series_cap, it_end, it_meas, sep2);
     }
 
     void LaunchSetSchedule(uint32_t* state, const uint32_t sweeps, const uint32_t warmup, const uint32_t n_sep, hipStream_t stream)

@@ -83,7 +83,8 @@ namespace swmi
             const uint64_t n = static_cast<uint64_t>(g.pitch) * n1;   // padded sites
             const bool pad = g.pitch != n0;
             *d_desc = c.Take<LatDesc>(1);
-            d.state = c.Take<uint32_t>(kLatStateWords);
+            d.state = c.Take<uint32_t>(kLatStateWords + kAuxWords);
+            d.aux = d.state + kLatStateWords;
             d.local = c.Take<uint16_t>(n);
             d.cpar = c.Take<uint64_t>(static_cast<size_t>(kWavesPerBlock) * g.n_blocks * g.edge_cap);
             d.bbits = c.Take<uint64_t>(static_cast<size_t>(kBbitWords) * g.n_blocks);
