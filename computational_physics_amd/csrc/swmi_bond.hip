@@ -34,6 +34,8 @@ namespace swmi
         // counter that a load waits on also counts the stores issued before it.
         constexpr uint32_t kCh = TWR_MAX < 16 ? TWR_MAX : 16;
         constexpr uint32_t kRows = TWR_MAX < 16 ? TWR_MAX : 16;   // rows resolved together at the end
+        // 64-wide tiles of at most kRows rows keep their rows' roots in registers from the row loop to the labels
+        constexpr bool kKeep = TW64 && TWR_MAX <= kRows;
         constexpr uint32_t kSites = kWavesPerBlock * TWR_MAX * 64;
         constexpr uint32_t kQw = 128u;                             // per-wave LDS words of Q
         constexpr uint32_t kPFlag = 1u << 17;
@@ -256,6 +258,9 @@ namespace swmi
         uint64_t last_B = 0, last_D = 0, down_bits = 0, right_bits = 0;
         uint32_t qlen = 0;
         uint32_t Rp = 0;   // 64-wide tiles: root of this lane's site in the previous row
+        uint32_t Rk[kKeep ? kRows / 2u + 1u : 1u];   // the rows' roots as they were labelled, two to a word
+        if (TW64)
+            Qw[lane] = 0u;   // run words of LabelRow64
         uint64_t prev_S = 0, prev_U2 = 0, prev_B = 0, prev_Ball = 0;
         uint32_t prev_site = 0;
         uint32_t colv = 0;   // 64-wide tiles: lane r collects the first-column spin of row r
@@ -296,7 +301,8 @@ namespace swmi
                     c.lab[i] = kPend ? __builtin_amdgcn_raw_buffer_load_b16(rs_local, lane * 2u, rowoff * 2u, 0) : 0u;
                 }
             };
-            const auto process = [&](const uint32_t r0, Chunk& c) {
+            const auto process = [&](const uint32_t r0, auto rc_t, Chunk& c) {
+                constexpr uint32_t rc = decltype(rc_t)::value;   // r0 where the rows' roots are kept
                 uint32_t(&sp)[kC] = c.sp;
                 const uint32_t(&aux)[kC] = c.aux;
                 const uint32_t(&lab)[kC] = c.lab;
@@ -393,7 +399,14 @@ namespace swmi
                             const uint64_t D = r == 0 ? 0ull : (injected ? prev_U2 : (~(prev_S ^ S) & prev_U2));
                             if (dump && r > 0)
                                 dump[prev_site] = static_cast<uint8_t>((LaneBit(prev_Ball) ? 1u : 0u) | (LaneBit(D) ? 2u : 0u));
-                            Rp = LabelRow64(P, Qw, dummy, row_b + lane4, B, D, Rp, r > 0);
+                            Rp = LabelRow64(P, Qw, dummy, row_b + lane4, B, D, Rp, RowBase(r + 1u));
+                            if (kKeep)
+                            {
+                                if (i % 2u == 0u)
+                                    Rk[(rc + i) / 2u] = Rp;
+                                else
+                                    Rk[(rc + i) / 2u] |= Rp << 16;
+                            }
                         }
                         else
                         {
@@ -440,13 +453,24 @@ namespace swmi
             meet();
             if (nrow == 0)
                 return;
-            process(0u, c0);
-            for (uint32_t r0 = kC; r0 < (TWR_MAX <= kC ? 0u : nrow); r0 += kC)
+            process(0u, std::integral_constant<uint32_t, 0>{}, c0);
+            if constexpr (kKeep)
             {
-                Chunk c;
-                load(r0, c);
-                process(r0, c);
+                // (a chunk has kC = kRows or kRows / 2 rows: at most one more, at a row known here)
+                if (TWR_MAX > kC && nrow > kC)
+                {
+                    Chunk c;
+                    load(kC, c);
+                    process(kC, std::integral_constant<uint32_t, TWR_MAX <= kC ? 0u : kC>{}, c);
+                }
             }
+            else
+                for (uint32_t r0 = kC; r0 < (TWR_MAX <= kC ? 0u : nrow); r0 += kC)
+                {
+                    Chunk c;
+                    load(r0, c);
+                    process(r0, std::integral_constant<uint32_t, 0>{}, c);
+                }
             };
             if (rot1 || rot2)
             {
@@ -518,108 +542,35 @@ namespace swmi
         }
         __syncthreads();
 
-        // every site's block-local root (kRows chases in flight per lane). A tile of at most kRows rows
-        // keeps its roots in registers; taller tiles write them back into P.
-        const bool one_chunk = TWR_MAX <= kRows || nrow <= kRows;
-        uint32_t xs[kRows];
-        // (a wave of a partial block may own no rows: its part of P was never written and is not chased)
-        for (uint32_t r0 = 0; r0 < (TWR_MAX <= kRows ? (nrow > 0 ? 1u : 0u) : nrow); r0 += kRows)
-        {
-#pragma unroll
-            for (uint32_t i = 0; i < kRows; ++i)
-                xs[i] = (r_begin + ((r0 + i < nrow) ? r0 + i : r0)) * 256u + lane4;
-            // two steps per round; a round ends the chase once a step moved no lane of any row. The
-            // differences are summed in vector registers (16 values below 2^17 cannot wrap to zero). Parents
-            // only decrease, so a chase ends within kSites steps; more rounds mean a broken forest, which is
-            // reported instead of followed.
-            for (uint32_t round = 0;; ++round)
-            {
-                if (round * 2u > kSites)
-                {
-                    if (lane == 0)
-                        (void)__hip_atomic_fetch_or(stp + kStErr, kErrLabelRange, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                    break;
-                }
-                uint32_t ys[kRows];
-                uint32_t moved = 0;
-#pragma unroll
-                for (uint32_t i = 0; i < kRows; ++i)
-                {
-                    ys[i] = LdsLoad(At(P, xs[i]));
-                    moved += ys[i] ^ xs[i];
-                }
-                if (!__ballot(moved != 0u))
-                    break;
-                moved = 0;
-#pragma unroll
-                for (uint32_t i = 0; i < kRows; ++i)
-                {
-                    xs[i] = LdsLoad(At(P, ys[i]));
-                    moved += xs[i] ^ ys[i];
-                }
-                if (!__ballot(moved != 0u))
-                    break;
-            }
-            if (!one_chunk)
-            {
-#pragma unroll
-                for (uint32_t i = 0; i < kRows; ++i)
-                    if (r0 + i < nrow)
-                        *At(Pl, (r_begin + r0 + i) * 256u) = xs[i];
-            }
-        }
-        // (taller tiles: a flagged entry is a root's own, first flagged by the edge marks, later holding its
-        // slot label; either way the site is its own root)
-        const auto root_of = [&](const uint32_t r) {
-            if (one_chunk)
-                return xs[r];
-            const uint32_t v = LdsLoad(At(Pl, (r_begin + r) * 256u));
-            return v >= kPFlag ? (r_begin + r) * 256u + lane4 : v;
-        };
-        __syncthreads();   // no chase may meet a flagged entry
-
-        // Sites on the block edge flag their root (lanes off the edge flag their own word of Q). The edge
-        // lanes of a row are `side`, plus every lane of the block's first and last lattice rows. The marks of
-        // up to kRows rows are issued together and return the root's entry as it was: the lane that found it
-        // unflagged (the cluster's first mark) gives the cluster the next slot of the block (one LDS counter,
-        // one addition per wave and chunk of rows), writes the slot's union-find entry (a root keyed by the
-        // root's site) and makes the root's entry in P kPFlag | (qcap + slot) << 2, so that after the barrier
-        // every site of the cluster reads the label 0x8000 | (qcap + slot). A block has at most as many edge
-        // roots as boundary sites, within its slot capacity; more would be a broken invariant, reported
-        // through the error flag.
-        const uint64_t side = TW64 ? (PAD ? (1ull | (1ull << elane)) : 0x8000000000000001ull) : __ballot(lx == 0 || rbound);
-        const uint64_t top_first = r_begin == 0 ? (TW64 ? vmask : (__ballot(lrow == 0) & vmask)) : 0ull;
-        const uint64_t bottom_last = last_wave ? (TW64 ? vmask : (__ballot(lrow == rpw - 1u) & vmask)) : 0ull;
         const uint32_t qcap = d.qcap, bslots = kWavesPerBlock * d.edge_cap;
         const Rsrc rs_cpar = MakeRsrc(d.cpar + bslots * bl.lb, bslots * 8u);
-        // full tiles (the rule) take the row count and the first/last row masks at compile time
-        const bool full = TWR_MAX <= kRows && nrow == kRows;
-        const auto mark_rows = [&](auto full_t, const uint32_t r0) {
-            constexpr bool kFull = decltype(full_t)::value;
-            uint32_t old[kRows], root[kRows];
-#pragma unroll
-            for (uint32_t i = 0; i < kRows; ++i)
-            {
-                old[i] = kPFlag;
-                root[i] = 0u;
-                const uint32_t r = r0 + i;
-                if (kFull || r < nrow)
-                {
-                    const bool last = kFull ? i + 1u == kRows : r + 1u == nrow;
-                    const uint64_t m = side | (r == 0u ? top_first : 0ull) | (last ? bottom_last : 0ull);
-                    root[i] = root_of(r);
-                    const uint32_t o = __hip_atomic_fetch_or(LaneBit(m) ? At(P, root[i]) : dummy, kPFlag, __ATOMIC_RELAXED,
-                                                             __HIP_MEMORY_SCOPE_WORKGROUP);
-                    old[i] = LaneBit(m) ? o : kPFlag;
-                }
-            }
-            uint64_t F[kRows];
+        const Rsrc rs_ecol = MakeRsrc(d.ecol + 2u * bl.lb * d.ecol_stride, 8u * d.ecol_stride);
+        const Rsrc rs_erow = MakeRsrc(d.erow + 2u * 64u * bl.lb, 2u * 64u * 4u);
+
+        // Edge marks: the lanes of m[k] flag their root[k], a site on the block edge (lanes off the edge flag their own
+        // word of Q). The marks of the K vectors are issued together and return the root's entry as it was: the lane
+        // that found it unflagged (the cluster's first mark) gives the cluster the next slot of the block (one LDS
+        // counter, one addition per wave), writes the slot's union-find entry (a root keyed by the root's site) and
+        // makes the root's entry in P kPFlag | (qcap + slot) << 2, so that after the barrier every site of the cluster
+        // reads the label 0x8000 | (qcap + slot). A block has at most as many edge roots as boundary sites, within its
+        // slot capacity; more would be a broken invariant, reported through the error flag.
+        const auto mark = [&](const auto& root, const auto& m, const auto K_t) {
+            constexpr uint32_t K = decltype(K_t)::value;
+            uint32_t old[K];
+            uint64_t F[K];
             uint32_t total = 0;
 #pragma unroll
-            for (uint32_t i = 0; i < kRows; ++i)
+            for (uint32_t k = 0; k < K; ++k)
             {
-                F[i] = __ballot(old[i] < kPFlag);
-                total += static_cast<uint32_t>(__popcll(F[i]));
+                const uint32_t o = __hip_atomic_fetch_or(LaneBit(m[k]) ? At(P, root[k]) : dummy, kPFlag, __ATOMIC_RELAXED,
+                                                         __HIP_MEMORY_SCOPE_WORKGROUP);
+                old[k] = LaneBit(m[k]) ? o : kPFlag;
+            }
+#pragma unroll
+            for (uint32_t k = 0; k < K; ++k)
+            {
+                F[k] = __ballot(old[k] < kPFlag);
+                total += static_cast<uint32_t>(__popcll(F[k]));
             }
             if (total == 0u)
                 return;
@@ -628,63 +579,225 @@ namespace swmi
                 base = __hip_atomic_fetch_add(&s_nslot, total, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
             base = __builtin_amdgcn_readfirstlane(base);
 #pragma unroll
-            for (uint32_t i = 0; i < kRows; ++i)
+            for (uint32_t k = 0; k < K; ++k)
             {
-                const bool first = LaneBit(F[i]);
-                const uint32_t pos = base + __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(F[i] >> 32),
-                                                                      __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(F[i]), 0u));
-                __hip_atomic_store(first ? At(P, root[i]) : dummy, kPFlag | ((qcap + min(pos, bslots - 1u)) << 2),
-                                   __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-                const u32x2 entry = {bslots * bl.lb + pos, SiteOf(bl.base, bl.stride, root[i] >> 2)};   // (site << 32) | slot
+                const bool first = LaneBit(F[k]);
+                const uint32_t pos = base + __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(F[k] >> 32),
+                                                                      __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(F[k]), 0u));
+                __hip_atomic_store(first ? At(P, root[k]) : dummy, kPFlag | ((qcap + min(pos, bslots - 1u)) << 2), __ATOMIC_RELAXED,
+                                   __HIP_MEMORY_SCOPE_WORKGROUP);
+                const u32x2 entry = {bslots * bl.lb + pos, SiteOf(bl.base, bl.stride, root[k] >> 2)};   // (site << 32) | slot
                 __builtin_amdgcn_raw_buffer_store_b64(entry, rs_cpar, first ? pos * 8u : kNoStore, 0, 0);
-                base += static_cast<uint32_t>(__popcll(F[i]));
+                base += static_cast<uint32_t>(__popcll(F[k]));
             }
         };
-        if (full)
-            mark_rows(std::true_type{}, 0u);
-        else if (one_chunk)
-            mark_rows(std::false_type{}, 0u);
-        else
-            for (uint32_t r0 = 0; r0 < nrow; r0 += kRows)
-                mark_rows(std::false_type{}, r0);
-        __syncthreads();   // every slot label in place
 
-        // labels out: the block-local labels, and (label << 16) | root index of the block's first and last
-        // column and first and last wave row for the merge and the halo flips. The outputs go through buffer
-        // views of this block's part of each array; a lane with nothing to store gets an offset past the
-        // view, and the hardware drops that store (no exec mask).
-        const Rsrc rs_ecol = MakeRsrc(d.ecol + 2u * bl.lb * d.ecol_stride, 8u * d.ecol_stride);
-        const uint32_t ecol_off = LaneBit(side) ? ((rbound ? d.ecol_stride : 0u) + r_begin * rpw + lrow) * 4u : kNoStore;
-        const Rsrc rs_erow = MakeRsrc(d.erow + 2u * 64u * bl.lb, 2u * 64u * 4u);
-        const auto emit = [&](const uint32_t r, const uint32_t root) {
-            const uint32_t wr = r_begin + r;
-            const uint32_t rowoff = wr * bl.stride;   // sites from the block's first site
-            const uint32_t lab = LdsLoad(At(P, root)) >> 2;
-            const uint32_t e = (lab << 16) | (root >> 2);
-            __builtin_amdgcn_raw_buffer_store_b16(static_cast<uint16_t>(lab), rs_local, lane * 2u, rowoff * 2u, 0);
-            __builtin_amdgcn_raw_buffer_store_b32(e, rs_ecol, ecol_off, r * rpw * 4u, 0);
-            if (wr == 0u)
-                __builtin_amdgcn_raw_buffer_store_b32(e, rs_erow, lane4, 0, 0);
-            if (wr + 1u == bl.nwr)
-                __builtin_amdgcn_raw_buffer_store_b32(e, rs_erow, lane4, 256u, 0);
-        };
-        const auto rows_do = [&](auto full_t, auto&& f) {
-            constexpr bool kFull = decltype(full_t)::value;
+        if constexpr (kKeep)
+        {
+            // Every site's block-local root, from the rows' roots as they were labelled, all rows of the tile in flight,
+            // and the root of one more site per lane: lane i < kRows row i's first column, lane kRows + i its last, so
+            // that one vector holds what the rows need for the block's edge columns.
+            constexpr uint32_t kSide = kRows;
+            const uint32_t srow = lane % kSide;
+            const bool sides = lane < 2u * kSide && srow < nrow;
+            uint32_t xs[kRows], xside = 0;
+            if (nrow > 0u)
+            {
 #pragma unroll
-            for (uint32_t i = 0; i < kRows; ++i)
-                if (kFull || i < nrow)
-                    f(i, xs[i]);
-        };
-        const auto for_rows = [&](auto&& f) {
-            if (full)
-                rows_do(std::true_type{}, f);
-            else if (one_chunk)
-                rows_do(std::false_type{}, f);
+                for (uint32_t i = 0; i < kRows; ++i)
+                    xs[i] = i < nrow ? (i % 2u == 0u ? Rk[i / 2u] & 0xFFFFu : Rk[i / 2u] >> 16) : r_begin * 256u;
+                xside = (r_begin + (sides ? srow : 0u)) * 256u + (sides && lane >= kSide ? elane * 4u : 0u);
+                // two steps per round; a round ends the chase once a step moved no lane of any row. The differences are
+                // summed in vector registers (17 values below 2^17 cannot wrap to zero). Parents only decrease, so a
+                // chase ends within kSites steps; more rounds mean a broken forest, which is reported instead of
+                // followed.
+                for (uint32_t round = 0;; ++round)
+                {
+                    if (round * 2u > kSites)
+                    {
+                        if (lane == 0)
+                            (void)__hip_atomic_fetch_or(stp + kStErr, kErrLabelRange, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                        break;
+                    }
+                    uint32_t ys[kRows];
+                    const uint32_t yside = LdsLoad(At(P, xside));
+                    uint32_t moved = yside ^ xside;
+#pragma unroll
+                    for (uint32_t i = 0; i < kRows; ++i)
+                    {
+                        ys[i] = LdsLoad(At(P, xs[i]));
+                        moved += ys[i] ^ xs[i];
+                    }
+                    if (!__ballot(moved != 0u))
+                        break;
+                    xside = LdsLoad(At(P, yside));
+                    moved = xside ^ yside;
+#pragma unroll
+                    for (uint32_t i = 0; i < kRows; ++i)
+                    {
+                        xs[i] = LdsLoad(At(P, ys[i]));
+                        moved += xs[i] ^ ys[i];
+                    }
+                    if (!__ballot(moved != 0u))
+                        break;
+                }
+            }
+            __syncthreads();   // no chase may meet a flagged entry
+            uint32_t xlast = xs[0];   // root in the tile's last row
+#pragma unroll
+            for (uint32_t i = 1; i < kRows; ++i)
+                xlast = i + 1u == nrow ? xs[i] : xlast;
+            if (nrow > 0u)
+            {
+                const uint32_t root[3] = {xside, xs[0], xlast};
+                const uint64_t m[3] = {__ballot(sides), r_begin == 0u ? vmask : 0ull, last_wave ? vmask : 0ull};
+                mark(root, m, std::integral_constant<uint32_t, 3>{});
+            }
+            __syncthreads();   // every slot label in place
+
+            // labels out: the block-local labels, and (label << 16) | root index of the block's first and last column and
+            // first and last wave row for the merge and the halo flips. The outputs go through buffer views of this
+            // block's part of each array; a lane with nothing to store gets an offset past the view, and the hardware
+            // drops that store (no exec mask).
+            if (nrow > 0u)
+            {
+                const auto entry = [&](const uint32_t root) { return ((LdsLoad(At(P, root)) >> 2) << 16) | (root >> 2); };
+                const auto emit = [&](auto full_t) {
+                    constexpr bool kFull = decltype(full_t)::value;
+#pragma unroll
+                    for (uint32_t i = 0; i < kRows; ++i)
+                        if (kFull || i < nrow)
+                            __builtin_amdgcn_raw_buffer_store_b16(static_cast<uint16_t>(LdsLoad(At(P, xs[i])) >> 2), rs_local, lane * 2u,
+                                                                  (r_begin + i) * bl.stride * 2u, 0);
+                };
+                if (nrow == kRows)
+                    emit(std::true_type{});
+                else
+                    emit(std::false_type{});
+                __builtin_amdgcn_raw_buffer_store_b32(entry(xside), rs_ecol,
+                                                      sides ? ((lane >= kSide ? d.ecol_stride : 0u) + r_begin + srow) * 4u : kNoStore, 0, 0);
+                if (r_begin == 0u)
+                    __builtin_amdgcn_raw_buffer_store_b32(entry(xs[0]), rs_erow, lane4, 0, 0);
+                if (last_wave)
+                    __builtin_amdgcn_raw_buffer_store_b32(entry(xlast), rs_erow, lane4, 256u, 0);
+            }
+        }
+        else
+        {
+            // every site's block-local root (kRows chases in flight per lane). A tile of at most kRows rows
+            // keeps its roots in registers; taller tiles write them back into P.
+            const bool one_chunk = TWR_MAX <= kRows || nrow <= kRows;
+            uint32_t xs[kRows];
+            // (a wave of a partial block may own no rows: its part of P was never written and is not chased)
+            for (uint32_t r0 = 0; r0 < (TWR_MAX <= kRows ? (nrow > 0 ? 1u : 0u) : nrow); r0 += kRows)
+            {
+#pragma unroll
+                for (uint32_t i = 0; i < kRows; ++i)
+                    xs[i] = (r_begin + ((r0 + i < nrow) ? r0 + i : r0)) * 256u + lane4;
+                // two steps per round; a round ends the chase once a step moved no lane of any row. The
+                // differences are summed in vector registers (16 values below 2^17 cannot wrap to zero). Parents
+                // only decrease, so a chase ends within kSites steps; more rounds mean a broken forest, which is
+                // reported instead of followed.
+                for (uint32_t round = 0;; ++round)
+                {
+                    if (round * 2u > kSites)
+                    {
+                        if (lane == 0)
+                            (void)__hip_atomic_fetch_or(stp + kStErr, kErrLabelRange, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                        break;
+                    }
+                    uint32_t ys[kRows];
+                    uint32_t moved = 0;
+#pragma unroll
+                    for (uint32_t i = 0; i < kRows; ++i)
+                    {
+                        ys[i] = LdsLoad(At(P, xs[i]));
+                        moved += ys[i] ^ xs[i];
+                    }
+                    if (!__ballot(moved != 0u))
+                        break;
+                    moved = 0;
+#pragma unroll
+                    for (uint32_t i = 0; i < kRows; ++i)
+                    {
+                        xs[i] = LdsLoad(At(P, ys[i]));
+                        moved += xs[i] ^ ys[i];
+                    }
+                    if (!__ballot(moved != 0u))
+                        break;
+                }
+                if (!one_chunk)
+                {
+#pragma unroll
+                    for (uint32_t i = 0; i < kRows; ++i)
+                        if (r0 + i < nrow)
+                            *At(Pl, (r_begin + r0 + i) * 256u) = xs[i];
+                }
+            }
+            // (taller tiles: a flagged entry is a root's own, first flagged by the edge marks, later holding its
+            // slot label; either way the site is its own root)
+            const auto root_of = [&](const uint32_t r) {
+                if (one_chunk)
+                    return xs[r];
+                const uint32_t v = LdsLoad(At(Pl, (r_begin + r) * 256u));
+                return v >= kPFlag ? (r_begin + r) * 256u + lane4 : v;
+            };
+            __syncthreads();   // no chase may meet a flagged entry
+
+            // Sites on the block edge flag their root: the edge lanes of a row are `side`, plus every lane of the block's first
+            // and last lattice rows.
+            const uint64_t side = TW64 ? (PAD ? (1ull | (1ull << elane)) : 0x8000000000000001ull) : __ballot(lx == 0 || rbound);
+            const uint64_t top_first = r_begin == 0 ? (TW64 ? vmask : (__ballot(lrow == 0) & vmask)) : 0ull;
+            const uint64_t bottom_last = last_wave ? (TW64 ? vmask : (__ballot(lrow == rpw - 1u) & vmask)) : 0ull;
+            const auto mark_rows = [&](const uint32_t r0) {
+                uint32_t root[kRows];
+                uint64_t m[kRows];
+#pragma unroll
+                for (uint32_t i = 0; i < kRows; ++i)
+                {
+                    const uint32_t r = r0 + i;
+                    root[i] = 0u;
+                    m[i] = 0ull;
+                    if (r < nrow)
+                    {
+                        m[i] = side | (r == 0u ? top_first : 0ull) | (r + 1u == nrow ? bottom_last : 0ull);
+                        root[i] = root_of(r);
+                    }
+                }
+                mark(root, m, std::integral_constant<uint32_t, kRows>{});
+            };
+            if (one_chunk)
+                mark_rows(0u);
+            else
+                for (uint32_t r0 = 0; r0 < nrow; r0 += kRows)
+                    mark_rows(r0);
+            __syncthreads();   // every slot label in place
+
+            // labels out, as above
+            const uint32_t ecol_off = LaneBit(side) ? ((rbound ? d.ecol_stride : 0u) + r_begin * rpw + lrow) * 4u : kNoStore;
+            const auto emit = [&](const uint32_t r, const uint32_t root) {
+                const uint32_t wr = r_begin + r;
+                const uint32_t rowoff = wr * bl.stride;   // sites from the block's first site
+                const uint32_t lab = LdsLoad(At(P, root)) >> 2;
+                const uint32_t e = (lab << 16) | (root >> 2);
+                __builtin_amdgcn_raw_buffer_store_b16(static_cast<uint16_t>(lab), rs_local, lane * 2u, rowoff * 2u, 0);
+                __builtin_amdgcn_raw_buffer_store_b32(e, rs_ecol, ecol_off, r * rpw * 4u, 0);
+                if (wr == 0u)
+                    __builtin_amdgcn_raw_buffer_store_b32(e, rs_erow, lane4, 0, 0);
+                if (wr + 1u == bl.nwr)
+                    __builtin_amdgcn_raw_buffer_store_b32(e, rs_erow, lane4, 256u, 0);
+            };
+            if (one_chunk)
+            {
+#pragma unroll
+                for (uint32_t i = 0; i < kRows; ++i)
+                    if (i < nrow)
+                        emit(i, xs[i]);
+            }
             else
                 for (uint32_t r = 0; r < nrow; ++r)
-                    f(r, root_of(r));
-        };
-        for_rows(emit);
+                    emit(r, root_of(r));
+        }
         const gptr<uint64_t> bb = Glob(d.bbits) + kBbitWords * bl.lb;
         if (lane == 0)
         {

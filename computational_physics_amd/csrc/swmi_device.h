@@ -184,23 +184,27 @@ namespace swmi
     // One row of a 64-wide tile joins the union-find: B are its bonds to the right (inside the tile), D the bonds
     // from the row above into it, Rp the root of this lane's site in the row above (resolved when that row was
     // labelled), self this lane's node. A row run's label is the minimum of its first site and the roots its down
-    // bonds reach (one LDS atomicMin per bonded lane into the run's slot of M); a bond to any other root links that
-    // root under the minimum with one atomicMin, and only a link that loses a race goes through the lockstep union.
-    // Returns the root of this lane's site. M: 64 words of the wave; dummy: a word of the lane's own, the target of
-    // LDS operations the lane has no use for. below: some row above may be bonded (D may be non-zero).
+    // bonds reach, taken by one LDS atomic per row: the run's word of M holds the maximum of base - node, and base
+    // grows from row to row by more than any node (bits 16 and up, the low 16 all ones), so what earlier rows left
+    // there is smaller than anything this row writes and no row clears its words. A bond to any other root links
+    // that root under the minimum with one atomicMin, and only a link that loses a race goes through the lockstep
+    // union. P[self] is left at the run's label, an ancestor; returns the root of this lane's site after the row's
+    // links. M: 64 words of the wave, below base at the start; dummy: a word of the lane's own, the target of LDS
+    // operations the lane has no use for.
+    // LDS operations are what bounds the labelling (one pipe per CU, about 7 cycles per operation of a wave with
+    // scattered roots): a row takes four and one per chase step, where clearing, minimum, entry and root as separate
+    // operations took eight.
     __device__ __forceinline__ uint32_t LabelRow64(uint32_t* P, uint32_t* M, uint32_t* dummy, const uint32_t self, const uint64_t B,
-                                                   const uint64_t D, const uint32_t Rp, const bool below)
+                                                   const uint64_t D, const uint32_t Rp, const uint32_t base)
     {
-        // slot of this lane's row run: the number of run starts after lane 0 up to this lane; the first lane of the
-        // run initialises it with its own node
+        // word of this lane's row run: the number of run starts after lane 0 up to this lane
         uint32_t* const Mk = M + __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(~B >> 32),
                                                            __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(~B), 0u));
-        __hip_atomic_store(LaneBit(~(B << 1)) ? Mk : dummy, self, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-        // the row's entries start as roots (overwritten below), so chases end on them
-        __hip_atomic_store(At(P, self), self, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-        if (below)
-            LdsMin(LaneBit(D) ? Mk : dummy, Rp);
-        uint32_t root = LdsLoad(Mk);
+        // a run's first lane brings its own node, a bonded lane the root above (an earlier row's node, so smaller)
+        const uint32_t x = LaneBit(D) ? Rp : self;
+        (void)__hip_atomic_fetch_max(LaneBit(~(B << 1) | D) ? Mk : dummy, base - x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        uint32_t root = base - LdsLoad(Mk);
+        __hip_atomic_store(At(P, self), root, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
         // bonds to a root other than the run's minimum link that root under it
         const uint64_t mg = D & __ballot(Rp != root);
         if (mg != 0ull)
@@ -223,9 +227,11 @@ namespace swmi
                 root = pr;
             }
         }
-        *At(P, self) = root;
         return root;
     }
+
+    // base of LabelRow64 for the k-th row a wave labels, k from 1 to 65535
+    __device__ __forceinline__ uint32_t RowBase(const uint32_t k) { return (k << 16) | 0xFFFFu; }
 
     // ---- union-find in HBM over the roots of edge-reaching clusters, one node per slot (every block numbers
     // its edge roots densely, so a block's nodes share a few cache lines). Entry of slot c: (key << 32) | parent

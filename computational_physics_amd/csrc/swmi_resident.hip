@@ -155,6 +155,8 @@ namespace swmi
         const uint32_t last_active = it_end > it ? (it_end - it - 1u) / 2u + 1u : 0u;   // sweeps until the schedule ends
         const uint32_t total = min(groups * sweeps, last_active);
         uint32_t done = 0;
+        uint32_t labelled = 0;   // rows the wave has labelled in this launch (kResidentRows * sweeps, below 2^16)
+        Qw[lane] = 0u;
 
         const auto first_col = [&]() -> uint64_t {   // bit i: spin of row i's right neighbour column
             uint32_t h = 0;
@@ -238,7 +240,7 @@ namespace swmi
                     {
                         right_bits |= ((Ball >> elane) & 1ull) << i;
                         const uint64_t D = i == 0u ? 0ull : (~(prev_S ^ S) & prev_U2);
-                        Rp = LabelRow64(P, Qw, dummy, node, B, D, Rp, i > 0u);
+                        Rp = LabelRow64(P, Qw, dummy, node, B, D, Rp, RowBase(++labelled));
                         if (i == 0u && lane == 0u)
                             sB[w] = B;
                     }
