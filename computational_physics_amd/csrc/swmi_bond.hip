@@ -26,7 +26,10 @@ namespace swmi
     // PAD: the lattice is stored with a row pitch d.n0 above its width d.n0v; in the last tile column only
     // the lanes up to d.elast hold sites (mask d.vlast), the rest are padding: they bond to nothing, their
     // draws are unused, and the row's last site bonds across the lattice edge instead of lane tw - 1.
-    template <uint32_t TWR_MAX, bool TW64, bool DBG, bool PAD>
+    // NW: waves of the workgroup, each with a strip of 4 * twr / NW wave rows of the block, at most TWR_MAX. Four
+    // waves label a tile each; sixteen label a quarter tile each, which shortens the chain of dependent LDS
+    // operations down a strip where a launch has too few blocks to fill the chip (LaunchBondLabelT).
+    template <uint32_t NW, uint32_t TWR_MAX, bool TW64, bool DBG, bool PAD>
     __device__ __forceinline__ void BondLabel(const LatDesc* __restrict__ descs, const uint32_t* __restrict__ block_lat,
                                               const uint32_t total_blocks)
     {
@@ -36,7 +39,8 @@ namespace swmi
         constexpr uint32_t kRows = TWR_MAX < 16 ? TWR_MAX : 16;   // rows resolved together at the end
         // 64-wide tiles of at most kRows rows keep their rows' roots in registers from the row loop to the labels
         constexpr bool kKeep = TW64 && TWR_MAX <= kRows;
-        constexpr uint32_t kSites = kWavesPerBlock * TWR_MAX * 64;
+        constexpr uint32_t kSites = NW * TWR_MAX * 64;
+        constexpr uint32_t kThreads = NW * 64u;
         constexpr uint32_t kQw = 128u;                             // per-wave LDS words of Q
         constexpr uint32_t kPFlag = 1u << 17;
         static_assert(kSites * 4u <= (1u << 16), "byte offsets must fit the 16-bit halves of a queue entry");
@@ -45,12 +49,13 @@ namespace swmi
         // per wave: 64-wide tiles keep the run minima of the current row in words 0-63 and give each lane a
         // word of its own in 64-127 (the target of LDS operations a lane has no use for, so that they need
         // no exec mask); narrow tiles keep their union queue here
-        __shared__ uint32_t Q[kWavesPerBlock * kQw];
+        __shared__ uint32_t Q[NW * kQw];
         __shared__ uint32_t FB[2u * kSites / 32u];   // flip bits of a pending flip, by label index (root or qcap + slot)
-        __shared__ uint64_t s_first_B[kWavesPerBlock];
+        __shared__ uint64_t s_first_B[NW];
         // Numerical Recipes pairs (c << 32 | a) by selector: words 0-7 one update, words 8-15 the jump from the stored
         // states to this sweep's
         __shared__ uint64_t AC[16];
+        __shared__ uint64_t s_right[NW == kWavesPerBlock ? 1u : kWavesPerBlock];   // bonds across the right edge, per tile
         __shared__ uint32_t s_nslot;            // slots given to the block's edge-reaching clusters
 
         const uint32_t b = RemapBlock(total_blocks);
@@ -58,13 +63,15 @@ namespace swmi
             return;
         if (threadIdx.x == 0)
             s_nslot = 0u;
+        if (NW != kWavesPerBlock && threadIdx.x < kWavesPerBlock)
+            s_right[threadIdx.x] = 0ull;
         const LatDesc& d = descs[LatticeOf(block_lat, b)];
         const Block bl = DecodeBlock(d, b);
         const uint32_t lane = threadIdx.x & 63u;
         const uint32_t lane4 = lane * 4u;
         const uint32_t w = Uniform(threadIdx.x >> 6);
 
-        const uint32_t n0 = d.n0, n1 = d.n1, twr = d.twr;
+        const uint32_t n0 = d.n0, n1 = d.n1, twr = d.twr * kWavesPerBlock / NW;   // wave rows of a strip
         const uint32_t tw = TW64 ? 64u : d.tw, rpw = TW64 ? 1u : d.rpw;
         const uint32_t lx = lane & (tw - 1u);
         const uint32_t lrow = TW64 ? 0u : lane / tw;
@@ -231,10 +238,10 @@ namespace swmi
                 if (threadIdx.x < d.fsw)
                     FB[d.qcap / 32u + threadIdx.x] = fbw;
                 if (d.flip_rule == 0u)
-                    for (uint32_t i = threadIdx.x; i < bl.nwr * 2u; i += 256u)   // bl.nwr * 64 root indices, 32 per word
+                    for (uint32_t i = threadIdx.x; i < bl.nwr * 2u; i += kThreads)   // bl.nwr * 64 root indices, 32 per word
                         FB[i] = RuleWord(d, bl, i, false, 0u);
                 else if (pending)   // the random rule's words, with the key of the pending flip's sweep
-                    for (uint32_t i = threadIdx.x; i < bl.nwr * 2u; i += 256u)
+                    for (uint32_t i = threadIdx.x; i < bl.nwr * 2u; i += kThreads)
                         FB[i] = RuleWord(d, bl, i, true, FlipKey(d.seed, it0 - 2u));
             }
             if (nrow > 0)
@@ -270,8 +277,8 @@ namespace swmi
             const auto chunks = [&](auto rotating, auto flipping) {
             constexpr bool kRot = decltype(rotating)::value;
             constexpr bool kPend = decltype(flipping)::value;
-            // rows loaded together: a flip on load also keeps the labels in flight, so half as many
-            constexpr uint32_t kC = kPend && kCh > 1u ? kCh / 2u : kCh;
+            // rows loaded together: a flip on load also keeps the labels in flight, so at most eight
+            constexpr uint32_t kC = kPend && kCh > 8u ? kCh / 2u : kCh;
             // what one chunk of rows loads per lane: the spin byte, the lcg32 state and, under a pending flip,
             // the label of its site in each row; one right-halo spin and one rotation offset per row (lane i:
             // row r0 + i of the chunk)
@@ -486,6 +493,9 @@ namespace swmi
         }
         if (nrow > 0)
         {
+            if (NW != kWavesPerBlock && lane == 0u && right_bits != 0ull)   // read after the last barrier
+                (void)__hip_atomic_fetch_or(&s_right[r_begin / d.twr], right_bits << (r_begin % d.twr), __ATOMIC_RELAXED,
+                                            __HIP_MEMORY_SCOPE_WORKGROUP);
             if (TW64 && !injected)   // first column of the tile's rows (rpw == 1): one store per wave
                 __builtin_amdgcn_raw_buffer_store_b8(static_cast<uint8_t>(colv & 1u), rs_halo, lane < nrow ? r_begin + lane : kNoStore, 0, 0);
 
@@ -803,8 +813,11 @@ namespace swmi
         {
             if (last_wave)
                 bb[0] = down_bits;
-            bb[1u + w] = right_bits;
+            if (NW == kWavesPerBlock)
+                bb[1u + w] = right_bits;
         }
+        if (NW != kWavesPerBlock && threadIdx.x < kWavesPerBlock)
+            bb[1u + threadIdx.x] = s_right[threadIdx.x];
         if (threadIdx.x == 0)
         {
             const uint32_t n = LdsLoad(&s_nslot);
@@ -814,30 +827,51 @@ namespace swmi
         }
     }
 
-    // 64-wide tiles of up to 16 rows: eight workgroups per CU (the register budget of 8 waves per SIMD is
-    // asked for explicitly; the compiler keeps the excess scalar registers in vector lanes). Narrow tiles
-    // keep the default budget (the cap would spill vector registers to scratch), and taller tiles are
-    // limited by their LDS anyway.
+    // 64-wide tiles of up to 16 rows: eight waves per SIMD (the register budget is asked for explicitly; the compiler
+    // keeps the excess scalar registers in vector lanes). Narrow tiles keep the default budget (the cap would spill
+    // vector registers to scratch), and taller tiles are limited by their LDS anyway.
     template <uint32_t TWR_MAX, bool DBG>
     __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8, 8))) void k_bond_label(
         const LatDesc* __restrict__ descs, const uint32_t* __restrict__ block_lat, const uint32_t total_blocks)
     {
-        BondLabel<TWR_MAX, true, DBG, false>(descs, block_lat, total_blocks);
+        BondLabel<kWavesPerBlock, TWR_MAX, true, DBG, false>(descs, block_lat, total_blocks);
+    }
+
+    // Sixteen waves per block, strips of up to 4 rows.
+    template <bool DBG, bool PAD>
+    __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(8, 8))) void k_bond_label_wide(
+        const LatDesc* __restrict__ descs, const uint32_t* __restrict__ block_lat, const uint32_t total_blocks)
+    {
+        BondLabel<16, 4, true, DBG, PAD>(descs, block_lat, total_blocks);
     }
 
     template <uint32_t TWR_MAX, bool TW64, bool DBG, bool PAD>
     __global__ __launch_bounds__(256) void k_bond_label_any(const LatDesc* __restrict__ descs, const uint32_t* __restrict__ block_lat,
                                                             const uint32_t total_blocks)
     {
-        BondLabel<TWR_MAX, TW64, DBG, PAD>(descs, block_lat, total_blocks);
+        BondLabel<kWavesPerBlock, TWR_MAX, TW64, DBG, PAD>(descs, block_lat, total_blocks);
     }
 
+    // Launches of at most this many blocks of 64-wide tiles, all of a height that four waves can share, give every
+    // block sixteen waves.
+    constexpr uint32_t kWideBlocks = 512;
+
     template <bool TW64, bool DBG>
-    void LaunchBondLabelT(const LatDesc* d_desc, const uint32_t* d_block_lat, const uint32_t total_blocks,
-                                 const uint32_t max_twr, const bool pad, hipStream_t stream)
+    void LaunchBondLabelT(const LatDesc* d_desc, const uint32_t* d_block_lat, const uint32_t total_blocks, const uint32_t max_twr,
+                          const bool quads, const bool pad, hipStream_t stream)
     {
         const uint32_t g = XcdGrid(total_blocks);
-        const auto launch = [&](auto kernel) { kernel<<<g, 256, 0, stream>>>(d_desc, d_block_lat, total_blocks); };
+        const auto launch = [&](auto kernel, const uint32_t threads = 256) {
+            kernel<<<g, threads, 0, stream>>>(d_desc, d_block_lat, total_blocks);
+        };
+        if constexpr (TW64)
+        {
+            if (quads && max_twr <= 16 && total_blocks <= kWideBlocks)
+            {
+                pad ? launch(k_bond_label_wide<DBG, true>, 1024) : launch(k_bond_label_wide<DBG, false>, 1024);
+                return;
+            }
+        }
         if (pad)   // padded lattices: two tile-height bounds
         {
             if (max_twr <= 16)
@@ -855,5 +889,5 @@ namespace swmi
             launch(k_bond_label_any<64, TW64, DBG, false>);
     }
 
-    template void LaunchBondLabelT<SWMI_BOND_TW64, SWMI_BOND_DBG>(const LatDesc*, const uint32_t*, uint32_t, uint32_t, bool, hipStream_t);
+    template void LaunchBondLabelT<SWMI_BOND_TW64, SWMI_BOND_DBG>(const LatDesc*, const uint32_t*, uint32_t, uint32_t, bool, bool, hipStream_t);
 }

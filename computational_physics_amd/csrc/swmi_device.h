@@ -212,7 +212,7 @@ namespace swmi
             const uint32_t old = __hip_atomic_fetch_min(LaneBit(mg) ? At(P, Rp) : dummy, root, __ATOMIC_RELAXED,
                                                         __HIP_MEMORY_SCOPE_WORKGROUP);
             // Rp was no longer a root (another lane linked it first): join the two trees
-            const uint64_t more = mg & __ballot(old != Rp && old != root);
+            const uint64_t more = mg & __ballot(old != Rp) & __ballot(old != root);
             if (more != 0ull)
             {
                 const bool mo = LaneBit(more);

@@ -217,7 +217,7 @@ namespace swmi
         const Geometry g = GeometryOf(c.n0, c.n1, c.tile_rows);
         const uint64_t n = static_cast<uint64_t>(g.pitch) * c.n1, groups = n / 64;
         return n * (1 + 4 + 2) + groups * (3 * 8 + 4) + static_cast<uint64_t>(kBbitWords) * 8 * g.n_blocks +
-               4ull * (kLatStateWords + 4ull * c.max_samples) + 4 * kAuxWords + 4ull * 2 * kWavesPerBlock * g.n_blocks +
+               4ull * (kLatStateWords + 4ull * c.max_samples) + 4 * kAuxWords + 4ull * 2 * g.n_blocks +
                static_cast<uint64_t>(kWavesPerBlock) * g.n_blocks * (8ull * g.edge_cap + 4) + 8ull * g.ecol_stride * g.n_blocks +
                4ull * 2 * 64 * g.n_blocks + 4ull * g.fsw * g.n_blocks + 2ull * g.halo_stride * g.n_blocks;
     }
@@ -253,7 +253,7 @@ namespace swmi
         bbits.allocate(static_cast<size_t>(kBbitWords) * g.n_blocks);
         state_words = kLatStateWords + 4u * c.max_samples;
         state.allocate(state_words);
-        partials.allocate(2ull * kWavesPerBlock * g.n_blocks);
+        partials.allocate(2ull * g.n_blocks);
         edge_count.allocate(static_cast<size_t>(kWavesPerBlock) * g.n_blocks);
         ecol.allocate(2ull * g.ecol_stride * g.n_blocks);
         erow.allocate(2ull * 64 * g.n_blocks);
@@ -410,6 +410,7 @@ void swmi_engine::Rebuild()
             it->twr_t = t;
             it->resident = resident;
         }
+        it->quads = it->quads && l.g.twr % 4u == 0u;
         it->max_rows = std::max(it->max_rows, rows);
         it->max_sites = std::max(it->max_sites, static_cast<uint32_t>(l.np));
         it->slots.push_back(i);
@@ -477,7 +478,7 @@ void swmi_engine::EnqueueSweeps(uint32_t n)
         hipStream_t s = ClassStream(c);
         for (uint32_t i = 0; i < n; ++i)
         {
-            LaunchBondLabel(k.Descs(d_desc.ptr), k.WorkList(), k.total_blocks, k.max_twr, k.tw64, k.pad, recording, s);
+            LaunchBondLabel(k.Descs(d_desc.ptr), k.WorkList(), k.total_blocks, k.max_twr, k.quads, k.tw64, k.pad, recording, s);
             LaunchMerge(k.Descs(d_desc.ptr), k.WorkList(), k.total_blocks, s);
             LaunchResolve(k.Descs(d_desc.ptr), k.WorkList(), k.total_blocks, s);
         }
@@ -549,7 +550,6 @@ void swmi_engine::EnqueueSample(uint32_t mode)
     for (size_t c = 0; c < n_tiled; ++c)
     {
         const KernelClass& k = classes[c];
-        LaunchMaterialize(k.Descs(d_desc.ptr), k.WorkList(), k.total_blocks, stream);
         LaunchObservables(k.Descs(d_desc.ptr), k.WorkList(), k.total_blocks, mode, stream);
         LaunchFinalizeSamples(d_desc.ptr, k.d_slots.ptr, k.n_lat, mode, stream);
     }
@@ -930,10 +930,10 @@ int swmi_observables(swmi_engine* engine, uint32_t lattice, int64_t* energy, int
 {
     return Guard([&] {
         Lattice& l = Eng(engine)->At(lattice);
-        engine->MaterializeOne(l);
+        engine->OneLattice(l, nullptr);
         LaunchObservables(engine->d_one_desc.ptr, nullptr, l.g.n_blocks, kSampleAlways, engine->stream);
         engine->LaunchCheck("observables launch");
-        std::vector<int32_t> p(2ull * kWavesPerBlock * l.g.n_blocks);
+        std::vector<int32_t> p(2ull * l.g.n_blocks);
         Check(hipMemcpyAsync(p.data(), l.partials.ptr, p.size() * 4, hipMemcpyDeviceToHost, engine->stream), "observables");
         Check(hipStreamSynchronize(engine->stream), "observables");
         int64_t e = 0, m = 0;
@@ -1076,7 +1076,7 @@ int swmi_label_bonds(swmi_engine* engine, uint32_t lattice, const uint8_t* bonds
         if (!l.parent.ptr)
             l.parent.allocate(l.np);
         engine->OneLattice(l, l.bond_in.ptr);
-        LaunchBondLabel(engine->d_one_desc.ptr, nullptr, l.g.n_blocks, l.g.twr, l.g.tw == 64, l.np != l.n, true,
+        LaunchBondLabel(engine->d_one_desc.ptr, nullptr, l.g.n_blocks, l.g.twr, l.g.twr % 4u == 0u, l.g.tw == 64, l.np != l.n, true,
                         engine->stream);
         LaunchMerge(engine->d_one_desc.ptr, nullptr, l.g.n_blocks, engine->stream);
         LaunchWriteLabels(engine->d_one_desc.ptr, nullptr, l.g.n_blocks, l.g.twr, engine->stream);
@@ -1329,7 +1329,7 @@ int swmi_time_kernels(swmi_engine* engine, uint32_t n_sweeps, float* ms)
         {
             Check(hipEventRecord(ev[0], engine->stream), "event");
             for (auto& k : engine->classes)
-                LaunchBondLabel(k.Descs(engine->d_desc.ptr), k.WorkList(), k.total_blocks, k.max_twr, k.tw64, k.pad, engine->recording,
+                LaunchBondLabel(k.Descs(engine->d_desc.ptr), k.WorkList(), k.total_blocks, k.max_twr, k.quads, k.tw64, k.pad, engine->recording,
                                 engine->stream);
             Check(hipEventRecord(ev[1], engine->stream), "event");
             for (auto& k : engine->classes)

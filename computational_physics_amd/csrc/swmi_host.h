@@ -174,6 +174,7 @@ namespace swmi
         bool pad = false;                    // padded lattices (the PAD specialisation of k_bond_label)
         uint32_t twr_t = 16;                 // k_bond_label TWR_MAX
         uint32_t max_twr = 1;
+        bool quads = true;                   // every tile height is a multiple of 4
         std::vector<uint32_t> block_lat;     // block -> lattice slot
         DeviceBuffer<uint32_t> d_block_lat;
         uint32_t total_blocks = 0;

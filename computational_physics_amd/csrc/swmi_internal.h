@@ -84,7 +84,7 @@ namespace swmi
         uint32_t* state;         // per-lattice device counters, see LatState
         uint8_t* bond_dump;      // per-site bond bytes of the last sweep (nullptr: not recorded)
         const uint8_t* bond_in;  // injected bond bytes (label-only mode), nullptr otherwise
-        int32_t* partials;       // 2 int32 (E, M) per tile for observables
+        int32_t* partials;       // 2 int32 (E, M) per block for observables
         uint32_t* edge_count;    // slots in use, word kWavesPerBlock * block
         uint32_t* ecol;          // block edge columns: [block][side][lattice row in block] of (label << 16) | q
         uint32_t* erow;          // block edge wave rows: [block][side][lane] of (label << 16) | q
@@ -158,10 +158,11 @@ namespace swmi
     // Launch wrappers (swmi_kernels.hip). Work list: block_lat[b] = lattice of global block b; a null work list
     // means every block belongs to descriptor 0.
     // all_tw64: every lattice of the work list has n0 % 64 == 0 (64-wide tiles); selects the specialised kernel
+    // quads: every lattice's tile height is a multiple of 4
     // debug: compiles in injected bonds (LatDesc::bond_in) and bond recording (LatDesc::bond_dump)
     // pad: some lattice of the work list is padded (selects the PAD specialisation, correct for every lattice)
     void LaunchBondLabel(const LatDesc* d_desc, const uint32_t* d_block_lat, uint32_t total_blocks, uint32_t max_twr,
-                         bool all_tw64, bool pad, bool debug, hipStream_t stream);
+                         bool quads, bool all_tw64, bool pad, bool debug, hipStream_t stream);
     void LaunchMerge(const LatDesc* d_desc, const uint32_t* d_block_lat, uint32_t total_blocks, hipStream_t stream);
     // n_lattices small lattices (descriptors d_slots[i]), one workgroup each: `groups` groups of `sweeps` sweeps with a
     // sample after each group when sample_mode >= 0. max_sites, max_rows: bounds on their padded sites and on the

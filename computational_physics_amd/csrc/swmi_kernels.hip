@@ -620,7 +620,7 @@ namespace swmi
     }
 
     // =============================================================================================
-    // Observables: per-tile partial sums of sum s(s_right + s_down) and sum s (lattice.cpp:29-67)
+    // Observables: per-block partial sums of sum s(s_right + s_down) and sum s (lattice.cpp:29-67)
     // =============================================================================================
     // A conditional sample is due when the lattice has advanced since its last sample, is past its warmup
     // and sits on its own n_sep grid.
@@ -630,71 +630,186 @@ namespace swmi
         return it > st[kStLastSample] && it > meas && sep2 != 0u && (it - meas) % sep2 == 0u;
     }
 
+    // A flip that is still pending is applied on the way (from the labels and the flip bits, as k_bond_label does) and
+    // not stored: the spin array is read once (1 byte a site, 3 with the labels of a pending flip) and left for the
+    // next sweep. Per wave one tile: spin masks of its rows by ballot, one per lane, the neighbours by shifts and from
+    // the next lane; the row below the tile is read again by the tile above it (or comes from the halo across the block
+    // edge). Summing row by row with scalar operations was bound by the scalar unit (104 us at 8192^2).
     __global__ __launch_bounds__(256) void k_observables(const LatDesc* __restrict__ descs, const uint32_t* __restrict__ block_lat,
                                                          const uint32_t total_blocks, const uint32_t sample_mode)
     {
+        constexpr uint32_t kCh = 8;   // rows loaded together
+        constexpr uint32_t kMaxSites = kWavesPerBlock * 64u * 64u;
+        __shared__ uint32_t fb[2u * kMaxSites / 32u];
+        __shared__ int32_t s_e[kWavesPerBlock], s_m[kWavesPerBlock];
         const uint32_t b = RemapBlock(total_blocks);
         if (b >= total_blocks)
             return;
         const LatDesc& d = descs[LatticeOf(block_lat, b)];
         if (sample_mode == kSampleDue && !SampleDue(d.state))
             return;
+        const gptr<const uint32_t> stp = Glob(static_cast<const uint32_t*>(d.state));
+        const bool pending = stp[kStApplied] != stp[kStIteration];
         const Block bl = DecodeBlock(d, b);
         const uint32_t lane = threadIdx.x & 63u;
         const uint32_t w = Uniform(threadIdx.x >> 6);
         const uint32_t r_begin = w * d.twr;
         const uint32_t nrow = bl.nwr > r_begin ? min(d.twr, bl.nwr - r_begin) : 0u;
-        const uint32_t pitch = d.n0, n0v = d.n0v, n1 = d.n1, tw = d.tw, rpw = d.rpw;
-        const uint32_t x = bl.sx * tw + (lane & (tw - 1u));
-        // padding columns (x >= n0v) hold no site; the right neighbour of column n0v - 1 is column 0
-        const bool valid = x < n0v;
-        const int32_t nv = __popcll(__ballot(valid));
-        const uint32_t xr = (x + 1u >= n0v) ? 0u : x + 1u;
-        int32_t e = 0, m = 0;
-        for (uint32_t r = 0; r < nrow; ++r)
+        const bool last_wave = r_begin + nrow >= bl.nwr;
+        const uint32_t pitch = d.n0, tw = d.tw, qcap = d.qcap;
+        const bool lastcol = bl.sx + 1u == d.tiles_x;
+        const uint64_t vmask = lastcol ? d.vlast : ~0ull;   // lanes that hold sites
+        const uint32_t elane = lastcol ? d.elast : tw - 1u;  // a lattice row's last site in this tile
+        uint64_t rowstart = 1;
+        for (uint32_t j = tw; j < 64u; j += tw)
+            rowstart |= 1ull << j;
+        const uint64_t redge = rowstart << elane;
+        const uint64_t low = Shr(~0ull, tw);   // lanes whose lower neighbour sits in the same wave row
+        const uint32_t sx_r = lastcol ? 0u : bl.sx + 1u;
+        const uint32_t sy_b = bl.sy + 1u == d.blocks_y ? 0u : bl.sy + 1u;
+        const gptr<const uint8_t> spins = Glob(static_cast<const uint8_t*>(d.spins));
+        const gptr<const uint16_t> local = Glob(static_cast<const uint16_t*>(d.local));
+        const gptr<const uint8_t> halo = Glob(static_cast<const uint8_t*>(d.halo)) + stp[kStHaloSide] * d.n_blocks * d.halo_stride;
+
+        if (pending)
         {
-            const uint32_t y = (bl.wyb + r_begin + r) * rpw + lane / tw;
-            const uint32_t s = d.spins[y * pitch + x] & 1u;
-            const uint32_t sr = d.spins[y * pitch + xr] & 1u;
-            const uint32_t sd = d.spins[((y + 1u == n1) ? 0u : y + 1u) * pitch + x] & 1u;
-            e += 2 * (__popcll(__ballot(valid && s == sr)) + __popcll(__ballot(valid && s == sd))) - 2 * nv;
-            m += 2 * __popcll(__ballot(valid && s != 0)) - nv;
+            const gptr<const uint32_t> fbits_g = Glob(static_cast<const uint32_t*>(d.fbits)) + bl.lb * d.fsw;
+            for (uint32_t i = threadIdx.x; i < d.fsw; i += 256u)
+                fb[qcap / 32u + i] = fbits_g[i];
+            const bool random_rule = d.flip_rule != 0u;
+            const uint32_t key = random_rule ? FlipKey(d.seed, stp[kStApplied]) : 0u;
+            for (uint32_t i = threadIdx.x; i < bl.nwr * 2u; i += 256u)
+                fb[i] = RuleWord(d, bl, i, random_rule, key);
         }
-        if (lane == 0)
+        // 64-wide tiles: lane r's hr is the spin to the right of the tile's row r (narrower ones wrap inside the row)
+        uint32_t hr = 0;
+        if (tw == 64u && lane < nrow)
+            hr = pending ? halo[(bl.sy * d.tiles_x + sx_r) * d.halo_stride + r_begin + lane]
+                         : spins[(bl.wyb + r_begin + lane) * pitch + sx_r * 64u];
+
+        // the row below the tile: the next tile's first row, or across the block edge the halo (the flipped spins of a
+        // pending flip); loaded without conditions, like the rows of a chunk, so that the loads overlap
+        const uint32_t r_below = r_begin + (last_wave ? 0u : nrow);   // in range either way
+        const uint32_t site_below = last_wave && !pending ? BlockBase(d, bl.sx, sy_b) + lane : bl.base + r_below * bl.stride + lane;
+        const uint32_t below_sp = spins[site_below], below_lab = local[site_below];
+        const uint32_t below_halo = halo[(sy_b * d.tiles_x + bl.sx) * d.halo_stride + d.ecol_stride + lane];
+        __syncthreads();
+
+        const auto flip_of = [&](const uint32_t lab) {
+            const uint32_t i = lab & 0x7FFFu;
+            return fb[min(i >> 5, 2u * kMaxSites / 32u - 1u)] >> (i & 31u);
+        };
+        const uint64_t Sbelow = __ballot((((pending ? (last_wave ? below_halo : below_sp ^ flip_of(below_lab)) : below_sp)) & 1u) != 0u);
+        // lane r collects the mask of the tile's row r (nrow <= 64): the sums are then one row per lane
+        uint32_t Slo = 0, Shi = 0;
+        const uint32_t span = (bl.nwr - 1u) * bl.stride + 64u;
+        const Rsrc rs_spins = MakeRsrc(d.spins + bl.base, span), rs_local = MakeRsrc(d.local + bl.base, span * 2u);
+        const auto rows = [&](auto pending_t) {
+            constexpr bool kPend = decltype(pending_t)::value;
+            for (uint32_t r0 = 0; r0 < nrow; r0 += kCh)
+            {
+                uint32_t sp[kCh], lab[kCh];
+#pragma unroll
+                for (uint32_t k = 0; k < kCh; ++k)
+                {
+                    const uint32_t off = Uniform((r_begin + min(r0 + k, nrow - 1u)) * bl.stride);
+                    sp[k] = __builtin_amdgcn_raw_buffer_load_b8(rs_spins, lane, off, 0);
+                    lab[k] = kPend ? __builtin_amdgcn_raw_buffer_load_b16(rs_local, lane * 2u, off * 2u, 0) : 0u;
+                }
+#pragma unroll
+                for (uint32_t k = 0; k < kCh; ++k)
+                {
+                    const uint32_t r = r0 + k;
+                    if (r < nrow)
+                    {
+                        const uint64_t S = __ballot(((kPend ? sp[k] ^ flip_of(lab[k]) : sp[k]) & 1u) != 0u);
+                        Slo = LaneBit(1ull << r) ? static_cast<uint32_t>(S) : Slo;
+                        Shi = LaneBit(1ull << r) ? static_cast<uint32_t>(S >> 32) : Shi;
+                    }
+                }
+            }
+        };
+        if (pending)
+            rows(std::true_type{});
+        else
+            rows(std::false_type{});
+        int32_t e = 0, m = 0;
         {
-            const uint32_t t = kWavesPerBlock * bl.lb + w;
-            d.partials[2u * t] = e;
-            d.partials[2u * t + 1u] = m;
+            const uint64_t S = (static_cast<uint64_t>(Shi) << 32) | Slo;
+            const bool last = lane + 1u >= nrow;
+            const uint32_t dlo = __shfl_down(Slo, 1), dhi = __shfl_down(Shi, 1);
+            const uint64_t Sn = last ? Sbelow : (static_cast<uint64_t>(dhi) << 32) | dlo;
+            const uint64_t RS = ((S >> 1) & ~redge) | (tw == 64u ? static_cast<uint64_t>(hr & 1u) << elane : (S << elane) & redge);
+            const uint64_t SD = (Shr(S, tw) & low) | Shl(Sn, 64u - tw);
+            const int32_t nv = __popcll(vmask);
+            if (lane < nrow)
+            {
+                e = 2 * (__popcll(~(S ^ RS) & vmask) + __popcll(~(S ^ SD) & vmask)) - 2 * nv;
+                m = 2 * __popcll(S & vmask) - nv;
+            }
+        }
+        for (uint32_t s = 32; s > 0; s >>= 1)
+        {
+            e += __shfl_down(e, s);
+            m += __shfl_down(m, s);
+        }
+        if (lane == 0u)
+        {
+            s_e[w] = e;
+            s_m[w] = m;
+        }
+        __syncthreads();
+        if (threadIdx.x == 0)
+        {
+            d.partials[2u * bl.lb] = s_e[0] + s_e[1] + s_e[2] + s_e[3];
+            d.partials[2u * bl.lb + 1u] = s_m[0] + s_m[1] + s_m[2] + s_m[3];
         }
     }
 
-    // One workgroup per lattice: reduce the tile partials in a fixed order, append (E, M) to the series
-    // and accumulate the FP64 moments (the only FP64 on the device).
-    __global__ __launch_bounds__(256) void k_finalize_samples(const LatDesc* __restrict__ descs, const uint32_t* __restrict__ slots,
-                                                              const uint32_t sample_mode)
+    // One workgroup per lattice: reduce the block partials (whole numbers: any order), append (E, M) to the series
+    // and accumulate the FP64 moments (the only FP64 of the tiled path).
+    __global__ __launch_bounds__(1024) void k_finalize_samples(const LatDesc* __restrict__ descs, const uint32_t* __restrict__ slots,
+                                                               const uint32_t sample_mode)
     {
-        __shared__ long long red_e[256], red_m[256];
+        constexpr uint32_t kWaves = 16, kCh = 8;   // entries loaded together per thread
+        __shared__ long long red_e[kWaves], red_m[kWaves];
         const LatDesc& d = descs[slots[blockIdx.x]];
         if (sample_mode == kSampleDue && !SampleDue(d.state))
             return;
         long long e = 0, m = 0;
-        for (uint32_t i = threadIdx.x; i < kWavesPerBlock * d.n_blocks; i += 256u)
+        const gptr<const u32x2> part = (gptr<const u32x2>)(d.partials);
+        const uint32_t n_blocks = d.n_blocks;
+        for (uint32_t i = threadIdx.x; i < n_blocks; i += kCh * 1024u)
         {
-            e += d.partials[2u * i];
-            m += d.partials[2u * i + 1u];
+            u32x2 v[kCh];
+#pragma unroll
+            for (uint32_t k = 0; k < kCh; ++k)
+                v[k] = part[min(i + k * 1024u, n_blocks - 1u)];
+#pragma unroll
+            for (uint32_t k = 0; k < kCh; ++k)
+                if (i + k * 1024u < n_blocks)
+                {
+                    e += static_cast<int32_t>(v[k].x);
+                    m += static_cast<int32_t>(v[k].y);
+                }
         }
-        red_e[threadIdx.x] = e;
-        red_m[threadIdx.x] = m;
+        for (uint32_t s = 32; s > 0; s >>= 1)
+        {
+            e += __shfl_down(e, s);
+            m += __shfl_down(m, s);
+        }
+        if ((threadIdx.x & 63u) == 0u)
+        {
+            red_e[threadIdx.x >> 6] = e;
+            red_m[threadIdx.x >> 6] = m;
+        }
         __syncthreads();
-        for (uint32_t s = 128; s > 0; s >>= 1)
-        {
-            if (threadIdx.x < s)
+        if (threadIdx.x == 0)
+            for (uint32_t k = 1; k < kWaves; ++k)
             {
-                red_e[threadIdx.x] += red_e[threadIdx.x + s];
-                red_m[threadIdx.x] += red_m[threadIdx.x + s];
+                red_e[0] += red_e[k];
+                red_m[0] += red_m[k];
             }
-            __syncthreads();
-        }
         if (threadIdx.x == 0)
         {
             LatState* st = reinterpret_cast<LatState*>(d.state);
@@ -944,23 +1059,23 @@ namespace swmi
     // =============================================================================================
     // defined in swmi_bond.hip, one part per combination
     template <bool TW64, bool DBG>
-    void LaunchBondLabelT(const LatDesc* d_desc, const uint32_t* d_block_lat, uint32_t total_blocks, uint32_t max_twr, bool pad,
+    void LaunchBondLabelT(const LatDesc* d_desc, const uint32_t* d_block_lat, uint32_t total_blocks, uint32_t max_twr, bool quads, bool pad,
                           hipStream_t stream);
 
     void LaunchBondLabel(const LatDesc* d_desc, const uint32_t* d_block_lat, const uint32_t total_blocks, const uint32_t max_twr,
-                         const bool all_tw64, const bool pad, const bool debug, hipStream_t stream)
+                         const bool quads, const bool all_tw64, const bool pad, const bool debug, hipStream_t stream)
     {
         if (debug)
         {
             if (all_tw64)
-                LaunchBondLabelT<true, true>(d_desc, d_block_lat, total_blocks, max_twr, pad, stream);
+                LaunchBondLabelT<true, true>(d_desc, d_block_lat, total_blocks, max_twr, quads, pad, stream);
             else
-                LaunchBondLabelT<false, true>(d_desc, d_block_lat, total_blocks, max_twr, pad, stream);
+                LaunchBondLabelT<false, true>(d_desc, d_block_lat, total_blocks, max_twr, quads, pad, stream);
         }
         else if (all_tw64)
-            LaunchBondLabelT<true, false>(d_desc, d_block_lat, total_blocks, max_twr, pad, stream);
+            LaunchBondLabelT<true, false>(d_desc, d_block_lat, total_blocks, max_twr, quads, pad, stream);
         else
-            LaunchBondLabelT<false, false>(d_desc, d_block_lat, total_blocks, max_twr, pad, stream);
+            LaunchBondLabelT<false, false>(d_desc, d_block_lat, total_blocks, max_twr, quads, pad, stream);
     }
 
     // Two-wave merge workgroups resident at once on MI355X: 256 CUs x 16 (8 waves per SIMD).
@@ -1035,7 +1150,7 @@ namespace swmi
     void LaunchFinalizeSamples(const LatDesc* d_desc, const uint32_t* d_slots, const uint32_t n_lattices, const uint32_t sample_mode,
                                hipStream_t stream)
     {
-        k_finalize_samples<<<n_lattices, 256, 0, stream>>>(d_desc, d_slots, sample_mode);
+        k_finalize_samples<<<n_lattices, 1024, 0, stream>>>(d_desc, d_slots, sample_mode);
     }
 
     void LaunchInitState(uint32_t* state, uint32_t* aux, const uint32_t words, const uint32_t series_cap, const uint32_t it_end,
