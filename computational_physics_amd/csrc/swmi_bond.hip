@@ -837,12 +837,12 @@ namespace swmi
         BondLabel<kWavesPerBlock, TWR_MAX, true, DBG, false>(descs, block_lat, total_blocks);
     }
 
-    // Sixteen waves per block, strips of up to 4 rows.
-    template <bool DBG, bool PAD>
-    __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(8, 8))) void k_bond_label_wide(
+    // Sixteen or eight waves per block, strips of up to 4 or 8 rows.
+    template <uint32_t NW, bool DBG, bool PAD>
+    __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(8, 8))) void k_bond_label_wide(
         const LatDesc* __restrict__ descs, const uint32_t* __restrict__ block_lat, const uint32_t total_blocks)
     {
-        BondLabel<16, 4, true, DBG, PAD>(descs, block_lat, total_blocks);
+        BondLabel<NW, 64 / NW, true, DBG, PAD>(descs, block_lat, total_blocks);
     }
 
     template <uint32_t TWR_MAX, bool TW64, bool DBG, bool PAD>
@@ -852,9 +852,11 @@ namespace swmi
         BondLabel<kWavesPerBlock, TWR_MAX, TW64, DBG, PAD>(descs, block_lat, total_blocks);
     }
 
-    // Launches of at most this many blocks of 64-wide tiles, all of a height that four waves can share, give every
-    // block sixteen waves.
-    constexpr uint32_t kWideBlocks = 512;
+    // Launches of few blocks of 64-wide tiles, all of a height that four waves can share, give every block more waves:
+    // sixteen up to one block per CU, eight up to two. Microseconds per sweep with 4 / 8 / 16 waves: 256 blocks
+    // (1024^2) 28.0 / - / 24.2, 352 blocks (1000 x 1350) 25.4 / 23.7 / 25.1, 1024 blocks (2048^2) 38.6 / 38.8 / 46.
+    constexpr uint32_t kWideBlocks = 256;
+    constexpr uint32_t kHalfBlocks = 512;
 
     template <bool TW64, bool DBG>
     void LaunchBondLabelT(const LatDesc* d_desc, const uint32_t* d_block_lat, const uint32_t total_blocks, const uint32_t max_twr,
@@ -868,7 +870,12 @@ namespace swmi
         {
             if (quads && max_twr <= 16 && total_blocks <= kWideBlocks)
             {
-                pad ? launch(k_bond_label_wide<DBG, true>, 1024) : launch(k_bond_label_wide<DBG, false>, 1024);
+                pad ? launch(k_bond_label_wide<16, DBG, true>, 1024) : launch(k_bond_label_wide<16, DBG, false>, 1024);
+                return;
+            }
+            if (quads && max_twr <= 16 && total_blocks <= kHalfBlocks)
+            {
+                pad ? launch(k_bond_label_wide<8, DBG, true>, 512) : launch(k_bond_label_wide<8, DBG, false>, 512);
                 return;
             }
         }

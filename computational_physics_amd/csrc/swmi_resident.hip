@@ -155,8 +155,7 @@ namespace swmi
         const uint32_t last_active = it_end > it ? (it_end - it - 1u) / 2u + 1u : 0u;   // sweeps until the schedule ends
         const uint32_t total = min(groups * sweeps, last_active);
         uint32_t done = 0;
-        uint32_t labelled = 0;   // rows the wave has labelled in this launch (kResidentRows * sweeps, below 2^16)
-        Qw[lane] = 0u;
+        Qw[lane] = 0u;   // run words of LabelRow64
 
         const auto first_col = [&]() -> uint64_t {   // bit i: spin of row i's right neighbour column
             uint32_t h = 0;
@@ -193,6 +192,13 @@ namespace swmi
                 drain64(qlen);
         };
 
+        const auto drain = [&](const uint32_t qlen) {
+            if (qlen == 0u)
+                return;
+            const uint32_t e = lane < qlen ? Qw[lane] : 0u;
+            LdsUnionLockstep(P, e >> 16, e & 0xFFFFu);
+        };
+
         const auto sweep = [&](const bool last) {
             const uint32_t it1 = it + 1u, it2 = it + 2u;
             const bool rot1 = it1 % 15u == 0u, rot2 = it2 % 15u == 0u;
@@ -200,6 +206,7 @@ namespace swmi
             const uint64_t Sbelow = nrow > 0u ? uniform64(sS[gbelow]) : 0ull;
             uint64_t right_bits = 0, prev_S = 0, prev_U2 = 0, prev_B = 0;
             uint32_t Rp = 0;
+            uint32_t xs[kR];   // every row's root: as the row was labelled, later the root of the whole forest
             uint64_t Snext = nrow > 0u ? __ballot((sp[0] & 1u) != 0u) : 0ull;
 #pragma unroll
             for (uint32_t i = 0; i < kR; ++i)
@@ -240,7 +247,8 @@ namespace swmi
                     {
                         right_bits |= ((Ball >> elane) & 1ull) << i;
                         const uint64_t D = i == 0u ? 0ull : (~(prev_S ^ S) & prev_U2);
-                        Rp = LabelRow64(P, Qw, dummy, node, B, D, Rp, RowBase(++labelled));
+                        Rp = LabelRow64(P, Qw, dummy, node, B, D, Rp, RowBase(i + 1u));
+                        xs[i] = Rp;
                         if (i == 0u && lane == 0u)
                             sB[w] = B;
                     }
@@ -273,12 +281,12 @@ namespace swmi
                     // down, into the first row of the strip below (this strip's own where it is alone in its column)
                     const uint64_t Dl = ~(prev_S ^ Sbelow) & prev_U2;
                     const uint64_t Bn = uniform64(sB[ybelow == 0u ? col : (strip + 1u) * tx + col]);
-                    const bool go = LaneBit(FirstBondPerInterval(Dl, prev_B & Bn, 1ull));
-                    LdsUnionLockstep(P, go ? node0 + (nrow - 1u) * rowb : 0u, go ? node_below : 0u);
+                    uint32_t qlen = 0;
+                    push(FirstBondPerInterval(Dl, prev_B & Bn, 1ull), Rp, node_below, qlen);
                     // right, one lane per row
-                    const bool gr = LaneBit(right_bits);
-                    const uint32_t a = ((y0 + lane) * tx + col) * 256u + elane * 4u, b = ((y0 + lane) * tx + cright) * 256u;
-                    LdsUnionLockstep(P, gr ? a : 0u, gr ? b : 0u);
+                    push(right_bits, ((y0 + lane) * tx + col) * 256u + elane * 4u, ((y0 + lane) * tx + cright) * 256u, qlen);
+                    drain(qlen);
+                    Qw[lane] = 0u;   // the queue took the run words' place
                 }
                 else
                 {
@@ -292,21 +300,17 @@ namespace swmi
                         push(K, top, lane < 64u - tw ? top + tw * 4u : yn * 256u + lane4 - (64u - tw) * 4u, qlen);
                         push(uniform64(sE[y]), top, top - elane * 4u, qlen);
                     }
-                    if (qlen > 0u)
-                    {
-                        const uint32_t e = lane < qlen ? Qw[lane] : 0u;
-                        LdsUnionLockstep(P, e >> 16, e & 0xFFFFu);
-                    }
+                    drain(qlen);
                 }
             }
             __syncthreads();   // the forest is complete
 
             if (nrow > 0u)
             {
-                uint32_t xs[kR];
 #pragma unroll
                 for (uint32_t i = 0; i < kR; ++i)
-                    xs[i] = node0 + (i < nrow ? i : 0u) * rowb;
+                    if (!TW64 || i >= nrow)
+                        xs[i] = node0 + (i < nrow ? i : 0u) * rowb;
                 // two steps per round, every row of the lane in flight (parents only decrease: a chase that does not
                 // end within the sites is a broken forest, reported instead of followed)
                 for (uint32_t round = 0;; ++round)
@@ -337,20 +341,34 @@ namespace swmi
                     if (!__ballot(moved != 0u))
                         break;
                 }
-                const uint32_t key = random_rule ? FlipKey(seed, it) : 0u;
+                // the flips; lane i collects the spin mask of row i and stores it
+                uint32_t Slo = 0, Shi = 0;
+                const auto flip = [&](const auto& bit_of) {
 #pragma unroll
-                for (uint32_t i = 0; i < kR; ++i)
-                {
-                    if (i < nrow)
+                    for (uint32_t i = 0; i < kR; ++i)
                     {
-                        sp[i] ^= FlipBit(d, xs[i] >> 2, random_rule, key);
+                        sp[i] ^= bit_of(xs[i] >> 2);
                         const uint64_t S = __ballot((sp[i] & 1u) != 0u);
-                        if (lane == 0u)
-                            sS[g0 + i * gstep] = S;
-                        if (last)
+                        Slo = LaneBit(1ull << i) ? static_cast<uint32_t>(S) : Slo;
+                        Shi = LaneBit(1ull << i) ? static_cast<uint32_t>(S >> 32) : Shi;
+                    }
+                };
+                if (random_rule)
+                {
+                    const uint32_t key = FlipKey(seed, it);
+                    flip([&](const uint32_t root) { return FlipBit(d, root, true, key); });
+                }
+                else
+                    flip([&](const uint32_t root) { return FlipBit(d, root, false, 0u); });
+                if (lane < nrow)
+                    sS[g0 + lane * gstep] = (static_cast<uint64_t>(Shi) << 32) | Slo;
+                if (last)
+                {
+#pragma unroll
+                    for (uint32_t i = 0; i < kR; ++i)
+                        if (i < nrow)
                             __builtin_amdgcn_raw_buffer_store_b16(static_cast<uint16_t>(xs[i] >> 2), rs_local, lane * 2u,
                                                                   (g0 + i * gstep) * 128u, 0);
-                    }
                 }
             }
             it = it2;
