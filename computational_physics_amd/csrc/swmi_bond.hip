@@ -29,7 +29,8 @@ namespace swmi
     // NW: waves of the workgroup, each with a strip of 4 * twr / NW wave rows of the block, at most TWR_MAX. Four
     // waves label a tile each; sixteen label a quarter tile each, which shortens the chain of dependent LDS
     // operations down a strip where a launch has too few blocks to fill the chip (LaunchBondLabelT).
-    template <uint32_t NW, uint32_t TWR_MAX, bool TW64, bool DBG, bool PAD>
+    // FULL: every strip of every block has exactly TWR_MAX rows, so that the row counts are constants.
+    template <uint32_t NW, uint32_t TWR_MAX, bool TW64, bool DBG, bool PAD, bool FULL>
     __device__ __forceinline__ void BondLabel(const LatDesc* __restrict__ descs, const uint32_t* __restrict__ block_lat,
                                               const uint32_t total_blocks)
     {
@@ -39,6 +40,8 @@ namespace swmi
         constexpr uint32_t kRows = TWR_MAX < 16 ? TWR_MAX : 16;   // rows resolved together at the end
         // 64-wide tiles of at most kRows rows keep their rows' roots in registers from the row loop to the labels
         constexpr bool kKeep = TW64 && TWR_MAX <= kRows;
+        // and collect what the edges of the tile need as bits of scalar words
+        constexpr bool kBits = kKeep && !PAD && !DBG;
         constexpr uint32_t kSites = NW * TWR_MAX * 64;
         constexpr uint32_t kThreads = NW * 64u;
         constexpr uint32_t kQw = 128u;                             // per-wave LDS words of Q
@@ -52,9 +55,9 @@ namespace swmi
         __shared__ uint32_t Q[NW * kQw];
         __shared__ uint32_t FB[2u * kSites / 32u];   // flip bits of a pending flip, by label index (root or qcap + slot)
         __shared__ uint64_t s_first_B[NW];
-        // Numerical Recipes pairs (c << 32 | a) by selector: words 0-7 one update, words 8-15 the jump from the stored
-        // states to this sweep's
-        __shared__ uint64_t AC[16];
+        // Numerical Recipes pairs (a << 32 | c: the loaded pair is the 64-bit addend of the multiply-add as it is) by
+        // selector: words 0-7 one update, words 8-15 the jump from the stored states to this sweep's
+        __shared__ __align__(128) uint64_t AC[16];
         __shared__ uint64_t s_right[NW == kWavesPerBlock ? 1u : kWavesPerBlock];   // bonds across the right edge, per tile
         __shared__ uint32_t s_nslot;            // slots given to the block's edge-reaching clusters
 
@@ -71,7 +74,8 @@ namespace swmi
         const uint32_t lane4 = lane * 4u;
         const uint32_t w = Uniform(threadIdx.x >> 6);
 
-        const uint32_t n0 = d.n0, n1 = d.n1, twr = d.twr * kWavesPerBlock / NW;   // wave rows of a strip
+        const uint32_t n0 = d.n0, n1 = d.n1, twr = FULL ? TWR_MAX : d.twr * kWavesPerBlock / NW;   // wave rows of a strip
+        const uint32_t bnwr = FULL ? NW * TWR_MAX : bl.nwr;                                          // and of the block
         const uint32_t tw = TW64 ? 64u : d.tw, rpw = TW64 ? 1u : d.rpw;
         const uint32_t lx = lane & (tw - 1u);
         const uint32_t lrow = TW64 ? 0u : lane / tw;
@@ -89,15 +93,15 @@ namespace swmi
         const gptr<const uint8_t> bond_in = Glob(d.bond_in);
 
         const uint32_t r_begin = w * twr;
-        const uint32_t nrow = bl.nwr > r_begin ? min(twr, bl.nwr - r_begin) : 0u;
+        const uint32_t nrow = FULL ? TWR_MAX : (bnwr > r_begin ? min(twr, bnwr - r_begin) : 0u);
         // buffer views of this block's part of the per-site arrays (row offsets in scalar registers, the lane
         // offset in a vector register, no per-row vector addresses)
-        const uint32_t span = (bl.nwr - 1u) * bl.stride + 64u;   // sites from the block's first to its last
+        const uint32_t span = (bnwr - 1u) * bl.stride + 64u;   // sites from the block's first to its last
         const Rsrc rs_spins = MakeRsrc(d.spins + bl.base, span);
         const Rsrc rs_rng = MakeRsrc(d.rng + bl.base, span * 4u);
         const Rsrc rs_local = MakeRsrc(d.local + bl.base, span * 2u);
         const gptr<const uint32_t> fbits_g = Glob(static_cast<const uint32_t*>(d.fbits)) + bl.lb * d.fsw;
-        const uint32_t nwaves = (bl.nwr + twr - 1u) / twr;
+        const uint32_t nwaves = (bnwr + twr - 1u) / twr;
         const bool last_wave = w + 1u == nwaves;
         const uint32_t sx_r = bl.sx + 1u == d.tiles_x ? 0u : bl.sx + 1u;   // block column to the right
         const uint32_t sy_b = bl.sy + 1u == d.blocks_y ? 0u : bl.sy + 1u;   // block row below
@@ -183,6 +187,7 @@ namespace swmi
         uint32_t* const Qw = Q + w * kQw;
         uint32_t* const Pl = At(P, lane4);   // this lane's entry of wave row 0
         uint32_t* const dummy = Qw + 64u + lane;
+        const uint32_t run_words = OffsetFrom(P, Qw), spare = OffsetFrom(P, dummy);
         // a full queue (>= 64 entries) is worked off right away; the tail moves to the front
         const auto drain64 = [&](uint32_t& qlen) {
             const uint32_t e = Qw[lane];
@@ -208,6 +213,12 @@ namespace swmi
         // pending flip: the block's flip bits (loaded into FB above), one per label index (k_resolve wrote the
         // bit of every cluster: by root index, or by qcap + slot for an edge-reaching one), so a site's flip is
         // the bit at its label's index
+        const uint32_t ac_at = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) uint64_t*)AC));
+        // the pair of the selector bits ks of a spin byte, in half `first` of AC (AC's alignment makes the sum an or)
+        const auto pair_of = [&](const uint32_t ks, const uint32_t first) {
+            static_assert(kSelMask == 7u * sizeof(uint64_t), "the selector bits are a byte offset into AC");
+            return ((__attribute__((address_space(3))) const uint64_t*)static_cast<uintptr_t>(ac_at | ks))[first];
+        };
         const auto flip_of = [&](const uint32_t lab) { return (LdsLoad(&FB[(lab & 0x7FFFu) >> 5]) >> (lab & 31u)) & 1u; };
 
         // spins below the tile (down halo), needed last but fetched first. Under a pending flip, below the
@@ -232,16 +243,16 @@ namespace swmi
                         ja *= a;
                         jc = a * jc + c;
                     }
-                    AC[threadIdx.x] = (static_cast<uint64_t>(c) << 32) | a;
-                    AC[8u + threadIdx.x] = (static_cast<uint64_t>(jc) << 32) | ja;
+                    AC[threadIdx.x] = (static_cast<uint64_t>(a) << 32) | c;
+                    AC[8u + threadIdx.x] = (static_cast<uint64_t>(ja) << 32) | jc;
                 }
                 if (threadIdx.x < d.fsw)
                     FB[d.qcap / 32u + threadIdx.x] = fbw;
                 if (d.flip_rule == 0u)
-                    for (uint32_t i = threadIdx.x; i < bl.nwr * 2u; i += kThreads)   // bl.nwr * 64 root indices, 32 per word
+                    for (uint32_t i = threadIdx.x; i < bnwr * 2u; i += kThreads)   // bl.nwr * 64 root indices, 32 per word
                         FB[i] = RuleWord(d, bl, i, false, 0u);
                 else if (pending)   // the random rule's words, with the key of the pending flip's sweep
-                    for (uint32_t i = threadIdx.x; i < bl.nwr * 2u; i += kThreads)
+                    for (uint32_t i = threadIdx.x; i < bnwr * 2u; i += kThreads)
                         FB[i] = RuleWord(d, bl, i, true, FlipKey(d.seed, it0 - 2u));
             }
             if (nrow > 0)
@@ -271,6 +282,9 @@ namespace swmi
         uint64_t prev_S = 0, prev_U2 = 0, prev_B = 0, prev_Ball = 0;
         uint32_t prev_site = 0;
         uint32_t colv = 0;   // 64-wide tiles: lane r collects the first-column spin of row r
+        // kBits: the rows' first-column spin, last-column spin and last-column draw, the latest row in bit 0, and the
+        // spins right of the tile (lane r: row r)
+        uint32_t col_b = 0, s63_b = 0, u63_b = 0, hright = 0;
         {
             // the chunk loop exists twice: sweeps without a group rotation (13 in 15) carry no rotation code
             // (and twice more for the sweeps that apply a pending flip on load, the rule after any sweep)
@@ -292,7 +306,7 @@ namespace swmi
                 const uint32_t lrow_ch = r_begin + min(r0 + (lane % kC), nrow - 1u);
                 // right halo of a 64-wide tile: under a pending flip the right neighbour's flipped first column
                 c.h = 0;
-                if (TW64)
+                if (TW64 && !kBits)
                     c.h = pending ? halo_g[(bl.sy * d.tiles_x + sx_r) * d.halo_stride + lrow_ch]
                                   : spins[(bl.wyb + lrow_ch) * n0 + sx_r * 64u];
                 // rotation offsets of the chunk's groups, needed on rotating sweeps only
@@ -320,7 +334,7 @@ namespace swmi
                     for (uint32_t i = 0; i < kC; ++i)
                         sp[i] ^= flip_of(lab[i]);
                 }
-                const uint64_t HR = TW64 ? __ballot((h & 1u) != 0u) : 0ull;
+                const uint64_t HR = TW64 && !kBits ? __ballot((h & 1u) != 0u) : 0ull;
 
 #pragma unroll
                 for (uint32_t i = 0; i < kC; ++i)
@@ -331,11 +345,16 @@ namespace swmi
                         const uint32_t wr = r_begin + r;
                         const uint32_t site = bl.base + wr * bl.stride + lane;
                         const uint64_t S = __ballot((sp[i] & 1u) != 0u);
-                        if (TW64)
+                        if (kBits)
+                        {
+                            col_b = (col_b << 1) + (static_cast<uint32_t>(S) & 1u);
+                            s63_b = (s63_b << 1) + static_cast<uint32_t>(S >> 63);
+                        }
+                        else if (TW64)
                             colv = LaneBit(1ull << r) ? static_cast<uint32_t>(S) : colv;   // bit 0 of S: lane 0's spin
                         else
                             __builtin_amdgcn_raw_buffer_store_b8(static_cast<uint8_t>(sp[i] & 1u), rs_halo, hcol_off, wr * rpw, 0);
-                        if (wr == 0 && !injected)
+                        if (r == 0 && r_begin == 0u && !injected)
                             __builtin_amdgcn_raw_buffer_store_b8(static_cast<uint8_t>(sp[i] & 1u), rs_halo, d.ecol_stride + lane, 0, 0);
                         uint64_t Ball, U2;
                         if (!injected)
@@ -344,20 +363,20 @@ namespace swmi
                             // (random/src/lcg32.cpp:51-84); a rotation by `shift` moves lane
                             // (i + shift) & 63's selector to lane i
                             uint32_t ks = sp[i] & kSelMask, shift = 0;
-                            const uint64_t jump = AC[8u + (ks >> kSelShift)];
-                            uint64_t ac = AC[ks >> kSelShift];
-                            uint32_t u1 = static_cast<uint32_t>(jump) * aux[i] + static_cast<uint32_t>(jump >> 32);
+                            const uint64_t jump = pair_of(ks, 8u);
+                            uint64_t ac = pair_of(ks, 0u);
+                            uint32_t u1 = static_cast<uint32_t>(jump >> 32) * aux[i] + static_cast<uint32_t>(jump);
                             if (kRot)
                             {
                                 // the state jumped to is the one the rotation works on and the one stored
                                 __builtin_amdgcn_raw_buffer_store_b32(u1, rs_rng, lane4, Uniform(wr * bl.stride) * 4u, 0);
                                 shift = ShuffleShift(u1, rot1 ? it1 : it2) & 63u;
                                 ks = static_cast<uint32_t>(__shfl(static_cast<int>(ks), static_cast<int>((lane + shift) & 63u)));
-                                ac = AC[ks >> kSelShift];
+                                ac = pair_of(ks, 0u);
                                 if (rot1)
-                                    u1 = static_cast<uint32_t>(ac) * u1 + static_cast<uint32_t>(ac >> 32);
+                                    u1 = static_cast<uint32_t>(ac >> 32) * u1 + static_cast<uint32_t>(ac);
                             }
-                            const uint32_t st = static_cast<uint32_t>(ac) * u1 + static_cast<uint32_t>(ac >> 32);
+                            const uint32_t st = static_cast<uint32_t>(ac >> 32) * u1 + static_cast<uint32_t>(ac);
                             if (kRot)
                             {
                                 spins[site] = static_cast<uint8_t>((sp[i] & 1u) | ks);
@@ -372,7 +391,12 @@ namespace swmi
                             // tiles) or the first column of the same lattice row (narrow tiles: one tile
                             // column)
                             uint64_t RS;
-                            if (!PAD)
+                            if (kBits)
+                            {
+                                RS = S >> 1;   // the last column's bond follows after the rows
+                                u63_b = (u63_b << 1) + static_cast<uint32_t>(U1 >> 63);
+                            }
+                            else if (!PAD)
                                 RS = TW64 ? ((S >> 1) | (((HR >> i) & 1ull) << 63))
                                           : (((S >> 1) & in_right) | ((S << (tw - 1u)) & ~in_right));
                             else
@@ -392,7 +416,10 @@ namespace swmi
                         }
                         const uint64_t B = Ball & in_right;
                         const uint64_t edge = Ball & redge;
-                        if (TW64)
+                        if (kBits)
+                        {
+                        }
+                        else if (TW64)
                             right_bits |= (PAD ? ((edge >> elane) & 1ull) : (edge >> 63)) << r;
                         else
                             for (uint32_t j = 0; j < rpw; ++j)
@@ -406,7 +433,7 @@ namespace swmi
                             const uint64_t D = r == 0 ? 0ull : (injected ? prev_U2 : (~(prev_S ^ S) & prev_U2));
                             if (dump && r > 0)
                                 dump[prev_site] = static_cast<uint8_t>((LaneBit(prev_Ball) ? 1u : 0u) | (LaneBit(D) ? 2u : 0u));
-                            Rp = LabelRow64(P, Qw, dummy, row_b + lane4, B, D, Rp, RowBase(r + 1u));
+                            Rp = LabelRow64(P, run_words, spare, row_b + lane4, B, D, Rp, RowBase(r + 1u));
                             if (kKeep)
                             {
                                 if (i % 2u == 0u)
@@ -444,6 +471,13 @@ namespace swmi
                                     dump[prev_site] = static_cast<uint8_t>((LaneBit(prev_Ball) ? 1u : 0u) | (LaneBit(D) ? 2u : 0u));
                             }
                         }
+                        if (kBits)   // the three words take this row's bits here (the compiler would keep every row's masks)
+                        {
+                            col_b = Uniform(col_b);
+                            s63_b = Uniform(s63_b);
+                            u63_b = Uniform(u63_b);
+                            asm volatile("" : "+s"(col_b), "+s"(s63_b), "+s"(u63_b));
+                        }
                         prev_S = S;
                         prev_U2 = U2;
                         prev_B = B;
@@ -457,6 +491,12 @@ namespace swmi
             Chunk c0;
             if (nrow > 0)
                 load(0u, c0);
+            if (kBits && nrow > 0)
+            {
+                // right halo of the tile's rows: under a pending flip the right neighbour's flipped first column
+                const uint32_t lr = r_begin + min(lane, nrow - 1u);
+                hright = kPend ? halo_g[(bl.sy * d.tiles_x + sx_r) * d.halo_stride + lr] : spins[(bl.wyb + lr) * n0 + sx_r * 64u];
+            }
             meet();
             if (nrow == 0)
                 return;
@@ -493,6 +533,14 @@ namespace swmi
         }
         if (nrow > 0)
         {
+            if (kBits)
+            {
+                // row r of the words is bit nrow - 1 - r
+                const uint32_t up = 32u - nrow;   // (nrow is 1 to 16)
+                const uint32_t h = static_cast<uint32_t>(__ballot((hright & 1u) != 0u));
+                right_bits = ~((__brev(s63_b) >> up) ^ h) & (__brev(u63_b) >> up);
+                colv = (__brev(col_b) >> up) >> (lane & 31u);
+            }
             if (NW != kWavesPerBlock && lane == 0u && right_bits != 0ull)   // read after the last barrier
                 (void)__hip_atomic_fetch_or(&s_right[r_begin / d.twr], right_bits << (r_begin % d.twr), __ATOMIC_RELAXED,
                                             __HIP_MEMORY_SCOPE_WORKGROUP);
@@ -794,7 +842,7 @@ namespace swmi
                 __builtin_amdgcn_raw_buffer_store_b32(e, rs_ecol, ecol_off, r * rpw * 4u, 0);
                 if (wr == 0u)
                     __builtin_amdgcn_raw_buffer_store_b32(e, rs_erow, lane4, 0, 0);
-                if (wr + 1u == bl.nwr)
+                if (wr + 1u == bnwr)
                     __builtin_amdgcn_raw_buffer_store_b32(e, rs_erow, lane4, 256u, 0);
             };
             if (one_chunk)
@@ -830,26 +878,19 @@ namespace swmi
     // 64-wide tiles of up to 16 rows: eight waves per SIMD (the register budget is asked for explicitly; the compiler
     // keeps the excess scalar registers in vector lanes). Narrow tiles keep the default budget (the cap would spill
     // vector registers to scratch), and taller tiles are limited by their LDS anyway.
-    template <uint32_t TWR_MAX, bool DBG>
-    __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8, 8))) void k_bond_label(
+    // NW waves per block: four take a tile each, eight and sixteen a half and a quarter of a tile.
+    template <uint32_t NW, uint32_t TWR_MAX, bool DBG, bool PAD, bool FULL>
+    __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(8, 8))) void k_bond_label(
         const LatDesc* __restrict__ descs, const uint32_t* __restrict__ block_lat, const uint32_t total_blocks)
     {
-        BondLabel<kWavesPerBlock, TWR_MAX, true, DBG, false>(descs, block_lat, total_blocks);
-    }
-
-    // Sixteen or eight waves per block, strips of up to 4 or 8 rows.
-    template <uint32_t NW, bool DBG, bool PAD>
-    __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(8, 8))) void k_bond_label_wide(
-        const LatDesc* __restrict__ descs, const uint32_t* __restrict__ block_lat, const uint32_t total_blocks)
-    {
-        BondLabel<NW, 64 / NW, true, DBG, PAD>(descs, block_lat, total_blocks);
+        BondLabel<NW, TWR_MAX, true, DBG, PAD, FULL>(descs, block_lat, total_blocks);
     }
 
     template <uint32_t TWR_MAX, bool TW64, bool DBG, bool PAD>
     __global__ __launch_bounds__(256) void k_bond_label_any(const LatDesc* __restrict__ descs, const uint32_t* __restrict__ block_lat,
                                                             const uint32_t total_blocks)
     {
-        BondLabel<kWavesPerBlock, TWR_MAX, TW64, DBG, PAD>(descs, block_lat, total_blocks);
+        BondLabel<kWavesPerBlock, TWR_MAX, TW64, DBG, PAD, false>(descs, block_lat, total_blocks);
     }
 
     // Launches of few blocks of 64-wide tiles, all of a height that four waves can share, give every block more waves:
@@ -860,7 +901,7 @@ namespace swmi
 
     template <bool TW64, bool DBG>
     void LaunchBondLabelT(const LatDesc* d_desc, const uint32_t* d_block_lat, const uint32_t total_blocks, const uint32_t max_twr,
-                          const bool quads, const bool pad, hipStream_t stream)
+                          const BondForm form, const bool pad, hipStream_t stream)
     {
         const uint32_t g = XcdGrid(total_blocks);
         const auto launch = [&](auto kernel, const uint32_t threads = 256) {
@@ -868,16 +909,24 @@ namespace swmi
         };
         if constexpr (TW64)
         {
-            if (quads && max_twr <= 16 && total_blocks <= kWideBlocks)
-            {
-                pad ? launch(k_bond_label_wide<16, DBG, true>, 1024) : launch(k_bond_label_wide<16, DBG, false>, 1024);
-                return;
-            }
-            if (quads && max_twr <= 16 && total_blocks <= kHalfBlocks)
-            {
-                pad ? launch(k_bond_label_wide<8, DBG, true>, 512) : launch(k_bond_label_wide<8, DBG, false>, 512);
-                return;
-            }
+            // NW waves per block
+            const auto launch_nw = [&](auto nw) {
+                constexpr uint32_t NW = decltype(nw)::value;
+                if (pad)
+                    launch(k_bond_label<NW, 64 / NW, DBG, true, false>, 64 * NW);
+                else if (!DBG && form == BondForm::kFull)
+                    launch(k_bond_label<NW, 64 / NW, DBG, false, !DBG>, 64 * NW);
+                else
+                    launch(k_bond_label<NW, 64 / NW, DBG, false, false>, 64 * NW);
+            };
+            if (form != BondForm::kAny && max_twr <= 16 && total_blocks <= kWideBlocks)
+                return launch_nw(std::integral_constant<uint32_t, 16>{});
+            if (form != BondForm::kAny && max_twr <= 16 && total_blocks <= kHalfBlocks)
+                return launch_nw(std::integral_constant<uint32_t, 8>{});
+            if (!pad && max_twr <= 8)
+                return launch(k_bond_label<kWavesPerBlock, 8, DBG, false, false>);
+            if (!pad && max_twr <= 16)
+                return launch_nw(std::integral_constant<uint32_t, kWavesPerBlock>{});
         }
         if (pad)   // padded lattices: two tile-height bounds
         {
@@ -886,15 +935,15 @@ namespace swmi
             else
                 launch(k_bond_label_any<64, TW64, DBG, true>);
         }
-        else if (max_twr <= 8)
-            TW64 ? launch(k_bond_label<8, DBG>) : launch(k_bond_label_any<8, false, DBG, false>);
-        else if (max_twr <= 16)
-            TW64 ? launch(k_bond_label<16, DBG>) : launch(k_bond_label_any<16, false, DBG, false>);
+        else if (!TW64 && max_twr <= 8)
+            launch(k_bond_label_any<8, false, DBG, false>);
+        else if (!TW64 && max_twr <= 16)
+            launch(k_bond_label_any<16, false, DBG, false>);
         else if (max_twr <= 32)
             launch(k_bond_label_any<32, TW64, DBG, false>);
         else
             launch(k_bond_label_any<64, TW64, DBG, false>);
     }
 
-    template void LaunchBondLabelT<SWMI_BOND_TW64, SWMI_BOND_DBG>(const LatDesc*, const uint32_t*, uint32_t, uint32_t, bool, bool, hipStream_t);
+    template void LaunchBondLabelT<SWMI_BOND_TW64, SWMI_BOND_DBG>(const LatDesc*, const uint32_t*, uint32_t, uint32_t, BondForm, bool, hipStream_t);
 }

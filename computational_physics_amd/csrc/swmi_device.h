@@ -101,6 +101,13 @@ namespace swmi
         return reinterpret_cast<uint32_t*>(reinterpret_cast<char*>(P) + off);
     }
 
+    // byte offset of the LDS word p from P
+    __device__ __forceinline__ uint32_t OffsetFrom(const uint32_t* P, const uint32_t* p)
+    {
+        return static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) const uint32_t*)p) -
+                                     reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) const uint32_t*)P));
+    }
+
     __device__ __forceinline__ uint32_t LdsLoad(const uint32_t* p)
     {
         return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
@@ -189,27 +196,28 @@ namespace swmi
     // there is smaller than anything this row writes and no row clears its words. A bond to any other root links
     // that root under the minimum with one atomicMin, and only a link that loses a race goes through the lockstep
     // union. P[self] is left at the run's label, an ancestor; returns the root of this lane's site after the row's
-    // links. M: 64 words of the wave, below base at the start; dummy: a word of the lane's own, the target of LDS
-    // operations the lane has no use for.
+    // links. M: 64 words of the wave, below base at the start; spare: a word of the lane's own, the target of LDS
+    // operations the lane has no use for (both as byte offsets from P: the selects below are between offsets, and P's
+    // address stays in the instructions' offset fields).
     // LDS operations are what bounds the labelling (one pipe per CU, about 7 cycles per operation of a wave with
     // scattered roots): a row takes four and one per chase step, where clearing, minimum, entry and root as separate
     // operations took eight.
-    __device__ __forceinline__ uint32_t LabelRow64(uint32_t* P, uint32_t* M, uint32_t* dummy, const uint32_t self, const uint64_t B,
-                                                   const uint64_t D, const uint32_t Rp, const uint32_t base)
+    __device__ __forceinline__ uint32_t LabelRow64(uint32_t* P, const uint32_t M, const uint32_t spare, const uint32_t self,
+                                                   const uint64_t B, const uint64_t D, const uint32_t Rp, const uint32_t base)
     {
         // word of this lane's row run: the number of run starts after lane 0 up to this lane
-        uint32_t* const Mk = M + __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(~B >> 32),
-                                                           __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(~B), 0u));
+        const uint32_t Mk = M + 4u * __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(~B >> 32),
+                                                               __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(~B), 0u));
         // a run's first lane brings its own node, a bonded lane the root above (an earlier row's node, so smaller)
         const uint32_t x = LaneBit(D) ? Rp : self;
-        (void)__hip_atomic_fetch_max(LaneBit(~(B << 1) | D) ? Mk : dummy, base - x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-        uint32_t root = base - LdsLoad(Mk);
+        (void)__hip_atomic_fetch_max(At(P, LaneBit(~(B << 1) | D) ? Mk : spare), base - x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        uint32_t root = base - LdsLoad(At(P, Mk));
         __hip_atomic_store(At(P, self), root, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
         // bonds to a root other than the run's minimum link that root under it
         const uint64_t mg = D & __ballot(Rp != root);
         if (mg != 0ull)
         {
-            const uint32_t old = __hip_atomic_fetch_min(LaneBit(mg) ? At(P, Rp) : dummy, root, __ATOMIC_RELAXED,
+            const uint32_t old = __hip_atomic_fetch_min(At(P, LaneBit(mg) ? Rp : spare), root, __ATOMIC_RELAXED,
                                                         __HIP_MEMORY_SCOPE_WORKGROUP);
             // Rp was no longer a root (another lane linked it first): join the two trees
             const uint64_t more = mg & __ballot(old != Rp) & __ballot(old != root);

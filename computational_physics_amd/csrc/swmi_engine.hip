@@ -188,6 +188,13 @@ namespace swmi
         return rows <= kResidentRows ? rows : 0;
     }
 
+    BondForm FormOf(const Geometry& g)
+    {
+        if (g.twr % 4u != 0u)
+            return BondForm::kAny;
+        return g.twr == 16u && g.nwr_y % (kWavesPerBlock * 16u) == 0u ? BondForm::kFull : BondForm::kQuads;
+    }
+
     LatDesc GeometryDesc(const Geometry& g, const uint32_t n0, const uint32_t n1)
     {
         LatDesc d{};
@@ -410,7 +417,7 @@ void swmi_engine::Rebuild()
             it->twr_t = t;
             it->resident = resident;
         }
-        it->quads = it->quads && l.g.twr % 4u == 0u;
+        it->form = std::min(it->form, FormOf(l.g));
         it->max_rows = std::max(it->max_rows, rows);
         it->max_sites = std::max(it->max_sites, static_cast<uint32_t>(l.np));
         it->slots.push_back(i);
@@ -478,7 +485,7 @@ void swmi_engine::EnqueueSweeps(uint32_t n)
         hipStream_t s = ClassStream(c);
         for (uint32_t i = 0; i < n; ++i)
         {
-            LaunchBondLabel(k.Descs(d_desc.ptr), k.WorkList(), k.total_blocks, k.max_twr, k.quads, k.tw64, k.pad, recording, s);
+            LaunchBondLabel(k.Descs(d_desc.ptr), k.WorkList(), k.total_blocks, k.max_twr, k.form, k.tw64, k.pad, recording, s);
             LaunchMerge(k.Descs(d_desc.ptr), k.WorkList(), k.total_blocks, s);
             LaunchResolve(k.Descs(d_desc.ptr), k.WorkList(), k.total_blocks, s);
         }
@@ -1076,7 +1083,7 @@ int swmi_label_bonds(swmi_engine* engine, uint32_t lattice, const uint8_t* bonds
         if (!l.parent.ptr)
             l.parent.allocate(l.np);
         engine->OneLattice(l, l.bond_in.ptr);
-        LaunchBondLabel(engine->d_one_desc.ptr, nullptr, l.g.n_blocks, l.g.twr, l.g.twr % 4u == 0u, l.g.tw == 64, l.np != l.n, true,
+        LaunchBondLabel(engine->d_one_desc.ptr, nullptr, l.g.n_blocks, l.g.twr, FormOf(l.g), l.g.tw == 64, l.np != l.n, true,
                         engine->stream);
         LaunchMerge(engine->d_one_desc.ptr, nullptr, l.g.n_blocks, engine->stream);
         LaunchWriteLabels(engine->d_one_desc.ptr, nullptr, l.g.n_blocks, l.g.twr, engine->stream);
@@ -1329,7 +1336,7 @@ int swmi_time_kernels(swmi_engine* engine, uint32_t n_sweeps, float* ms)
         {
             Check(hipEventRecord(ev[0], engine->stream), "event");
             for (auto& k : engine->classes)
-                LaunchBondLabel(k.Descs(engine->d_desc.ptr), k.WorkList(), k.total_blocks, k.max_twr, k.quads, k.tw64, k.pad, engine->recording,
+                LaunchBondLabel(k.Descs(engine->d_desc.ptr), k.WorkList(), k.total_blocks, k.max_twr, k.form, k.tw64, k.pad, engine->recording,
                                 engine->stream);
             Check(hipEventRecord(ev[1], engine->stream), "event");
             for (auto& k : engine->classes)

@@ -126,6 +126,7 @@ namespace swmi
     uint32_t DefaultTileRows(uint32_t n0, uint32_t n1);
     // Rows of the strips in which k_resident sweeps a lattice of this geometry: 0 if it does not take it.
     uint32_t ResidentRows(const Geometry& g, uint32_t n1);
+    BondForm FormOf(const Geometry& g);
     // k_bond_label specialisation bound for a tile height: 8, 16, 32 or 64.
     uint32_t TwrClass(uint32_t twr);
 
@@ -174,7 +175,7 @@ namespace swmi
         bool pad = false;                    // padded lattices (the PAD specialisation of k_bond_label)
         uint32_t twr_t = 16;                 // k_bond_label TWR_MAX
         uint32_t max_twr = 1;
-        bool quads = true;                   // every tile height is a multiple of 4
+        BondForm form = BondForm::kFull;     // what its lattices' tile heights have in common
         std::vector<uint32_t> block_lat;     // block -> lattice slot
         DeviceBuffer<uint32_t> d_block_lat;
         uint32_t total_blocks = 0;

@@ -153,16 +153,24 @@ namespace swmi
     };
 
 
+    // What the tile heights of a launch's lattices allow k_bond_label (64-wide tiles)
+    enum class BondForm : uint32_t
+    {
+        kAny,     // nothing
+        kQuads,   // every tile height is a multiple of 4: a block's rows can be shared by 8 or 16 waves
+        kFull     // and every tile is exactly 16 rows, every block 4 tiles
+    };
+
     constexpr uint32_t kErrLabelRange = 1u;  // a label chase left [0, n) or met an unflagged root
 
     // Launch wrappers (swmi_kernels.hip). Work list: block_lat[b] = lattice of global block b; a null work list
     // means every block belongs to descriptor 0.
     // all_tw64: every lattice of the work list has n0 % 64 == 0 (64-wide tiles); selects the specialised kernel
-    // quads: every lattice's tile height is a multiple of 4
+    // form: what all lattices of the work list have in common
     // debug: compiles in injected bonds (LatDesc::bond_in) and bond recording (LatDesc::bond_dump)
     // pad: some lattice of the work list is padded (selects the PAD specialisation, correct for every lattice)
     void LaunchBondLabel(const LatDesc* d_desc, const uint32_t* d_block_lat, uint32_t total_blocks, uint32_t max_twr,
-                         bool quads, bool all_tw64, bool pad, bool debug, hipStream_t stream);
+                         BondForm form, bool all_tw64, bool pad, bool debug, hipStream_t stream);
     void LaunchMerge(const LatDesc* d_desc, const uint32_t* d_block_lat, uint32_t total_blocks, hipStream_t stream);
     // n_lattices small lattices (descriptors d_slots[i]), one workgroup each: `groups` groups of `sweeps` sweeps with a
     // sample after each group when sample_mode >= 0. max_sites, max_rows: bounds on their padded sites and on the

@@ -1059,23 +1059,23 @@ namespace swmi
     // =============================================================================================
     // defined in swmi_bond.hip, one part per combination
     template <bool TW64, bool DBG>
-    void LaunchBondLabelT(const LatDesc* d_desc, const uint32_t* d_block_lat, uint32_t total_blocks, uint32_t max_twr, bool quads, bool pad,
+    void LaunchBondLabelT(const LatDesc* d_desc, const uint32_t* d_block_lat, uint32_t total_blocks, uint32_t max_twr, BondForm form, bool pad,
                           hipStream_t stream);
 
     void LaunchBondLabel(const LatDesc* d_desc, const uint32_t* d_block_lat, const uint32_t total_blocks, const uint32_t max_twr,
-                         const bool quads, const bool all_tw64, const bool pad, const bool debug, hipStream_t stream)
+                         const BondForm form, const bool all_tw64, const bool pad, const bool debug, hipStream_t stream)
     {
         if (debug)
         {
             if (all_tw64)
-                LaunchBondLabelT<true, true>(d_desc, d_block_lat, total_blocks, max_twr, quads, pad, stream);
+                LaunchBondLabelT<true, true>(d_desc, d_block_lat, total_blocks, max_twr, form, pad, stream);
             else
-                LaunchBondLabelT<false, true>(d_desc, d_block_lat, total_blocks, max_twr, quads, pad, stream);
+                LaunchBondLabelT<false, true>(d_desc, d_block_lat, total_blocks, max_twr, form, pad, stream);
         }
         else if (all_tw64)
-            LaunchBondLabelT<true, false>(d_desc, d_block_lat, total_blocks, max_twr, quads, pad, stream);
+            LaunchBondLabelT<true, false>(d_desc, d_block_lat, total_blocks, max_twr, form, pad, stream);
         else
-            LaunchBondLabelT<false, false>(d_desc, d_block_lat, total_blocks, max_twr, quads, pad, stream);
+            LaunchBondLabelT<false, false>(d_desc, d_block_lat, total_blocks, max_twr, form, pad, stream);
     }
 
     // Two-wave merge workgroups resident at once on MI355X: 256 CUs x 16 (8 waves per SIMD).

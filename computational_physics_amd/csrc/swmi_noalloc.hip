@@ -136,7 +136,7 @@ extern "C" int swmi_label_bonds_noalloc(const uint8_t* bonds, uint32_t n0, uint3
         LaunchNoAllocSetup(d, d_desc, s);
         if (pad)
             LaunchPadBytes(const_cast<uint8_t*>(d.bond_in), bonds, np, n0, g.pitch, s);
-        LaunchBondLabel(d_desc, nullptr, g.n_blocks, g.twr, g.twr % 4u == 0u, g.tw == 64, pad, true, s);
+        LaunchBondLabel(d_desc, nullptr, g.n_blocks, g.twr, FormOf(g), g.tw == 64, pad, true, s);
         LaunchMerge(d_desc, nullptr, g.n_blocks, s);
         LaunchWriteLabels(d_desc, nullptr, g.n_blocks, g.twr, s);
         if (pad)

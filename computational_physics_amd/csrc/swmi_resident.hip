@@ -148,7 +148,7 @@ namespace swmi
         __syncthreads();   // sS
 
         uint32_t* const Qw = Q + w * kQw;
-        uint32_t* const dummy = Qw + 64u + lane;
+        const uint32_t run_words = OffsetFrom(P, Qw), spare = OffsetFrom(P, Qw + 64u + lane);
         const uint32_t rowb = n0 * 4u * rpw;                // P bytes between consecutive rows of a strip
         const uint32_t node0 = g0 * 256u + lane4;           // this lane's node of the strip's first row
         const uint32_t node_below = gbelow * 256u + lane4;
@@ -247,7 +247,7 @@ namespace swmi
                     {
                         right_bits |= ((Ball >> elane) & 1ull) << i;
                         const uint64_t D = i == 0u ? 0ull : (~(prev_S ^ S) & prev_U2);
-                        Rp = LabelRow64(P, Qw, dummy, node, B, D, Rp, RowBase(i + 1u));
+                        Rp = LabelRow64(P, run_words, spare, node, B, D, Rp, RowBase(i + 1u));
                         xs[i] = Rp;
                         if (i == 0u && lane == 0u)
                             sB[w] = B;
