@@ -418,6 +418,8 @@ void swmi_engine::Rebuild()
             it->resident = resident;
         }
         it->form = std::min(it->form, FormOf(l.g));
+        it->max_blocks = std::max(it->max_blocks, l.g.n_blocks);
+        it->max_block_rows = std::max(it->max_block_rows, l.g.ecol_stride);
         it->max_rows = std::max(it->max_rows, rows);
         it->max_sites = std::max(it->max_sites, static_cast<uint32_t>(l.np));
         it->slots.push_back(i);
@@ -486,8 +488,13 @@ void swmi_engine::EnqueueSweeps(uint32_t n)
         for (uint32_t i = 0; i < n; ++i)
         {
             LaunchBondLabel(k.Descs(d_desc.ptr), k.WorkList(), k.total_blocks, k.max_twr, k.form, k.tw64, k.pad, recording, s);
+            if (k.Joined())
+            {
+                LaunchJoin(d_desc.ptr, k.d_slots.ptr, k.n_lat, k.max_blocks, s);
+                continue;
+            }
             LaunchMerge(k.Descs(d_desc.ptr), k.WorkList(), k.total_blocks, s);
-            LaunchResolve(k.Descs(d_desc.ptr), k.WorkList(), k.total_blocks, s);
+            LaunchResolve(k.Descs(d_desc.ptr), k.WorkList(), k.total_blocks, k.max_block_rows, s);
         }
     }
     Join(0, n_tiled - 1);
@@ -1340,10 +1347,14 @@ int swmi_time_kernels(swmi_engine* engine, uint32_t n_sweeps, float* ms)
                                 engine->stream);
             Check(hipEventRecord(ev[1], engine->stream), "event");
             for (auto& k : engine->classes)
-                LaunchMerge(k.Descs(engine->d_desc.ptr), k.WorkList(), k.total_blocks, engine->stream);
+                if (k.Joined())
+                    LaunchJoin(engine->d_desc.ptr, k.d_slots.ptr, k.n_lat, k.max_blocks, engine->stream);
+                else
+                    LaunchMerge(k.Descs(engine->d_desc.ptr), k.WorkList(), k.total_blocks, engine->stream);
             Check(hipEventRecord(ev[2], engine->stream), "event");
             for (auto& k : engine->classes)
-                LaunchResolve(k.Descs(engine->d_desc.ptr), k.WorkList(), k.total_blocks, engine->stream);
+                if (!k.Joined())
+                    LaunchResolve(k.Descs(engine->d_desc.ptr), k.WorkList(), k.total_blocks, k.max_block_rows, engine->stream);
             Check(hipEventRecord(ev[3], engine->stream), "event");
             Check(hipEventSynchronize(ev[3]), "event sync");
             for (int k = 0; k < 3; ++k)

@@ -175,6 +175,10 @@ namespace swmi
         bool pad = false;                    // padded lattices (the PAD specialisation of k_bond_label)
         uint32_t twr_t = 16;                 // k_bond_label TWR_MAX
         uint32_t max_twr = 1;
+        uint32_t max_block_rows = 0;         // lattice rows of the tallest block
+        uint32_t max_blocks = 0;             // blocks of the largest lattice
+        // every lattice's slots fit one workgroup: k_join takes the place of k_merge and k_resolve
+        bool Joined() const { return tw64 && max_block_rows <= 64u && max_blocks <= swmi::kJoinBlocks; }
         BondForm form = BondForm::kFull;     // what its lattices' tile heights have in common
         std::vector<uint32_t> block_lat;     // block -> lattice slot
         DeviceBuffer<uint32_t> d_block_lat;

@@ -63,6 +63,7 @@ namespace swmi
     constexpr uint32_t kResidentSites = 16384;  // largest (padded) lattice that one workgroup sweeps alone (k_resident)
     constexpr uint32_t kResidentWaves = 16;     // its waves, each with a strip of at most kResidentRows rows
     constexpr uint32_t kResidentRows = 16;
+    constexpr uint32_t kJoinBlocks = 16;        // most blocks of a lattice whose slots one workgroup joins (k_join)
     constexpr uint32_t kNumXcd = 8;          // MI355X: 8 XCDs, workgroups dispatched round-robin
     constexpr uint16_t kEdgeFlag = 0x8000u;  // cluster reaches the block edge
     constexpr uint32_t kRightWords = kWavesPerBlock;
@@ -177,8 +178,12 @@ namespace swmi
     // rows of a strip (ResidentRows).
     void LaunchResident(const LatDesc* d_desc, const uint32_t* d_slots, uint32_t n_lattices, uint32_t max_sites, uint32_t max_rows,
                         bool tw64, bool pad, uint32_t sweeps, uint32_t groups, int32_t sample_mode, hipStream_t stream);
+    // k_merge and k_resolve of n_lattices lattices of 64-wide tiles, blocks of at most 64 rows and at most
+    // max_blocks <= kJoinBlocks blocks, one workgroup each
+    void LaunchJoin(const LatDesc* d_desc, const uint32_t* d_slots, uint32_t n_lattices, uint32_t max_blocks, hipStream_t stream);
     // end of a sweep: flip bits and halos of every block, then iteration += 2
-    void LaunchResolve(const LatDesc* d_desc, const uint32_t* d_block_lat, uint32_t total_blocks, hipStream_t stream);
+    // max_rows: lattice rows of the tallest block
+    void LaunchResolve(const LatDesc* d_desc, const uint32_t* d_block_lat, uint32_t total_blocks, uint32_t max_rows, hipStream_t stream);
     // apply a pending flip to the spin array (no-op for lattices without one)
     void LaunchMaterialize(const LatDesc* d_desc, const uint32_t* d_block_lat, uint32_t total_blocks, hipStream_t stream);
     // canonical label (minimum site index) of every site into parent[] (inspection)

@@ -315,12 +315,27 @@ namespace swmi
             f(i, slots * bl.lb + i);
     }
 
+    // The lattice's counters at the end of the sweep that began at iteration `it`.
+    __device__ __forceinline__ void AdvanceIteration(const LatDesc& d, const uint32_t it)
+    {
+        const gptr<uint32_t> stp = Glob(d.state);
+        stp[kStApplied] = it;
+        stp[kStIteration] = it + 2u;
+        // a rotating sweep stored the states at which its lanes' pairs changed
+        if ((it + 1u) % 15u == 0u)
+            Glob(d.aux)[kAuxRngIt] = it;
+        else if ((it + 2u) % 15u == 0u)
+            Glob(d.aux)[kAuxRngIt] = it + 1u;
+    }
+
     // End of a sweep, per block (two waves): the slots of the block's edge-reaching clusters are chased in the
     // slot union-find, and each slot's bit becomes the flip rule applied to its canonical root; then the
     // block's flip bitmap and the flipped spins of its first column and first wave row (the halos its left
     // and upper neighbours read in the next sweep) are written out, and the lattice's counters move on:
     // applied = the iteration whose spins the array holds, iteration += 2. The spin array itself is left for
     // the next sweep to flip.
+    // kMaxRows: lattice rows of the tallest block.
+    template <uint32_t kMaxRows>
     __global__ __launch_bounds__(128) void k_resolve(const LatDesc* __restrict__ descs, const uint32_t* __restrict__ block_lat,
                                                      const uint32_t total_blocks)
     {
@@ -343,8 +358,7 @@ namespace swmi
         // loaded with the lattice's counters; their spins (written into the halo by this sweep's
         // k_bond_label) follow with the first entries of the slot chases. The halo is flipped in place.
         const uint32_t rows = bl.nwr * d.rpw;
-        // rows <= kWavesPerBlock * 64 (a tile has twr <= tw wave rows of rpw = 64 / tw lattice rows)
-        constexpr uint32_t kHaloPer = (kWavesPerBlock * 64u + 64u + kThreads - 1u) / kThreads;
+        constexpr uint32_t kHaloPer = (kMaxRows + 64u + kThreads - 1u) / kThreads;
         // (straight-line loads from a selected address, every one in range, so that they are all in flight
         // at once; hoff is the entry's offset in the halo)
         uint32_t hs[kHaloPer], hl[kHaloPer], hoff[kHaloPer];
@@ -433,16 +447,191 @@ namespace swmi
         if (!ok)
             (void)__hip_atomic_fetch_or(stp + kStErr, kErrLabelRange, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         if (bl.lb == 0 && threadIdx.x == 0)
+            AdvanceIteration(d, stp[kStIteration]);
+    }
+
+    // =============================================================================================
+    // k_join: k_merge and k_resolve of a lattice of few blocks, in one workgroup
+    // =============================================================================================
+    // For a lattice of few blocks the two kernels are launch time and chains of memory round trips. Here one workgroup of 16 waves holds the whole lattice's slot union-find in LDS: node 256 * block + slot (a block
+    // of 64 columns and at most 64 rows has at most 252 boundary sites, so at most 252 slots). The edges, the halo
+    // labels and the counters are read in one round trip; the unions are LDS operations; the flip bits, the flipped
+    // halos and every slot's root go out as k_resolve and k_merge leave them (the root directly as parent).
+    // A wave takes two edges and one block, so at most 16 blocks: one CU reads about 8 KB per microsecond from the other
+    // CUs' results, which bounds it (microseconds per sweep at T_c with k_merge and k_resolve / with k_join: 6 blocks
+    // 17.5 / 13.9, 16 blocks 18.8 / 16.2, and with more edges per wave 24 blocks 19.3 / 20.0, 64 blocks 20.1 / 32.1).
+    __global__ __launch_bounds__(1024) void k_join(const LatDesc* __restrict__ descs, const uint32_t* __restrict__ slots)
+    {
+        constexpr uint32_t kWaves = 16, kEdges = 2u, kNodes = 256u;
+        extern __shared__ uint64_t L[];            // kNodes entries per block: (key of the parent << 32) | parent
+        __shared__ uint32_t sw[kWaves * 8u];       // flip bits by node
+        const LatDesc& d = descs[slots[blockIdx.x]];
+        const gptr<uint32_t> stp = Glob(d.state);
+        const uint32_t lane = threadIdx.x & 63u, w = Uniform(threadIdx.x >> 6);
+        const uint32_t tx = d.tiles_x, nb = d.n_blocks, brows = kWavesPerBlock * d.twr, stride = 64u * tx, qcap = d.qcap;
+        const uint32_t bslots = kWavesPerBlock * d.edge_cap, es = d.ecol_stride;
+        const gptr<const uint32_t> ec = Glob(static_cast<const uint32_t*>(d.ecol)), er = Glob(static_cast<const uint32_t*>(d.erow));
+        const gptr<const uint64_t> bb = Glob(static_cast<const uint64_t*>(d.bbits));
+        const gptr<const uint32_t> counts = Glob(static_cast<const uint32_t*>(d.edge_count));
+        bool ok = true;
+        const auto rows_of = [&](const uint32_t sy) { return min(brows, d.nwr_y - sy * brows); };
+
+        // edge e = w + 16 k: block e / 2, its right edge (lane = row) or its down edge (lane = column)
+        uint32_t va[kEdges], vb[kEdges], lbb[kEdges];
+        uint64_t word[kEdges];
+#pragma unroll
+        for (uint32_t k = 0; k < kEdges; ++k)
         {
-            const uint32_t it = stp[kStIteration];
-            stp[kStApplied] = it;
-            stp[kStIteration] = it + 2u;
-            // a rotating sweep stored the states at which its lanes' pairs changed
-            if ((it + 1u) % 15u == 0u)
-                Glob(d.aux)[kAuxRngIt] = it;
-            else if ((it + 2u) % 15u == 0u)
-                Glob(d.aux)[kAuxRngIt] = it + 1u;
+            const uint32_t e = min(w + kWaves * k, 2u * nb - 1u), lb = e >> 1;
+            const uint32_t sx = lb % tx, sy = lb / tx;
+            const bool down = (e & 1u) != 0u;
+            lbb[k] = down ? (sy + 1u == d.blocks_y ? 0u : sy + 1u) * tx + sx : sy * tx + (sx + 1u == tx ? 0u : sx + 1u);
+            const uint32_t row = min(lane, rows_of(sy) - 1u);
+            va[k] = *(down ? er + 128u * lb + 64u + lane : ec + (2u * lb + 1u) * es + row);
+            vb[k] = *(down ? er + 128u * lbb[k] + lane : ec + 2u * lbb[k] * es + row);
+            word[k] = bb[kBbitWords * lb + (down ? 0u : 1u + row / d.twr)];
         }
+        // block w: its slots and its halo (first column, first row)
+        const uint32_t blk = min(w, nb - 1u), blk_rows = rows_of(blk / tx);
+        const uint32_t cnt = counts[kWavesPerBlock * blk];
+        const uint32_t hc = ec[2u * blk * es + min(lane, blk_rows - 1u)] >> 16, hr = er[128u * blk + lane] >> 16;
+        const uint32_t active = stp[kStActive], hside = stp[kStHaloSide], fkey = stp[kStFlipKey], it = stp[kStIteration];
+        if (active == 0u)
+            return;
+        const gptr<uint8_t> halo = Glob(d.halo) + (hside * nb + blk) * d.halo_stride;
+        const uint32_t sc = halo[min(lane, blk_rows - 1u)], sr = halo[es + lane];
+
+        // every slot's node, a root keyed by its site (the edge entries of a block name all of its slots)
+        const auto node_of = [&](const uint32_t lb, const uint32_t v) { return lb * kNodes + min((v >> 16 & 0x7FFFu) - qcap, kNodes - 1u); };
+        const auto key_of = [&](const uint32_t lb, const uint32_t v) {
+            return SiteOf((lb / tx) * brows * stride + (lb % tx) * 64u, stride, v & 0xFFFFu);
+        };
+        const auto put = [&](const uint32_t lb, const uint32_t v) {
+            if ((v >> 16) & kEdgeFlag)
+            {
+                const uint32_t n = node_of(lb, v);
+                __hip_atomic_store(&L[n], SlotEntry(key_of(lb, v), n), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+            }
+        };
+#pragma unroll
+        for (uint32_t k = 0; k < kEdges; ++k)
+            if (w + kWaves * k < 2u * nb)
+            {
+                put((w + kWaves * k) >> 1, va[k]);
+                put(lbb[k], vb[k]);
+            }
+        __syncthreads();
+
+        // unions of the bonded pairs, one lane each (the loop of k_merge's local unions)
+#pragma unroll
+        for (uint32_t k = 0; k < kEdges; ++k)
+        {
+            const uint32_t e = w + kWaves * k;
+            if (e < 2u * nb)
+            {
+                const uint32_t lb = e >> 1;
+                const bool down = (e & 1u) != 0u;
+                const uint32_t bit = down ? lane : lane % d.twr;
+                bool open = ((word[k] >> bit) & 1ull) != 0ull && (down || lane < rows_of(lb / tx));
+                // both ends of a bond across an edge belong to edge-reaching clusters
+                if (open && !((va[k] >> 16) & (vb[k] >> 16) & kEdgeFlag))
+                {
+                    ok = false;
+                    open = false;
+                }
+                uint32_t a = node_of(lb, va[k]), b = node_of(lbb[k], vb[k]);
+                while (__ballot(open))
+                {
+                    if (open)
+                    {
+                        uint64_t ea = LocalEntry(L, a), eb = LocalEntry(L, b);
+                        while (static_cast<uint32_t>(ea) != a || static_cast<uint32_t>(eb) != b)
+                        {
+                            a = static_cast<uint32_t>(ea);
+                            b = static_cast<uint32_t>(eb);
+                            ea = LocalEntry(L, a);
+                            eb = LocalEntry(L, b);
+                        }
+                        if (a == b)
+                            open = false;
+                        else
+                        {
+                            if ((ea >> 32) > (eb >> 32))   // roots hold their own keys; link the larger under the smaller
+                            {
+                                const uint32_t t = a;
+                                a = b;
+                                b = t;
+                                const uint64_t te = ea;
+                                ea = eb;
+                                eb = te;
+                            }
+                            const uint64_t old = __hip_atomic_fetch_min(&L[b], SlotEntry(static_cast<uint32_t>(ea >> 32), a),
+                                                                        __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                            if (old == eb)
+                                open = false;
+                            else   // b had been linked under old's parent (which this link may have displaced): unite with it
+                                b = static_cast<uint32_t>(old);
+                        }
+                    }
+                }
+            }
+        }
+        __syncthreads();
+
+        const bool random_rule = d.flip_rule != 0u;
+        const uint32_t key = random_rule ? fkey : 0u;
+        if (w < nb)
+        {
+            const uint32_t nslot = Uniform(min(cnt, kNodes));
+            uint32_t* const bits = sw + blk * 8u;
+            for (uint32_t s0 = 0; s0 < nslot; s0 += 64u)
+            {
+                const uint32_t i = s0 + lane;
+                uint32_t bit = 0;
+                if (i < nslot)
+                {
+                    uint32_t n = blk * kNodes + i;
+                    uint64_t e = LocalEntry(L, n);
+                    while (static_cast<uint32_t>(e) != n)
+                    {
+                        n = static_cast<uint32_t>(e);
+                        e = LocalEntry(L, n);
+                    }
+                    const uint32_t root = static_cast<uint32_t>(e >> 32);
+                    bit = FlipBit(d, root, random_rule, key);
+                    Glob(d.cpar)[bslots * blk + i] = SlotEntry(root, bslots * (n / kNodes) + n % kNodes);
+                }
+                const uint64_t m = __ballot(bit != 0u);
+                if (lane < 2u)
+                {
+                    const uint32_t v = lane ? static_cast<uint32_t>(m >> 32) : static_cast<uint32_t>(m);
+                    bits[(s0 >> 5) + lane] = v;
+                    if ((s0 >> 5) + lane < d.fsw)
+                        Glob(d.fbits)[blk * d.fsw + (s0 >> 5) + lane] = v;
+                }
+            }
+            const auto flip = [&](const uint32_t lab) -> uint32_t {
+                const uint32_t i = lab & 0x7FFFu;
+                if (lab & kEdgeFlag)
+                {
+                    const uint32_t s = i - qcap;
+                    if (s >= nslot)
+                    {
+                        ok = false;
+                        return 0u;
+                    }
+                    return (LdsLoad(&bits[s >> 5]) >> (s & 31u)) & 1u;
+                }
+                return FlipBit(d, SiteOf((blk / tx) * brows * stride + (blk % tx) * 64u, stride, i), random_rule, key);
+            };
+            if (lane < blk_rows)
+                halo[lane] = static_cast<uint8_t>((sc ^ flip(hc)) & 1u);
+            halo[es + lane] = static_cast<uint8_t>((sr ^ flip(hr)) & 1u);
+        }
+        if (!ok)
+            (void)__hip_atomic_fetch_or(stp + kStErr, kErrLabelRange, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (threadIdx.x == 0)
+            AdvanceIteration(d, it);
     }
 
     // Applies a pending flip to the spin array (lattices without one return at once): per block (two
@@ -1102,9 +1291,19 @@ namespace swmi
             LaunchMergeAs<false>(d_desc, d_block_lat, total_blocks, stream);
     }
 
-    void LaunchResolve(const LatDesc* d_desc, const uint32_t* d_block_lat, const uint32_t total_blocks, hipStream_t stream)
+    void LaunchResolve(const LatDesc* d_desc, const uint32_t* d_block_lat, const uint32_t total_blocks, const uint32_t max_rows,
+                       hipStream_t stream)
     {
-        k_resolve<<<XcdGrid(total_blocks), 128, 0, stream>>>(d_desc, d_block_lat, total_blocks);
+        // (a tile has at most 64 lattice rows, a block of 16-row tiles 64: one halo entry per thread instead of three)
+        if (max_rows > 64u)
+            k_resolve<kWavesPerBlock * 64u><<<XcdGrid(total_blocks), 128, 0, stream>>>(d_desc, d_block_lat, total_blocks);
+        else
+            k_resolve<64><<<XcdGrid(total_blocks), 128, 0, stream>>>(d_desc, d_block_lat, total_blocks);
+    }
+
+    void LaunchJoin(const LatDesc* d_desc, const uint32_t* d_slots, const uint32_t n_lattices, const uint32_t max_blocks, hipStream_t stream)
+    {
+        k_join<<<n_lattices, 1024, max_blocks * 256u * sizeof(uint64_t), stream>>>(d_desc, d_slots);
     }
 
     void LaunchMaterialize(const LatDesc* d_desc, const uint32_t* d_block_lat, const uint32_t total_blocks, hipStream_t stream)

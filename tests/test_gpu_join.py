@@ -1,0 +1,39 @@
+"""Lattices of few blocks merge and resolve in one workgroup (k_join); with 17 blocks and more the two kernels do. Both
+against the oracle: one block, sixteen, the first count past it, partial and padded blocks, tall tiles that keep the two
+kernels, both flip rules, and a mixed engine."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("n0,n1,tile_rows", [(64, 64, 16), (256, 256, 0), (64, 1024, 16), (1024, 64, 16), (64, 1030, 16), (1088, 64, 16),
+                                             (130, 300, 0), (192, 200, 4), (128, 512, 64), (256, 250, 1)])
+@pytest.mark.parametrize("T,rule", [(2.0, 0), (2.2691853, 1), (2.6, 0)])
+def test_merge_and_flip_match_the_oracle(swmi, oracle, n0, n1, tile_rows, T, rule):
+    print(f"join {n0}x{n1} tile_rows {tile_rows} T {T} rule {rule}", flush=True)
+    ref = oracle.PerSite(n0, n1, T, seed=n1, spin_seed=2, flip_rule=rule)
+    with swmi.Engine(swmi.LatticeConfig(n0, n1, T, seed=n1, spin_seed=2, tile_rows=tile_rows, flip_rule=rule)) as e:
+        for k in range(8):
+            _, labels = ref.sweep(record=True)
+            e.sweep(1)
+            if k % 3 == 1:
+                np.testing.assert_array_equal(e.labels(), labels, err_msg=f"labels, sweep {k + 1}")
+                assert e.energy_magnetization() == oracle.observables(n0, n1, ref.spins)   # the pending flip, not stored
+        np.testing.assert_array_equal(e.spins(), ref.spins)
+        assert e.error_flags() == 0
+
+
+def test_lattices_of_a_joined_engine_equal_their_lone_runs(swmi):
+    print("join batch", flush=True)
+    cfgs = [swmi.LatticeConfig(n0, n1, T, seed=k, flip_rule=k % 2)
+            for k, (n0, n1, T) in enumerate([(256, 256, 2.2), (192, 320, 2.0), (128, 130, 2.5), (64, 300, 2.27), (256, 192, 2.8)])]
+    with swmi.Engine(cfgs) as e:
+        e.set_schedule(1, sweeps=13)
+        e.sweep(40)
+        got = [e.spins(i) for i in range(len(cfgs))]
+    for k, c in enumerate(cfgs):
+        with swmi.Engine(c) as alone:
+            alone.sweep(13 if k == 1 else 40)
+            np.testing.assert_array_equal(alone.spins(), got[k], err_msg=f"lattice {k}")
+            assert alone.error_flags() == 0
