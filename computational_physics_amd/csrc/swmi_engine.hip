@@ -417,10 +417,12 @@ void swmi_engine::Rebuild()
             it->twr_t = t;
             it->resident = resident;
         }
+        it->max_rows = std::max(it->max_rows, rows);
+        it->full = it->full && !pad && (rows == 4u || rows == kResidentRows) && rows == it->max_rows &&
+                   l.np == 64ull * rows * kResidentWaves;
         it->form = std::min(it->form, FormOf(l.g));
         it->max_blocks = std::max(it->max_blocks, l.g.n_blocks);
         it->max_block_rows = std::max(it->max_block_rows, l.g.ecol_stride);
-        it->max_rows = std::max(it->max_rows, rows);
         it->max_sites = std::max(it->max_sites, static_cast<uint32_t>(l.np));
         it->slots.push_back(i);
         d[i] = Desc(l, static_cast<uint32_t>(it->block_lat.size()));
@@ -535,7 +537,7 @@ void swmi_engine::EnqueueResident(const uint32_t sweeps, const uint32_t groups, 
     {
         const KernelClass& k = classes[c];
         const auto launch = [&](uint32_t per_group, uint32_t n_groups, int32_t mode) {
-            LaunchResident(d_desc.ptr, k.d_slots.ptr, k.n_lat, k.max_sites, k.max_rows, k.tw64, k.pad, per_group, n_groups, mode,
+            LaunchResident(d_desc.ptr, k.d_slots.ptr, k.n_lat, k.max_sites, k.max_rows, k.full, k.tw64, k.pad, per_group, n_groups, mode,
                            ClassStream(n_tiled));
         };
         if (sample_mode < 0 || sweeps > kResidentLaunchSweeps)

@@ -175,12 +175,21 @@ namespace swmi
     void LaunchMerge(const LatDesc* d_desc, const uint32_t* d_block_lat, uint32_t total_blocks, hipStream_t stream);
     // n_lattices small lattices (descriptors d_slots[i]), one workgroup each: `groups` groups of `sweeps` sweeps with a
     // sample after each group when sample_mode >= 0. max_sites, max_rows: bounds on their padded sites and on the
-    // rows of a strip (ResidentRows).
+    // rows of a strip (ResidentRows). full: no padding, and every wave of every lattice has exactly max_rows rows, 4 or
+    // kResidentRows.
     void LaunchResident(const LatDesc* d_desc, const uint32_t* d_slots, uint32_t n_lattices, uint32_t max_sites, uint32_t max_rows,
-                        bool tw64, bool pad, uint32_t sweeps, uint32_t groups, int32_t sample_mode, hipStream_t stream);
+                        bool full, bool tw64, bool pad, uint32_t sweeps, uint32_t groups, int32_t sample_mode, hipStream_t stream);
     // k_merge and k_resolve of n_lattices lattices of 64-wide tiles, blocks of at most 64 rows and at most
     // max_blocks <= kJoinBlocks blocks, one workgroup each
     void LaunchJoin(const LatDesc* d_desc, const uint32_t* d_slots, uint32_t n_lattices, uint32_t max_blocks, hipStream_t stream);
+    // Geometry of a lattice that one workgroup labels (ResidentRows): n0 the caller's width, the rest as in LatDesc.
+    struct WholeGeometry
+    {
+        uint32_t n0, tiles_x, tw, nwr_y, elast;
+        uint64_t vlast;
+    };
+    // canonical labels of the device bond field `bonds` into `labels`, both n0 wide
+    void LaunchLabelWhole(const WholeGeometry& g, const uint8_t* bonds, uint32_t* labels, hipStream_t stream);
     // end of a sweep: flip bits and halos of every block, then iteration += 2
     // max_rows: lattice rows of the tallest block
     void LaunchResolve(const LatDesc* d_desc, const uint32_t* d_block_lat, uint32_t total_blocks, uint32_t max_rows, hipStream_t stream);

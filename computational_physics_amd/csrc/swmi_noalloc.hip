@@ -129,6 +129,13 @@ extern "C" int swmi_label_bonds_noalloc(const uint8_t* bonds, uint32_t n0, uint3
         carve.base = ScratchOf(device);
         const LatDesc d = NoAllocDesc(g, n0, n1, bonds, labels, carve, &d_desc);
         hipStream_t s = static_cast<hipStream_t>(stream);
+        if (ResidentRows(g, n1) != 0u)
+        {
+            // one workgroup labels it in one launch, in LDS
+            LaunchLabelWhole(WholeGeometry{n0, g.tiles_x, g.tw, g.nwr_y, g.elast, g.vlast}, bonds, labels, s);
+            Check(hipGetLastError(), "label launch");
+            return;
+        }
         const bool pad = g.pitch != n0;
         const uint64_t np = static_cast<uint64_t>(g.pitch) * n1, n = static_cast<uint64_t>(n0) * n1;
         // descriptor and fresh counters are written by a kernel (no memset, no host copy); the kernels run with
