@@ -35,6 +35,10 @@ namespace swmi
         // Captured measurement graphs hold groups of (n_sep sweeps + sample) up to about this many sweeps.
         constexpr uint32_t kGraphGroupSweeps = 64;
         constexpr size_t kMaxGraphs = 6;
+        // Spins unpacked at a time on their way to the host (a multiple of 64)
+        constexpr uint64_t kStageBytes = 16ull << 20;
+        // Samples of a series read with the lattice's counters (64 KiB)
+        constexpr uint32_t kSeriesFirst = 4096;
         // Sweeps of one k_resident launch (a few milliseconds at most).
         constexpr uint32_t kResidentLaunchSweeps = 500;
     }
@@ -394,7 +398,7 @@ void swmi_engine::Rebuild()
     // workgroup sweeps (tile_rows 0: the caller asks for no tiles of its own) the k_resident build it needs. While
     // bonds are recorded every lattice is tiled: only k_bond_label records them.
     std::vector<KernelClass> next;
-    std::vector<LatDesc> d(lattices.size());
+    std::vector<LatDesc> d(2 * lattices.size());
     for (uint32_t i = 0; i < lattices.size(); ++i)
     {
         const Lattice& l = *lattices[i];
@@ -425,7 +429,9 @@ void swmi_engine::Rebuild()
         it->max_block_rows = std::max(it->max_block_rows, l.g.ecol_stride);
         it->max_sites = std::max(it->max_sites, static_cast<uint32_t>(l.np));
         it->slots.push_back(i);
+        lattices[i]->slot = i;
         d[i] = Desc(l, static_cast<uint32_t>(it->block_lat.size()));
+        d[lattices.size() + i] = Desc(l, 0);
         if (it->n_lat++ == 0)
             it->first_slot = i;
         it->block_lat.insert(it->block_lat.end(), l.g.n_blocks, i);
@@ -684,8 +690,7 @@ void swmi_engine::AdvanceRng(const Lattice& l)
 
 void swmi_engine::MaterializeOne(const Lattice& l)
 {
-    OneLattice(l, nullptr);
-    LaunchMaterialize(d_one_desc.ptr, nullptr, l.g.n_blocks, stream);
+    LaunchMaterialize(Solo(l), nullptr, l.g.n_blocks, stream);
     LaunchCheck("flip launch");
 }
 
@@ -826,10 +831,18 @@ int swmi_download_spins(swmi_engine* engine, uint32_t lattice, uint8_t* spins)
             throw SwmiError(SWMI_ERR_INVALID, "null argument");
         Lattice& l = Eng(engine)->At(lattice);
         engine->MaterializeOne(l);
-        std::vector<uint8_t> buf(l.np);
-        Check(hipMemcpyAsync(buf.data(), l.spins.ptr, l.np, hipMemcpyDeviceToHost, engine->stream), "spin download");
+        // unpacked on the device, piece by piece, straight into the caller's array
+        const uint64_t piece = std::min<uint64_t>(l.n, kStageBytes);
+        if (engine->stage.count < piece)
+            engine->stage.allocate(piece);
+        for (uint64_t first = 0; first < l.n; first += piece)
+        {
+            const uint64_t now = std::min(piece, l.n - first);
+            LaunchGetSpins(engine->stage.ptr, l.spins.ptr, first, now, l.cfg.n0, l.g.pitch, engine->stream);
+            engine->LaunchCheck("spin download");
+            Check(hipMemcpyAsync(spins + first, engine->stage.ptr, now, hipMemcpyDeviceToHost, engine->stream), "spin download");
+        }
         Check(hipStreamSynchronize(engine->stream), "spin download");
-        UnpadRows(l, buf.data(), spins, [](uint8_t v) { return static_cast<uint8_t>(v & 1u); });   // bits 3-5: selectors
     });
 }
 
@@ -839,12 +852,14 @@ int swmi_set_temperature(swmi_engine* engine, uint32_t lattice, float temperatur
         Lattice& l = Eng(engine)->At(lattice);
         if (!(temperature > 0.0f) || !std::isfinite(temperature))
             throw SwmiError(SWMI_ERR_INVALID, "temperature must be positive and finite");
-        Check(hipStreamSynchronize(engine->stream), "set temperature");
         l.cfg.temperature = temperature;
         l.p_add = BondProbability(temperature);
         l.threshold = BondThreshold(l.p_add);
-        engine->Rebuild();
-        Check(hipStreamSynchronize(engine->stream), "set temperature");
+        // the threshold lives in the descriptors, which the captured graphs read where they are
+        const uint32_t n = static_cast<uint32_t>(engine->lattices.size());
+        engine->descs[l.slot].threshold = engine->descs[n + l.slot].threshold = static_cast<uint32_t>(l.threshold);
+        LaunchSetThreshold(engine->d_desc.ptr + l.slot, engine->d_desc.ptr + n + l.slot, static_cast<uint32_t>(l.threshold), engine->stream);
+        engine->LaunchCheck("set temperature");
     });
 }
 
@@ -946,8 +961,7 @@ int swmi_observables(swmi_engine* engine, uint32_t lattice, int64_t* energy, int
 {
     return Guard([&] {
         Lattice& l = Eng(engine)->At(lattice);
-        engine->OneLattice(l, nullptr);
-        LaunchObservables(engine->d_one_desc.ptr, nullptr, l.g.n_blocks, kSampleAlways, engine->stream);
+        LaunchObservables(engine->Solo(l), nullptr, l.g.n_blocks, kSampleAlways, engine->stream);
         engine->LaunchCheck("observables launch");
         std::vector<int32_t> p(2ull * l.g.n_blocks);
         Check(hipMemcpyAsync(p.data(), l.partials.ptr, p.size() * 4, hipMemcpyDeviceToHost, engine->stream), "observables");
@@ -996,9 +1010,13 @@ int swmi_get_series(swmi_engine* engine, uint32_t lattice, int64_t* energy, int6
 {
     return Guard([&] {
         Lattice& l = Eng(engine)->At(lattice);
-        LatState st{};
-        Check(hipMemcpyAsync(&st, l.state.ptr, sizeof(st), hipMemcpyDeviceToHost, engine->stream), "series");
+        // the counters and the series behind them in one copy; what exceeds it in a second one
+        const uint32_t room = std::min(l.cfg.max_samples, max), first = std::min(room, kSeriesFirst);
+        std::vector<uint32_t> words(kLatStateWords + 4ull * first);
+        Check(hipMemcpyAsync(words.data(), l.state.ptr, words.size() * 4, hipMemcpyDeviceToHost, engine->stream), "series");
         Check(hipStreamSynchronize(engine->stream), "series");
+        LatState st{};
+        std::memcpy(&st, words.data(), sizeof(st));
         const uint32_t stored = std::min(st.n_samples, st.series_cap);
         const uint32_t n = std::min(stored, max);
         if (count)
@@ -1006,8 +1024,15 @@ int swmi_get_series(swmi_engine* engine, uint32_t lattice, int64_t* energy, int6
         if (n == 0)
             return;
         std::vector<int64_t> buf(2ull * n);
-        Check(hipMemcpyAsync(buf.data(), l.state.ptr + kLatStateWords, buf.size() * 8, hipMemcpyDeviceToHost, engine->stream), "series");
-        Check(hipStreamSynchronize(engine->stream), "series");
+        const uint32_t have = std::min(n, first);
+        std::memcpy(buf.data(), words.data() + kLatStateWords, 16ull * have);
+        if (n > have)
+        {
+            Check(hipMemcpyAsync(buf.data() + 2ull * have, l.state.ptr + kLatStateWords + 4ull * have, 16ull * (n - have),
+                                 hipMemcpyDeviceToHost, engine->stream),
+                  "series");
+            Check(hipStreamSynchronize(engine->stream), "series");
+        }
         for (uint32_t i = 0; i < n; ++i)
         {
             if (energy)
@@ -1021,14 +1046,8 @@ int swmi_get_series(swmi_engine* engine, uint32_t lattice, int64_t* energy, int6
 int swmi_reset_measurements(swmi_engine* engine)
 {
     return Guard([&] {
-        for (auto& l : Eng(engine)->lattices)
-        {
-            if (!l)
-                continue;
-            Check(hipMemsetAsync(reinterpret_cast<uint8_t*>(l->state.ptr) + 4 * kStSamples, 0, 4, engine->stream), "reset");
-            Check(hipMemsetAsync(reinterpret_cast<uint8_t*>(l->state.ptr) + 4 * kStMoments, 0, sizeof(LatState::moments), engine->stream),
-                  "reset");
-        }
+        LaunchResetMeasurements(Eng(engine)->d_desc.ptr, static_cast<uint32_t>(engine->lattices.size()), engine->stream);
+        engine->LaunchCheck("reset");
         Check(hipStreamSynchronize(engine->stream), "reset");
     });
 }

@@ -136,6 +136,7 @@ namespace swmi
         uint64_t n = 0;            // sites, n0 * n1
         uint64_t np = 0;           // padded sites, pitch * n1 (the per-site arrays hold np entries)
         uint32_t n_groups = 0;     // np / 64
+        uint32_t slot = 0;         // index among the engine's lattices (set by Rebuild)
         Geometry g;
         float p_add = 0.0f;
         uint64_t threshold = 0;
@@ -210,8 +211,11 @@ struct swmi_engine
     int device = 0;
     hipStream_t stream = nullptr;
     std::vector<std::unique_ptr<swmi::Lattice>> lattices;
+    // descriptors of all lattices, for the work lists, then once more each lattice's own with block_base 0, for launches
+    // over one lattice (with a null work list)
     std::vector<swmi::LatDesc> descs;
     swmi::DeviceBuffer<swmi::LatDesc> d_desc;
+    swmi::DeviceBuffer<uint8_t> stage;   // spins on their way to the host, kept between calls
     std::vector<swmi::KernelClass> classes;   // the tiled ones first
     size_t n_tiled = 0;                       // classes the tiled kernels sweep; the rest are resident
     bool recording = false;   // some lattice records its bonds (selects the inspection build of k_bond_label)
@@ -223,7 +227,7 @@ struct swmi_engine
     std::vector<hipStream_t> side_streams;
     std::vector<hipEvent_t> join_events;
     hipEvent_t fork_event = nullptr;
-    // single-lattice descriptor for the inspection hooks (launched with a null work list)
+    // single-lattice descriptor for the inspection hooks, whose buffers are not in the descriptors above
     swmi::DeviceBuffer<swmi::LatDesc> d_one_desc;
 
     swmi_engine();
@@ -266,7 +270,9 @@ struct swmi_engine
     void OneLattice(const swmi::Lattice& l, const uint8_t* bond_in);
     // brings lattice l's stored lcg32 states to its current iteration
     void AdvanceRng(const swmi::Lattice& l);
-    // OneLattice, then applies lattice l's pending flip
+    // lattice l's own descriptor
+    const swmi::LatDesc* Solo(const swmi::Lattice& l) const { return d_desc.ptr + lattices.size() + l.slot; }
+    // applies lattice l's pending flip
     void MaterializeOne(const swmi::Lattice& l);
     uint64_t TotalSites() const;
 };

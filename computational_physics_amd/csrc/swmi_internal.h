@@ -218,6 +218,12 @@ namespace swmi
                        hipStream_t stream);
     // n row-major spins (width n0v) into the padded spin bytes (pitch), keeping the selector bits
     void LaunchSetSpins(uint8_t* spins, const uint8_t* src, uint64_t n, uint32_t n0v, uint32_t pitch, hipStream_t stream);
+    // the spins of row-major sites [first, first + n) (width n0v) from the padded spin bytes (pitch); without padding first
+    // and n are multiples of 64
+    void LaunchGetSpins(uint8_t* dst, const uint8_t* spins, uint64_t first, uint64_t n, uint32_t n0v, uint32_t pitch, hipStream_t stream);
+    void LaunchSetThreshold(LatDesc* a, LatDesc* b, uint32_t threshold, hipStream_t stream);
+    // samples and moments of n lattices back to zero
+    void LaunchResetMeasurements(const LatDesc* d_desc, uint32_t n, hipStream_t stream);
     // row-major bytes (width n0v) to np padded bytes (pitch), padding 0
     void LaunchPadBytes(uint8_t* dst, const uint8_t* src, uint64_t np, uint32_t n0v, uint32_t pitch, hipStream_t stream);
     // padded canonical labels to the n row-major labels of the row-major sites

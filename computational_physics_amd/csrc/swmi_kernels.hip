@@ -1205,6 +1205,39 @@ namespace swmi
         }
     }
 
+    // Download of row-major spins [first, first + n), bit 0 of the spin bytes: sixteen sites per thread where no row is
+    // padded (first and n are then multiples of 64).
+    __global__ __launch_bounds__(256) void k_get_spins(uint8_t* __restrict__ dst, const uint8_t* __restrict__ spins, const uint64_t first,
+                                                       const uint64_t n,
+                                                       const uint32_t n0v, const uint32_t pitch)
+    {
+        const uint64_t i = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+        if (n0v == pitch)
+        {
+            if (16u * i < n)
+                reinterpret_cast<u32x4*>(dst)[i] = reinterpret_cast<const u32x4*>(spins + first)[i] & 0x01010101u;
+        }
+        else if (i < n)
+            dst[i] = spins[((first + i) / n0v) * pitch + (first + i) % n0v] & 1u;
+    }
+
+    __global__ void k_set_threshold(LatDesc* __restrict__ a, LatDesc* __restrict__ b, const uint32_t threshold)
+    {
+        a->threshold = threshold;
+        b->threshold = threshold;
+    }
+
+    __global__ __launch_bounds__(64) void k_reset_measurements(const LatDesc* __restrict__ descs, const uint32_t n)
+    {
+        const uint32_t i = blockIdx.x * 64u + threadIdx.x;
+        if (i >= n)
+            return;
+        uint32_t* const state = descs[i].state;
+        state[kStSamples] = 0u;
+        for (uint32_t w = kStMoments; w < kLatStateWords; ++w)
+            state[w] = 0u;
+    }
+
     // Row-major bytes (n0v wide) to the padded layout (pitch wide, padding columns 0), and back.
     __global__ __launch_bounds__(256) void k_pad_bytes(uint8_t* __restrict__ dst, const uint8_t* __restrict__ src, const uint64_t np,
                                                        const uint32_t n0v, const uint32_t pitch)
@@ -1373,6 +1406,23 @@ namespace swmi
                         hipStream_t stream)
     {
         k_set_spins<<<static_cast<uint32_t>((n + 255) / 256), 256, 0, stream>>>(spins, src, n, n0v, pitch);
+    }
+
+    void LaunchGetSpins(uint8_t* dst, const uint8_t* spins, const uint64_t first, const uint64_t n, const uint32_t n0v, const uint32_t pitch,
+                        hipStream_t stream)
+    {
+        const uint64_t threads = n0v == pitch ? n / 16u : n;
+        k_get_spins<<<static_cast<uint32_t>((threads + 255) / 256), 256, 0, stream>>>(dst, spins, first, n, n0v, pitch);
+    }
+
+    void LaunchSetThreshold(LatDesc* a, LatDesc* b, const uint32_t threshold, hipStream_t stream)
+    {
+        k_set_threshold<<<1, 1, 0, stream>>>(a, b, threshold);
+    }
+
+    void LaunchResetMeasurements(const LatDesc* d_desc, const uint32_t n, hipStream_t stream)
+    {
+        k_reset_measurements<<<(n + 63u) / 64u, 64, 0, stream>>>(d_desc, n);
     }
 
     void LaunchPadBytes(uint8_t* dst, const uint8_t* src, const uint64_t np, const uint32_t n0v, const uint32_t pitch,
