@@ -501,7 +501,7 @@ void swmi_engine::EnqueueSweeps(uint32_t n)
                 LaunchJoin(d_desc.ptr, k.d_slots.ptr, k.n_lat, k.max_blocks, s);
                 continue;
             }
-            LaunchMerge(k.Descs(d_desc.ptr), k.WorkList(), k.total_blocks, s);
+            LaunchMerge(k.Descs(d_desc.ptr), k.WorkList(), k.total_blocks, k.tw64, k.max_block_rows, s);
             LaunchResolve(k.Descs(d_desc.ptr), k.WorkList(), k.total_blocks, k.max_block_rows, s);
         }
     }
@@ -1113,7 +1113,7 @@ int swmi_label_bonds(swmi_engine* engine, uint32_t lattice, const uint8_t* bonds
         engine->OneLattice(l, l.bond_in.ptr);
         LaunchBondLabel(engine->d_one_desc.ptr, nullptr, l.g.n_blocks, l.g.twr, FormOf(l.g), l.g.tw == 64, l.np != l.n, true,
                         engine->stream);
-        LaunchMerge(engine->d_one_desc.ptr, nullptr, l.g.n_blocks, engine->stream);
+        LaunchMerge(engine->d_one_desc.ptr, nullptr, l.g.n_blocks, l.g.tw == 64, l.g.ecol_stride, engine->stream);
         LaunchWriteLabels(engine->d_one_desc.ptr, nullptr, l.g.n_blocks, l.g.twr, engine->stream);
         engine->LaunchCheck("label launch");
         Check(hipStreamSynchronize(engine->stream), "label");
@@ -1371,7 +1371,7 @@ int swmi_time_kernels(swmi_engine* engine, uint32_t n_sweeps, float* ms)
                 if (k.Joined())
                     LaunchJoin(engine->d_desc.ptr, k.d_slots.ptr, k.n_lat, k.max_blocks, engine->stream);
                 else
-                    LaunchMerge(k.Descs(engine->d_desc.ptr), k.WorkList(), k.total_blocks, engine->stream);
+                    LaunchMerge(k.Descs(engine->d_desc.ptr), k.WorkList(), k.total_blocks, k.tw64, k.max_block_rows, engine->stream);
             Check(hipEventRecord(ev[2], engine->stream), "event");
             for (auto& k : engine->classes)
                 if (!k.Joined())

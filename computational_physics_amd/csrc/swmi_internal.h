@@ -172,7 +172,9 @@ namespace swmi
     // pad: some lattice of the work list is padded (selects the PAD specialisation, correct for every lattice)
     void LaunchBondLabel(const LatDesc* d_desc, const uint32_t* d_block_lat, uint32_t total_blocks, uint32_t max_twr,
                          BondForm form, bool all_tw64, bool pad, bool debug, hipStream_t stream);
-    void LaunchMerge(const LatDesc* d_desc, const uint32_t* d_block_lat, uint32_t total_blocks, hipStream_t stream);
+    // max_rows: lattice rows of the tallest block
+    void LaunchMerge(const LatDesc* d_desc, const uint32_t* d_block_lat, uint32_t total_blocks, bool all_tw64, uint32_t max_rows,
+                     hipStream_t stream);
     // n_lattices small lattices (descriptors d_slots[i]), one workgroup each: `groups` groups of `sweeps` sweeps with a
     // sample after each group when sample_mode >= 0. max_sites, max_rows: bounds on their padded sites and on the
     // rows of a strip (ResidentRows). full: no padding, and every wave of every lattice has exactly max_rows rows, 4 or

@@ -279,6 +279,175 @@ namespace swmi
         }
     }
 
+    // k_merge for 64-wide tiles and blocks of at most 64 rows (at most 252 boundary sites, so 252 slots): one wave per
+    // block takes both of its edges. The bonded pairs are first united in LDS, in a table indexed by slot (256 entries
+    // each for the block, its right and its lower neighbour: no hashing), so that pairs that share a cluster, also
+    // across the two edges, cost one lattice-wide union per non-root slot and no two lanes race on one slot; a slot
+    // that several lanes hold is claimed by the last of them to write its mark.
+    template <bool FRESH>
+    __global__ __launch_bounds__(64) void k_merge_block(const LatDesc* __restrict__ descs, const uint32_t* __restrict__ block_lat,
+                                                        const uint32_t total_blocks)
+    {
+        constexpr uint32_t kN = 256u;
+        __shared__ uint64_t L[3u * kN];   // (key of the parent << 32) | parent; later the list of unions
+        const uint32_t b = RemapBlock(total_blocks);
+        if (b >= total_blocks)
+            return;
+        const LatDesc& d = descs[LatticeOf(block_lat, b)];
+        const gptr<const uint32_t> active = Glob(static_cast<const uint32_t*>(d.state)) + kStActive;
+        const Block bl = DecodeBlock(d, b);
+        const uint32_t lane = threadIdx.x;
+        const gptr<const uint64_t> bb = Glob(static_cast<const uint64_t*>(d.bbits)) + kBbitWords * bl.lb;
+        const gptr<const uint32_t> ec = Glob(static_cast<const uint32_t*>(d.ecol)), er = Glob(static_cast<const uint32_t*>(d.erow));
+        const gptr<uint32_t> err = Glob(d.state) + kStErr;
+        const uint32_t es = d.ecol_stride, twr = d.twr, qcap = d.qcap, slots = kWavesPerBlock * d.edge_cap;
+        const uint32_t sx_r = (bl.sx + 1u == d.tiles_x) ? 0u : bl.sx + 1u, sy_b = bl.sy + 1u == d.blocks_y ? 0u : bl.sy + 1u;
+        const uint32_t lb_r = bl.sy * d.tiles_x + sx_r, lb_b = sy_b * d.tiles_x + bl.sx;
+        const uint32_t row = min(lane, bl.nwr - 1u);
+        // pair 0: the right edge at lattice row `lane`; pair 1: the down edge at column `lane`
+        uint32_t va[2], vb[2];
+        va[0] = ec[(2u * bl.lb + 1u) * es + row];
+        vb[0] = ec[2u * lb_r * es + row];
+        va[1] = er[2u * 64u * bl.lb + 64u + lane];
+        vb[1] = er[2u * 64u * lb_b + lane];
+        const uint64_t right = bb[1u + row / twr], down = bb[0];
+        const uint32_t act = *active;
+        Issued(va[0]);
+        Issued(vb[0]);
+        Issued(va[1]);
+        Issued(vb[1]);
+        Issued(right);
+        Issued(down);
+        bool bit[2] = {lane < bl.nwr && ((right >> (row % twr)) & 1ull) != 0ull, ((down >> lane) & 1ull) != 0ull};
+        if (act == 0u || !__ballot(bit[0] || bit[1]))
+            return;
+
+        uint32_t n[4], k[4];   // nodes and keys: a and b of pair 0, a and b of pair 1
+#pragma unroll
+        for (uint32_t p = 0; p < 2u; ++p)
+        {
+            const uint32_t region = (1u + p) * kN, base = BlockBase(d, p ? bl.sx : sx_r, p ? sy_b : bl.sy);
+            const uint32_t sa = ((va[p] >> 16) & 0x7FFFu) - qcap, sb = ((vb[p] >> 16) & 0x7FFFu) - qcap;
+            // both ends of a bond across an edge belong to edge-reaching clusters
+            const bool good = ((va[p] >> 16) & (vb[p] >> 16) & kEdgeFlag) && sa < min(slots, kN) && sb < min(slots, kN);
+            if (bit[p] && !good)
+            {
+                (void)__hip_atomic_fetch_or(err, kErrLabelRange, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                bit[p] = false;
+            }
+            n[2u * p] = bit[p] ? sa : 0u;
+            n[2u * p + 1u] = bit[p] ? region + sb : 0u;
+            k[2u * p] = SiteOf(bl.base, bl.stride, va[p] & 0xFFFFu);
+            k[2u * p + 1u] = SiteOf(base, bl.stride, vb[p] & 0xFFFFu);
+            if (bit[p])
+            {
+                __hip_atomic_store(&L[n[2u * p]], SlotEntry(k[2u * p], n[2u * p]), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                __hip_atomic_store(&L[n[2u * p + 1u]], SlotEntry(k[2u * p + 1u], n[2u * p + 1u]), __ATOMIC_RELAXED,
+                                   __HIP_MEMORY_SCOPE_WORKGROUP);
+            }
+        }
+#pragma unroll
+        for (uint32_t p = 0; p < 2u; ++p)
+        {
+            uint32_t x = n[2u * p], y = n[2u * p + 1u];
+            bool open = bit[p];
+            while (__ballot(open))
+            {
+                if (open)
+                {
+                    uint64_t ex = LocalEntry(L, x), ey = LocalEntry(L, y);
+                    while (static_cast<uint32_t>(ex) != x || static_cast<uint32_t>(ey) != y)
+                    {
+                        x = static_cast<uint32_t>(ex);
+                        y = static_cast<uint32_t>(ey);
+                        ex = LocalEntry(L, x);
+                        ey = LocalEntry(L, y);
+                    }
+                    if (x == y)
+                        open = false;
+                    else
+                    {
+                        // roots hold their own entries; link the larger under the smaller (a lattice one block wide or
+                        // high has the same slot in two of the table's parts: equal keys, ordered by node)
+                        if (ex > ey)
+                        {
+                            const uint32_t t = x;
+                            x = y;
+                            y = t;
+                            const uint64_t te = ex;
+                            ex = ey;
+                            ey = te;
+                        }
+                        const uint64_t old = __hip_atomic_fetch_min(&L[y], ex, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                        if (old == ey)
+                            open = false;
+                        else   // y had been linked under old's parent (which this link may have displaced): unite with it
+                            y = static_cast<uint32_t>(old);
+                    }
+                }
+            }
+        }
+        // the roots of the lane's nodes, chased together (a lane without a pair sits on no node: done at once)
+        uint64_t e[4];
+        uint32_t r[4];
+#pragma unroll
+        for (uint32_t i = 0; i < 4u; ++i)
+        {
+            r[i] = n[i];
+            e[i] = bit[i >> 1] ? LocalEntry(L, n[i]) : static_cast<uint64_t>(n[i]);
+        }
+        for (;;)
+        {
+            bool moved = false;
+#pragma unroll
+            for (uint32_t i = 0; i < 4u; ++i)
+                if (static_cast<uint32_t>(e[i]) != r[i])
+                {
+                    r[i] = static_cast<uint32_t>(e[i]);
+                    e[i] = LocalEntry(L, r[i]);
+                    moved = true;
+                }
+            if (!__ballot(moved))
+                break;
+        }
+        // one lane claims each node that is not its component's root
+        bool has[4];
+#pragma unroll
+        for (uint32_t i = 0; i < 4u; ++i)
+            if (r[i] != n[i])
+                __hip_atomic_store(&L[n[i]], static_cast<uint64_t>(lane * 4u + i), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+#pragma unroll
+        for (uint32_t i = 0; i < 4u; ++i)
+            has[i] = r[i] != n[i] && LocalEntry(L, n[i]) == static_cast<uint64_t>(lane * 4u + i);
+        const auto slot_of = [&](const uint32_t node) {
+            return (node < kN ? bl.lb : (node < 2u * kN ? lb_r : lb_b)) * slots + (node & (kN - 1u));
+        };
+        // the unions, listed one per lane: two words (slot, key) each for the node and its root. At most one per link
+        // made above, so at most 128.
+        uint32_t total = 0;
+#pragma unroll
+        for (uint32_t i = 0; i < 4u; ++i)
+        {
+            const uint64_t f = __ballot(has[i]);
+            const uint32_t at = total + __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(f >> 32), __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(f), 0u));
+            if (has[i] && at < 128u)
+            {
+                __hip_atomic_store(&L[2u * at], SlotEntry(k[i], slot_of(n[i])), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                __hip_atomic_store(&L[2u * at + 1u], SlotEntry(static_cast<uint32_t>(e[i] >> 32), slot_of(r[i])), __ATOMIC_RELAXED,
+                                   __HIP_MEMORY_SCOPE_WORKGROUP);
+            }
+            total += static_cast<uint32_t>(__popcll(f));
+        }
+        for (uint32_t i = lane; i < min(total, 128u); i += 64u)
+        {
+            const uint64_t x = LocalEntry(L, 2u * i), y = LocalEntry(L, 2u * i + 1u);
+            SlotUnion<FRESH>(Glob(d.cpar), static_cast<uint32_t>(x), static_cast<uint32_t>(x >> 32), static_cast<uint32_t>(y),
+                             static_cast<uint32_t>(y >> 32), d.n_blocks * slots, err);
+        }
+        if (total > 128u && lane == 0u)
+            (void)__hip_atomic_fetch_or(err, kErrLabelRange, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+
     // =============================================================================================
     // k_resolve / k_flip: resolve + flip (reference ResolveLabels_Kernel / FlipClusters_Kernel,
     // swendsen_wang_amd_gpu.cpp:403-467), split into the decision (k_resolve, end of every sweep) and its
@@ -1303,8 +1472,10 @@ namespace swmi
     // Two-wave merge workgroups resident at once on MI355X: 256 CUs x 16 (8 waves per SIMD).
     constexpr uint32_t kOneRoundMergeBlocks = 4096;
     // Launches of at least this many blocks unite each edge's pairs in LDS before the lattice-wide unions: many
-    // blocks race on the memory-side atomics there. Smaller launches see few races and only the added latency
-    // (measured at 512 to 2048 blocks: 1024^2 and 2048^2 lattices are faster without).
+    // blocks race on the memory-side atomics there. Smaller launches see few races and only the added latency.
+    // Microseconds per sweep without / with, both edges of a block in one wave (k_merge_block) at T_c: 36 blocks 19.6 /
+    // 21.0, 256 blocks 21.8 / 23.4, 1024 blocks 32.6 / 33.5, 4096 blocks (with each edge's own local unions before, which
+    // narrow and tall tiles keep) 67.4 / 66.9, 16384 blocks 234.8 / 224.8.
     constexpr uint32_t kLocalUnionBlocks = 4096;
 
     template <bool FRESH>
@@ -1316,8 +1487,17 @@ namespace swmi
             k_merge<FRESH, false><<<XcdGrid(total_blocks), 128, 0, stream>>>(d_desc, d_block_lat, total_blocks);
     }
 
-    void LaunchMerge(const LatDesc* d_desc, const uint32_t* d_block_lat, const uint32_t total_blocks, hipStream_t stream)
+    void LaunchMerge(const LatDesc* d_desc, const uint32_t* d_block_lat, const uint32_t total_blocks, const bool all_tw64,
+                     const uint32_t max_rows, hipStream_t stream)
     {
+        if (all_tw64 && max_rows <= 64u && total_blocks >= kLocalUnionBlocks)
+        {
+            if (total_blocks <= kOneRoundMergeBlocks)
+                k_merge_block<true><<<XcdGrid(total_blocks), 64, 0, stream>>>(d_desc, d_block_lat, total_blocks);
+            else
+                k_merge_block<false><<<XcdGrid(total_blocks), 64, 0, stream>>>(d_desc, d_block_lat, total_blocks);
+            return;
+        }
         if (total_blocks <= kOneRoundMergeBlocks)
             LaunchMergeAs<true>(d_desc, d_block_lat, total_blocks, stream);
         else

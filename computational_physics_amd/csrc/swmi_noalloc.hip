@@ -144,7 +144,7 @@ extern "C" int swmi_label_bonds_noalloc(const uint8_t* bonds, uint32_t n0, uint3
         if (pad)
             LaunchPadBytes(const_cast<uint8_t*>(d.bond_in), bonds, np, n0, g.pitch, s);
         LaunchBondLabel(d_desc, nullptr, g.n_blocks, g.twr, FormOf(g), g.tw == 64, pad, true, s);
-        LaunchMerge(d_desc, nullptr, g.n_blocks, s);
+        LaunchMerge(d_desc, nullptr, g.n_blocks, g.tw == 64, g.ecol_stride, s);
         LaunchWriteLabels(d_desc, nullptr, g.n_blocks, g.twr, s);
         if (pad)
             LaunchUnpadLabels(labels, d.parent, n, n0, g.pitch, s);

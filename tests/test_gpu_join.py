@@ -37,3 +37,35 @@ def test_lattices_of_a_joined_engine_equal_their_lone_runs(swmi):
             alone.sweep(13 if k == 1 else 40)
             np.testing.assert_array_equal(alone.spins(), got[k], err_msg=f"lattice {k}")
             assert alone.error_flags() == 0
+
+
+@pytest.mark.parametrize("n0,n1", [(64, 262144), (262144, 64), (128, 131074)])
+@pytest.mark.parametrize("T", [2.0, 2.2691853])
+def test_launches_of_4096_blocks_one_or_two_wide(swmi, oracle, n0, n1, T):
+    """From 4096 blocks one wave unites both edges of a block in LDS (k_merge_block). A block that is its own right or
+    lower neighbour has each slot twice in that table."""
+    print(f"block merge {n0}x{n1} T {T}", flush=True)
+    ref = oracle.PerSite(n0, n1, T, seed=3)
+    with swmi.Engine(swmi.LatticeConfig(n0, n1, T, seed=3)) as e:
+        e.sweep(1)
+        _, labels = ref.sweep(record=True)
+        np.testing.assert_array_equal(e.labels(), labels)
+        np.testing.assert_array_equal(e.spins(), ref.spins)
+        e.sweep(1)
+        ref.sweep()
+        np.testing.assert_array_equal(e.spins(), ref.spins)
+        assert e.error_flags() == 0
+
+
+def test_many_small_tiled_lattices_equal_their_lone_runs(swmi):
+    """1040 lattices of two by two blocks in one launch of 4160 blocks: every block meets the same neighbour twice."""
+    print("block merge, 1040 lattices", flush=True)
+    cfgs = [swmi.LatticeConfig(128, 128, 1.9 + 0.001 * i, seed=i, tile_rows=16, flip_rule=i % 2) for i in range(1040)]
+    with swmi.Engine(cfgs) as e:
+        e.sweep(12)
+        got = {i: e.spins(i) for i in range(0, 1040, 13)}
+        assert all(e.error_flags(i) == 0 for i in got)
+    for i, spins in got.items():
+        with swmi.Engine(cfgs[i]) as alone:
+            alone.sweep(12)
+            np.testing.assert_array_equal(alone.spins(), spins, err_msg=f"lattice {i}")
