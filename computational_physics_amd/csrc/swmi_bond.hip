@@ -596,7 +596,8 @@ namespace swmi
             const uint64_t tgtB = TW64 ? Bbot : Shl(Bbot, 64u - tw);
             const bool go = LaneBit(FirstBondPerInterval(last_D, last_B & tgtB, rowstart));
             const uint32_t top = wr * 256u + lane4;
-            LdsUnionLockstep(P, go ? top : 0u, go ? top + 256u - (64u - tw) * 4u : 0u);
+            // (64-wide tiles: from the root the last row was labelled with)
+            LdsUnionLockstep(P, go ? (TW64 ? Rp : top) : 0u, go ? top + 256u - (64u - tw) * 4u : 0u);
         }
         __syncthreads();
 
