@@ -56,8 +56,8 @@ def _run(cmd: list[str]) -> None:
 def build_library() -> Path:
     LIB_DIR.mkdir(exist_ok=True)
     parts = [(src, []) for src in ("swmi_kernels.hip", "swmi_resident.hip", "swmi_engine.hip", "swmi_noalloc.hip", "swmi_server.cpp")]
-    parts += [("swmi_bond.hip", [f"-DSWMI_BOND_TW64={tw64}", f"-DSWMI_BOND_DBG={dbg}"])
-              for tw64 in ("true", "false") for dbg in ("true", "false")]
+    parts += [("swmi_bond.hip", [f"-DSWMI_BOND_TW64={tw64}", f"-DSWMI_BOND_MODE={mode}"])
+              for tw64 in ("true", "false") for mode in (0, 1, 2)]
     with tempfile.TemporaryDirectory() as tmp, ThreadPoolExecutor(min(8, os.cpu_count() or 1)) as pool:
         objects = [str(Path(tmp) / f"{i}.o") for i in range(len(parts))]
         compiles = [pool.submit(_run, [HIPCC, *HIP_FLAGS, *defs, "-I", str(ROOT / "include"), "-c", str(CSRC / src), "-o", obj])

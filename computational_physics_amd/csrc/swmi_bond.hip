@@ -1,7 +1,6 @@
 // swmi_bond.hip -- k_bond_label: bond activation and tile labelling (the first kernel of a sweep, see
-// swmi_kernels.hip). Compiled once per SWMI_BOND_TW64 (64-wide tiles or narrow ones) and SWMI_BOND_DBG (the
-// inspection build or the sweep proper): the specialisations take most of the build and these parts build in
-// parallel.
+// swmi_kernels.hip). Compiled once per SWMI_BOND_TW64 (64-wide tiles or narrow ones) and SWMI_BOND_MODE (a BondMode): the
+// specialisations take most of the build and these parts build in parallel.
 #include "swmi_device.h"
 
 namespace swmi
@@ -21,8 +20,8 @@ namespace swmi
     // Nodes of the LDS union-find are byte offsets into P. After the final find, the root of every
     // cluster that reaches the block edge carries kPFlag in its own entry, so a site's label (root index,
     // plus kEdgeFlag) is P[root] >> 2.
-    // DBG: the inspection modes (injected bonds instead of generated ones, bond recording) are compiled in;
-    // the sweep kernel proper has neither branch.
+    // MODE: the sweep proper; the inspection build, in which bonds may be injected instead of generated and may be
+    // recorded; or the labelling of an injected bond field alone.
     // PAD: the lattice is stored with a row pitch d.n0 above its width d.n0v; in the last tile column only
     // the lanes up to d.elast hold sites (mask d.vlast), the rest are padding: they bond to nothing, their
     // draws are unused, and the row's last site bonds across the lattice edge instead of lane tw - 1.
@@ -30,12 +29,13 @@ namespace swmi
     // waves label a tile each; sixteen label a quarter tile each, which shortens the chain of dependent LDS
     // operations down a strip where a launch has too few blocks to fill the chip (LaunchBondLabelT).
     // FULL: every strip of every block has exactly TWR_MAX rows, so that the row counts are constants.
-    template <uint32_t NW, uint32_t TWR_MAX, bool TW64, bool DBG, bool PAD, bool FULL>
+    template <uint32_t NW, uint32_t TWR_MAX, bool TW64, BondMode MODE, bool PAD, bool FULL>
     __device__ __forceinline__ void BondLabel(const LatDesc* __restrict__ descs, const uint32_t* __restrict__ block_lat,
                                               const uint32_t total_blocks)
     {
         // All loads of a chunk of rows are issued before its first store: on this hardware the memory
         // counter that a load waits on also counts the stores issued before it.
+        constexpr bool DBG = MODE == BondMode::kInspect;
         constexpr uint32_t kCh = TWR_MAX < 16 ? TWR_MAX : 16;
         constexpr uint32_t kRows = TWR_MAX < 16 ? TWR_MAX : 16;   // rows resolved together at the end
         // 64-wide tiles of at most kRows rows keep their rows' roots in registers from the row loop to the labels
@@ -84,7 +84,7 @@ namespace swmi
         const uint64_t vmask = lastcol ? d.vlast : ~0ull;   // lanes that hold sites
         const uint32_t elane = lastcol ? d.elast : tw - 1u;  // lx of a lattice row's last site in this tile
         const bool rbound = lx == elane;
-        const bool injected = DBG && d.bond_in != nullptr;
+        const bool injected = MODE == BondMode::kLabel || (DBG && d.bond_in != nullptr);
         const uint32_t thr = d.threshold;
         const gptr<uint32_t> stp = Glob(d.state);
         const gptr<uint8_t> dump = DBG ? Glob(d.bond_dump) : nullptr;
@@ -134,7 +134,7 @@ namespace swmi
         const uint32_t y_below = nrow > 0 ? ((y_last + 1u == n1) ? 0u : y_last + 1u) : 0u;
         const uint32_t below = (r_begin + nrow) * bl.stride + lx;   // the site below the tile, inside the block
         const uint32_t below_halo = (sy_b * d.tiles_x + bl.sx) * d.halo_stride + d.ecol_stride + lx;
-        const uint32_t hd_spin = spins[y_below * n0 + x];
+        const uint32_t hd_spin = MODE == BondMode::kLabel ? 0u : spins[y_below * n0 + x];
         // (the label-only pass over injected bonds has no flip bits and no halos: those loads belong to the sweep,
         // where `injected` is false at compile time)
         uint32_t fbw = 0, hd_lab = 0, hd_sv = 0, hd_h0 = 0, hd_h1 = 0;
@@ -408,6 +408,8 @@ namespace swmi
                         {
                             Ball = __ballot((aux[i] & 1u) != 0u);
                             U2 = __ballot((aux[i] & 2u) != 0u);
+                            if (kBits)
+                                u63_b = (u63_b << 1) + static_cast<uint32_t>(Ball >> 63);
                         }
                         if (PAD)
                         {
@@ -491,7 +493,7 @@ namespace swmi
             Chunk c0;
             if (nrow > 0)
                 load(0u, c0);
-            if (kBits && nrow > 0)
+            if (kBits && MODE != BondMode::kLabel && nrow > 0)
             {
                 // right halo of the tile's rows: under a pending flip the right neighbour's flipped first column
                 const uint32_t lr = r_begin + min(lane, nrow - 1u);
@@ -538,7 +540,7 @@ namespace swmi
                 // row r of the words is bit nrow - 1 - r
                 const uint32_t up = 32u - nrow;   // (nrow is 1 to 16)
                 const uint32_t h = static_cast<uint32_t>(__ballot((hright & 1u) != 0u));
-                right_bits = ~((__brev(s63_b) >> up) ^ h) & (__brev(u63_b) >> up);
+                right_bits = (MODE == BondMode::kLabel ? ~0u : ~((__brev(s63_b) >> up) ^ h)) & (__brev(u63_b) >> up);
                 colv = (__brev(col_b) >> up) >> (lane & 31u);
             }
             if (NW != kWavesPerBlock && lane == 0u && right_bits != 0ull)   // read after the last barrier
@@ -880,27 +882,77 @@ namespace swmi
     // keeps the excess scalar registers in vector lanes). Narrow tiles keep the default budget (the cap would spill
     // vector registers to scratch), and taller tiles are limited by their LDS anyway.
     // NW waves per block: four take a tile each, eight and sixteen a half and a quarter of a tile.
-    template <uint32_t NW, uint32_t TWR_MAX, bool DBG, bool PAD, bool FULL>
+    template <uint32_t NW, uint32_t TWR_MAX, BondMode MODE, bool PAD, bool FULL>
     __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(8, 8))) void k_bond_label(
         const LatDesc* __restrict__ descs, const uint32_t* __restrict__ block_lat, const uint32_t total_blocks)
     {
-        BondLabel<NW, TWR_MAX, true, DBG, PAD, FULL>(descs, block_lat, total_blocks);
+        BondLabel<NW, TWR_MAX, true, MODE, PAD, FULL>(descs, block_lat, total_blocks);
     }
 
-    template <uint32_t TWR_MAX, bool TW64, bool DBG, bool PAD>
+    template <uint32_t TWR_MAX, bool TW64, BondMode MODE, bool PAD>
     __global__ __launch_bounds__(256) void k_bond_label_any(const LatDesc* __restrict__ descs, const uint32_t* __restrict__ block_lat,
                                                             const uint32_t total_blocks)
     {
-        BondLabel<kWavesPerBlock, TWR_MAX, TW64, DBG, PAD, false>(descs, block_lat, total_blocks);
+        BondLabel<kWavesPerBlock, TWR_MAX, TW64, MODE, PAD, false>(descs, block_lat, total_blocks);
+    }
+
+    // The labelling of one bond field alone: the descriptor comes with the launch, not from memory.
+    template <uint32_t NW, uint32_t TWR_MAX, bool PAD, bool FULL>
+    __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(8, 8))) void k_label_blocks(const LatDesc d, const uint32_t total_blocks)
+    {
+        BondLabel<NW, TWR_MAX, true, BondMode::kLabel, PAD, FULL>(&d, nullptr, total_blocks);
+    }
+
+    template <bool PAD>
+    __global__ __launch_bounds__(256) void k_label_blocks_narrow(const LatDesc d, const uint32_t total_blocks)
+    {
+        BondLabel<kWavesPerBlock, 16, false, BondMode::kLabel, PAD, false>(&d, nullptr, total_blocks);
     }
 
     // Launches of few blocks of 64-wide tiles, all of a height that four waves can share, give every block more waves:
-    // sixteen up to one block per CU, eight up to two. Microseconds per sweep with 4 / 8 / 16 waves: 256 blocks
-    // (1024^2) 28.0 / - / 24.2, 352 blocks (1000 x 1350) 25.4 / 23.7 / 25.1, 1024 blocks (2048^2) 38.6 / 38.8 / 46.
+    // sixteen up to one block per CU, eight up to three. Microseconds per sweep with 4 / 8 / 16 waves: 256 blocks
+    // (1024^2) 28.0 / - / 24.2, 352 blocks (1000 x 1350) 25.4 / 23.7 / 25.1, 484 (1408^2) - / 25.5 / 26.9, 676 (1664^2)
+    // 29.2 / 28.8 / -, 1024 (2048^2) 32.6 / 33.3 / 46.
     constexpr uint32_t kWideBlocks = 256;
-    constexpr uint32_t kHalfBlocks = 512;
+    constexpr uint32_t kHalfBlocks = 768;
 
-    template <bool TW64, bool DBG>
+    // f(NW) with the waves per block for a launch of 64-wide tiles of at most 16 rows
+    template <typename F>
+    static void WithWaves(const uint32_t total_blocks, const BondForm form, F&& f)
+    {
+        if (form != BondForm::kAny && total_blocks <= kWideBlocks)
+            f(std::integral_constant<uint32_t, 16>{});
+        else if (form != BondForm::kAny && total_blocks <= kHalfBlocks)
+            f(std::integral_constant<uint32_t, 8>{});
+        else
+            f(std::integral_constant<uint32_t, kWavesPerBlock>{});
+    }
+
+#if SWMI_BOND_MODE == 2
+    // tiles of at most 16 rows
+    template <bool TW64>
+    void LaunchLabelBlocksT(const LatDesc& d, const uint32_t total_blocks, const BondForm form, const bool pad, hipStream_t stream)
+    {
+        const uint32_t g = XcdGrid(total_blocks);
+        if constexpr (TW64)
+            WithWaves(total_blocks, form, [&](auto nw) {
+                constexpr uint32_t NW = decltype(nw)::value;
+                if (pad)
+                    k_label_blocks<NW, 64 / NW, true, false><<<g, 64 * NW, 0, stream>>>(d, total_blocks);
+                else if (form == BondForm::kFull)
+                    k_label_blocks<NW, 64 / NW, false, true><<<g, 64 * NW, 0, stream>>>(d, total_blocks);
+                else
+                    k_label_blocks<NW, 64 / NW, false, false><<<g, 64 * NW, 0, stream>>>(d, total_blocks);
+            });
+        else if (pad)
+            k_label_blocks_narrow<true><<<g, 256, 0, stream>>>(d, total_blocks);
+        else
+            k_label_blocks_narrow<false><<<g, 256, 0, stream>>>(d, total_blocks);
+    }
+
+    template void LaunchLabelBlocksT<SWMI_BOND_TW64>(const LatDesc&, uint32_t, BondForm, bool, hipStream_t);
+#else
+    template <bool TW64, BondMode MODE>
     void LaunchBondLabelT(const LatDesc* d_desc, const uint32_t* d_block_lat, const uint32_t total_blocks, const uint32_t max_twr,
                           const BondForm form, const bool pad, hipStream_t stream)
     {
@@ -910,41 +962,39 @@ namespace swmi
         };
         if constexpr (TW64)
         {
-            // NW waves per block
-            const auto launch_nw = [&](auto nw) {
-                constexpr uint32_t NW = decltype(nw)::value;
-                if (pad)
-                    launch(k_bond_label<NW, 64 / NW, DBG, true, false>, 64 * NW);
-                else if (!DBG && form == BondForm::kFull)
-                    launch(k_bond_label<NW, 64 / NW, DBG, false, !DBG>, 64 * NW);
-                else
-                    launch(k_bond_label<NW, 64 / NW, DBG, false, false>, 64 * NW);
-            };
-            if (form != BondForm::kAny && max_twr <= 16 && total_blocks <= kWideBlocks)
-                return launch_nw(std::integral_constant<uint32_t, 16>{});
-            if (form != BondForm::kAny && max_twr <= 16 && total_blocks <= kHalfBlocks)
-                return launch_nw(std::integral_constant<uint32_t, 8>{});
-            if (!pad && max_twr <= 8)
-                return launch(k_bond_label<kWavesPerBlock, 8, DBG, false, false>);
-            if (!pad && max_twr <= 16)
-                return launch_nw(std::integral_constant<uint32_t, kWavesPerBlock>{});
+            if (!pad && max_twr <= 8 && (form == BondForm::kAny || total_blocks > kHalfBlocks))
+                return launch(k_bond_label<kWavesPerBlock, 8, MODE, false, false>);
+            // (padded lattices of many blocks keep the registers of k_bond_label_any)
+            if (max_twr <= 16 && (!pad || (form != BondForm::kAny && total_blocks <= kHalfBlocks)))
+                return WithWaves(total_blocks, form, [&](auto nw) {
+                    constexpr uint32_t NW = decltype(nw)::value;
+                    constexpr bool kSweep = MODE == BondMode::kSweep;
+                    if (pad)
+                        launch(k_bond_label<NW, 64 / NW, MODE, true, false>, 64 * NW);
+                    else if (kSweep && form == BondForm::kFull)
+                        launch(k_bond_label<NW, 64 / NW, MODE, false, kSweep>, 64 * NW);
+                    else
+                        launch(k_bond_label<NW, 64 / NW, MODE, false, false>, 64 * NW);
+                });
         }
         if (pad)   // padded lattices: two tile-height bounds
         {
             if (max_twr <= 16)
-                launch(k_bond_label_any<16, TW64, DBG, true>);
+                launch(k_bond_label_any<16, TW64, MODE, true>);
             else
-                launch(k_bond_label_any<64, TW64, DBG, true>);
+                launch(k_bond_label_any<64, TW64, MODE, true>);
         }
         else if (!TW64 && max_twr <= 8)
-            launch(k_bond_label_any<8, false, DBG, false>);
+            launch(k_bond_label_any<8, false, MODE, false>);
         else if (!TW64 && max_twr <= 16)
-            launch(k_bond_label_any<16, false, DBG, false>);
+            launch(k_bond_label_any<16, false, MODE, false>);
         else if (max_twr <= 32)
-            launch(k_bond_label_any<32, TW64, DBG, false>);
+            launch(k_bond_label_any<32, TW64, MODE, false>);
         else
-            launch(k_bond_label_any<64, TW64, DBG, false>);
+            launch(k_bond_label_any<64, TW64, MODE, false>);
     }
 
-    template void LaunchBondLabelT<SWMI_BOND_TW64, SWMI_BOND_DBG>(const LatDesc*, const uint32_t*, uint32_t, uint32_t, BondForm, bool, hipStream_t);
+    template void LaunchBondLabelT<SWMI_BOND_TW64, static_cast<BondMode>(SWMI_BOND_MODE)>(const LatDesc*, const uint32_t*, uint32_t, uint32_t,
+                                                                                       BondForm, bool, hipStream_t);
+#endif
 }

@@ -154,6 +154,14 @@ namespace swmi
     };
 
 
+    // What k_bond_label does
+    enum class BondMode : uint32_t
+    {
+        kSweep,     // the bond phase of a sweep
+        kInspect,   // the same, with bonds injected (LatDesc::bond_in) or recorded (LatDesc::bond_dump)
+        kLabel      // only the labelling of injected bonds
+    };
+
     // What the tile heights of a launch's lattices allow k_bond_label (64-wide tiles)
     enum class BondForm : uint32_t
     {
@@ -206,8 +214,8 @@ namespace swmi
     void LaunchSetRngCurrent(const uint32_t* state, uint32_t* aux, hipStream_t stream);
     // brings the rng array of np sites to the lattice's current iteration
     void LaunchAdvanceRng(const uint8_t* spins, uint32_t* rng, uint64_t np, const uint32_t* state, uint32_t* aux, hipStream_t stream);
-    // allocation-free labelling: descriptor d into d_desc, fresh d.state
-    void LaunchNoAllocSetup(const LatDesc& d, LatDesc* d_desc, hipStream_t stream);
+    // labelling of the bond field d.bond_in of one lattice (tiles of at most 16 rows) into d.parent
+    void LaunchLabelBlocks(const LatDesc& d, BondForm form, bool pad, hipStream_t stream);
     void LaunchObservables(const LatDesc* d_desc, const uint32_t* d_block_lat, uint32_t total_blocks, uint32_t sample_mode,
                            hipStream_t stream);
     // lattices d_slots[0 .. n_lattices)

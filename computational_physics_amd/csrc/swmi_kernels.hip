@@ -214,13 +214,8 @@ namespace swmi
     }
 
     template <bool FRESH, bool LOCAL>
-    __global__ __launch_bounds__(128) void k_merge(const LatDesc* __restrict__ descs, const uint32_t* __restrict__ block_lat,
-                                                   const uint32_t total_blocks)
+    __device__ __forceinline__ void MergeEdges(const LatDesc& d, const uint32_t b)
     {
-        const uint32_t b = RemapBlock(total_blocks);
-        if (b >= total_blocks)
-            return;
-        const LatDesc& d = descs[LatticeOf(block_lat, b)];
         // the lattice's active flag is loaded with the edge data (an inactive lattice links nothing)
         const gptr<const uint32_t> active = Glob(static_cast<const uint32_t*>(d.state)) + kStActive;
         const Block bl = DecodeBlock(d, b);
@@ -277,6 +272,24 @@ namespace swmi
             if (down_bits && act != 0u)
                 MergeEdge<FRESH, LOCAL>(d, bl, down_bits, va, vb, lb_b, BlockBase(d, bl.sx, sy_b), err, HS[1], SS[1], SK[1], SW[1]);
         }
+    }
+
+    template <bool FRESH, bool LOCAL>
+    __global__ __launch_bounds__(128) void k_merge(const LatDesc* __restrict__ descs, const uint32_t* __restrict__ block_lat,
+                                                   const uint32_t total_blocks)
+    {
+        const uint32_t b = RemapBlock(total_blocks);
+        if (b < total_blocks)
+            MergeEdges<FRESH, LOCAL>(descs[LatticeOf(block_lat, b)], b);
+    }
+
+    // of one lattice whose descriptor comes with the launch
+    template <bool FRESH>
+    __global__ __launch_bounds__(128) void k_merge_one(const LatDesc d, const uint32_t total_blocks)
+    {
+        const uint32_t b = RemapBlock(total_blocks);
+        if (b < total_blocks)
+            MergeEdges<FRESH, false>(d, b);
     }
 
     // k_merge for 64-wide tiles and blocks of at most 64 rows (at most 252 boundary sites, so 252 slots): one wave per
@@ -903,16 +916,11 @@ namespace swmi
 
     // Inspection kernel: the canonical label (minimum site index) of every site, written to parent[]: the
     // canonical root of every slot of the block (kept in LDS, one word per slot), then every site's label.
-    __global__ __launch_bounds__(256) void k_write_labels(const LatDesc* __restrict__ descs, const uint32_t* __restrict__ block_lat,
-                                                          const uint32_t total_blocks)
+    __device__ __forceinline__ void WriteLabels(const LatDesc& d, const uint32_t b)
     {
         constexpr uint32_t kPass = 16;   // wave rows per pass of the workgroup (16 lanes per wave row)
         constexpr uint32_t kCh = 4;      // passes loaded together
         extern __shared__ uint32_t R[];  // kWavesPerBlock * edge_cap entries (at most the block's sites)
-        const uint32_t b = RemapBlock(total_blocks);
-        if (b >= total_blocks)
-            return;
-        const LatDesc& d = descs[LatticeOf(block_lat, b)];
         const Block bl = DecodeBlock(d, b);
         const gptr<uint32_t> L = Glob(d.parent);
         const gptr<uint16_t> local = Glob(d.local);
@@ -975,6 +983,21 @@ namespace swmi
         }
         if (!ok)
             (void)__hip_atomic_fetch_or(Glob(d.state) + kStErr, kErrLabelRange, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+
+    __global__ __launch_bounds__(256) void k_write_labels(const LatDesc* __restrict__ descs, const uint32_t* __restrict__ block_lat,
+                                                          const uint32_t total_blocks)
+    {
+        const uint32_t b = RemapBlock(total_blocks);
+        if (b < total_blocks)
+            WriteLabels(descs[LatticeOf(block_lat, b)], b);
+    }
+
+    __global__ __launch_bounds__(256) void k_write_labels_one(const LatDesc d, const uint32_t total_blocks)
+    {
+        const uint32_t b = RemapBlock(total_blocks);
+        if (b < total_blocks)
+            WriteLabels(d, b);
     }
 
     // =============================================================================================
@@ -1266,17 +1289,6 @@ namespace swmi
         state[kStLastSample] = it;
     }
 
-    // Set-up of the allocation-free labelling (swmi_label_bonds_noalloc): the descriptor and fresh counters,
-    // written by this kernel into the scratch memory.
-    __global__ __launch_bounds__(64) void k_noalloc_setup(const LatDesc d, LatDesc* __restrict__ desc_out)
-    {
-        const uint32_t i = threadIdx.x;
-        if (i == 0)
-            *desc_out = d;
-        if (i < kLatStateWords)
-            d.state[i] = i == kStItEnd ? 0xFFFFFFFFu : (i == kStActive ? 1u : 0u);
-    }
-
     // =============================================================================================
     // Initialisation
     // =============================================================================================
@@ -1449,9 +1461,12 @@ namespace swmi
     // launch wrappers
     // =============================================================================================
     // defined in swmi_bond.hip, one part per combination
-    template <bool TW64, bool DBG>
+    template <bool TW64, BondMode MODE>
     void LaunchBondLabelT(const LatDesc* d_desc, const uint32_t* d_block_lat, uint32_t total_blocks, uint32_t max_twr, BondForm form, bool pad,
                           hipStream_t stream);
+
+    template <bool TW64>
+    void LaunchLabelBlocksT(const LatDesc& d, uint32_t total_blocks, BondForm form, bool pad, hipStream_t stream);
 
     void LaunchBondLabel(const LatDesc* d_desc, const uint32_t* d_block_lat, const uint32_t total_blocks, const uint32_t max_twr,
                          const BondForm form, const bool all_tw64, const bool pad, const bool debug, hipStream_t stream)
@@ -1459,14 +1474,14 @@ namespace swmi
         if (debug)
         {
             if (all_tw64)
-                LaunchBondLabelT<true, true>(d_desc, d_block_lat, total_blocks, max_twr, form, pad, stream);
+                LaunchBondLabelT<true, BondMode::kInspect>(d_desc, d_block_lat, total_blocks, max_twr, form, pad, stream);
             else
-                LaunchBondLabelT<false, true>(d_desc, d_block_lat, total_blocks, max_twr, form, pad, stream);
+                LaunchBondLabelT<false, BondMode::kInspect>(d_desc, d_block_lat, total_blocks, max_twr, form, pad, stream);
         }
         else if (all_tw64)
-            LaunchBondLabelT<true, false>(d_desc, d_block_lat, total_blocks, max_twr, form, pad, stream);
+            LaunchBondLabelT<true, BondMode::kSweep>(d_desc, d_block_lat, total_blocks, max_twr, form, pad, stream);
         else
-            LaunchBondLabelT<false, false>(d_desc, d_block_lat, total_blocks, max_twr, form, pad, stream);
+            LaunchBondLabelT<false, BondMode::kSweep>(d_desc, d_block_lat, total_blocks, max_twr, form, pad, stream);
     }
 
     // Two-wave merge workgroups resident at once on MI355X: 256 CUs x 16 (8 waves per SIMD).
@@ -1547,10 +1562,18 @@ namespace swmi
         LaunchSetRngCurrent(state, aux, stream);
     }
 
-    void LaunchNoAllocSetup(const LatDesc& d, LatDesc* d_desc, hipStream_t stream)
+    void LaunchLabelBlocks(const LatDesc& d, const BondForm form, const bool pad, hipStream_t stream)
     {
-        static_assert(kLatStateWords <= 64, "one wave writes the counters");
-        k_noalloc_setup<<<1, 64, 0, stream>>>(d, d_desc);
+        const uint32_t g = XcdGrid(d.n_blocks);
+        if (d.tw == 64u)
+            LaunchLabelBlocksT<true>(d, d.n_blocks, form, pad, stream);
+        else
+            LaunchLabelBlocksT<false>(d, d.n_blocks, form, pad, stream);
+        if (d.n_blocks <= kOneRoundMergeBlocks)
+            k_merge_one<true><<<g, 128, 0, stream>>>(d, d.n_blocks);
+        else
+            k_merge_one<false><<<g, 128, 0, stream>>>(d, d.n_blocks);
+        k_write_labels_one<<<g, 256, d.qcap * sizeof(uint32_t), stream>>>(d, d.n_blocks);
     }
 
     void LaunchObservables(const LatDesc* d_desc, const uint32_t* d_block_lat, const uint32_t total_blocks, const uint32_t sample_mode,

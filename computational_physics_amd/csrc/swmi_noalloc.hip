@@ -4,7 +4,7 @@
 //
 // The caller passes the bond field and the label array in device memory. Every other buffer the kernels
 // need (block-local labels, the union-find over edge-root slots, block-edge bond bits, slot counts, edge
-// columns and rows, per-lattice counters and the lattice descriptor) is carved out of one file-scope device array, `scratch`,
+// columns and rows and per-lattice counters) is carved out of one file-scope device array, `scratch`,
 // which every GPU holds for the life of the process. For a lattice that needs no row padding the last kernel
 // writes the canonical labels straight into the caller's label array; a padded lattice gets its bond field
 // padded into scratch and its labels written into scratch, and a last kernel writes the unpadded labels. The call enqueues kernels on the caller's stream and returns: no
@@ -77,12 +77,12 @@ namespace swmi
         // The label-only descriptor over a carve (spins alias the bond field: the injected pass reads spin
         // bytes but uses none of them; it reads no lcg32 state and writes no spin, halo or flip bit).
         LatDesc NoAllocDesc(const Geometry& g, const uint32_t n0, const uint32_t n1, const uint8_t* bonds, uint32_t* labels,
-                            Carve& c, LatDesc** d_desc)
+                            Carve& c)
         {
             LatDesc d = GeometryDesc(g, n0, n1);
             const uint64_t n = static_cast<uint64_t>(g.pitch) * n1;   // padded sites
             const bool pad = g.pitch != n0;
-            *d_desc = c.Take<LatDesc>(1);
+            (void)c.Take<LatDesc>(1);   // kept free: the largest lattice the array takes is part of the interface
             d.state = c.Take<uint32_t>(kLatStateWords + kAuxWords);
             d.aux = d.state + kLatStateWords;
             d.local = c.Take<uint16_t>(n);
@@ -116,8 +116,7 @@ extern "C" int swmi_label_bonds_noalloc(const uint8_t* bonds, uint32_t n0, uint3
                                                   " sites (got " + std::to_string(n0) + " x " + std::to_string(n1) + ")");
         const Geometry g = GeometryOf(n0, n1, kNoAllocTileRows);
         Carve size;
-        LatDesc* d_desc = nullptr;
-        (void)NoAllocDesc(g, n0, n1, bonds, labels, size, &d_desc);
+        (void)NoAllocDesc(g, n0, n1, bonds, labels, size);
         if (size.used > kScratchBytes)
             throw SwmiError(SWMI_ERR_INVALID, "lattice needs " + std::to_string(size.used) + " bytes of scratch, more than the " +
                                                   std::to_string(kScratchBytes) + " the static array holds");
@@ -127,7 +126,7 @@ extern "C" int swmi_label_bonds_noalloc(const uint8_t* bonds, uint32_t n0, uint3
             throw SwmiError(SWMI_ERR_NO_DEVICE, "device index " + std::to_string(device) + " out of range");
         Carve carve;
         carve.base = ScratchOf(device);
-        const LatDesc d = NoAllocDesc(g, n0, n1, bonds, labels, carve, &d_desc);
+        const LatDesc d = NoAllocDesc(g, n0, n1, bonds, labels, carve);
         hipStream_t s = static_cast<hipStream_t>(stream);
         if (ResidentRows(g, n1) != 0u)
         {
@@ -138,14 +137,10 @@ extern "C" int swmi_label_bonds_noalloc(const uint8_t* bonds, uint32_t n0, uint3
         }
         const bool pad = g.pitch != n0;
         const uint64_t np = static_cast<uint64_t>(g.pitch) * n1, n = static_cast<uint64_t>(n0) * n1;
-        // descriptor and fresh counters are written by a kernel (no memset, no host copy); the kernels run with
-        // a null work list (every block belongs to the one lattice)
-        LaunchNoAllocSetup(d, d_desc, s);
         if (pad)
             LaunchPadBytes(const_cast<uint8_t*>(d.bond_in), bonds, np, n0, g.pitch, s);
-        LaunchBondLabel(d_desc, nullptr, g.n_blocks, g.twr, FormOf(g), g.tw == 64, pad, true, s);
-        LaunchMerge(d_desc, nullptr, g.n_blocks, g.tw == 64, g.ecol_stride, s);
-        LaunchWriteLabels(d_desc, nullptr, g.n_blocks, g.twr, s);
+        // (the descriptor goes with every launch; the counters a labelling uses are written by its first kernel)
+        LaunchLabelBlocks(d, FormOf(g), pad, s);
         if (pad)
             LaunchUnpadLabels(labels, d.parent, n, n0, g.pitch, s);
         Check(hipGetLastError(), "label launch");

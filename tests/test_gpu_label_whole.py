@@ -12,7 +12,9 @@ from test_zz_no_alloc import _bonds, _Hip
 pytestmark = pytest.mark.gpu
 
 EXTENTS = [(2, 2), (16, 6), (6, 8), (32, 32), (30, 200), (32, 512), (48, 34), (62, 2), (64, 2), (64, 64), (64, 256), (64, 258), (66, 50),
-           (126, 100), (128, 128), (130, 18), (192, 64), (1000, 6), (1024, 16), (1026, 14)]
+           (126, 100), (128, 128), (130, 18), (192, 64), (1000, 6), (1024, 16), (1026, 14),
+           # tiled: partial and padded blocks, 16, 8 and 4 waves per block, narrow rows
+           (300, 300), (64, 1000), (512, 320), (1000, 1350), (1536, 1024), (2048, 1024), (1100, 3000), (32, 2048), (30, 1000), (16, 4096)]
 
 
 def test_small_bond_fields_match_the_oracle(swmi, oracle):
