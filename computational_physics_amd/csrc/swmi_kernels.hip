@@ -1070,7 +1070,9 @@ namespace swmi
 
         // the row below the tile: the next tile's first row, or across the block edge the halo (the flipped spins of a
         // pending flip); loaded without conditions, like the rows of a chunk, so that the loads overlap
-        const uint32_t r_below = r_begin + (last_wave ? 0u : nrow);   // in range either way
+        // (in range for every wave: the last tile and the waves past it, which own no rows in a partial block, read the
+        // block's last row and do not use it)
+        const uint32_t r_below = min(r_begin + nrow, bl.nwr - 1u);
         const uint32_t site_below = last_wave && !pending ? BlockBase(d, bl.sx, sy_b) + lane : bl.base + r_below * bl.stride + lane;
         const uint32_t below_sp = spins[site_below], below_lab = local[site_below];
         const uint32_t below_halo = halo[(sy_b * d.tiles_x + bl.sx) * d.halo_stride + d.ecol_stride + lane];

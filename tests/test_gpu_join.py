@@ -69,3 +69,23 @@ def test_many_small_tiled_lattices_equal_their_lone_runs(swmi):
         with swmi.Engine(cfgs[i]) as alone:
             alone.sweep(12)
             np.testing.assert_array_equal(alone.spins(), spins, err_msg=f"lattice {i}")
+
+
+@pytest.mark.parametrize("n0,n1,T,rule", [(1006, 270, 2.392, 1), (130, 300, 2.0, 0), (256, 258, 2.2691853, 1)])
+def test_samples_of_a_partial_last_block_match_the_oracle(swmi, oracle, n0, n1, T, rule):
+    """A last block row of few rows leaves tiles without rows; the sample reads nothing past the lattice for them (their
+    unused row below the tile used to be read beyond the end of the spin array)."""
+    print(f"partial block samples {n0}x{n1} T {T} rule {rule}", flush=True)
+    ref = oracle.PerSite(n0, n1, T, seed=6, flip_rule=rule)
+    with swmi.Engine(swmi.LatticeConfig(n0, n1, T, seed=6, flip_rule=rule, max_samples=8)) as e:
+        e.run(12, 3)
+        want = []
+        for k in range(12):
+            ref.sweep()
+            if k % 3 == 2:
+                want.append(oracle.observables(n0, n1, ref.spins))
+        E, M = e.series()
+        assert list(zip(E.tolist(), M.tolist())) == want
+        e.spins()   # no flip pending any more
+        e.sample()
+        assert e.energy_magnetization() == want[-1] and e.moments()[0] == 5 and e.error_flags() == 0
