@@ -41,7 +41,7 @@ namespace swmi
         // 64-wide tiles of at most kRows rows keep their rows' roots in registers from the row loop to the labels
         constexpr bool kKeep = TW64 && TWR_MAX <= kRows;
         // and collect what the edges of the tile need as bits of scalar words
-        constexpr bool kBits = kKeep && !PAD && !DBG;
+        constexpr bool kBits = kKeep && !DBG;
         constexpr uint32_t kSites = NW * TWR_MAX * 64;
         constexpr uint32_t kThreads = NW * 64u;
         constexpr uint32_t kQw = 128u;                             // per-wave LDS words of Q
@@ -285,6 +285,7 @@ namespace swmi
         // kBits: the rows' first-column spin, last-column spin and last-column draw, the latest row in bit 0, and the
         // spins right of the tile (lane r: row r)
         uint32_t col_b = 0, s63_b = 0, u63_b = 0, hright = 0;
+        const auto last_bit = [&](const uint64_t m) { return static_cast<uint32_t>(PAD ? (m >> elane) & 1ull : m >> 63); };
         {
             // the chunk loop exists twice: sweeps without a group rotation (13 in 15) carry no rotation code
             // (and twice more for the sweeps that apply a pending flip on load, the rule after any sweep)
@@ -348,7 +349,7 @@ namespace swmi
                         if (kBits)
                         {
                             col_b = (col_b << 1) + (static_cast<uint32_t>(S) & 1u);
-                            s63_b = (s63_b << 1) + static_cast<uint32_t>(S >> 63);
+                            s63_b = (s63_b << 1) + last_bit(S);
                         }
                         else if (TW64)
                             colv = LaneBit(1ull << r) ? static_cast<uint32_t>(S) : colv;   // bit 0 of S: lane 0's spin
@@ -394,7 +395,7 @@ namespace swmi
                             if (kBits)
                             {
                                 RS = S >> 1;   // the last column's bond follows after the rows
-                                u63_b = (u63_b << 1) + static_cast<uint32_t>(U1 >> 63);
+                                u63_b = (u63_b << 1) + last_bit(U1);
                             }
                             else if (!PAD)
                                 RS = TW64 ? ((S >> 1) | (((HR >> i) & 1ull) << 63))
@@ -409,7 +410,7 @@ namespace swmi
                             Ball = __ballot((aux[i] & 1u) != 0u);
                             U2 = __ballot((aux[i] & 2u) != 0u);
                             if (kBits)
-                                u63_b = (u63_b << 1) + static_cast<uint32_t>(Ball >> 63);
+                                u63_b = (u63_b << 1) + last_bit(Ball);
                         }
                         if (PAD)
                         {
@@ -915,7 +916,6 @@ namespace swmi
     // 29.2 / 28.8 / -, 1024 (2048^2) 32.6 / 33.3 / 46.
     constexpr uint32_t kWideBlocks = 256;
     constexpr uint32_t kHalfBlocks = 768;
-
     // f(NW) with the waves per block for a launch of 64-wide tiles of at most 16 rows
     template <typename F>
     static void WithWaves(const uint32_t total_blocks, const BondForm form, F&& f)
@@ -952,6 +952,11 @@ namespace swmi
 
     template void LaunchLabelBlocksT<SWMI_BOND_TW64>(const LatDesc&, uint32_t, BondForm, bool, hipStream_t);
 #else
+    // Padded lattices of more blocks run with the default register budget (seven blocks per CU) up to two rounds of
+    // blocks, with eight blocks per CU above: 2209 blocks (3000^2) 51.2 against 51.7 us per sweep, 3969 (4000^2) 73.3
+    // against 70.5, 15625 (8000^2) 205.1 against 205.0.
+    constexpr uint32_t kPadRounds = 2u * 7u * 256u;
+
     template <bool TW64, BondMode MODE>
     void LaunchBondLabelT(const LatDesc* d_desc, const uint32_t* d_block_lat, const uint32_t total_blocks, const uint32_t max_twr,
                           const BondForm form, const bool pad, hipStream_t stream)
@@ -964,8 +969,7 @@ namespace swmi
         {
             if (!pad && max_twr <= 8 && (form == BondForm::kAny || total_blocks > kHalfBlocks))
                 return launch(k_bond_label<kWavesPerBlock, 8, MODE, false, false>);
-            // (padded lattices of many blocks keep the registers of k_bond_label_any)
-            if (max_twr <= 16 && (!pad || (form != BondForm::kAny && total_blocks <= kHalfBlocks)))
+            if (max_twr <= 16 && (!pad || (form != BondForm::kAny && total_blocks <= kHalfBlocks) || total_blocks > kPadRounds))
                 return WithWaves(total_blocks, form, [&](auto nw) {
                     constexpr uint32_t NW = decltype(nw)::value;
                     constexpr bool kSweep = MODE == BondMode::kSweep;
