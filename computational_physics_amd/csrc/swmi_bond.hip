@@ -11,15 +11,16 @@ namespace swmi
     // Per wavefront (tile) the rows are processed top to bottom with the loads of the next kCh rows in
     // flight together. Bonds are computed on wave-uniform 64-bit masks: S (spin up), U1/U2 (draw below
     // threshold), B (bond to the right neighbour inside the tile), D (bond to the site below).
-    // 64-wide tiles keep the previous row's roots resolved in registers (Rp). A row run's label is the
-    // minimum of its first site and the roots its down bonds reach (one LDS atomicMin per bonded lane into
-    // the run's slot); a bond to any other root links that root under the minimum with one atomicMin, and
-    // only a link that loses a race goes through the lockstep union.
+    // 64-wide tiles keep the previous row's roots resolved in registers (Rp) and label a row with LabelRow64.
     // Narrow tiles record one union per overlap interval of consecutive rows in a per-wave LDS queue,
     // worked off 64 at a time whenever it fills.
     // Nodes of the LDS union-find are byte offsets into P. After the final find, the root of every
     // cluster that reaches the block edge carries kPFlag in its own entry, so a site's label (root index,
     // plus kEdgeFlag) is P[root] >> 2.
+    // What bounds it: at 4096^2 (45.5 us, 10.5 B a site moved, 3.9 TB/s from the memory-side cache) instruction issue
+    // and the LDS pipe, about 60 instructions and 11 LDS operations per 64-site row where 90 and 18 took 55.9 us; at 8192^2
+    // (171 us, 4.1 TB/s) HBM, where a large copy reaches 5.0, and 14.6 B a site took 227; below 1024^2 the chain of LDS
+    // round trips down a strip (256^2 9.6 us with 4-row strips, 14.7 with 16).
     // MODE: the sweep proper; the inspection build, in which bonds may be injected instead of generated and may be
     // recorded; or the labelling of an injected bond field alone.
     // PAD: the lattice is stored with a row pitch d.n0 above its width d.n0v; in the last tile column only

@@ -181,9 +181,9 @@ namespace swmi
 
     // One workgroup of kResidentWaves waves takes a lattice whose sites fit its LDS union-find and whose rows, split
     // into strips over the waves left per tile column, leave at most kResidentRows per strip. Every lattice it takes
-    // is faster there than tiled: 64^2 3 against 24 us per sweep, 128^2 9 against 24 (a 16-row strip is as long a
-    // chain as a 16-row tile, and the sweep has no launches, merge or resolve); a larger one would leave the other
-    // 255 CUs idle for longer.
+    // is faster there than tiled: 64^2 4.3 against 24 us per sweep, 128^2 11.5 against 24 (a 16-row strip is as long a
+    // chain as a 16-row tile, and the sweep has no launches, merge or resolve). Four times the sites would take four
+    // times as long on the one CU, 46 us, where the tiled kernels take 16 (256^2).
     uint32_t ResidentRows(const Geometry& g, const uint32_t n1)
     {
         if (static_cast<uint64_t>(g.pitch) * n1 > kResidentSites || g.tiles_x > kResidentWaves)

@@ -1,23 +1,24 @@
 // swmi_kernels.hip -- gfx950 kernels of the Swendsen-Wang engine.
 //
-// One sweep = three launches over the engine's block work list (all lattices of the engine at once):
-//   k_bond_label  per block (one workgroup, 4 wavefronts, one tile each): applies the previous sweep's
+// One sweep of tiled lattices = three launches over the engine's block work list (all lattices of the engine at once):
+//   k_bond_label  (swmi_bond.hip) per block (one workgroup of 4, 8 or 16 wavefronts): applies the previous sweep's
 //                 cluster flip to each site as it loads it (label -> bit of the block's flip bitmap) and
-//                 stores the flipped spin; two lcg32 updates per site; bond activation against the integer
+//                 stores the flipped spin; two lcg32 draws per site; bond activation against the integer
 //                 threshold on 64-bit ballot masks (scalar unit); row runs from the masks, unions in an LDS
 //                 union-find (atomicMin keeps parent <= child, so roots are cluster minima); block-local
 //                 uint16 labels with an edge flag; the block-edge bond bits and the block's halo spins.
-//   k_merge       per block (two waves): unions across block edges by atomicMin on the uint32 parent
-//                 array in HBM, over the roots of edge-reaching clusters only.
-//   k_resolve     per block (two waves): the listed edge-cluster roots are chased in the global parent
-//                 array (one chase per root); the block's flip bitmap (the flip rule applied to every
-//                 cluster's canonical root) is written out and the block's halo spins are flipped in place.
-//                 Advances the lcg32 iteration count; the spin array waits for the next k_bond_label.
-// k_flip applies a pending flip to the spin array; it runs only before something reads the spins.
+//   k_merge       per block: unions across block edges by 64-bit atomicMin in a union-find in HBM over the slots
+//                 of the edge-reaching clusters (two waves per block; k_merge_block with one for large launches).
+//   k_resolve     per block (two waves): the block's slots are chased in that union-find, their flip bits written
+//                 out and the block's halo spins flipped in place. Advances the lcg32 iteration count; the spin
+//                 array waits for the next k_bond_label.
+// k_join does the work of k_merge and k_resolve for lattices of few blocks, and k_resident (swmi_resident.hip) sweeps
+// small lattices whole, without any of these launches. k_flip applies a pending flip to the spin array; it runs only
+// before something reads the spins. k_observables takes a sample without storing the flip.
 // Spin bytes: bit 0 is the spin, bits 3-5 hold the site's current lcg32 parameter selector, i.e. the
 // index k of the Numerical Recipes pair (a_k, c_k) that lane i of its group uses after the group's
 // rotations (sel0[(i + rot) & 63]). The byte is read every sweep anyway, so the generator needs no other
-// per-group data except on the sweeps that rotate (one in 7.5).
+// per-group data except on the sweeps that rotate (one in 7.5); only those store lcg32 states.
 // Reference behaviour: ising/src/swendsen_wang_amd_gpu.cpp:78-467 (four kernels per sweep) and the CPU
 // labeller ising/src/swendsen_wang_cpu.cpp:13-205; the kernels here are written for wave64 CDNA4.
 #include "swmi_device.h"
@@ -1013,7 +1014,8 @@ namespace swmi
 
     // A flip that is still pending is applied on the way (from the labels and the flip bits, as k_bond_label does) and
     // not stored: the spin array is read once (1 byte a site, 3 with the labels of a pending flip) and left for the
-    // next sweep. Per wave one tile: spin masks of its rows by ballot, one per lane, the neighbours by shifts and from
+    // next sweep (8192^2: 206 us per sample with k_flip, k_set_applied and three reads per spin, now 75 with the final
+    // sum, 68 of them here for 3 bytes a site, 2.9 TB/s). Per wave one tile: spin masks of its rows by ballot, one per lane, the neighbours by shifts and from
     // the next lane; the row below the tile is read again by the tile above it (or comes from the halo across the block
     // edge). Summing row by row with scalar operations was bound by the scalar unit (104 us at 8192^2).
     __global__ __launch_bounds__(256) void k_observables(const LatDesc* __restrict__ descs, const uint32_t* __restrict__ block_lat,

@@ -2,6 +2,8 @@
 // allocate device memory (code under HIP graph capture, tight serving loops, harnesses that forbid
 // hipMalloc).
 //
+// A lattice that one workgroup holds is labelled by k_label_whole (swmi_resident.hip) in one launch. For larger ones:
+//
 // The caller passes the bond field and the label array in device memory. Every other buffer the kernels
 // need (block-local labels, the union-find over edge-root slots, block-edge bond bits, slot counts, edge
 // columns and rows and per-lattice counters) is carved out of one file-scope device array, `scratch`,

@@ -59,7 +59,8 @@ typedef struct
     float temperature;    /* T > 0 */
     uint32_t seed;        /* lcg32 group seeds: seed*0x9E3779B1 + g + 1 (seed 0: g + 1) */
     uint32_t spin_seed;   /* hot start: srand48(spin_seed); spin = drand48() < 0.5 ? 0 : 1 (1: reference) */
-    uint32_t tile_rows;   /* tile height in 64-site wave rows (0: default); results do not depend on it */
+    uint32_t tile_rows;   /* tile height in 64-site wave rows (0: default, and lattices of up to 16384 sites may be swept
+                           * untiled, one workgroup each); results do not depend on it */
     uint32_t flip_rule;   /* SWMI_FLIP_PARITY or SWMI_FLIP_RANDOM */
     uint32_t max_samples; /* capacity of the on-device (E, M) time series (0: no series, moments only) */
 } swmi_lattice_config;
@@ -106,7 +107,8 @@ int swmi_get_threshold(const swmi_engine* engine, uint32_t lattice, float* p_add
  * SwendsenWang_2D::Update (ising/src/swendsen_wang.cpp:94-112). Asynchronous on the engine stream. ---- */
 int swmi_sweep(swmi_engine* engine, uint32_t n_sweeps);
 /* Launch mode: captured hipGraphs of 16 sweeps (or of sample groups) replayed for long sweep loops
- * (enable = 1, the default) or every kernel launched one by one (0). Results are identical. The
+ * (enable = 1, the default) or every kernel launched one by one (0). Results are identical. Lattices that one
+ * workgroup sweeps take one launch per 500 sweeps either way. The
  * reference launches every kernel and synchronises after each (swendsen_wang_amd_gpu.cpp:253-492).
  * New engines start with graphs unless the environment variable SWMI_GRAPHS is "0". */
 int swmi_set_graphs(swmi_engine* engine, int enable);
@@ -169,8 +171,9 @@ int swmi_download_labels(swmi_engine* engine, uint32_t lattice, uint32_t* labels
  * n0 x n1 lattice (the extents swmi_lattice_config allows, at most 2^22 sites) and writes the canonical
  * labels into `labels` (device memory, n0*n1 uint32), exactly as swmi_label_bonds + swmi_download_labels.
  * The kernels are enqueued on `stream` (a hipStream_t; NULL is the default stream) and the call returns
- * without waiting; it allocates nothing, issues no memset and copies nothing to or from the host. Every
- * buffer beyond the two arrays comes from a 48 MiB static device array that each GPU holds until the
+ * without waiting; it allocates nothing, issues no memset and copies nothing to or from the host. A lattice of
+ * up to 16384 sites that one workgroup labels needs no memory beyond the two arrays. For a larger one every
+ * buffer beyond them comes from a 48 MiB static device array that each GPU holds until the
  * process ends, shared by all calls on that GPU: calls that overlap on one GPU (other streams, other
  * threads) race, calls on one stream are ordered. An unpadded lattice needs about 2.5 bytes of it per
  * site; one whose rows are padded (swmi_get_layout) about 7 per padded site, and one that needs more than
