@@ -184,12 +184,14 @@ namespace swmi
     // is faster there than tiled: 64^2 4.3 against 24 us per sweep, 128^2 11.5 against 24 (a 16-row strip is as long a
     // chain as a 16-row tile, and the sweep has no launches, merge or resolve). Four times the sites would take four
     // times as long on the one CU, 46 us, where the tiled kernels take 16 (256^2).
+    // Wave rows of very narrow lattices join through many more unions: 16 x 1024 (16 wave rows per strip) takes 27.4
+    // against 36.9 us tiled, but 4 x 4096 28.2 against 23.3, so below 16 columns only strips of up to 8 go here.
     uint32_t ResidentRows(const Geometry& g, const uint32_t n1)
     {
         if (static_cast<uint64_t>(g.pitch) * n1 > kResidentSites || g.tiles_x > kResidentWaves)
             return 0;
         const uint32_t strips = kResidentWaves / g.tiles_x, rows = (g.nwr_y + strips - 1u) / strips;
-        return rows <= kResidentRows ? rows : 0;
+        return rows <= (g.tw < 16u ? kResidentRows / 2u : kResidentRows) ? rows : 0;
     }
 
     BondForm FormOf(const Geometry& g)

@@ -10,7 +10,8 @@ pytestmark = pytest.mark.gpu
 TC = 2.2691853
 
 EXTENTS = [(64, 2), (64, 64), (64, 256), (192, 64), (1024, 16), (128, 128), (126, 100), (130, 18), (100, 162), (32, 32), (32, 512),
-           (16, 6), (48, 34), (2, 2), (30, 200), (64, 258)]
+           (16, 6), (48, 34), (2, 2), (30, 200), (64, 258),
+           (4, 2048), (4, 2064)]   # below 16 columns: the last lattice of eight rows per strip and the first past it
 
 
 @pytest.mark.parametrize("n0,n1", EXTENTS)
