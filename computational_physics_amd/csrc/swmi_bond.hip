@@ -176,7 +176,8 @@ namespace swmi
         // The stored states are those of iteration rng_it: a lane's (a, c) stays the same until the next rotation,
         // so the state after the sweep's first update is one affine step away, u1 = A st + C with (A, C) the pair
         // applied it1 - rng_it times, and the sweep needs to store no state. A rotating sweep stores the state at
-        // which the pairs change (it0, or it1 when the second update rotates): at most 15 updates are jumped.
+        // which the pairs change (it0, or it1 when the second update rotates): at most 15 updates are jumped. Both
+        // updates rotate only in the sweep in which the 32-bit update count wraps (2^32 - 1 is a multiple of 15).
         const uint32_t n_jump = min((rot1 ? it0 : it1) - rng_it, 15u);
 
         // halos: this sweep writes the block's first column and first wave row into its side of the halo
@@ -377,6 +378,14 @@ namespace swmi
                                 ac = pair_of(ks, 0u);
                                 if (rot1)
                                     u1 = static_cast<uint32_t>(ac >> 32) * u1 + static_cast<uint32_t>(ac);
+                                if (rot1 && rot2)   // the sweep in which the update count wraps to 0
+                                {
+                                    __builtin_amdgcn_raw_buffer_store_b32(u1, rs_rng, lane4, Uniform(wr * bl.stride) * 4u, 0);
+                                    const uint32_t second = ShuffleShift(u1, it2) & 63u;
+                                    ks = static_cast<uint32_t>(__shfl(static_cast<int>(ks), static_cast<int>((lane + second) & 63u)));
+                                    ac = pair_of(ks, 0u);
+                                    shift += second;
+                                }
                             }
                             const uint32_t st = static_cast<uint32_t>(ac >> 32) * u1 + static_cast<uint32_t>(ac);
                             if (kRot)

@@ -504,11 +504,11 @@ namespace swmi
         const gptr<uint32_t> stp = Glob(d.state);
         stp[kStApplied] = it;
         stp[kStIteration] = it + 2u;
-        // a rotating sweep stored the states at which its lanes' pairs changed
-        if ((it + 1u) % 15u == 0u)
-            Glob(d.aux)[kAuxRngIt] = it;
-        else if ((it + 2u) % 15u == 0u)
+        // a rotating sweep stored the states at which its lanes' pairs changed (last)
+        if ((it + 2u) % 15u == 0u)
             Glob(d.aux)[kAuxRngIt] = it + 1u;
+        else if ((it + 1u) % 15u == 0u)
+            Glob(d.aux)[kAuxRngIt] = it;
     }
 
     // End of a sweep, per block (two waves): the slots of the block's edge-reaching clusters are chased in the

@@ -254,7 +254,8 @@ namespace swmi
         const uint32_t rowb = n0 * 4u * rpw;                // P bytes between consecutive rows of a strip
         const uint32_t node0 = g0 * 256u + lane4;           // this lane's node of the strip's first row
         const uint32_t node_below = gbelow * 256u + lane4;
-        const uint32_t last_active = it_end > it ? (it_end - it - 1u) / 2u + 1u : 0u;   // sweeps until the schedule ends
+        // sweeps until the schedule ends (without one the update count may wrap)
+        const uint32_t last_active = it_end == 0xFFFFFFFFu ? 0xFFFFFFFFu : (it_end > it ? (it_end - it - 1u) / 2u + 1u : 0u);
         const uint32_t total = min(groups * sweeps, last_active);
         uint32_t done = 0;
         Qw[lane] = 0u;   // run words of LabelRow64
@@ -304,11 +305,12 @@ namespace swmi
                     uint64_t ac = pair_of(ks);
                     st = static_cast<uint32_t>(ac >> 32) * st + static_cast<uint32_t>(ac);
                     const uint64_t U1 = __ballot(st < thr);
-                    if (rot2)
+                    if (rot2)   // (both rotate in the sweep in which the update count wraps to 0)
                     {
-                        shift = ShuffleShift(st, it2) & 63u;
-                        ks = static_cast<uint32_t>(__shfl(static_cast<int>(ks), static_cast<int>((lane + shift) & 63u)));
+                        const uint32_t second = ShuffleShift(st, it2) & 63u;
+                        ks = static_cast<uint32_t>(__shfl(static_cast<int>(ks), static_cast<int>((lane + second) & 63u)));
                         ac = pair_of(ks);
+                        shift += second;
                     }
                     st = static_cast<uint32_t>(ac >> 32) * st + static_cast<uint32_t>(ac);
                     const uint64_t U2 = __ballot(st < thr) & vmask;
