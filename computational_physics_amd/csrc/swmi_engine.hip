@@ -584,13 +584,13 @@ void swmi_engine::Run(uint32_t n, uint32_t sep, int32_t sample_mode)
 {
     if (classes.empty() || n == 0)
         return;
-    // the resident classes beside the tiled ones
-    if (sample_mode >= 0)
-        EnqueueResident(sep, (n + sep - 1) / sep, sample_mode);   // ising_2d.cpp:132: i += N_Sep while i < n
-    else
-        EnqueueResident(n, 1, -1);
-    RunTiled(n, sep, sample_mode);
-    JoinResident();
+    BesideResident([&] {
+        if (sample_mode >= 0)
+            EnqueueResident(sep, (n + sep - 1) / sep, sample_mode);   // ising_2d.cpp:132: i += N_Sep while i < n
+        else
+            EnqueueResident(n, 1, -1);
+        RunTiled(n, sep, sample_mode);
+    });
 }
 
 void swmi_engine::RunTiled(uint32_t n, uint32_t sep, int32_t sample_mode)
@@ -914,9 +914,10 @@ int swmi_sweep(swmi_engine* engine, uint32_t n_sweeps)
 int swmi_sample(swmi_engine* engine)
 {
     return Guard([&] {
-        Eng(engine)->EnqueueResident(0, 1, kSampleAlways);
-        engine->EnqueueSample(kSampleAlways);
-        engine->JoinResident();
+        Eng(engine)->BesideResident([&] {
+            engine->EnqueueResident(0, 1, kSampleAlways);
+            engine->EnqueueSample(kSampleAlways);
+        });
     });
 }
 

@@ -253,6 +253,28 @@ struct swmi_engine
     // from the engine stream; JoinResident joins them back
     void EnqueueResident(uint32_t sweeps, uint32_t groups, int32_t sample_mode);
     void JoinResident();
+    // f launches on the resident classes (EnqueueResident) and the tiled ones; whatever f throws, the engine stream goes on
+    // after the resident classes' launches
+    template <typename F>
+    void BesideResident(F&& f)
+    {
+        try
+        {
+            f();
+        }
+        catch (...)
+        {
+            try
+            {
+                JoinResident();
+            }
+            catch (...)
+            {
+            }
+            throw;
+        }
+        JoinResident();
+    }
     // Run for the tiled classes
     void RunTiled(uint32_t n, uint32_t sep, int32_t sample_mode);
     // work on side streams [first, last) starts after what the engine stream holds now, and the engine stream goes on

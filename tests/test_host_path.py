@@ -1,0 +1,71 @@
+"""The engine's host side on a machine without a GPU: libswmi.so over a recorder that stands in for the HIP runtime
+(hip_recorder.cpp) and runs no kernel. Checks which kernels a call launches, in which order over the streams, and what it
+does when a runtime call fails."""
+import subprocess
+import sys
+import textwrap
+from pathlib import Path
+
+import pytest
+
+ROOT = Path(__file__).resolve().parent.parent
+PRELUDE = """
+import ctypes, re, sys
+sys.path.insert(0, {root!r})
+rec = ctypes.CDLL({recorder!r}, mode=ctypes.RTLD_GLOBAL)
+rec.rec_take.restype = ctypes.c_char_p
+rec.rec_fail.argtypes = [ctypes.c_char_p, ctypes.c_size_t]
+rec.rec_cost.argtypes = [ctypes.c_char_p, ctypes.c_double]
+import computational_physics_amd as cpa
+
+def take():
+    return rec.rec_take().decode().splitlines()
+
+def fail(name, least=0):
+    rec.rec_fail(name.encode(), least)
+
+def launched(lines):
+    return [m.group(1) for l in lines for m in [re.match(r"(?:captured )?launch \\\\S*?(k_[a-z_]+?)(?:I|E|P)", l)] if m]
+"""
+
+
+@pytest.fixture(scope="module")
+def recorded(tmp_path_factory):
+    lib = tmp_path_factory.mktemp("recorder") / "hip_recorder.so"
+    subprocess.run(["g++", "-std=c++17", "-O1", "-shared", "-fPIC", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include", "-Wno-deprecated-declarations",
+                    "-o", str(lib), str(ROOT / "tests" / "hip_recorder.cpp")], check=True, timeout=300)
+
+    def run(script):
+        code = PRELUDE.format(root=str(ROOT), recorder=str(lib)).replace("\\\\", "\\") + textwrap.dedent(script)
+        got = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=120)
+        assert got.returncode == 0, got.stdout[-3000:] + got.stderr[-3000:]
+
+    return run
+
+
+@pytest.mark.parametrize("call", ["e.sweep(64)", "e.run(640, 10)"])
+@pytest.mark.parametrize("failing", ["hipStreamBeginCapture", "hipGraphInstantiate"])
+def test_a_failed_call_still_joins_the_resident_stream(recorded, call, failing):
+    """A 64^2 lattice is swept on a side stream beside a 256^2 one; whatever fails after its launch, the engine stream
+    waits for it before the call returns, so that a later read on that stream sees the sweeps."""
+    recorded(f"""
+        e = cpa.Engine([cpa.LatticeConfig(64, 64), cpa.LatticeConfig(256, 256)])
+        take()
+        fail({failing!r})
+        try:
+            {call}
+            raise SystemExit("the call did not fail")
+        except cpa.SwmiError:
+            pass
+        lines = take()
+        last = max(i for i, l in enumerate(lines) if "k_resident" in l)
+        side = lines[last].rsplit(" ", 1)[1]
+        records = [(i, l.split()[2]) for i, l in enumerate(lines) if i > last and l.startswith("record") and l.endswith(" stream " + side)]
+        assert records, lines
+        at, event = records[-1]
+        waits = [l.split()[2] for l in lines[at:] if l.startswith("wait") and l.endswith(" event " + event)]
+        assert waits and waits[0] != side, lines
+        fail("")
+        e.sweep(64)
+        assert "k_resident" in launched(take())
+    """)
