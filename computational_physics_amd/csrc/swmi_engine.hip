@@ -500,7 +500,7 @@ void swmi_engine::EnqueueSweeps(uint32_t n)
             LaunchBondLabel(k.Descs(d_desc.ptr), k.WorkList(), k.total_blocks, k.max_twr, k.form, k.tw64, k.pad, recording, s);
             if (k.Joined())
             {
-                LaunchJoin(d_desc.ptr, k.d_slots.ptr, k.n_lat, k.max_blocks, s);
+                LaunchJoin(k.Descs(d_desc.ptr), k.Slots(), k.n_lat, k.max_blocks, s);
                 continue;
             }
             LaunchMerge(k.Descs(d_desc.ptr), k.WorkList(), k.total_blocks, k.tw64, k.max_block_rows, s);
@@ -1372,7 +1372,7 @@ int swmi_time_kernels(swmi_engine* engine, uint32_t n_sweeps, float* ms)
             Check(hipEventRecord(ev[1], engine->stream), "event");
             for (auto& k : engine->classes)
                 if (k.Joined())
-                    LaunchJoin(engine->d_desc.ptr, k.d_slots.ptr, k.n_lat, k.max_blocks, engine->stream);
+                    LaunchJoin(k.Descs(engine->d_desc.ptr), k.Slots(), k.n_lat, k.max_blocks, engine->stream);
                 else
                     LaunchMerge(k.Descs(engine->d_desc.ptr), k.WorkList(), k.total_blocks, k.tw64, k.max_block_rows, engine->stream);
             Check(hipEventRecord(ev[2], engine->stream), "event");

@@ -197,6 +197,7 @@ namespace swmi
         // null work list (the kernels then skip the work-list load), a larger class all descriptors and its list.
         const LatDesc* Descs(const LatDesc* all) const { return n_lat == 1 ? all + first_slot : all; }
         const uint32_t* WorkList() const { return n_lat == 1 ? nullptr : d_block_lat.ptr; }
+        const uint32_t* Slots() const { return n_lat == 1 ? nullptr : d_slots.ptr; }
     };
 
     struct GraphEntry

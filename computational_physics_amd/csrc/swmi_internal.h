@@ -190,7 +190,7 @@ namespace swmi
     void LaunchResident(const LatDesc* d_desc, const uint32_t* d_slots, uint32_t n_lattices, uint32_t max_sites, uint32_t max_rows,
                         bool full, bool tw64, bool pad, uint32_t sweeps, uint32_t groups, int32_t sample_mode, hipStream_t stream);
     // k_merge and k_resolve of n_lattices lattices of 64-wide tiles, blocks of at most 64 rows and at most
-    // max_blocks <= kJoinBlocks blocks, one workgroup each
+    // max_blocks <= kJoinBlocks blocks, one workgroup each (d_slots null: the one lattice of *d_desc)
     void LaunchJoin(const LatDesc* d_desc, const uint32_t* d_slots, uint32_t n_lattices, uint32_t max_blocks, hipStream_t stream);
     // Geometry of a lattice that one workgroup labels (ResidentRows): n0 the caller's width, the rest as in LatDesc.
     struct WholeGeometry

@@ -648,7 +648,7 @@ namespace swmi
         constexpr uint32_t kWaves = 16, kEdges = 2u, kNodes = 256u;
         extern __shared__ uint64_t L[];            // kNodes entries per block: (key of the parent << 32) | parent
         __shared__ uint32_t sw[kWaves * 8u];       // flip bits by node
-        const LatDesc& d = descs[slots[blockIdx.x]];
+        const LatDesc& d = descs[LatticeOf(slots, blockIdx.x)];
         const gptr<uint32_t> stp = Glob(d.state);
         const uint32_t lane = threadIdx.x & 63u, w = Uniform(threadIdx.x >> 6);
         const uint32_t tx = d.tiles_x, nb = d.n_blocks, brows = kWavesPerBlock * d.twr, stride = 64u * tx, qcap = d.qcap;
@@ -660,7 +660,7 @@ namespace swmi
         const auto rows_of = [&](const uint32_t sy) { return min(brows, d.nwr_y - sy * brows); };
 
         // edge e = w + 16 k: block e / 2, its right edge (lane = row) or its down edge (lane = column)
-        uint32_t va[kEdges], vb[kEdges], lbb[kEdges];
+        uint32_t va[kEdges], vb[kEdges], lbb[kEdges], base_a[kEdges], base_b[kEdges];   // base: first site of the block
         uint64_t word[kEdges];
 #pragma unroll
         for (uint32_t k = 0; k < kEdges; ++k)
@@ -668,7 +668,10 @@ namespace swmi
             const uint32_t e = min(w + kWaves * k, 2u * nb - 1u), lb = e >> 1;
             const uint32_t sx = lb % tx, sy = lb / tx;
             const bool down = (e & 1u) != 0u;
-            lbb[k] = down ? (sy + 1u == d.blocks_y ? 0u : sy + 1u) * tx + sx : sy * tx + (sx + 1u == tx ? 0u : sx + 1u);
+            const uint32_t sx_b = down ? sx : (sx + 1u == tx ? 0u : sx + 1u), sy_b = !down ? sy : (sy + 1u == d.blocks_y ? 0u : sy + 1u);
+            lbb[k] = sy_b * tx + sx_b;
+            base_a[k] = sy * brows * stride + sx * 64u;
+            base_b[k] = sy_b * brows * stride + sx_b * 64u;
             const uint32_t row = min(lane, rows_of(sy) - 1u);
             va[k] = *(down ? er + 128u * lb + 64u + lane : ec + (2u * lb + 1u) * es + row);
             vb[k] = *(down ? er + 128u * lbb[k] + lane : ec + 2u * lbb[k] * es + row);
@@ -685,23 +688,22 @@ namespace swmi
         const uint32_t sc = halo[min(lane, blk_rows - 1u)], sr = halo[es + lane];
 
         // every slot's node, a root keyed by its site (the edge entries of a block name all of its slots)
-        const auto node_of = [&](const uint32_t lb, const uint32_t v) { return lb * kNodes + min((v >> 16 & 0x7FFFu) - qcap, kNodes - 1u); };
-        const auto key_of = [&](const uint32_t lb, const uint32_t v) {
-            return SiteOf((lb / tx) * brows * stride + (lb % tx) * 64u, stride, v & 0xFFFFu);
-        };
-        const auto put = [&](const uint32_t lb, const uint32_t v) {
-            if ((v >> 16) & kEdgeFlag)
+        const uint32_t max_slots = min(bslots, kNodes);
+        const auto slot_of = [&](const uint32_t v) { return (v >> 16) - (kEdgeFlag + qcap); };   // of no slot: past them all
+        const auto node_of = [&](const uint32_t lb, const uint32_t v) { return lb * kNodes + slot_of(v); };
+        const auto put = [&](const uint32_t lb, const uint32_t base, const uint32_t v) {
+            if (slot_of(v) < max_slots)
             {
                 const uint32_t n = node_of(lb, v);
-                __hip_atomic_store(&L[n], SlotEntry(key_of(lb, v), n), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                __hip_atomic_store(&L[n], SlotEntry(SiteOf(base, stride, v & 0xFFFFu), n), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
             }
         };
 #pragma unroll
         for (uint32_t k = 0; k < kEdges; ++k)
             if (w + kWaves * k < 2u * nb)
             {
-                put((w + kWaves * k) >> 1, va[k]);
-                put(lbb[k], vb[k]);
+                put((w + kWaves * k) >> 1, base_a[k], va[k]);
+                put(lbb[k], base_b[k], vb[k]);
             }
         __syncthreads();
 
@@ -717,11 +719,12 @@ namespace swmi
                 const uint32_t bit = down ? lane : lane % d.twr;
                 bool open = ((word[k] >> bit) & 1ull) != 0ull && (down || lane < rows_of(lb / tx));
                 // both ends of a bond across an edge belong to edge-reaching clusters
-                if (open && !((va[k] >> 16) & (vb[k] >> 16) & kEdgeFlag))
+                if (open && max(slot_of(va[k]), slot_of(vb[k])) >= max_slots)
                 {
                     ok = false;
                     open = false;
                 }
+                // (a lane that takes part follows only nodes written above, whose parents are such nodes)
                 uint32_t a = node_of(lb, va[k]), b = node_of(lbb[k], vb[k]);
                 while (__ballot(open))
                 {
@@ -765,32 +768,58 @@ namespace swmi
         const uint32_t key = random_rule ? fkey : 0u;
         if (w < nb)
         {
-            const uint32_t nslot = Uniform(min(cnt, kNodes));
+            const uint32_t nslot = Uniform(min(cnt, max_slots));
             uint32_t* const bits = sw + blk * 8u;
-            for (uint32_t s0 = 0; s0 < nslot; s0 += 64u)
+            // two slots per lane, their chases in flight together
+            for (uint32_t s0 = 0; s0 < nslot; s0 += 128u)
             {
-                const uint32_t i = s0 + lane;
-                uint32_t bit = 0;
-                if (i < nslot)
+                uint32_t n[2];
+                uint64_t e[2];
+#pragma unroll
+                for (uint32_t j = 0; j < 2u; ++j)
                 {
-                    uint32_t n = blk * kNodes + i;
-                    uint64_t e = LocalEntry(L, n);
-                    while (static_cast<uint32_t>(e) != n)
-                    {
-                        n = static_cast<uint32_t>(e);
-                        e = LocalEntry(L, n);
-                    }
-                    const uint32_t root = static_cast<uint32_t>(e >> 32);
-                    bit = FlipBit(d, root, random_rule, key);
-                    Glob(d.cpar)[bslots * blk + i] = SlotEntry(root, bslots * (n / kNodes) + n % kNodes);
+                    n[j] = blk * kNodes + min(s0 + 64u * j + lane, nslot - 1u);
+                    e[j] = LocalEntry(L, n[j]);
                 }
-                const uint64_t m = __ballot(bit != 0u);
-                if (lane < 2u)
+                // (a node that no edge named, of a count that is too large, holds whatever the LDS held: its chase stays in
+                // the table and ends by its length; roots read themselves again)
+                uint32_t left = nb * kNodes;
+                for (; left != 0u; --left)
                 {
-                    const uint32_t v = lane ? static_cast<uint32_t>(m >> 32) : static_cast<uint32_t>(m);
-                    bits[(s0 >> 5) + lane] = v;
-                    if ((s0 >> 5) + lane < d.fsw)
-                        Glob(d.fbits)[blk * d.fsw + (s0 >> 5) + lane] = v;
+                    uint32_t moved = 0;
+#pragma unroll
+                    for (uint32_t j = 0; j < 2u; ++j)
+                    {
+                        const uint32_t up = min(static_cast<uint32_t>(e[j]), nb * kNodes - 1u);
+                        moved |= up ^ n[j];
+                        n[j] = up;
+                    }
+                    if (!__ballot(moved != 0u))
+                        break;
+#pragma unroll
+                    for (uint32_t j = 0; j < 2u; ++j)
+                        e[j] = LocalEntry(L, n[j]);
+                }
+                ok = ok && left != 0u;
+#pragma unroll
+                for (uint32_t j = 0; j < 2u; ++j)
+                {
+                    const uint32_t first = s0 + 64u * j, i = first + lane;
+                    uint32_t bit = 0;
+                    if (i < nslot)
+                    {
+                        const uint32_t root = static_cast<uint32_t>(e[j] >> 32);
+                        bit = FlipBit(d, root, random_rule, key);
+                        Glob(d.cpar)[bslots * blk + i] = SlotEntry(root, bslots * (n[j] / kNodes) + n[j] % kNodes);
+                    }
+                    const uint64_t m = __ballot(bit != 0u);
+                    if (first < nslot && lane < 2u)
+                    {
+                        const uint32_t v = lane ? static_cast<uint32_t>(m >> 32) : static_cast<uint32_t>(m);
+                        bits[(first >> 5) + lane] = v;
+                        if ((first >> 5) + lane < d.fsw)
+                            Glob(d.fbits)[blk * d.fsw + (first >> 5) + lane] = v;
+                    }
                 }
             }
             const auto flip = [&](const uint32_t lab) -> uint32_t {
@@ -804,6 +833,11 @@ namespace swmi
                         return 0u;
                     }
                     return (LdsLoad(&bits[s >> 5]) >> (s & 31u)) & 1u;
+                }
+                if (i >= blk_rows * 64u)
+                {
+                    ok = false;
+                    return 0u;
                 }
                 return FlipBit(d, SiteOf((blk / tx) * brows * stride + (blk % tx) * 64u, stride, i), random_rule, key);
             };

@@ -25,6 +25,7 @@ class _Hip:
         self.lib.hipStreamCreate.argtypes = [ctypes.POINTER(vp)]
         self.lib.hipStreamSynchronize.argtypes = [vp]
         self.lib.hipStreamDestroy.argtypes = [vp]
+        self.lib.hipDeviceSynchronize.argtypes = []
 
     def check(self, status, what):
         assert status == 0, f"{what}: hip error {status}"
