@@ -1114,8 +1114,13 @@ namespace swmi
         const uint32_t below_halo = halo[(sy_b * d.tiles_x + bl.sx) * d.halo_stride + d.ecol_stride + lane];
         __syncthreads();
 
+        // (a label outside the block's range is a broken invariant, as in k_flip)
+        const uint32_t qmax = bl.nwr * 64u, slots = kWavesPerBlock * d.edge_cap;
+        bool bad = false;
         const auto flip_of = [&](const uint32_t lab) {
             const uint32_t i = lab & 0x7FFFu;
+            const bool edge = (lab & kEdgeFlag) != 0u;
+            bad = bad || (edge ? i - qcap : i) >= (edge ? slots : qmax);
             return fb[min(i >> 5, 2u * kMaxSites / 32u - 1u)] >> (i & 31u);
         };
         const uint64_t Sbelow = __ballot((((pending ? (last_wave ? below_halo : below_sp ^ flip_of(below_lab)) : below_sp)) & 1u) != 0u);
@@ -1152,6 +1157,8 @@ namespace swmi
             rows(std::true_type{});
         else
             rows(std::false_type{});
+        if (__ballot(bad) && lane == 0u)
+            (void)__hip_atomic_fetch_or(Glob(d.state) + kStErr, kErrLabelRange, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         int32_t e = 0, m = 0;
         {
             const uint64_t S = (static_cast<uint64_t>(Shi) << 32) | Slo;

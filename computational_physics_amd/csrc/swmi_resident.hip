@@ -117,17 +117,20 @@ namespace swmi
     }
 
     // Flip of a site of the tiled path's last sweep that is still pending: the rule at the root of a cluster inside
-    // its block, or the bit k_resolve wrote for the slot of an edge-reaching cluster.
+    // its block, or the bit k_resolve wrote for the slot of an edge-reaching cluster. A label outside the block's range
+    // (a broken invariant) clears ok.
     __device__ uint32_t PendingFlip(const LatDesc& d, const uint32_t wr, const uint32_t sx, const uint32_t lab, const bool random_rule,
-                                    const uint32_t key)
+                                    const uint32_t key, bool& ok)
     {
-        const uint32_t sy = wr / (kWavesPerBlock * d.twr);
+        const uint32_t brows = kWavesPerBlock * d.twr, sy = wr / brows;
         const uint32_t i = lab & 0x7FFFu;
         if (lab & kEdgeFlag)
         {
-            const uint32_t s = min(i - d.qcap, kWavesPerBlock * d.edge_cap - 1u);
+            const uint32_t slots = kWavesPerBlock * d.edge_cap, s = min(i - d.qcap, slots - 1u);
+            ok = ok && i - d.qcap < slots;
             return (Glob(static_cast<const uint32_t*>(d.fbits))[(sy * d.tiles_x + sx) * d.fsw + (s >> 5)] >> (s & 31u)) & 1u;
         }
+        ok = ok && i < min(brows, d.nwr_y - sy * brows) * 64u;
         return FlipBit(d, SiteOf(BlockBase(d, sx, sy), 64u * d.tiles_x, i), random_rule, key);
     }
 
@@ -218,6 +221,7 @@ namespace swmi
         const gptr<uint32_t> rotp = Glob(d.rot);
         const bool pending = applied != it;
         const uint32_t pkey = pending && random_rule ? FlipKey(seed, applied) : 0u;
+        bool ok = true;
 #pragma unroll
         for (uint32_t i = 0; i < kR; ++i)
         {
@@ -230,11 +234,13 @@ namespace swmi
                 rs[i] = __builtin_amdgcn_raw_buffer_load_b32(rs_rng, lane4, first * 4u, 0);
                 if (pending)
                     sp[i] ^= PendingFlip(d, y0 + i, col, __builtin_amdgcn_raw_buffer_load_b16(rs_local, lane * 2u, first * 2u, 0),
-                                         random_rule, pkey);
+                                         random_rule, pkey, ok);
             }
         }
         uint32_t grot = lane < nrow ? rotp[g0 + lane * gstep] : 0u;   // lane i: row i
-        __syncthreads();   // AC, JAC
+        __syncthreads();   // AC, JAC, sErr
+        if (!ok)
+            sErr = kErrLabelRange;
 #pragma unroll
         for (uint32_t i = 0; i < kR; ++i)
         {

@@ -56,3 +56,34 @@ def test_join_reports_broken_labels(swmi, fault):
     r.close()
     assert state[ERRORS] == (1 if bad else 0) or fault == "unnamed slot"
     assert state[ITERATION] == 2
+
+
+def _pending(swmi):
+    """128 x 128 in four blocks, the last sweep's flip pending: every site a cluster of its own block's root 0."""
+    r = RawLattice(swmi, 128, 128, 16)
+    r.a["state"][[ITERATION, APPLIED]] = 4, 2
+    r.a["aux"][0] = 4
+    return r
+
+
+# (label, is it in its range): roots of a block of 64 x 64 sites, then slots
+LABELS = [(4095, True), (4096, False), (0x7FFF, False), ("slot 0", True), ("slot 251", True), ("last slot", True), ("past the slots", False),
+          (EDGE, False)]
+
+
+@pytest.mark.parametrize("label,good", LABELS)
+@pytest.mark.parametrize("reader", ["sample", "resident"])
+def test_readers_of_a_pending_flip_report_broken_labels(swmi, label, good, reader):
+    print(f"pending flip, label {label}, {reader}", flush=True)
+    r = _pending(swmi)
+    slots = 4 * r.g.edge_cap
+    index = {"slot 0": 0, "slot 251": 251, "last slot": slots - 1, "past the slots": slots}
+    r.a["local"][128 * 100 + 77] = EDGE | (r.g.qcap + index[label]) if label in index else label
+    if reader == "sample":
+        state = r.launch("_ZN4swmi17LaunchObservablesEPKNS_7LatDescEPKjjjP12ihipStream_t", [u32, u32], 4, 0)
+    else:
+        state = r.launch("_ZN4swmi14LaunchResidentEPKNS_7LatDescEPKjjjjbbbjjiP12ihipStream_t",
+                         [u32, u32, u32, flag, flag, flag, u32, u32, i32], 1, 16384, 16, True, True, False, 1, 1, -1)
+    r.close()
+    assert state[ERRORS] == (0 if good else 1)
+    assert state[ITERATION] == (4 if reader == "sample" else 6)
