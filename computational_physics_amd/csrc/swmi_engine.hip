@@ -836,7 +836,21 @@ int swmi_download_spins(swmi_engine* engine, uint32_t lattice, uint8_t* spins)
         // unpacked on the device, piece by piece, straight into the caller's array
         const uint64_t piece = std::min<uint64_t>(l.n, kStageBytes);
         if (engine->stage.count < piece)
-            engine->stage.allocate(piece);
+        {
+            try
+            {
+                engine->stage.allocate(piece);
+            }
+            catch (const SwmiError&)
+            {
+                // no device memory left for a piece: the padded spin bytes as they are, unpacked here
+                std::vector<uint8_t> buf(l.np);
+                Check(hipMemcpyAsync(buf.data(), l.spins.ptr, l.np, hipMemcpyDeviceToHost, engine->stream), "spin download");
+                Check(hipStreamSynchronize(engine->stream), "spin download");
+                UnpadRows(l, buf.data(), spins, [](uint8_t v) { return static_cast<uint8_t>(v & 1u); });
+                return;
+            }
+        }
         for (uint64_t first = 0; first < l.n; first += piece)
         {
             const uint64_t now = std::min(piece, l.n - first);

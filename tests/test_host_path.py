@@ -69,3 +69,24 @@ def test_a_failed_call_still_joins_the_resident_stream(recorded, call, failing):
         e.sweep(64)
         assert "k_resident" in launched(take())
     """)
+
+
+@pytest.mark.parametrize("n0,n1", [(128, 256), (100, 300)])
+def test_spins_are_read_back_when_no_device_memory_is_left(recorded, n0, n1):
+    """An engine that fills the device still returns its spins: the download then needs no memory there."""
+    recorded(f"""
+        import numpy as np
+        n0, n1 = {n0}, {n1}
+        e = cpa.Engine(cpa.LatticeConfig(n0, n1))
+        pitch, _ = e.layout()
+        data = bytearray(e.checkpoint())
+        padded = np.random.default_rng(1).integers(0, 64, pitch * n1).astype(np.uint8)   # spins and selector bits
+        data[64:64 + pitch * n1] = padded.tobytes()
+        e.restore(bytes(data))
+        fail("hipMalloc", 64)
+        np.testing.assert_array_equal(e.spins().reshape(n1, n0), padded.reshape(n1, pitch)[:, :n0] & 1)
+        fail("")
+        take()
+        e.spins()
+        assert "k_get_spins" in launched(take())
+    """)
