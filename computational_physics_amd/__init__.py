@@ -177,8 +177,9 @@ def copy_calibration(nbytes: int, repeats: int = 10) -> float:
 
 
 def autotune(config: "LatticeConfig", sweeps: int = 20) -> tuple[int, list[float]]:
-    """Time plain sweeps for tile heights 1..64 (wave rows); the fastest is used from now on in this process
-    for lattices of this extent created with tile_rows=0. Returns (best, ms per sweep per height; -1 = skipped)."""
+    """Time plain sweeps for tile heights 1..64 (wave rows) and, for a lattice that one workgroup can sweep, untiled;
+    the fastest is used from now on in this process for lattices of this extent created with tile_rows=0. Returns
+    (best, ms per sweep per height; -1 = skipped), best a value for tile_rows: 0 where untiled is fastest."""
     best = ctypes.c_uint32()
     ms = (ctypes.c_float * 7)()
     _check(load_library().swmi_autotune(ctypes.byref(config._c()), sweeps, ctypes.byref(best), ms))
@@ -186,8 +187,8 @@ def autotune(config: "LatticeConfig", sweeps: int = 20) -> tuple[int, list[float
 
 
 def autotune_batch(configs, sweeps: int = 20) -> tuple[int, list[float]]:
-    """Time plain sweeps of the whole batch with one tile height for all lattices (1..64); returns the fastest
-    height and the ms per sweep of each."""
+    """Time plain sweeps of the whole batch with one tile height for all lattices (1..64) and, if some of them can be
+    swept untiled, with tile_rows=0 for all; returns the fastest tile_rows and the ms per sweep of each height."""
     arr = (_Config * len(configs))(*[c._c() for c in configs])
     best = ctypes.c_uint32()
     ms = (ctypes.c_float * 7)()

@@ -25,7 +25,14 @@ namespace swmi
         thread_local std::string g_error;
 
         std::mutex g_tune_mutex;
-        std::map<std::pair<uint32_t, uint32_t>, uint32_t> g_tuned;   // (n0, n1) -> tile rows
+        // What swmi_autotune measured for an extent: the fastest tile height, and whether a lattice of tile_rows 0 is to run
+        // with it although one workgroup could sweep it whole.
+        struct Tuned
+        {
+            uint32_t rows;
+            bool tiled;
+        };
+        std::map<std::pair<uint32_t, uint32_t>, Tuned> g_tuned;   // by (n0, n1)
 
         // Sweeps per captured graph of plain sweeps; a sweep loop of fewer sweeps runs eagerly. Loops of at least
         // two long units replay long graphs (each replay boundary costs a few microseconds of idle GPU), the
@@ -113,7 +120,22 @@ namespace swmi
     {
         std::lock_guard<std::mutex> lock(g_tune_mutex);
         const auto it = g_tuned.find({n0, n1});
-        return it == g_tuned.end() ? 16u : it->second;
+        return it == g_tuned.end() ? 16u : it->second.rows;
+    }
+
+    // k_resident's strips for a lattice of this configuration (ResidentRows), 0 if it runs tiled: an explicit tile height,
+    // or an extent that the autotuner found faster tiled
+    static uint32_t StripRows(const swmi_lattice_config& c, const Geometry& g)
+    {
+        if (c.tile_rows != 0u)
+            return 0u;
+        {
+            std::lock_guard<std::mutex> lock(g_tune_mutex);
+            const auto it = g_tuned.find({c.n0, c.n1});
+            if (it != g_tuned.end() && it->second.tiled)
+                return 0u;
+        }
+        return ResidentRows(g, c.n1);
     }
 
     uint32_t TwrClass(const uint32_t twr)
@@ -408,7 +430,7 @@ void swmi_engine::Rebuild()
         const bool pad = l.np != l.n;
         // padded lattices have two tile-height classes (16 and 64)
         const uint32_t t = pad ? (l.g.twr <= 16 ? 16u : 64u) : TwrClass(l.g.twr);
-        const uint32_t rows = recording || l.cfg.tile_rows != 0u ? 0u : ResidentRows(l.g, l.cfg.n1);
+        const uint32_t rows = recording ? 0u : StripRows(l.cfg, l.g);
         const bool resident = rows != 0u;
         const auto same = [&](const KernelClass& k) {
             return k.tw64 == tw64 && k.pad == pad && k.twr_t == t && k.resident == resident && (!resident || (k.max_rows <= 4u) == (rows <= 4u));
@@ -1441,7 +1463,21 @@ int swmi_autotune(const swmi_lattice_config* config, uint32_t sweeps, uint32_t* 
         }
         {
             std::lock_guard<std::mutex> lock(g_tune_mutex);
-            g_tuned[{config->n0, config->n1}] = best;
+            g_tuned[{config->n0, config->n1}] = Tuned{best, false};
+        }
+        // one workgroup for the whole lattice, where it fits: what tile_rows 0 stands for then
+        swmi_lattice_config c = *config;
+        c.tile_rows = 0;
+        c.max_samples = 0;
+        if (StripRows(c, GeometryOf(c.n0, c.n1, 0)) != 0u)
+        {
+            if (TimeSweeps(&c, 1, sweeps) < best_ms)
+                best = 0;
+            else
+            {
+                std::lock_guard<std::mutex> lock(g_tune_mutex);
+                g_tuned[{config->n0, config->n1}].tiled = true;
+            }
         }
         if (best_tile_rows)
             *best_tile_rows = best;
@@ -1476,6 +1512,15 @@ int swmi_autotune_batch(const swmi_lattice_config* configs, uint32_t n_lattices,
                 best_ms = ms;
             }
         }
+        // every lattice on its own: one workgroup where it fits, else the default height of its extent
+        bool whole = false;
+        for (auto& c : cs)
+        {
+            c.tile_rows = 0;
+            whole = whole || StripRows(c, GeometryOf(c.n0, c.n1, 0)) != 0u;
+        }
+        if (whole && TimeSweeps(cs.data(), n_lattices, sweeps) < best_ms)
+            best = 0;
         if (best_tile_rows)
             *best_tile_rows = best;
     });

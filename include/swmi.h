@@ -120,13 +120,14 @@ int swmi_get_tile_rows(const swmi_engine* engine, uint32_t lattice, uint32_t* ti
 int swmi_get_layout(const swmi_engine* engine, uint32_t lattice, uint32_t* pitch, uint32_t* n_groups);
 /* Tile-height autotuner: times plain sweeps of this configuration for each tile height in
  * {1, 2, 4, 8, 16, 32, 64} (clamped to the lattice; ms_per_sweep[i] = -1 for a height clamped to one already
- * measured), returns the fastest and remembers it for this extent, so that later lattices created with
+ * measured) and, where one workgroup can sweep the lattice untiled, for that too. Returns the fastest as a value for
+ * tile_rows (0: untiled) and remembers it for this extent, so that later lattices created with
  * tile_rows = 0 use it. Spins, labels and random streams do not depend on the tile height. The
  * reference fixes the tile from the wavefront size (ising/src/swendsen_wang.cpp:16-31). */
 int swmi_autotune(const swmi_lattice_config* config, uint32_t sweeps, uint32_t* best_tile_rows, float* ms_per_sweep);
 /* Batch autotuner: times plain sweeps of an engine holding all n_lattices lattices with one tile height
- * for all of them (each of {1, 2, 4, 8, 16, 32, 64}, clamped per lattice) and returns the height with the
- * highest aggregate throughput. A batch prefers taller tiles than its small lattices would alone: its
+ * for all of them (each of {1, 2, 4, 8, 16, 32, 64}, clamped per lattice) and, if it holds lattices that one workgroup can
+ * sweep, with tile_rows 0 for all, and returns the tile_rows with the highest aggregate throughput (0 for the last). A batch prefers taller tiles than its small lattices would alone: its
  * blocks already fill the device, and taller tiles mean fewer block edges to merge. */
 int swmi_autotune_batch(const swmi_lattice_config* configs, uint32_t n_lattices, uint32_t sweeps, uint32_t* best_tile_rows,
                         float* ms_per_sweep);

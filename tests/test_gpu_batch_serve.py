@@ -240,7 +240,7 @@ def test_batch_autotune_returns_a_height_and_results_do_not_depend_on_it(swmi):
     cfgs = [_cfg(swmi, n0, n1, T, seed=30 + i, spin_seed=40 + i) for i, (n0, n1, T, _) in enumerate(MIXED[:6])]
     best, ms = swmi.autotune_batch(cfgs, sweeps=3)
     print(f"batch autotune: best {best}, ms {ms}", flush=True)
-    assert best in (1, 2, 4, 8, 16, 32, 64) and all(m > 0 for m in ms)
+    assert best in (0, 1, 2, 4, 8, 16, 32, 64) and all(m > 0 for m in ms)   # 0: every lattice on its own
     tuned = [_cfg(swmi, c.n0, c.n1, c.temperature, seed=c.seed, spin_seed=c.spin_seed, tile_rows=best) for c in cfgs]
     with swmi.Engine(tuned) as a, swmi.Engine(cfgs) as b:
         a.sweep(12)

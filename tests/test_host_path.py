@@ -90,3 +90,27 @@ def test_spins_are_read_back_when_no_device_memory_is_left(recorded, n0, n1):
         e.spins()
         assert "k_get_spins" in launched(take())
     """)
+
+
+@pytest.mark.parametrize("untiled_wins", [True, False])
+def test_autotuners_measure_and_return_the_untiled_path(recorded, untiled_wins):
+    """A lattice that one workgroup sweeps is timed that way too: tile_rows 0 comes back when it is the fastest, and a
+    height found faster is what a later lattice of this extent runs with."""
+    recorded(f"""
+        wins = {untiled_wins}
+        rec.rec_cost(b"k_resident", 1.0 if wins else 1e5)
+        small = cpa.LatticeConfig(64, 64)
+        best, ms = cpa.autotune(small, sweeps=20)
+        assert (best == 0) == wins and len(ms) == 7 and best in (0, 1, 2, 4, 8, 16, 32, 64), (best, ms)
+        take()
+        e = cpa.Engine(small)
+        e.sweep(3)
+        assert ("k_resident" in launched(take())) == wins
+        assert wins or e.tile_rows() == best
+        batch = [cpa.LatticeConfig(48, 48), cpa.LatticeConfig(256, 256)]
+        best, ms = cpa.autotune_batch(batch, sweeps=20)
+        assert (best == 0) == wins and len(ms) == 7 and min(ms) > 0, (best, ms)
+        # nothing to sweep untiled: always a height
+        assert cpa.autotune(cpa.LatticeConfig(256, 256), sweeps=20)[0] > 0
+        assert cpa.autotune_batch([cpa.LatticeConfig(256, 256), cpa.LatticeConfig(512, 320)], sweeps=20)[0] > 0
+    """)
