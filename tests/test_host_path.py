@@ -114,3 +114,22 @@ def test_autotuners_measure_and_return_the_untiled_path(recorded, untiled_wins):
         assert cpa.autotune(cpa.LatticeConfig(256, 256), sweeps=20)[0] > 0
         assert cpa.autotune_batch([cpa.LatticeConfig(256, 256), cpa.LatticeConfig(512, 320)], sweeps=20)[0] > 0
     """)
+
+
+@pytest.mark.parametrize("sizes", [[(64, 64)], [(256, 256)], [(2048, 512)], [(64, 64), (32, 32), (256, 256), (2048, 512)]])
+def test_time_kernels_times_the_kernels_of_a_sweep(recorded, sizes):
+    """The same launches as a sweep loop's, each counted in its figure (one microsecond a launch here)."""
+    recorded(f"""
+        from collections import Counter
+        e = cpa.Engine([cpa.LatticeConfig(n0, n1) for n0, n1 in {sizes}])
+        take()
+        e.set_graphs(False)
+        e.sweep(12)
+        want = Counter(launched(take()))
+        ms = e.time_kernels(12)
+        assert Counter(launched(take())) == want
+        parts = [("k_bond_label", "k_resident"), ("k_merge", "k_join"), ("k_resolve",)]
+        for figure, names in zip(ms, parts):
+            launches = sum(n for k, n in want.items() if k.startswith(names))
+            assert abs(figure * 12 - launches * 1e-3) < 1e-6, (ms, want)
+    """)
