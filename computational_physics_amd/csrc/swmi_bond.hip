@@ -914,10 +914,11 @@ namespace swmi
         BondLabel<NW, TWR_MAX, true, BondMode::kLabel, PAD, FULL>(&d, nullptr, total_blocks);
     }
 
-    template <bool PAD>
+    // (TWR_MAX 8 has half the LDS and rows of 16: 2 x 2^20 at bond density 0.95 74 against 83 us, the whole call 93 and 100)
+    template <uint32_t TWR_MAX, bool PAD>
     __global__ __launch_bounds__(256) void k_label_blocks_narrow(const LatDesc d, const uint32_t total_blocks)
     {
-        BondLabel<kWavesPerBlock, 16, false, BondMode::kLabel, PAD, false>(&d, nullptr, total_blocks);
+        BondLabel<kWavesPerBlock, TWR_MAX, false, BondMode::kLabel, PAD, false>(&d, nullptr, total_blocks);
     }
 
     // Launches of few blocks of 64-wide tiles, all of a height that four waves can share, give every block more waves:
@@ -955,9 +956,11 @@ namespace swmi
                     k_label_blocks<NW, 64 / NW, false, false><<<g, 64 * NW, 0, stream>>>(d, total_blocks);
             });
         else if (pad)
-            k_label_blocks_narrow<true><<<g, 256, 0, stream>>>(d, total_blocks);
+            k_label_blocks_narrow<16, true><<<g, 256, 0, stream>>>(d, total_blocks);
+        else if (d.twr <= 8u)
+            k_label_blocks_narrow<8, false><<<g, 256, 0, stream>>>(d, total_blocks);
         else
-            k_label_blocks_narrow<false><<<g, 256, 0, stream>>>(d, total_blocks);
+            k_label_blocks_narrow<16, false><<<g, 256, 0, stream>>>(d, total_blocks);
     }
 
     template void LaunchLabelBlocksT<SWMI_BOND_TW64>(const LatDesc&, uint32_t, BondForm, bool, hipStream_t);
