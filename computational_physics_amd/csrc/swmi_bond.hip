@@ -1006,9 +1006,11 @@ namespace swmi
                         launch(k_bond_label<NW, 64 / NW, MODE, false, false>, 64 * NW);
                 });
         }
-        if (pad)   // padded lattices: two tile-height bounds
+        if (pad)   // padded lattices: two tile-height bounds (and the small one of narrow tiles)
         {
-            if (max_twr <= 16)
+            if (!TW64 && max_twr <= 4)
+                launch(k_bond_label_any<4, false, MODE, true>);
+            else if (max_twr <= 16)
                 launch(k_bond_label_any<16, TW64, MODE, true>);
             else
                 launch(k_bond_label_any<64, TW64, MODE, true>);

@@ -180,8 +180,15 @@ namespace swmi
         uint32_t max_twr = 1;
         uint32_t max_block_rows = 0;         // lattice rows of the tallest block
         uint32_t max_blocks = 0;             // blocks of the largest lattice
-        // every lattice's slots fit one workgroup: k_join takes the place of k_merge and k_resolve
-        bool Joined() const { return tw64 && max_block_rows <= 64u && max_blocks <= swmi::kJoinBlocks; }
+        // Every lattice's slots fit one workgroup: k_join takes the place of k_merge and k_resolve, except for many
+        // lattices of few blocks, where its sixteen waves per lattice (512 lattices fill the chip) have too little to do.
+        // Microseconds per sweep with k_join / without, lattices of one block 512 19.4 / 21.9, 1024 30.3 / 28.7, 4096 84 /
+        // 61; of two blocks 512 25.1 / 29.0, 1024 38.5 / 39.9, 2048 66 / 60; of four 2048 108 / 112, 4096 214 / 214; of
+        // six 2048 150 / 158; of sixteen 2048 357 / 402.
+        bool Joined() const
+        {
+            return tw64 && max_block_rows <= 64u && max_blocks <= swmi::kJoinBlocks && (n_lat <= 512u || total_blocks >= 4u * n_lat);
+        }
         BondForm form = BondForm::kFull;     // what its lattices' tile heights have in common
         std::vector<uint32_t> block_lat;     // block -> lattice slot
         DeviceBuffer<uint32_t> d_block_lat;

@@ -133,3 +133,15 @@ def test_time_kernels_times_the_kernels_of_a_sweep(recorded, sizes):
             launches = sum(n for k, n in want.items() if k.startswith(names))
             assert abs(figure * 12 - launches * 1e-3) < 1e-6, (ms, want)
     """)
+
+
+@pytest.mark.parametrize("n0,n1,count,joined", [(64, 64, 512, True), (64, 64, 513, False), (64, 256, 600, True), (64, 128, 600, False),
+                                                (256, 256, 600, True), (64, 1088, 1, False), (64, 1024, 1, True)])
+def test_many_lattices_of_few_blocks_merge_and_resolve_block_by_block(recorded, n0, n1, count, joined):
+    recorded(f"""
+        e = cpa.Engine([cpa.LatticeConfig({n0}, {n1}, tile_rows=16) for _ in range({count})])
+        take()
+        e.sweep(1)
+        kernels = launched(take())
+        assert kernels == ["k_bond_label", "k_join"] if {joined} else kernels[-1] == "k_resolve" and "k_join" not in kernels, kernels
+    """)
