@@ -48,6 +48,14 @@ namespace swmi
         constexpr uint32_t kSeriesFirst = 4096;
         // Sweeps of one k_resident launch (a few milliseconds at most).
         constexpr uint32_t kResidentLaunchSweeps = 500;
+        // Lattices of one block that leave most of k_resident's sixteen waves without work, by what they are: one column of
+        // 64-wide tiles, and up to four narrow wave rows. 512 workgroups fill the chip; an engine of this many such lattices
+        // sweeps them tiled, a block each. Microseconds per sweep resident / tiled: 64 x 8, 2048 lattices 21.2 / 21.6, 4096
+        // 42.2 / 33.4; 64 x 64, 2048 34.8 / 39.3, 4096 69.3 / 61.2; 8 x 8, 2048 17.1 / 21.8, 4096 34.1 / 33.0, 8192 68.0 /
+        // 55.7; 16 x 16, 4096 44.2 / 41.5. Larger ones stay: 16 x 32, 8192 lattices 101 / 105, 32 x 32 120 / 152, 128 x 8,
+        // 4096 48 / 57, 128 x 128 187 / 214.
+        constexpr uint32_t kManyColumns = 2560;
+        constexpr uint32_t kManyNarrow = 4096;
     }
 
     void SetLastError(const std::string& m) { g_error = m; }
@@ -202,8 +210,8 @@ namespace swmi
     }
 
     // One workgroup of kResidentWaves waves takes a lattice whose sites fit its LDS union-find and whose rows, split
-    // into strips over the waves left per tile column, leave at most kResidentRows per strip. Every lattice it takes
-    // is faster there than tiled: 64^2 4.3 against 24 us per sweep, 128^2 11.5 against 24 (a 16-row strip is as long a
+    // into strips over the waves left per tile column, leave at most kResidentRows per strip. Alone, every lattice it takes
+    // is faster there than tiled (for very many of the smallest see kManyColumns): 64^2 4.3 against 24 us per sweep, 128^2 11.5 against 24 (a 16-row strip is as long a
     // chain as a 16-row tile, and the sweep has no launches, merge or resolve). Four times the sites would take four
     // times as long on the one CU, 46 us, where the tiled kernels take 16 (256^2).
     // Wave rows of very narrow lattices join through many more unions: 16 x 1024 (16 wave rows per strip) takes 27.4
@@ -423,6 +431,14 @@ void swmi_engine::Rebuild()
     // bonds are recorded every lattice is tiled: only k_bond_label records them.
     std::vector<KernelClass> next;
     std::vector<LatDesc> d(2 * lattices.size());
+    const auto column = [](const Geometry& g) { return g.tw == 64u && g.n_blocks == 1u; };
+    const auto few_rows = [](const Geometry& g) { return g.tw < 64u && g.nwr_y <= 4u; };
+    uint32_t columns = 0, narrow = 0;
+    for (const auto& l : lattices)
+    {
+        columns += l->cfg.tile_rows == 0u && column(l->g) ? 1u : 0u;
+        narrow += l->cfg.tile_rows == 0u && few_rows(l->g) ? 1u : 0u;
+    }
     for (uint32_t i = 0; i < lattices.size(); ++i)
     {
         const Lattice& l = *lattices[i];
@@ -430,7 +446,8 @@ void swmi_engine::Rebuild()
         const bool pad = l.np != l.n;
         // padded lattices have two tile-height classes (16 and 64)
         const uint32_t t = pad ? (l.g.twr <= 16 ? 16u : 64u) : TwrClass(l.g.twr);
-        const uint32_t rows = recording ? 0u : StripRows(l.cfg, l.g);
+        const bool many = (columns >= kManyColumns && column(l.g)) || (narrow >= kManyNarrow && few_rows(l.g));
+        const uint32_t rows = recording || many ? 0u : StripRows(l.cfg, l.g);
         const bool resident = rows != 0u;
         const auto same = [&](const KernelClass& k) {
             return k.tw64 == tw64 && k.pad == pad && k.twr_t == t && k.resident == resident && (!resident || (k.max_rows <= 4u) == (rows <= 4u));

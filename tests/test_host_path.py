@@ -145,3 +145,14 @@ def test_many_lattices_of_few_blocks_merge_and_resolve_block_by_block(recorded, 
         kernels = launched(take())
         assert kernels == ["k_bond_label", "k_join"] if {joined} else kernels[-1] == "k_resolve" and "k_join" not in kernels, kernels
     """)
+
+
+@pytest.mark.parametrize("n0,n1,least", [(64, 64, 2560), (34, 6, 2560), (8, 8, 4096), (16, 16, 4096), (32, 32, 0), (128, 8, 0)])
+def test_very_many_of_the_smallest_lattices_are_swept_tiled(recorded, n0, n1, least):
+    recorded(f"""
+        for count in ({least} - 1, {least}) if {least} else (4200,):
+            e = cpa.Engine([cpa.LatticeConfig({n0}, {n1}) for _ in range(count)])
+            take()
+            e.sweep(2)
+            assert ("k_resident" in launched(take())) == (count != {least}), count
+    """)
