@@ -114,8 +114,9 @@ def test_mixed_batch_equals_alone_and_oracle(swmi, oracle):
             np.testing.assert_array_equal(ref.spins, got[i], err_msg=f"oracle, lattice {i}")
 
 
-def test_schedule_stops_one_lattice(swmi):
-    cfgs = [_cfg(swmi, 128, 128, seed=1), _cfg(swmi, 64, 64, 2.0, seed=2)]
+@pytest.mark.parametrize("tile_rows", [0, 16])   # swept whole, and tiled
+def test_schedule_stops_one_lattice(swmi, tile_rows):
+    cfgs = [_cfg(swmi, 128, 128, seed=1, tile_rows=tile_rows), _cfg(swmi, 64, 64, 2.0, seed=2, tile_rows=tile_rows)]
     with swmi.Engine(cfgs) as e:
         e.set_schedule(0, sweeps=7)
         e.sweep(20)
@@ -127,9 +128,10 @@ def test_schedule_stops_one_lattice(swmi):
 
 
 @pytest.mark.parametrize("sweeps,warmup,extra", [(100, 20, 0), (100, 30, 47), (60, 0, 13)])
-def test_scheduled_samples_equal_plain_protocol(swmi, sweeps, warmup, extra):
+@pytest.mark.parametrize("tile_rows", [0, 16])
+def test_scheduled_samples_equal_plain_protocol(swmi, sweeps, warmup, extra, tile_rows):
     """warmup + sweeps with a sample every 10th, run inside a longer loop, equals the plain protocol."""
-    c = _cfg(swmi, 128, 64, 2.1, seed=5, spin_seed=6, max_samples=32)
+    c = _cfg(swmi, 128, 64, 2.1, seed=5, spin_seed=6, max_samples=32, tile_rows=tile_rows)
     with swmi.Engine([c, _cfg(swmi, 64, 64, seed=7)]) as e:
         e.set_schedule(0, sweeps=warmup + sweeps, warmup=warmup, n_sep=10)
         e.run_scheduled(warmup + sweeps + extra, 10)

@@ -8,15 +8,16 @@ TC = 2.2691853
 
 
 @pytest.mark.parametrize("n0,n1,rule", [(128, 128, 0), (256, 64, 1), (32, 32, 0)])
-def test_restore_continues_bit_for_bit(swmi, n0, n1, rule):
+@pytest.mark.parametrize("tile_rows", [0, 16])
+def test_restore_continues_bit_for_bit(swmi, n0, n1, rule, tile_rows):
     """30 sweeps, checkpoint, 40 more (crossing lcg32 rotations) == restore into a fresh lattice + 40."""
-    cfg = swmi.LatticeConfig(n0, n1, 2.1, seed=5, spin_seed=7, flip_rule=rule, max_samples=16)
+    cfg = swmi.LatticeConfig(n0, n1, 2.1, seed=5, spin_seed=7, flip_rule=rule, max_samples=16, tile_rows=tile_rows)
     with swmi.Engine(cfg) as a:
         a.run(30, 10)
         ck = a.checkpoint()
         a.run(40, 10)
         want_spins, want_rng, want_mom, want_ser = a.spins(), a.rng_state(), a.moments(), a.series()
-    other = swmi.LatticeConfig(n0, n1, 2.9, seed=99, spin_seed=3, flip_rule=1 - rule, max_samples=16)
+    other = swmi.LatticeConfig(n0, n1, 2.9, seed=99, spin_seed=3, flip_rule=1 - rule, max_samples=16, tile_rows=tile_rows)
     with swmi.Engine([swmi.LatticeConfig(64, 64, 2.0), other]) as b:
         b.restore(ck, 1)
         b.run(40, 10)

@@ -58,12 +58,14 @@ def test_launches_of_4096_blocks_one_or_two_wide(swmi, oracle, n0, n1, T):
 
 
 def test_many_small_tiled_lattices_equal_their_lone_runs(swmi):
-    """1040 lattices of two by two blocks in one launch of 4160 blocks: every block meets the same neighbour twice."""
+    """1040 lattices of two by two blocks in one launch of 4177 blocks: every block meets the same neighbour twice. (The
+    lattice of 17 blocks keeps the class off k_join.)"""
     print("block merge, 1040 lattices", flush=True)
     cfgs = [swmi.LatticeConfig(128, 128, 1.9 + 0.001 * i, seed=i, tile_rows=16, flip_rule=i % 2) for i in range(1040)]
+    cfgs.append(swmi.LatticeConfig(64, 1088, 2.2, seed=3, tile_rows=16))
     with swmi.Engine(cfgs) as e:
         e.sweep(12)
-        got = {i: e.spins(i) for i in range(0, 1040, 13)}
+        got = {i: e.spins(i) for i in range(0, 1041, 13)}
         assert all(e.error_flags(i) == 0 for i in got)
     for i, spins in got.items():
         with swmi.Engine(cfgs[i]) as alone:

@@ -208,6 +208,57 @@ def test_large_padded_lattice_one_sweep_bit_exact(swmi, oracle, T):
         assert e.error_flags() == 0
 
 
+@pytest.mark.parametrize("n0,n1", [(1000, 1350), (1100, 1090), (2500, 1100), (2100, 2500)])
+@pytest.mark.parametrize("rule", [0, 1])
+def test_padded_lattices_of_some_hundred_to_some_thousand_blocks(swmi, oracle, n0, n1, rule):
+    """352, 324 and 720 blocks (eight waves per block) and 1320 (four, the build of the default register budget): rows
+    padded, with partial last block rows. Spins over eight sweeps, across the rotation at update 15; the labels of the
+    last."""
+    print(f"padded {n0}x{n1} rule {rule}", flush=True)
+    ref = oracle.PerSite(n0, n1, TC, seed=4, spin_seed=6, flip_rule=rule)
+    with swmi.Engine(swmi.LatticeConfig(n0, n1, TC, seed=4, spin_seed=6, flip_rule=rule)) as e:
+        assert e.layout()[0] > n0
+        e.sweep(7)
+        e.sweep(1)
+        for _ in range(7):
+            ref.sweep()
+        _, labels = ref.sweep(record=True)
+        np.testing.assert_array_equal(e.labels(), labels)
+        np.testing.assert_array_equal(e.spins(), ref.spins)
+        assert e.energy_magnetization() == oracle.observables(n0, n1, ref.spins)
+        assert e.error_flags() == 0
+
+
+@pytest.mark.parametrize("n0,n1", [(256, 256), (192, 130), (64, 64), (32, 32), (100, 100)])
+def test_a_new_temperature_holds_for_captured_graphs_and_for_one_lattice_only(swmi, oracle, n0, n1):
+    """The threshold is changed in the descriptors that captured graphs go on reading: sweeps through the same graphs
+    before and after the change, on a lattice that is not the engine's first, equal an oracle given the same change; the
+    other lattice keeps its own."""
+    print(f"new temperature {n0}x{n1}", flush=True)
+    t = [2.1, 2.5]
+    refs = [oracle.PerSite(n0, n1, t[i], seed=20 + i, spin_seed=3) for i in range(2)]
+    with swmi.Engine([swmi.LatticeConfig(n0, n1, t[i], seed=20 + i, spin_seed=3) for i in range(2)]) as e:
+        def both(k):
+            e.sweep(k)
+            for r in refs:
+                for _ in range(k):
+                    r.sweep()
+            for i, r in enumerate(refs):
+                np.testing.assert_array_equal(e.spins(i), r.spins, err_msg=f"lattice {i}")
+
+        both(40)                       # two replays of a 16-sweep graph and eager sweeps
+        e.set_temperature(1.9, 1)
+        refs[1].threshold = oracle.threshold(1.9)
+        assert e.threshold(1)[1] == refs[1].threshold != e.threshold(0)[1]
+        both(40)
+        e.energy_magnetization(1)      # launches over one lattice read its other descriptor
+        e.set_temperature(2.7, 1)
+        e.set_temperature(2.3, 0)
+        refs[1].threshold, refs[0].threshold = oracle.threshold(2.7), oracle.threshold(2.3)
+        both(40)
+        assert e.error_flags(0) == 0 and e.error_flags(1) == 0
+
+
 @pytest.mark.parametrize("n0,n1,T,tile_rows", [(64, 64, TC, 0), (128, 96, 2.0, 4), (32, 32, 2.6, 0), (256, 128, TC, 16),
                                                (16, 64, 1.5, 2), (512, 64, 3.0, 64)])
 def test_random_flip_rule_bit_exact(swmi, oracle, n0, n1, T, tile_rows):
