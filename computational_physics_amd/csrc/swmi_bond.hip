@@ -934,9 +934,11 @@ namespace swmi
     }
 
     // Launches of few blocks of 64-wide tiles, all of a height that four waves can share, give every block more waves:
-    // sixteen up to one block per CU, eight up to three. Microseconds per sweep with 4 / 8 / 16 waves: 256 blocks
-    // (1024^2) 28.0 / - / 24.2, 352 blocks (1000 x 1350) 25.4 / 23.7 / 25.1, 484 (1408^2) - / 25.5 / 26.9, 676 (1664^2)
-    // 29.2 / 28.8 / -, 1024 (2048^2) 32.6 / 33.3 / 46.
+    // sixteen up to one block per CU, eight up to three. Microseconds per sweep at T_c with 4 / 8 / 16 waves: 6 blocks
+    // (128 x 192) 17.0 / 14.4 / 13.9, 16 (256^2) 19.1 / 16.5 / 16.2, 36 (384^2) 22.6 / 20.0 / 19.6, 64 (512^2) 22.9 / 20.3 /
+    // 20.0, 132 (768 x 704) 23.9 / 21.3 / 20.9, 256 (1024^2) 24.7 / 22.1 / 21.8, 256 padded (1000^2) 25.2 / 22.8 / 22.4; with
+    // builds of before the constant row counts 352 padded blocks (1000 x 1350) 25.4 / 23.7 / 25.1, 484 (1408^2) - / 25.5 / 26.9,
+    // 676 (1664^2) 29.2 / 28.8 / -, 1024 (2048^2) 32.6 / 33.3 / 46.
     constexpr uint32_t kWideBlocks = 256;
     constexpr uint32_t kHalfBlocks = 768;
     // f(NW) with the waves per block for a launch of 64-wide tiles of at most 16 rows

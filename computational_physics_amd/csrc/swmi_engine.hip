@@ -46,7 +46,8 @@ namespace swmi
         constexpr uint64_t kStageBytes = 16ull << 20;
         // Samples of a series read with the lattice's counters (64 KiB)
         constexpr uint32_t kSeriesFirst = 4096;
-        // Sweeps of one k_resident launch (a few milliseconds at most).
+        // Sweeps of one k_resident launch: 2 to 14 ms (3.7 us a sweep at 32^2, 27.4 at 16 x 1024), times the rounds of 512
+        // workgroups that an engine of more lattices takes.
         constexpr uint32_t kResidentLaunchSweeps = 500;
         // Lattices of one block that leave most of k_resident's sixteen waves without work, by what they are: one column of
         // 64-wide tiles, and up to four narrow wave rows. 512 workgroups fill the chip; an engine of this many such lattices
@@ -201,7 +202,6 @@ namespace swmi
         g.ecol_stride = kWavesPerBlock * g.twr * g.rpw;
         g.halo_stride = g.ecol_stride + 64u;
         g.qcap = kWavesPerBlock * g.twr * 64u;
-        g.fbw = (g.qcap + kWavesPerBlock * g.edge_cap + 31u) / 32u;
         g.fsw = (kWavesPerBlock * g.edge_cap + 31u) / 32u;
         // the bond pass loads a block's slot flip bits one word per thread of its 256
         if (g.fsw > 256u)
@@ -211,11 +211,12 @@ namespace swmi
 
     // One workgroup of kResidentWaves waves takes a lattice whose sites fit its LDS union-find and whose rows, split
     // into strips over the waves left per tile column, leave at most kResidentRows per strip. Alone, every lattice it takes
-    // is faster there than tiled (for very many of the smallest see kManyColumns): 64^2 4.3 against 24 us per sweep, 128^2 11.5 against 24 (a 16-row strip is as long a
-    // chain as a 16-row tile, and the sweep has no launches, merge or resolve). Four times the sites would take four
-    // times as long on the one CU, 46 us, where the tiled kernels take 16 (256^2).
-    // Wave rows of very narrow lattices join through many more unions: 16 x 1024 (16 wave rows per strip) takes 27.4
-    // against 36.9 us tiled, but 4 x 4096 28.2 against 23.3, so below 16 columns only strips of up to 8 go here.
+    // is faster there than tiled (for very many of the smallest see kManyColumns): 64^2 4.3 against 12.8 us per sweep, 128^2
+    // 11.6 against 13.7 (a 16-row strip is as long a chain as a 16-row tile, and the sweep has no launches, merge or
+    // resolve). Four times the sites would take four times as long on the one CU, 46 us, where the tiled kernels take 16
+    // (256^2). Wave rows of very narrow lattices join through many more unions: 16 x 1024 (16 wave rows per strip) takes
+    // 27.7 against 35.1 us tiled and 4 x 2048 (8 per strip) 16.9 against 22.4, but 4 x 4096 28.2 against 22.7, so below 16
+    // columns only strips of up to 8 go here.
     uint32_t ResidentRows(const Geometry& g, const uint32_t n1)
     {
         if (static_cast<uint64_t>(g.pitch) * n1 > kResidentSites || g.tiles_x > kResidentWaves)
@@ -250,7 +251,6 @@ namespace swmi
         d.n_blocks = g.n_blocks;
         d.halo_stride = g.halo_stride;
         d.qcap = g.qcap;
-        d.fbw = g.fbw;
         d.fsw = g.fsw;
         return d;
     }

@@ -112,7 +112,7 @@ namespace swmi
     struct Geometry
     {
         uint32_t pitch = 0, tw = 0, rpw = 0, twr = 0, tiles_x = 0, blocks_y = 0, nwr_y = 0, n_blocks = 0, edge_cap = 0,
-                 ecol_stride = 0, halo_stride = 0, elast = 0, qcap = 0, fbw = 0, fsw = 0;
+                 ecol_stride = 0, halo_stride = 0, elast = 0, qcap = 0, fsw = 0;
         uint64_t vlast = 0;
     };
     // Row pitch of an n0 x n1 lattice: n0 when the wave64 tiling takes it as it is, else the next width it
@@ -189,7 +189,9 @@ namespace swmi
         {
             return tw64 && max_block_rows <= 64u && max_blocks <= swmi::kJoinBlocks && (n_lat <= 512u || total_blocks >= 4u * n_lat);
         }
-        BondForm form = BondForm::kFull;     // what its lattices' tile heights have in common
+        // What its lattices' tile heights have in common: one lattice of another height takes the build of constant row counts
+        // (below: `full`, one of another size) from its whole class, which is one launch.
+        BondForm form = BondForm::kFull;
         std::vector<uint32_t> block_lat;     // block -> lattice slot
         DeviceBuffer<uint32_t> d_block_lat;
         uint32_t total_blocks = 0;
@@ -247,8 +249,8 @@ struct swmi_engine
 
     swmi::Lattice& At(uint32_t i);
     swmi::LatDesc Desc(const swmi::Lattice& l, uint32_t block_base) const;
-    // Rebuilds descriptors and class work lists after a change of the lattice set, a temperature or the
-    // recording mode, and drops the captured graphs. The uploads are ordered on the engine stream; the
+    // Rebuilds descriptors and class work lists after a change of the lattice set or the recording mode, and drops
+    // the captured graphs. The uploads are ordered on the engine stream; the
     // host copies stay alive until the next rebuild.
     void Rebuild();
     void DropGraphs();

@@ -41,8 +41,9 @@
 // leaves the spins as they were; the next sweep's k_bond_label flips each site as it loads it (from its
 // label and the block's flip bits) and stores the flipped spin. LatState::applied is the iteration at
 // which the spin array holds the chain's state; applied != iteration means the last sweep's flip is still
-// pending, and every reader of spins (observables, downloads, checkpoints, the inspection hooks) first
-// runs k_flip, which applies it.
+// pending. Whatever reads spins takes it into account: k_observables and k_resident apply it to what they
+// load, as the next sweep does, and downloads, checkpoints and the inspection hooks first run k_flip, which
+// applies it to the array.
 //
 // Tiling. A "wave row" is 64 consecutive row-major sites, which is exactly one lcg32 group:
 //   n0 >= 64 (n0 % 64 == 0): a wave row is 64 columns of one lattice row;
@@ -92,7 +93,6 @@ namespace swmi
         uint32_t ecol_stride;    // lattice rows per block: kWavesPerBlock * twr * rpw
         uint32_t edge_cap;       // slots of one tile: min(tile sites, block boundary sites)
         uint32_t qcap;           // block-local indices of a block: kWavesPerBlock * twr * 64
-        uint32_t fbw;            // flip-bit words per block: (qcap + 4 * edge_cap) / 32, rounded up
         uint32_t fsw;            // slot flip-bit words of a block: 4 * edge_cap / 32, rounded up
         uint32_t n0, n1;         // row pitch (padded width) and height
         uint32_t n0v;            // lattice width: columns [n0v, n0) are padding
@@ -240,5 +240,4 @@ namespace swmi
     void LaunchUnpadLabels(uint32_t* dst, const uint32_t* src, uint64_t n, uint32_t n0v, uint32_t pitch, hipStream_t stream);
     void LaunchHotStart(uint8_t* spins, uint64_t n, uint32_t spin_seed, uint32_t n0v, uint32_t pitch, hipStream_t stream);
     void LaunchCopy(const uint4* src, uint4* dst, uint64_t n16, hipStream_t stream);
-    void LaunchIota(uint32_t* labels, uint64_t n, hipStream_t stream);
 }

@@ -14,7 +14,7 @@
 //                 array waits for the next k_bond_label.
 // k_join does the work of k_merge and k_resolve for lattices of few blocks, and k_resident (swmi_resident.hip) sweeps
 // small lattices whole, without any of these launches. k_flip applies a pending flip to the spin array; it runs only
-// before something reads the spins. k_observables takes a sample without storing the flip.
+// before the array itself is read (downloads, checkpoints, inspection). k_observables takes a sample without storing the flip.
 // Spin bytes: bit 0 is the spin, bits 3-5 hold the site's current lcg32 parameter selector, i.e. the
 // index k of the Numerical Recipes pair (a_k, c_k) that lane i of its group uses after the group's
 // rotations (sel0[(i + rot) & 63]). The byte is read every sweep anyway, so the generator needs no other
@@ -465,7 +465,7 @@ namespace swmi
     // =============================================================================================
     // k_resolve / k_flip: resolve + flip (reference ResolveLabels_Kernel / FlipClusters_Kernel,
     // swendsen_wang_amd_gpu.cpp:403-467), split into the decision (k_resolve, end of every sweep) and its
-    // application to the spin array (the next sweep's k_bond_label, or k_flip when something reads spins)
+    // application to the spin array (the next sweep's k_bond_label, or k_flip before the array itself is read)
     // =============================================================================================
     // Bitmap index of a label: the root index, or qcap + slot for an edge-reaching cluster. An index outside
     // the block's range (a broken invariant) clears ok and reads bit 0.
@@ -636,7 +636,8 @@ namespace swmi
     // =============================================================================================
     // k_join: k_merge and k_resolve of a lattice of few blocks, in one workgroup
     // =============================================================================================
-    // For a lattice of few blocks the two kernels are launch time and chains of memory round trips. Here one workgroup of 16 waves holds the whole lattice's slot union-find in LDS: node 256 * block + slot (a block
+    // For a lattice of few blocks the two kernels are launch time and chains of memory round trips. Here one workgroup of
+    // 16 waves holds the whole lattice's slot union-find in LDS: node 256 * block + slot (a block
     // of 64 columns and at most 64 rows has at most 252 boundary sites, so at most 252 slots). The edges, the halo
     // labels and the counters are read in one round trip; the unions are LDS operations; the flip bits, the flipped
     // halos and every slot's root go out as k_resolve and k_merge leave them (the root directly as parent).
@@ -1049,8 +1050,8 @@ namespace swmi
     // A flip that is still pending is applied on the way (from the labels and the flip bits, as k_bond_label does) and
     // not stored: the spin array is read once (1 byte a site, 3 with the labels of a pending flip) and left for the
     // next sweep (8192^2: 206 us per sample with k_flip, k_set_applied and three reads per spin, now 75 with the final
-    // sum, 68 of them here for 3 bytes a site, 2.9 TB/s). Per wave one tile: spin masks of its rows by ballot, one per lane, the neighbours by shifts and from
-    // the next lane; the row below the tile is read again by the tile above it (or comes from the halo across the block
+    // sum, 68 of them here for 3 bytes a site, 2.9 TB/s). Per wave one tile: spin masks of its rows by ballot, one per
+    // lane, the neighbours by shifts and from the next lane; the row below the tile is read again by the tile above it (or comes from the halo across the block
     // edge). Summing row by row with scalar operations was bound by the scalar unit (104 us at 8192^2).
     __global__ __launch_bounds__(256) void k_observables(const LatDesc* __restrict__ descs, const uint32_t* __restrict__ block_lat,
                                                          const uint32_t total_blocks, const uint32_t sample_mode)
@@ -1115,12 +1116,11 @@ namespace swmi
         __syncthreads();
 
         // (a label outside the block's range is a broken invariant, as in k_flip)
-        const uint32_t qmax = bl.nwr * 64u, slots = kWavesPerBlock * d.edge_cap;
-        bool bad = false;
+        const uint32_t qmax = bl.nwr * 64u, slots = kWavesPerBlock * d.edge_cap, first_slot = kEdgeFlag + qcap;
+        uint64_t bad = 0;   // lanes
         const auto flip_of = [&](const uint32_t lab) {
             const uint32_t i = lab & 0x7FFFu;
-            const bool edge = (lab & kEdgeFlag) != 0u;
-            bad = bad || (edge ? i - qcap : i) >= (edge ? slots : qmax);
+            bad |= __ballot(lab >= qmax) & __ballot(lab - first_slot >= slots);
             return fb[min(i >> 5, 2u * kMaxSites / 32u - 1u)] >> (i & 31u);
         };
         const uint64_t Sbelow = __ballot((((pending ? (last_wave ? below_halo : below_sp ^ flip_of(below_lab)) : below_sp)) & 1u) != 0u);
@@ -1157,7 +1157,7 @@ namespace swmi
             rows(std::true_type{});
         else
             rows(std::false_type{});
-        if (__ballot(bad) && lane == 0u)
+        if (bad != 0ull && lane == 0u)
             (void)__hip_atomic_fetch_or(Glob(d.state) + kStErr, kErrLabelRange, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         int32_t e = 0, m = 0;
         {
@@ -1488,13 +1488,6 @@ namespace swmi
         }
     }
 
-    __global__ __launch_bounds__(256) void k_iota(uint32_t* __restrict__ labels, const uint64_t n)
-    {
-        const uint64_t i = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-        if (i < n)
-            labels[i] = static_cast<uint32_t>(i);
-    }
-
     __global__ __launch_bounds__(256) void k_copy(const uint4* __restrict__ src, uint4* __restrict__ dst, const uint64_t n16)
     {
         for (uint64_t i = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < n16;
@@ -1690,11 +1683,6 @@ namespace swmi
     {
         const uint64_t threads = (n + 63) / 64;
         k_hot_start<<<static_cast<uint32_t>((threads + 255) / 256), 256, 0, stream>>>(spins, n, spin_seed, n0v, pitch);
-    }
-
-    void LaunchIota(uint32_t* labels, const uint64_t n, hipStream_t stream)
-    {
-        k_iota<<<static_cast<uint32_t>((n + 255) / 256), 256, 0, stream>>>(labels, n);
     }
 
     void LaunchCopy(const uint4* src, uint4* dst, const uint64_t n16, hipStream_t stream)

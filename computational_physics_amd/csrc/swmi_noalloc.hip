@@ -9,7 +9,8 @@
 // columns and rows and per-lattice counters) is carved out of one file-scope device array, `scratch`,
 // which every GPU holds for the life of the process. For a lattice that needs no row padding the last kernel
 // writes the canonical labels straight into the caller's label array; a padded lattice gets its bond field
-// padded into scratch and its labels written into scratch, and a last kernel writes the unpadded labels. The call enqueues kernels on the caller's stream and returns: no
+// padded into scratch and its labels written into scratch, and a last kernel writes the unpadded labels. The call
+// enqueues kernels on the caller's stream and returns: no
 // allocation, no memset, no host synchronisation.
 //
 // Every call on a GPU shares that GPU's copy of the array, so two calls that overlap on one GPU (two

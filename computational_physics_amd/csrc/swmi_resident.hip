@@ -5,8 +5,8 @@
 // samples, where the tiled path (swmi_kernels.hip) needs three launches per sweep and three more kernels per sample.
 // What bounds it is the chain of dependent LDS operations per row of a wave's strip, so sixteen waves (the largest
 // workgroup) share the lattice's rows: strips of at most 16 rows of one tile column (64-wide tiles) or 16 wave rows
-// (narrower lattices). Microseconds per sweep at T_c, tiled with launches / here: 32^2 35 / 3.7, 64^2 24 / 4.3, 128^2
-// 24 / 11.5; of the 128^2 sweep the rows take 6, the strip edges 1.3, the final roots 2, the flips 0.9, waiting the rest.
+// (narrower lattices). Microseconds per sweep at T_c, tiled / here: 32^2 24.4 / 3.8, 64^2 12.8 / 4.3, 128^2
+// 13.7 / 11.6 (before the tiled path had its builds for launches of few blocks 35, 24 and 24); of the 128^2 sweep the rows take 6, the strip edges 1.3, the final roots 2, the flips 0.9, waiting the rest.
 #include "swmi_device.h"
 
 namespace swmi

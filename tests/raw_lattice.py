@@ -11,13 +11,13 @@ u32, u64, vp = ctypes.c_uint32, ctypes.c_uint64, ctypes.c_void_p
 
 class Geometry(ctypes.Structure):
     _fields_ = [(f, u32) for f in ("pitch", "tw", "rpw", "twr", "tiles_x", "blocks_y", "nwr_y", "n_blocks", "edge_cap", "ecol_stride",
-                                   "halo_stride", "elast", "qcap", "fbw", "fsw")] + [("vlast", u64)]
+                                   "halo_stride", "elast", "qcap", "fsw")] + [("vlast", u64)]
 
 
 class LatDesc(ctypes.Structure):
     _fields_ = [(f, vp) for f in ("spins", "rng", "aux", "masks", "rot", "local", "parent", "cpar", "bbits", "state", "bond_dump", "bond_in",
                                   "partials", "edge_count", "ecol", "erow")] + \
-               [(f, u32) for f in ("ecol_stride", "edge_cap", "qcap", "fbw", "fsw", "n0", "n1", "n0v", "elast")] + [("vlast", u64)] + \
+               [(f, u32) for f in ("ecol_stride", "edge_cap", "qcap", "fsw", "n0", "n1", "n0v", "elast")] + [("vlast", u64)] + \
                [(f, u32) for f in ("tw", "rpw", "twr", "tiles_x", "blocks_y", "nwr_y", "threshold", "block_base", "n_blocks", "flip_rule", "seed")] + \
                [("fbits", vp), ("halo", vp), ("halo_stride", u32)]
 
