@@ -13,6 +13,7 @@
 #include <memory>
 #include <mutex>
 #include <string>
+#include <tuple>
 #include <utility>
 #include <vector>
 
@@ -57,6 +58,9 @@ namespace swmi
         // 4096 48 / 57, 128 x 128 187 / 214.
         constexpr uint32_t kManyColumns = 2560;
         constexpr uint32_t kManyNarrow = 4096;
+        // Resident lattices of several kinds go into one launch of k_resident_mixed up to one per CU (the LDS of its largest
+        // lattices leaves a CU one workgroup); beyond that each kind has a launch of its own.
+        constexpr uint32_t kMixedLattices = 256;
     }
 
     void SetLastError(const std::string& m) { g_error = m; }
@@ -431,6 +435,12 @@ void swmi_engine::Rebuild()
     // bonds are recorded every lattice is tiled: only k_bond_label records them.
     std::vector<KernelClass> next;
     std::vector<LatDesc> d(2 * lattices.size());
+    using TiledKey = std::tuple<bool, bool, uint32_t>;   // 64-wide tiles, padding, tile-height bound
+    const auto key_of = [](const Lattice& l) {
+        const bool pad = l.np != l.n;
+        // padded lattices have two tile-height classes (16 and 64)
+        return TiledKey{l.g.tw == 64u, pad, pad ? (l.g.twr <= 16 ? 16u : 64u) : TwrClass(l.g.twr)};
+    };
     const auto column = [](const Geometry& g) { return g.tw == 64u && g.n_blocks == 1u; };
     const auto few_rows = [](const Geometry& g) { return g.tw < 64u && g.nwr_y <= 4u; };
     uint32_t columns = 0, narrow = 0;
@@ -439,18 +449,33 @@ void swmi_engine::Rebuild()
         columns += l->cfg.tile_rows == 0u && column(l->g) ? 1u : 0u;
         narrow += l->cfg.tile_rows == 0u && few_rows(l->g) ? 1u : 0u;
     }
+    std::vector<uint32_t> strip_rows(lattices.size());   // of k_resident's strips; 0: tiled
+    for (size_t i = 0; i < lattices.size(); ++i)
+    {
+        const Lattice& l = *lattices[i];
+        const bool many = (columns >= kManyColumns && column(l.g)) || (narrow >= kManyNarrow && few_rows(l.g));
+        strip_rows[i] = recording || many ? 0u : StripRows(l.cfg, l.g);
+    }
+    uint32_t kinds = 0, n_resident = 0;   // kinds: bit 4 * (64-wide) + 2 * padded + (more than 4 rows)
+    for (size_t i = 0; i < lattices.size(); ++i)
+    {
+        const Lattice& l = *lattices[i];
+        if (strip_rows[i] == 0u)
+            continue;
+        kinds |= 1u << ((l.g.tw == 64u ? 4u : 0u) + (l.np != l.n ? 2u : 0u) + (strip_rows[i] > 4u ? 1u : 0u));
+        ++n_resident;
+    }
+    const bool mixed = (kinds & (kinds - 1u)) != 0u && n_resident <= kMixedLattices;
     for (uint32_t i = 0; i < lattices.size(); ++i)
     {
         const Lattice& l = *lattices[i];
-        const bool tw64 = l.g.tw == 64;
-        const bool pad = l.np != l.n;
-        // padded lattices have two tile-height classes (16 and 64)
-        const uint32_t t = pad ? (l.g.twr <= 16 ? 16u : 64u) : TwrClass(l.g.twr);
-        const bool many = (columns >= kManyColumns && column(l.g)) || (narrow >= kManyNarrow && few_rows(l.g));
-        const uint32_t rows = recording || many ? 0u : StripRows(l.cfg, l.g);
+        const auto [tw64, pad, t] = key_of(l);
+        const uint32_t rows = strip_rows[i];
         const bool resident = rows != 0u;
-        const auto same = [&](const KernelClass& k) {
-            return k.tw64 == tw64 && k.pad == pad && k.twr_t == t && k.resident == resident && (!resident || (k.max_rows <= 4u) == (rows <= 4u));
+        const auto same = [&, tw64 = tw64, pad = pad, t = t](const KernelClass& k) {
+            if (resident)
+                return k.resident && (mixed || (k.tw64 == tw64 && k.pad == pad && (k.max_rows <= 4u) == (rows <= 4u)));
+            return !k.resident && k.tw64 == tw64 && k.pad == pad && k.twr_t == t;
         };
         auto it = std::find_if(next.begin(), next.end(), same);
         if (it == next.end())
@@ -461,6 +486,7 @@ void swmi_engine::Rebuild()
             it->pad = pad;
             it->twr_t = t;
             it->resident = resident;
+            it->mixed = resident && mixed;
         }
         it->max_rows = std::max(it->max_rows, rows);
         it->full = it->full && !pad && (rows == 4u || rows == kResidentRows) && rows == it->max_rows &&
@@ -584,7 +610,7 @@ void swmi_engine::EnqueueResident(const uint32_t sweeps, const uint32_t groups, 
     {
         const KernelClass& k = classes[c];
         const auto launch = [&](uint32_t per_group, uint32_t n_groups, int32_t mode) {
-            LaunchResident(d_desc.ptr, k.d_slots.ptr, k.n_lat, k.max_sites, k.max_rows, k.full, k.tw64, k.pad, per_group, n_groups, mode,
+            LaunchResident(d_desc.ptr, k.d_slots.ptr, k.n_lat, k.max_sites, k.max_rows, k.full, k.tw64, k.pad, k.mixed, per_group, n_groups, mode,
                            ClassStream(n_tiled));
         };
         if (sample_mode < 0 || sweeps > kResidentLaunchSweeps)

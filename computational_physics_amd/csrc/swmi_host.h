@@ -196,6 +196,7 @@ namespace swmi
         DeviceBuffer<uint32_t> d_block_lat;
         uint32_t total_blocks = 0;
         bool resident = false;               // small lattices that k_resident sweeps, one workgroup each
+        bool mixed = false;                  // resident: of several kinds, all of the engine's in one launch
         bool full = true;                    // resident: every wave of every lattice has exactly max_rows rows
         uint32_t max_sites = 0, max_rows = 0;   // resident: bounds on the padded sites and the rows of a strip
         std::vector<uint32_t> slots;         // descriptor slots of the class's lattices

@@ -186,9 +186,9 @@ namespace swmi
     // n_lattices small lattices (descriptors d_slots[i]), one workgroup each: `groups` groups of `sweeps` sweeps with a
     // sample after each group when sample_mode >= 0. max_sites, max_rows: bounds on their padded sites and on the
     // rows of a strip (ResidentRows). full: no padding, and every wave of every lattice has exactly max_rows rows, 4 or
-    // kResidentRows.
+    // kResidentRows. mixed: lattices of any kinds (the other properties do not matter).
     void LaunchResident(const LatDesc* d_desc, const uint32_t* d_slots, uint32_t n_lattices, uint32_t max_sites, uint32_t max_rows,
-                        bool full, bool tw64, bool pad, uint32_t sweeps, uint32_t groups, int32_t sample_mode, hipStream_t stream);
+                        bool full, bool tw64, bool pad, bool mixed, uint32_t sweeps, uint32_t groups, int32_t sample_mode, hipStream_t stream);
     // k_merge and k_resolve of n_lattices lattices of 64-wide tiles, blocks of at most 64 rows and at most
     // max_blocks <= kJoinBlocks blocks, one workgroup each (d_slots null: the one lattice of *d_desc)
     void LaunchJoin(const LatDesc* d_desc, const uint32_t* d_slots, uint32_t n_lattices, uint32_t max_blocks, hipStream_t stream);

@@ -50,15 +50,16 @@ class RawLattice:
         self.memory = []
 
     def launch(self, name, argtypes, *args):
-        """Uploads the arrays and the descriptor, launches name(descriptors, list of lattice 0, *args, stream 0) and returns the
-        state words."""
+        """Uploads the arrays and the descriptor, launches name(descriptors, list, *args, stream 0) and returns the state words.
+        The list names lattice 0 once per block: it serves the kernels that read one entry per lattice and those that read
+        one per block."""
         for field, array in self.a.items():
             p = self.hip.malloc(array.nbytes)
             self.memory.append(p)
             self.hip.h2d(p, array)
             setattr(self.d, field, p.value)
-        zero = np.zeros(1, np.uint32)
-        desc, slots = self.hip.malloc(ctypes.sizeof(LatDesc)), self.hip.malloc(4)
+        zero = np.zeros(self.g.n_blocks, np.uint32)
+        desc, slots = self.hip.malloc(ctypes.sizeof(LatDesc)), self.hip.malloc(zero.nbytes)
         self.memory += [desc, slots]
         self.hip.h2d(desc, np.frombuffer(bytes(self.d), np.uint8).copy())
         self.hip.h2d(slots, zero)

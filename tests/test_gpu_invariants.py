@@ -82,8 +82,8 @@ def test_readers_of_a_pending_flip_report_broken_labels(swmi, label, good, reade
     if reader == "sample":
         state = r.launch("_ZN4swmi17LaunchObservablesEPKNS_7LatDescEPKjjjP12ihipStream_t", [u32, u32], 4, 0)
     else:
-        state = r.launch("_ZN4swmi14LaunchResidentEPKNS_7LatDescEPKjjjjbbbjjiP12ihipStream_t",
-                         [u32, u32, u32, flag, flag, flag, u32, u32, i32], 1, 16384, 16, True, True, False, 1, 1, -1)
+        state = r.launch("_ZN4swmi14LaunchResidentEPKNS_7LatDescEPKjjjjbbbbjjiP12ihipStream_t",
+                         [u32, u32, u32, flag, flag, flag, flag, u32, u32, i32], 1, 16384, 16, True, True, False, False, 1, 1, -1)
     r.close()
     assert state[ERRORS] == (0 if good else 1)
     assert state[ITERATION] == (4 if reader == "sample" else 6)

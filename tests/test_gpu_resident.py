@@ -86,6 +86,33 @@ def test_the_two_paths_take_over_from_each_other(swmi, oracle, n0, n1, rule):
         assert e.error_flags() == 0
 
 
+@pytest.mark.parametrize("rule", [0, 1])
+def test_lattices_of_every_kind_in_one_launch_match_the_oracle(swmi, oracle, rule):
+    """k_resident_mixed: all the extents above in one engine, their labels, samples and generators included."""
+    extents = [x for x in EXTENTS if x not in ((64, 258), (4, 2064))]
+    print(f"resident, every kind, rule {rule}", flush=True)
+    T = [2.0 + 0.1 * (i % 6) for i in range(len(extents))]
+    refs = [oracle.PerSite(n0, n1, T[i], seed=i, spin_seed=3, flip_rule=rule) for i, (n0, n1) in enumerate(extents)]
+    with swmi.Engine([swmi.LatticeConfig(n0, n1, T[i], seed=i, spin_seed=3, flip_rule=rule, max_samples=8)
+                      for i, (n0, n1) in enumerate(extents)]) as e:
+        e.sweep(3)
+        e.run(20, 5)
+        for i, ((n0, n1), ref) in enumerate(zip(extents, refs)):
+            samples = []
+            for k in range(23):
+                _, labels = ref.sweep(record=True)
+                if k >= 3 and (k - 3) % 5 == 4:
+                    samples.append(oracle.observables(n0, n1, ref.spins))
+            E, M = e.series(i)
+            assert list(zip(E.tolist(), M.tolist())) == samples, (n0, n1)
+            np.testing.assert_array_equal(e.labels(i), labels, err_msg=f"labels {n0}x{n1}")
+            np.testing.assert_array_equal(e.spins(i), ref.spins, err_msg=f"spins {n0}x{n1}")
+            st = e.rng_state(i)
+            np.testing.assert_array_equal(st["states"], ref.states)
+            np.testing.assert_array_equal(st["rot"], ref.rot)
+            assert e.error_flags(i) == 0
+
+
 def test_schedules_and_long_loops_of_a_mixed_engine(swmi):
     """Resident, tiled and scheduled lattices in one engine equal their lone runs; loops longer than one launch."""
     print("resident mixed engine", flush=True)

@@ -156,3 +156,25 @@ def test_very_many_of_the_smallest_lattices_are_swept_tiled(recorded, n0, n1, le
             e.sweep(2)
             assert ("k_resident" in launched(take())) == (count != {least}), count
     """)
+
+
+def _routes(recorded, sizes, want):
+    """Kernels of one sweep of an engine of these lattices against `want`, a list of name and grid pairs."""
+    recorded(f"""
+        e = cpa.Engine([cpa.LatticeConfig(n0, n1) for n0, n1 in {sizes}])
+        take()
+        e.sweep(1)
+        lines = [l for l in take() if l.startswith("launch")]
+        got = sorted((k, int(re.search(r" grid (\\d+)", l).group(1))) for k, l in zip(launched(lines), lines))
+        assert got == sorted({want}), got
+    """)
+
+
+def test_resident_lattices_of_several_kinds_share_one_launch(recorded):
+    small = [(32, 32), (64, 64), (128, 128), (100, 100), (48, 48)]
+    _routes(recorded, small, [("k_resident_mixed", 5)])
+    _routes(recorded, [(64, 64)] * 7, [("k_resident", 7)])
+    _routes(recorded, [(64, 64)] * 200 + [(128, 128)] * 56, [("k_resident_mixed", 256)])
+    _routes(recorded, [(64, 64)] * 200 + [(128, 128)] * 57, [("k_resident", 200), ("k_resident", 57)])
+    # one tiled class beside them changes nothing
+    _routes(recorded, small + [(512, 512)], [("k_resident_mixed", 5), ("k_bond_label", 64), ("k_merge", 64), ("k_resolve", 64)])
