@@ -450,16 +450,24 @@ void swmi_engine::Rebuild()
         narrow += l->cfg.tile_rows == 0u && few_rows(l->g) ? 1u : 0u;
     }
     std::vector<uint32_t> strip_rows(lattices.size());   // of k_resident's strips; 0: tiled
+    std::map<TiledKey, uint32_t> tiled_blocks, small_blocks;
     for (size_t i = 0; i < lattices.size(); ++i)
     {
         const Lattice& l = *lattices[i];
         const bool many = (columns >= kManyColumns && column(l.g)) || (narrow >= kManyNarrow && few_rows(l.g));
         strip_rows[i] = recording || many ? 0u : StripRows(l.cfg, l.g);
+        (strip_rows[i] ? small_blocks : tiled_blocks)[key_of(l)] += l.g.n_blocks;
     }
+    // With two tiled classes and more, their branches and the resident launch have more streams than the device has hardware
+    // queues for, and a branch may have to wait for the whole resident launch. A small lattice whose tiled class is there
+    // anyway, with as many blocks at least, costs next to nothing in its launches and goes along.
     uint32_t kinds = 0, n_resident = 0;   // kinds: bit 4 * (64-wide) + 2 * padded + (more than 4 rows)
     for (size_t i = 0; i < lattices.size(); ++i)
     {
         const Lattice& l = *lattices[i];
+        const TiledKey key = key_of(l);
+        if (tiled_blocks.size() >= 2u && tiled_blocks.count(key) != 0u && small_blocks[key] <= tiled_blocks[key])
+            strip_rows[i] = 0u;
         if (strip_rows[i] == 0u)
             continue;
         kinds |= 1u << ((l.g.tw == 64u ? 4u : 0u) + (l.np != l.n ? 2u : 0u) + (strip_rows[i] > 4u ? 1u : 0u));

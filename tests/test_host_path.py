@@ -178,3 +178,13 @@ def test_resident_lattices_of_several_kinds_share_one_launch(recorded):
     _routes(recorded, [(64, 64)] * 200 + [(128, 128)] * 57, [("k_resident", 200), ("k_resident", 57)])
     # one tiled class beside them changes nothing
     _routes(recorded, small + [(512, 512)], [("k_resident_mixed", 5), ("k_bond_label", 64), ("k_merge", 64), ("k_resolve", 64)])
+
+
+def test_small_lattices_go_along_with_a_tiled_class_where_there_are_several(recorded):
+    tiled = [("k_bond_label", 72), ("k_merge", 72), ("k_resolve", 72), ("k_bond_label", 264), ("k_merge", 264), ("k_resolve", 264)]
+    # 128^2 joins 512^2 (4 + 64 blocks) and 100^2 joins 1000^2 (4 + 256); 32^2 has no tiled class of its own
+    _routes(recorded, [(128, 128), (100, 100), (512, 512), (1000, 1000)], tiled)
+    _routes(recorded, [(128, 128), (100, 100), (512, 512), (1000, 1000), (32, 32)], tiled + [("k_resident", 1)])
+    # more blocks than the tiled class has: resident
+    _routes(recorded, [(128, 128)] * 17 + [(512, 512), (1000, 1000)],
+            [("k_resident", 17), ("k_bond_label", 64), ("k_merge", 64), ("k_resolve", 64), ("k_bond_label", 256), ("k_merge", 256), ("k_resolve", 256)])
