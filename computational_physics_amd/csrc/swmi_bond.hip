@@ -17,8 +17,10 @@ namespace swmi
     // Nodes of the LDS union-find are byte offsets into P. After the final find, the root of every
     // cluster that reaches the block edge carries kPFlag in its own entry, so a site's label (root index,
     // plus kEdgeFlag) is P[root] >> 2.
-    // What bounds it: at 4096^2 (45.5 us, 10.5 B a site moved, 3.9 TB/s from the memory-side cache) instruction issue
-    // and the LDS pipe, about 60 instructions and 11 LDS operations per 64-site row where 90 and 18 took 55.9 us; at 8192^2
+    // What bounds it: at 4096^2 (46.1 us, 10.5 B a site moved, 4.0 TB/s from the memory-side cache) the dependent
+    // operations down a strip at eight waves per SIMD, with vector issue 50 %, the LDS pipe 48 % (a third of it bank
+    // conflicts) and the scalar unit 37 % busy: 59.9 vector, 45.0 scalar and 15.7 LDS instructions per 64-site row (about 11
+    // of the LDS ones in the row loop), where 81, 72 and 19.3 took 55.9 us; at 8192^2
     // (171 us, 4.1 TB/s) HBM, where a large copy reaches 5.0, and 14.6 B a site took 227; below 1024^2 the chain of LDS
     // round trips down a strip (256^2 9.6 us with 4-row strips, 14.7 with 16).
     // MODE: the sweep proper; the inspection build, in which bonds may be injected instead of generated and may be

@@ -199,9 +199,9 @@ namespace swmi
     // links. M: 64 words of the wave, below base at the start; spare: a word of the lane's own, the target of LDS
     // operations the lane has no use for (both as byte offsets from P: the selects below are between offsets, and P's
     // address stays in the instructions' offset fields).
-    // LDS operations are what bounds the labelling (one pipe per CU, about 7 cycles per operation of a wave with
-    // scattered roots): a row takes four and one per chase step, where clearing, minimum, entry and root as separate
-    // operations took eight.
+    // LDS operations are what a row waits for (about 7 cycles of the CU's one pipe per operation of a wave with scattered
+    // roots, and the round trip): a row takes four and one per chase step, where clearing, minimum, entry and root as
+    // separate operations took eight.
     __device__ __forceinline__ uint32_t LabelRow64(uint32_t* P, const uint32_t M, const uint32_t spare, const uint32_t self,
                                                    const uint64_t B, const uint64_t D, const uint32_t Rp, const uint32_t base)
     {
