@@ -648,7 +648,7 @@ void swmi_engine::EnqueueSample(uint32_t mode)
     {
         const KernelClass& k = classes[c];
         LaunchObservables(k.Descs(d_desc.ptr), k.WorkList(), k.total_blocks, mode, stream);
-        LaunchFinalizeSamples(d_desc.ptr, k.d_slots.ptr, k.n_lat, mode, stream);
+        LaunchFinalizeSamples(d_desc.ptr, k.d_slots.ptr, k.n_lat, k.max_blocks, mode, stream);
     }
     LaunchCheck("sample launch");
 }

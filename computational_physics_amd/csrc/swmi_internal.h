@@ -218,8 +218,8 @@ namespace swmi
     void LaunchLabelBlocks(const LatDesc& d, BondForm form, bool pad, hipStream_t stream);
     void LaunchObservables(const LatDesc* d_desc, const uint32_t* d_block_lat, uint32_t total_blocks, uint32_t sample_mode,
                            hipStream_t stream);
-    // lattices d_slots[0 .. n_lattices)
-    void LaunchFinalizeSamples(const LatDesc* d_desc, const uint32_t* d_slots, uint32_t n_lattices, uint32_t sample_mode,
+    // lattices d_slots[0 .. n_lattices), of at most max_blocks blocks
+    void LaunchFinalizeSamples(const LatDesc* d_desc, const uint32_t* d_slots, uint32_t n_lattices, uint32_t max_blocks, uint32_t sample_mode,
                                hipStream_t stream);
     void LaunchInitState(uint32_t* state, uint32_t* aux, uint32_t words, uint32_t series_cap, uint32_t it_end, uint32_t it_meas,
                          uint32_t sep2, hipStream_t stream);

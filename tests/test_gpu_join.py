@@ -73,7 +73,8 @@ def test_many_small_tiled_lattices_equal_their_lone_runs(swmi):
             np.testing.assert_array_equal(alone.spins(), spins, err_msg=f"lattice {i}")
 
 
-@pytest.mark.parametrize("n0,n1,T,rule", [(1006, 270, 2.392, 1), (130, 300, 2.0, 0), (256, 258, 2.2691853, 1)])
+@pytest.mark.parametrize("n0,n1,T,rule", [(1006, 270, 2.392, 1), (130, 300, 2.0, 0), (256, 258, 2.2691853, 1),
+                                          (512, 512, 2.2, 0), (320, 832, 2.2, 1)])   # 64 and 65 blocks: one wave sums, sixteen
 def test_samples_of_a_partial_last_block_match_the_oracle(swmi, oracle, n0, n1, T, rule):
     """A last block row of few rows leaves tiles without rows; the sample reads nothing past the lattice for them (their
     unused row below the tile used to be read beyond the end of the spin array)."""
