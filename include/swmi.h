@@ -112,7 +112,8 @@ int swmi_sweep(swmi_engine* engine, uint32_t n_sweeps);
  * reference launches every kernel and synchronises after each (swendsen_wang_amd_gpu.cpp:253-492).
  * New engines start with graphs unless the environment variable SWMI_GRAPHS is "0". */
 int swmi_set_graphs(swmi_engine* engine, int enable);
-/* Tile height (in 64-site wave rows) the lattice runs with. */
+/* Tile height (in 64-site wave rows) the lattice runs with wherever it is tiled (a lattice that is swept untiled is while
+ * its bonds are recorded or injected). */
 int swmi_get_tile_rows(const swmi_engine* engine, uint32_t lattice, uint32_t* tile_rows);
 /* Row pitch P of the lattice's padded layout and its number of lcg32 groups, P*n1/64 (the sizes of the
  * swmi_rng_export arrays). The reference stores the lattice unpadded (ising/include/lattice.hpp:24); P = n0
